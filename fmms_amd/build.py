@@ -44,6 +44,7 @@ SOURCES = {
     "m2l_p7_8.hip": "fast",
     "m2l_p9.hip": "fast",
     "m2l_p10.hip": "fast",
+    "m2l_rot.hip": "fast",
     "downward.hip": "fast",
     "near.hip": "fast",
     "direct.hip": "fast",

@@ -117,10 +117,10 @@ struct fmmh_ctx {
   Buf m2l_lam, m2l_m32;                     // mixed form: FP32 M2L scales, scaled moments
   Buf loc32;                                // mixed form: FP32 locals scaled by lam^n
   uint32_t p_nitems = 0, p_nsplit = 0;
-  Buf rt_sw, rt_swt, rt_din, rt_dout, rt_fin, rt_fout, rt_fact;
+  Buf rt_tab;  // p > TEMPLATED_MAX_P: the rotation M2L's tables
   Buf ctrace, clap;  // softened far field: q = sum m |x - z|^2; L, G, H per cell
   int rot_p = -1;
-  std::vector<char> rot_struct;
+  std::vector<uint32_t> rot_off;
   Buf direct_ids, direct_out, direct_part;
   Buf pinned;
 
@@ -135,8 +135,7 @@ struct fmmh_ctx {
                   &moments, &locals, &pows, &fvals, &fmin, &fact, &binom, &front_a, &front_b,
                   &m2l, &p2p, &ctr, &mkeys, &mkeys_alt, &tptr, &pkeys, &pkeys_alt, &pptr, &list_tot,
                   &nch, &choff, &chunks, &part, &far, &p2p_work, &walkrec, &walk_code, &walk_blk, &pl_n, &pl_items,
-                  &pl_reds, &pl_partial, &m2l_lam, &m2l_m32, &loc32, &rt_sw, &rt_swt, &rt_din, &rt_dout, &rt_fin, &rt_fout,
-                  &rt_fact, &direct_ids, &direct_out, &direct_part, &lf_part, &lf_state, &lf_flag, &ctrace, &clap,
+                  &pl_reds, &pl_partial, &m2l_lam, &m2l_m32, &loc32, &rt_tab, &direct_ids, &direct_out, &direct_part, &lf_part, &lf_state, &lf_flag, &ctrace, &clap,
                   &d_sysoff};
     bufs.assign(std::begin(all), std::end(all));
   }
@@ -521,34 +520,31 @@ struct fmmh_ctx {
     uint32_t* dtot = (uint32_t*)list_tot.p;
     HCHECK(hipMemsetAsync(dtot, 0, 16, s));
     plan_p2p_count(dtot);
-    if (p <= TEMPLATED_MAX_P) {
-      const uint32_t ch = (uint32_t)tun.m2l_chunk;
-      size_t maxck = m2l_max_chunks(2 * n_m2l, nc, ch);
-      ensure(nch, ((size_t)nc + 1) * 4);
-      ensure(choff, ((size_t)nc + 1) * 4);
-      ensure(chunks, maxck * m2l_chunk_bytes());
-      ensure_scan(nc + 1);
-      uint32_t* tot = nullptr;
-      m2l_build_chunks((uint32_t*)tptr.p, nc, ch, (uint32_t*)nch.p, (uint32_t*)choff.p,
-                       (uint32_t*)scan_tmp.p, chunks.p, s, &tot);
-      // choff[nc] = total chunks (the reduce reads choff[t+1])
-      HCHECK(hipMemcpyAsync((uint32_t*)choff.p + nc, tot, 4, hipMemcpyDeviceToDevice, s));
-      HCHECK(hipMemcpyAsync(dtot + 3, tot, 4, hipMemcpyDeviceToDevice, s));
-    }
+    const uint32_t ch =
+        p <= TEMPLATED_MAX_P ? (uint32_t)tun.m2l_chunk : m2l_rot_chunk(2 * n_m2l);
+    size_t maxck = m2l_max_chunks(2 * n_m2l, nc, ch);
+    ensure(nch, ((size_t)nc + 1) * 4);
+    ensure(choff, ((size_t)nc + 1) * 4);
+    ensure(chunks, maxck * m2l_chunk_bytes());
+    ensure_scan(nc + 1);
+    uint32_t* tot = nullptr;
+    m2l_build_chunks((uint32_t*)tptr.p, nc, ch, (uint32_t*)nch.p, (uint32_t*)choff.p,
+                     (uint32_t*)scan_tmp.p, chunks.p, s, &tot);
+    // choff[nc] = total chunks (the reduce reads choff[t+1])
+    HCHECK(hipMemcpyAsync((uint32_t*)choff.p + nc, tot, 4, hipMemcpyDeviceToDevice, s));
+    HCHECK(hipMemcpyAsync(dtot + 3, tot, 4, hipMemcpyDeviceToDevice, s));
     const uint4 t = read1((const uint4*)dtot);
     p_nitems = t.x;
     p_nsplit = t.z;
     plan_p2p_emit(t.y);
-    if (p <= TEMPLATED_MAX_P) {
-      nchunks = t.w;
-      ensure(part, m2l_part_bytes(p, std::max<size_t>(nchunks, 1)));
-      if (prm.precision == FMMH_PREC_FP32BULK) {
-        ensure(m2l_lam, (size_t)nc * sizeof(double));
-        ensure(m2l_m32, (size_t)nc * m2l32_moment_bytes(p));
-        ensure(loc32, (size_t)nc * m2l32_moment_bytes(p));
-      }
-    } else if (p >= 20) {
+    nchunks = t.w;
+    ensure(part, m2l_part_bytes(p, std::max<size_t>(nchunks, 1)));
+    if (p > TEMPLATED_MAX_P) {
       rot_tables();
+    } else if (prm.precision == FMMH_PREC_FP32BULK) {
+      ensure(m2l_lam, (size_t)nc * sizeof(double));
+      ensure(m2l_m32, (size_t)nc * m2l32_moment_bytes(p));
+      ensure(loc32, (size_t)nc * m2l32_moment_bytes(p));
     }
     ensure(far, n * sizeof(double4));
   }
@@ -614,8 +610,8 @@ struct fmmh_ctx {
       mark(ST_M2L_REDUCE);
       launch_m2l_reduce(p, nc, (uint32_t*)choff.p, (cplx*)part.p, loc, s);
     } else {
-      launch_m2l_gen(p, nc, (uint32_t*)tptr.p, msorted, sbits, c, mom, soft2, rot_struct.data(),
-                     loc, s);
+      HCHECK(launch_m2l_rot(p, nc, chunks.p, nchunks, (uint32_t*)choff.p, msorted, sbits, c, mom,
+                            soft2, (const double*)rt_tab.p, rot_off, (cplx*)part.p, loc, s));
       mark(ST_M2L_REDUCE);
     }
     double* lap = nullptr;
@@ -660,7 +656,6 @@ struct fmmh_ctx {
 
   void evaluate(const double* pos, const double* mass, double* acc, double* pot, bool regather) {
     const size_t D = (size_t)hdim(prm.p);
-    rot_struct.resize(std::max(rot_struct.size(), rot_tables_struct_bytes()));
     lists_ok = false;
     drop_graph();
     ensure(moments, nc * D * sizeof(cplx));
@@ -814,23 +809,10 @@ struct fmmh_ctx {
   void rot_tables() {
     const int p = prm.p;
     if (rot_p == p) return;
-    std::vector<double> sw, swt, fact;
-    std::vector<cplx> din, dout, fin, fout;
-    rot_tables_host(p, sw, swt, din, dout, fin, fout, fact);
-    auto up = [&](Buf& b, const void* src, size_t bytes) {
-      ensure(b, bytes);
-      HCHECK(hipMemcpy(b.p, src, bytes, hipMemcpyHostToDevice));
-    };
-    up(rt_sw, sw.data(), sw.size() * 8);
-    up(rt_swt, swt.data(), swt.size() * 8);
-    up(rt_din, din.data(), din.size() * sizeof(cplx));
-    up(rt_dout, dout.data(), dout.size() * sizeof(cplx));
-    up(rt_fin, fin.data(), fin.size() * sizeof(cplx));
-    up(rt_fout, fout.data(), fout.size() * sizeof(cplx));
-    up(rt_fact, fact.data(), fact.size() * 8);
-    rot_struct.resize(rot_tables_struct_bytes());
-    make_rot_tables((double*)rt_sw.p, (double*)rt_swt.p, (cplx*)rt_din.p, (cplx*)rt_dout.p,
-                    (cplx*)rt_fin.p, (cplx*)rt_fout.p, (double*)rt_fact.p, rot_struct.data());
+    std::vector<double> tab;
+    rot_tables_host(p, tab, rot_off);
+    ensure(rt_tab, tab.size() * 8);
+    HCHECK(hipMemcpy(rt_tab.p, tab.data(), tab.size() * 8, hipMemcpyHostToDevice));
     rot_p = p;
   }
 

@@ -212,15 +212,15 @@ void launch_p2m_gen(int p, const uint32_t* leaf_ids, uint32_t nleaves, DevCells 
                     cplx* moments, hipStream_t s);
 void launch_m2m_gen(int p, const uint32_t* cells, uint32_t cnt, DevCells c, cplx* moments,
                     hipStream_t s);
-void rot_tables_host(int p, std::vector<double>& sw, std::vector<double>& swt,
-                     std::vector<cplx>& din, std::vector<cplx>& dout, std::vector<cplx>& fin,
-                     std::vector<cplx>& fout, std::vector<double>& fact);
-size_t rot_tables_struct_bytes();
-void make_rot_tables(const double* sw, const double* swt, const cplx* din, const cplx* dout,
-                     const cplx* fin, const cplx* fout, const double* fact, void* out);
-void launch_m2l_gen(int p, uint32_t nc, const uint32_t* tptr, const uint64_t* skeys, int sbits,
-                    DevCells c, const cplx* moments, double soft2, const void* rot_tables,
-                    cplx* locals, hipStream_t s);
+// m2l_rot.hip: the swap matrices and scale factors of order p (host), the
+// sources per chunk, and the M2L (chunk partials in part, then the locals).
+void rot_tables_host(int p, std::vector<double>& tab, std::vector<uint32_t>& off);
+uint32_t m2l_rot_chunk(uint32_t ndirected);
+hipError_t launch_m2l_rot(int p, uint32_t nc, const void* chunks, uint32_t nchunks,
+                          const uint32_t* choff, const uint64_t* skeys, int sbits, DevCells c,
+                          const cplx* moments, double soft2, const double* tab,
+                          const std::vector<uint32_t>& off, cplx* part, cplx* locals,
+                          hipStream_t s);
 void launch_l2l_gen(int p, const uint32_t* cells, uint32_t cnt, DevCells c, cplx* locals,
                     hipStream_t s);
 void launch_l2p_gen(int p, const uint32_t* leaf_ids, uint32_t nleaves, DevCells c, DevBodies b,

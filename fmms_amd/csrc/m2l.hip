@@ -2,7 +2,9 @@
 // the per-target reduction of chunk partials and the order dispatch. The
 // contraction kernels live in m2l_kernel.h, instantiated per range of orders
 // by m2l_p*.hip (separate translation units so they build in parallel).
-#include "m2l_kernel.h"
+#include "common.h"
+#include "internal.h"
+#include "m2l_chunk.h"
 
 namespace fmmh {
 

@@ -16,6 +16,7 @@
 #pragma once
 #include "common.h"
 #include "internal.h"
+#include "m2l_chunk.h"
 
 namespace fmmh {
 
@@ -144,12 +145,6 @@ __device__ __forceinline__ void m2l_accumulate(R x, R y, R z, R soft2, const C* 
     }
   }
 }
-
-struct M2lChunk {
-  uint32_t target;
-  uint32_t begin;
-  uint32_t end;
-};
 
 template <int P, int H>
 __device__ __forceinline__ void m2l_chunk(const M2lChunk ck, uint32_t ci,
