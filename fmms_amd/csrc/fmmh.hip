@@ -423,7 +423,6 @@ struct fmmh_ctx {
   // levels go straight into m2l_m32.
   void upward(const double* pos, const double* mass, bool regather) {
     const int p = prm.p;
-    const size_t D = (size_t)hdim(p);
     DevCells c = cells();
     DevBodies b = bodies();
     if (regather) launch_gather(pos, mass, order, n, b, s);
@@ -446,7 +445,6 @@ struct fmmh_ctx {
       for (int L = (int)max_level - 1; L >= 0; L--)
         launch_m2m(p, (uint32_t*)int_cells.p + int_off[L], int_off[L + 1] - int_off[L], c, mom, s);
     } else {
-      launch_fill_u64(mom, nc * D * 2, 0, s);  // kernel fill: safe under graph capture
       launch_p2m_gen(p, (uint32_t*)leaf_ids.p, nleaves, c, b, mom, s);
       for (int L = (int)max_level - 1; L >= 0; L--)
         launch_m2m_gen(p, (uint32_t*)lvl_cells.p + lvl_off[L], lvl_off[L + 1] - lvl_off[L], c, mom,
