@@ -518,8 +518,7 @@ struct fmmh_ctx {
     uint32_t* dtot = (uint32_t*)list_tot.p;
     HCHECK(hipMemsetAsync(dtot, 0, 16, s));
     plan_p2p_count(dtot);
-    const uint32_t ch =
-        p <= TEMPLATED_MAX_P ? (uint32_t)tun.m2l_chunk : m2l_rot_chunk(2 * n_m2l);
+    const uint32_t ch = p <= TEMPLATED_MAX_P ? (uint32_t)tun.m2l_chunk : M2L_ROT_CHUNK;
     size_t maxck = m2l_max_chunks(2 * n_m2l, nc, ch);
     ensure(nch, ((size_t)nc + 1) * 4);
     ensure(choff, ((size_t)nc + 1) * 4);

@@ -212,10 +212,12 @@ void launch_p2m_gen(int p, const uint32_t* leaf_ids, uint32_t nleaves, DevCells 
                     cplx* moments, hipStream_t s);
 void launch_m2m_gen(int p, const uint32_t* cells, uint32_t cnt, DevCells c, cplx* moments,
                     hipStream_t s);
-// m2l_rot.hip: the swap matrices and scale factors of order p (host), the
-// sources per chunk, and the M2L (chunk partials in part, then the locals).
+// m2l_rot.hip: the swap matrices and scale factors of order p (host), and the
+// M2L (chunk partials in part, then the locals). Sources per chunk: four
+// batches. A fixed length, since a target's sums are grouped by it and a system
+// in an ensemble has to get its standalone sums bit for bit.
+constexpr uint32_t M2L_ROT_CHUNK = 64;
 void rot_tables_host(int p, std::vector<double>& tab, std::vector<uint32_t>& off);
-uint32_t m2l_rot_chunk(uint32_t ndirected);
 hipError_t launch_m2l_rot(int p, uint32_t nc, const void* chunks, uint32_t nchunks,
                           const uint32_t* choff, const uint64_t* skeys, int sbits, DevCells c,
                           const cplx* moments, double soft2, const double* tab,

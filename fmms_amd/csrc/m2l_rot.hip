@@ -538,14 +538,6 @@ static RotTables rot_view(int p, const double* tab, const std::vector<uint32_t>&
   return r;
 }
 
-// Sources per chunk: enough chunks to fill the chip several times over (8192,
-// about 8 rounds of 4 blocks per CU) where the lists allow it, in whole batches; long lists keep
-// long chunks, so the partials stay a small part of the locals' memory.
-uint32_t m2l_rot_chunk(uint32_t ndirected) {
-  const uint32_t ch = (ndirected / 8192u + 15u) / 16u * 16u;
-  return std::min(1024u, std::max(16u, ch));
-}
-
 template <int STMAX>
 static hipError_t rot_t(int p, const M2lChunk* ck, uint32_t nchunks, const uint64_t* skeys,
                         uint64_t smask, DevCells c, const cplx* moments, double soft2,
