@@ -115,6 +115,7 @@ struct fmmh_ctx {
   Buf walk_code, walk_blk;  // the walk's per-pair decisions, per-block counts
   Buf pl_n, pl_items, pl_reds, pl_partial;  // P2P work plan
   Buf m2l_lam, m2l_m32;                     // mixed form: FP32 M2L scales, scaled moments
+  Buf m2l_rows;                             // FP64 form: source rows
   Buf loc32;                                // mixed form: FP32 locals scaled by lam^n
   uint32_t p_nitems = 0, p_nsplit = 0;
   Buf rt_tab;  // p > TEMPLATED_MAX_P: the rotation M2L's tables
@@ -135,7 +136,7 @@ struct fmmh_ctx {
                   &moments, &locals, &pows, &fvals, &fmin, &fact, &binom, &front_a, &front_b,
                   &m2l, &p2p, &ctr, &mkeys, &mkeys_alt, &tptr, &pkeys, &pkeys_alt, &pptr, &list_tot,
                   &nch, &choff, &chunks, &part, &far, &p2p_work, &walkrec, &walk_code, &walk_blk, &pl_n, &pl_items,
-                  &pl_reds, &pl_partial, &m2l_lam, &m2l_m32, &loc32, &rt_tab, &direct_ids, &direct_out, &direct_part, &lf_part, &lf_state, &lf_flag, &ctrace, &clap,
+                  &pl_reds, &pl_partial, &m2l_lam, &m2l_m32, &m2l_rows, &loc32, &rt_tab, &direct_ids, &direct_out, &direct_part, &lf_part, &lf_state, &lf_flag, &ctrace, &clap,
                   &d_sysoff};
     bufs.assign(std::begin(all), std::end(all));
   }
@@ -535,10 +536,12 @@ struct fmmh_ctx {
     p_nsplit = t.z;
     plan_p2p_emit(t.y);
     nchunks = t.w;
-    ensure(part, m2l_part_bytes(p, std::max<size_t>(nchunks, 1)));
+    ensure(part, m2l_part_bytes(p, std::max<size_t>(nchunks, 1), mixed32()));
     if (p > TEMPLATED_MAX_P) {
       rot_tables();
-    } else if (prm.precision == FMMH_PREC_FP32BULK) {
+    } else if (!mixed32()) {
+      ensure(m2l_rows, (size_t)nc * m2l_row_bytes(p));
+    } else {
       ensure(m2l_lam, (size_t)nc * sizeof(double));
       ensure(m2l_m32, (size_t)nc * m2l32_moment_bytes(p));
       ensure(loc32, (size_t)nc * m2l32_moment_bytes(p));
@@ -603,9 +606,10 @@ struct fmmh_ctx {
       mark(ST_M2L_REDUCE);
       launch_m2l_reduce32(p, nc, (uint32_t*)choff.p, part.p, (const double*)m2l_lam.p, loc, s);
     } else if (!gen) {
-      launch_m2l_kernel(p, chunks.p, nchunks, msorted, sbits, c, mom, soft2, (cplx*)part.p, s);
+      launch_m2l_kernel(p, nc, chunks.p, nchunks, msorted, sbits, c, mom, soft2,
+                        (double*)m2l_rows.p, (double*)part.p, s);
       mark(ST_M2L_REDUCE);
-      launch_m2l_reduce(p, nc, (uint32_t*)choff.p, (cplx*)part.p, loc, s);
+      launch_m2l_reduce(p, nc, (uint32_t*)choff.p, (const double*)part.p, loc, s);
     } else {
       HCHECK(launch_m2l_rot(p, nc, chunks.p, nchunks, (uint32_t*)choff.p, msorted, sbits, c, mom,
                             soft2, (const double*)rt_tab.p, rot_off, (cplx*)part.p, loc, s));

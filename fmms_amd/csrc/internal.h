@@ -166,14 +166,17 @@ void launch_csr_ptr(const uint64_t* keys, uint32_t nnz, int sbits, uint32_t ntar
 // --------------------------------------------------------------- m2l.hip
 // Chunks of at most `ch` sources per target (the M2L work unit).
 size_t m2l_max_chunks(uint32_t nnz, uint32_t nc, uint32_t ch);
-size_t m2l_part_bytes(int p, size_t maxchunks);
+size_t m2l_part_bytes(int p, size_t maxchunks, bool fp32);
 size_t m2l_chunk_bytes();
 void m2l_build_chunks(const uint32_t* tptr, uint32_t nc, uint32_t ch, uint32_t* nch,
                       uint32_t* choff, uint32_t* scan_tmp, void* chunks, hipStream_t s,
                       uint32_t** total_dev);
-bool launch_m2l_kernel(int p, const void* chunks, uint32_t nchunks, const uint64_t* skeys,
-                       int sbits, DevCells c, const cplx* moments, double soft2, cplx* part,
-                       hipStream_t s);
+// FP64 form, p <= 10: rows [nc] x m2l_row_bytes(p) is scratch (the sources'
+// multipoles and centres as contiguous rows), part gets the chunk partials.
+size_t m2l_row_bytes(int p);
+bool launch_m2l_kernel(int p, uint32_t nc, const void* chunks, uint32_t nchunks,
+                       const uint64_t* skeys, int sbits, DevCells c, const cplx* moments,
+                       double soft2, double* rows, double* part, hipStream_t s);
 // Mixed form: the same M2L on radius-scaled FP32 operands (m2l_kernel.h);
 // lam [nc] doubles and m32 [nc] x m2l32_moment_bytes(p) are scratch.
 // prep_below: FP32 moments are made from the FP64 ones for the cells above
@@ -189,7 +192,7 @@ void launch_m2l_scale(uint32_t nc, DevCells c, const BBox* bb, const uint64_t* k
 size_t m2l32_moment_bytes(int p);
 bool launch_m2l_reduce32(int p, uint32_t nc, const uint32_t* choff, const void* part,
                          const double* lam, cplx* locals, hipStream_t s);
-bool launch_m2l_reduce(int p, uint32_t nc, const uint32_t* choff, const cplx* part, cplx* locals,
+bool launch_m2l_reduce(int p, uint32_t nc, const uint32_t* choff, const double* part, cplx* locals,
                        hipStream_t s);
 
 // ----------------------------------------------------------- upward32.hip

@@ -10,7 +10,8 @@ namespace fmmh {
 
 template <int P>
 void m2l_t(const M2lChunk* chunks, uint32_t nchunks, const uint64_t* skeys, uint64_t smask,
-           DevCells c, const cplx* moments, double soft2, cplx* part, hipStream_t s);
+           uint32_t nc, DevCells c, const cplx* moments, double soft2, double* rows, double* part,
+           hipStream_t s);
 template <int P>
 void m2l32_t(const M2lChunk* chunks, uint32_t nchunks, const uint64_t* skeys, uint64_t smask,
              DevCells c, const double* lam, const cplxf* m32, double soft2, cplxf* part,
@@ -80,11 +81,13 @@ __global__ void __launch_bounds__(256) k_m2l_emit(const uint32_t* __restrict__ t
 
 constexpr int RED_AHEAD = 8;  // chunk partials loaded ahead of the in-order sum
 
-// locals[t] = sum over the target's chunk partials in chunk order; both
-// halves of m written (F_n^{-m} = (-1)^m conj(F_n^m)); empty targets get 0.
+// locals[t] = sum over the target's chunk partials in chunk order (partials
+// in the real layout, (P+1)^2 doubles: degree n at n^2, m = 0, then re, im of
+// each m); both halves of m written (F_n^{-m} = (-1)^m conj(F_n^m)); empty
+// targets get 0.
 template <int P>
 __global__ void __launch_bounds__(256) k_m2l_reduce(uint32_t nc, const uint32_t* __restrict__ choff,
-                                                   const cplx* __restrict__ part,
+                                                   const double* __restrict__ part,
                                                    cplx* __restrict__ locals) {
   constexpr int D = hdim(P), NF = hnpos(P);
   size_t g = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -95,23 +98,28 @@ __global__ void __launch_bounds__(256) k_m2l_reduce(uint32_t nc, const uint32_t*
   while ((n + 1) * (n + 2) / 2 <= e) n++;
   int m = e - n * (n + 1) / 2;
   cplx s = cplx{0.0, 0.0};
+  constexpr int W = (P + 1) * (P + 1);
+  const int ir = n * n + (m ? 2 * m - 1 : 0), ii = n * n + 2 * m;  // m = 0: ii unused
   const uint32_t c0 = choff[t], c1 = choff[t + 1];
   uint32_t c = c0;
   for (; c + RED_AHEAD <= c1; c += RED_AHEAD) {  // loads issued together, added in order
-    cplx v[RED_AHEAD];
-#pragma unroll
-    for (int j = 0; j < RED_AHEAD; j++) v[j] = part[(size_t)(c + j) * NF + e];
+    double vr[RED_AHEAD], vi[RED_AHEAD];
 #pragma unroll
     for (int j = 0; j < RED_AHEAD; j++) {
-      s.re += v[j].re;
-      s.im += v[j].im;
+      vr[j] = part[(size_t)(c + j) * W + ir];
+      vi[j] = part[(size_t)(c + j) * W + ii];
+    }
+#pragma unroll
+    for (int j = 0; j < RED_AHEAD; j++) {
+      s.re += vr[j];
+      s.im += vi[j];
     }
   }
   for (; c < c1; c++) {
-    cplx v = part[(size_t)c * NF + e];
-    s.re += v.re;
-    s.im += v.im;
+    s.re += part[(size_t)c * W + ir];
+    s.im += part[(size_t)c * W + ii];
   }
+  if (m == 0) s.im = 0.0;
   cplx* out = locals + (size_t)t * D;
   out[hidx(n, m)] = s;
   if (m > 0) {
@@ -168,10 +176,17 @@ __global__ void __launch_bounds__(256) k_m2l_reduce32(uint32_t nc, const uint32_
 // Scratch layout handed in by the context: nch/choff (nc+1 words each) and
 // chunk/partial arrays sized for the worst case sum_t ceil(S_t/CH).
 size_t m2l_max_chunks(uint32_t nnz, uint32_t nc, uint32_t ch) { return (size_t)nnz / ch + nc + 1; }
-size_t m2l_part_bytes(int p, size_t maxchunks) { return maxchunks * hnpos(p) * sizeof(cplx); }
+// One chunk's partial: FP32 complex halves in the mixed form, (p+1)^2 doubles
+// in the FP64 form, complex halves in the runtime orders' kernel.
+size_t m2l_part_bytes(int p, size_t maxchunks, bool fp32) {
+  const size_t one = p > TEMPLATED_MAX_P ? hnpos(p) * sizeof(cplx)
+                     : fp32              ? hnpos(p) * sizeof(cplxf)
+                                         : hdim(p) * sizeof(double);
+  return maxchunks * one;
+}
 
 template <int P>
-static void m2l_reduce_t(uint32_t nc, const uint32_t* choff, const cplx* part, cplx* locals,
+static void m2l_reduce_t(uint32_t nc, const uint32_t* choff, const double* part, cplx* locals,
                          hipStream_t s) {
   size_t th = (size_t)nc * hnpos(P);
   hipLaunchKernelGGL(k_m2l_reduce<P>, dim3((th + 255) / 256), dim3(256), 0, s, nc, choff, part,
@@ -202,15 +217,21 @@ void m2l_build_chunks(const uint32_t* tptr, uint32_t nc, uint32_t ch, uint32_t* 
     default: return false;      \
   }
 
-bool launch_m2l_kernel(int p, const void* chunks, uint32_t nchunks, const uint64_t* skeys,
-                       int sbits, DevCells c, const cplx* moments, double soft2, cplx* part,
-                       hipStream_t s) {
+bool launch_m2l_kernel(int p, uint32_t nc, const void* chunks, uint32_t nchunks,
+                       const uint64_t* skeys, int sbits, DevCells c, const cplx* moments,
+                       double soft2, double* rows, double* part, hipStream_t s) {
   const uint64_t smask = (1ull << sbits) - 1ull;
   const M2lChunk* ck = (const M2lChunk*)chunks;
-#define CALL(P) m2l_t<P>(ck, nchunks, skeys, smask, c, moments, soft2, part, s)
+#define CALL(P) m2l_t<P>(ck, nchunks, skeys, smask, nc, c, moments, soft2, rows, part, s)
   FMMH_P_SWITCH3(p, CALL)
 #undef CALL
   return true;
+}
+
+// Bytes of one cell's source row (M2lRow<p>), p <= 10.
+size_t m2l_row_bytes(int p) {
+  const int nm = hdim(p), ndir = p <= 7 ? 1 : p == 8 ? 9 : nm;
+  return (size_t)((nm - ndir + 7) / 8 * 8 + (3 + ndir + 7) / 8 * 8) * sizeof(double);
 }
 
 void launch_m2l_scale(uint32_t nc, DevCells c, const BBox* bb, const uint64_t* keys_sorted,
@@ -249,7 +270,7 @@ bool launch_m2l_reduce32(int p, uint32_t nc, const uint32_t* choff, const void* 
   return true;
 }
 
-bool launch_m2l_reduce(int p, uint32_t nc, const uint32_t* choff, const cplx* part, cplx* locals,
+bool launch_m2l_reduce(int p, uint32_t nc, const uint32_t* choff, const double* part, cplx* locals,
                        hipStream_t s) {
 #define CALL(P) m2l_reduce_t<P>(nc, choff, part, locals, s)
   FMMH_P_SWITCH3(p, CALL)

@@ -1,4 +1,5 @@
-// m2l_kernel.h — far-field M2L on gfx950 (FP64, FMA contraction on).
+// m2l_kernel.h — far-field M2L on gfx950 (FP64, and FP32 in the mixed form;
+// FMA contraction on).
 //
 // F_B[n,m] += sum_{k<=p-n} sum_{|l|<=k} conj(M_A[k,l]) Theta_{n+k}^{m+l}(s_B - z_A)
 // (crates/fmm translate.rs:47-136). The reference evaluates each accepted
@@ -23,13 +24,6 @@ namespace fmmh {
 // The chunk length (sources per thread) is a context parameter,
 // fmmh_tuning.m2l_chunk (default 32).
 
-__device__ __forceinline__ void cmac(cplx& f, double ar, double ai, double br, double bi) {
-  f.re = fma(ar, br, f.re);
-  f.re = fma(-ai, bi, f.re);
-  f.im = fma(ar, bi, f.im);
-  f.im = fma(ai, br, f.im);
-}
-
 __device__ __forceinline__ void cmac(cplxf& f, float ar, float ai, float br, float bi) {
   f.re = fmaf(ar, br, f.re);
   f.re = fmaf(-ai, bi, f.re);
@@ -38,10 +32,6 @@ __device__ __forceinline__ void cmac(cplxf& f, float ar, float ai, float br, flo
 }
 
 // f += a * (br + i bi) for a real factor a.
-__device__ __forceinline__ void cmac_real(cplx& f, double a, double br, double bi) {
-  f.re = fma(a, br, f.re);
-  f.im = fma(a, bi, f.im);
-}
 __device__ __forceinline__ void cmac_real(cplxf& f, float a, float br, float bi) {
   f.re = fmaf(a, br, f.re);
   f.im = fmaf(a, bi, f.im);
@@ -53,15 +43,10 @@ __device__ __forceinline__ float m2l_rsqrt(float x) {
   return y * fmaf(-0.5f * x * y, y, 1.5f);  // one Newton step on the hardware estimate
 }
 
-// F (m>=0 half, hpos layout) += M2L of source multipole M (m>=0 half) at r.
-// H = 2: every degree n of F; H = 0 / 1: only even / odd n (the two halves
-// of a chunk, run by two waves: about equal work, half the accumulators).
+// FP32 (mixed form): F (m>=0 half, hpos layout) += M2L of source multipole M
+// (m>=0 half) at r, term by term (softening as in m2l_accumulate64).
 template <int P, int H, typename R, typename C>
 __device__ __forceinline__ void m2l_accumulate(R x, R y, R z, R soft2, const C* M, C* F) {
-  // Softening: the harmonic derivatives of the Plummer kernel are those of
-  // 1/r times (r/s)^{2n+1}, s^2 = r^2 + eps^2; in the recursion that is
-  // 1/r^2 -> 1/s^2 and the (n-2) term scaled by ks = r^2/s^2 (soft2 = 0:
-  // ks = 1, pure 1/r).
   const R rr2 = x * x + y * y + z * z;
   const R r2 = rr2 + soft2;
   const R ir = m2l_rsqrt(r2);
@@ -146,83 +131,340 @@ __device__ __forceinline__ void m2l_accumulate(R x, R y, R z, R soft2, const C* 
   }
 }
 
-template <int P, int H>
-__device__ __forceinline__ void m2l_chunk(const M2lChunk ck, uint32_t ci,
-                                          const uint64_t* __restrict__ skeys, uint64_t smask,
-                                          const double* __restrict__ ccx,
-                                          const double* __restrict__ ccy,
-                                          const double* __restrict__ ccz,
-                                          const cplx* __restrict__ moments, double soft2,
-                                          cplx* __restrict__ part) {
-  constexpr int D = hdim(P), NF = hnpos(P);
-  const double tx = ccx[ck.target], ty = ccy[ck.target], tz = ccz[ck.target];
-  cplx F[NF];
+// ------------------------------------------------------------------- FP64
+// Real-valued layout of an m >= 0 half: (P+1)^2 doubles, degree n at n^2:
+// X_n^0 (real), then (re, im) of X_n^m, m = 1..n.
+__host__ __device__ constexpr int rre(int n, int m) { return n * n + (m ? 2 * m - 1 : 0); }
+__host__ __device__ constexpr int rim(int n, int m) { return n * n + 2 * m; }
+
+// F += M2L of source multipole M at r, both in the real layout, with the
+// terms of +l and -l taken together. With M_k^l = a + ib, M_k^{-l} =
+// (-1)^l conj(M_k^l) and
+//   S = Theta^{m+l} + (-1)^l Theta^{m-l},  D = Theta^{m+l} - (-1)^l Theta^{m-l},
+// the two terms of F_n^m are a S - i b D: four multiply-adds instead of
+// eight, and S, D depend on n + k, m and l alone, so one set serves every
+// (n, k) of a degree, and the set of (m, l) serves (l, m) with the imaginary
+// parts exchanged. F_n^0 is real: 2 Re(conj(M_k^l) Theta^l), accumulated
+// halved (the caller doubles it). At P = 7: 876 multiply-adds and 112 adds
+// for the sums, against 2100 term by term.
+// H = 2: every degree n of F; H = 0 / 1: only even / odd n (the two halves
+// of a chunk, run by two waves: about equal work, half the accumulators).
+// on: whether the lane has a pair (else Theta is 0 and nothing is added).
+// mid() runs between the degrees s = 0..2 and the others.
+template <int P, int H, class Mid>
+__device__ __forceinline__ void m2l_accumulate64(bool on, double x, double y, double z,
+                                                 double soft2, const double* M, double* F,
+                                                 Mid mid) {
+  // Softening: the harmonic derivatives of the Plummer kernel are those of
+  // 1/r times (r/s)^{2n+1}, s^2 = r^2 + eps^2; in the recursion that is
+  // 1/r^2 -> 1/s^2 and the (n-2) term scaled by r^2/s^2 (soft2 = 0: 1).
+  const double rr2 = x * x + y * y + z * z;
+  const double r2 = rr2 + soft2;
+  const double ir = m2l_rsqrt(r2);
+  const double ir2 = ir * ir;
+  const double kir = soft2 > 0.0 ? rr2 * ir2 * ir2 : ir2;
+  const double xs = x * ir2, ys = y * ir2, zs = z * ir2;
+  double Tr[P + 1], Ti[P + 1], Ar[P + 1], Ai[P + 1], Br[P + 1], Bi[P + 1];  // Theta_s, _{s-1}, _{s-2}
 #pragma unroll
-  for (int i = 0; i < NF; i++) F[i] = cz();
-  for (uint32_t j = ck.begin; j < ck.end; j++) {
-    const uint32_t src = (uint32_t)(skeys[j] & smask);
-    const cplx* ms = moments + (size_t)src * D;
-    cplx M[NF];
+  for (int s = 0; s <= P; s++) {
+    // Theta_s^q, q = 0..s (harmonic.rs:91-129 recursion, Dehnen eq. 52/54)
+    if (s == 0) {
+      Tr[0] = on ? ir : 0.0;
+      Ti[0] = 0.0;
+    } else {
+      const double a = (double)(2 * s - 1) * zs;
 #pragma unroll
-    for (int k = 0; k <= P; k++)
+      for (int q = 0; q <= P; q++) {
+        if (q > s) continue;
+        if (q + 2 <= s) {
+          const double bq = (double)((s - 1) * (s - 1) - q * q) * kir;
+          Tr[q] = fma(a, Ar[q], -(bq * Br[q]));
+          Ti[q] = q == 0 ? 0.0 : fma(a, Ai[q], -(bq * Bi[q]));
+        } else if (q == s - 1) {
+          Tr[q] = a * Ar[q];
+          Ti[q] = q == 0 ? 0.0 : a * Ai[q];
+        } else {  // q == s: (2s-1)(x+iy)/r^2 * Theta_{s-1}^{s-1}
+          const double wr = (double)(2 * s - 1) * xs, wi = (double)(2 * s - 1) * ys;
+          Tr[q] = s == 1 ? wr * Ar[0] : fma(wr, Ar[s - 1], -(wi * Ai[s - 1]));
+          Ti[q] = s == 1 ? wi * Ar[0] : fma(wr, Ai[s - 1], wi * Ar[s - 1]);
+        }
+      }
+    }
+    // all terms with n + k == s: l = 0, and m = 0
+    const double t0 = 0.5 * Tr[0];
 #pragma unroll
-      for (int l = 0; l <= k; l++) M[hpos(k, l)] = ms[hidx(k, l)];
-    m2l_accumulate<P, H, double, cplx>(tx - ccx[src], ty - ccy[src], tz - ccz[src], soft2, M, F);
+    for (int n = 0; n <= P; n++) {
+      if (n > s) continue;
+      if (H != 2 && (n & 1) != H) continue;
+      const int k = s - n;
+      F[rre(n, 0)] = fma(M[rre(k, 0)], t0, F[rre(n, 0)]);
+#pragma unroll
+      for (int l = 1; l <= P; l++) {
+        if (l > k) continue;
+        F[rre(n, 0)] = fma(M[rre(k, l)], Tr[l], F[rre(n, 0)]);
+        F[rre(n, 0)] = fma(M[rim(k, l)], Ti[l], F[rre(n, 0)]);
+      }
+#pragma unroll
+      for (int m = 1; m <= P; m++) {
+        if (m > n) continue;
+        F[rre(n, m)] = fma(M[rre(k, 0)], Tr[m], F[rre(n, m)]);
+        F[rim(n, m)] = fma(M[rre(k, 0)], Ti[m], F[rim(n, m)]);
+      }
+    }
+    // m, l >= 1: one set of sums per unordered {u, v}, u >= v, for (m, l) =
+    // (u, v) and (v, u)
+#pragma unroll
+    for (int u = 1; u <= P; u++) {
+#pragma unroll
+      for (int v = 1; v <= P; v++) {
+        if (v > u || u + v > s) continue;
+        const double pr = Tr[u + v], pi = Ti[u + v];
+        const double mr = (v & 1) ? -Tr[u - v] : Tr[u - v];
+        const double mi = u == v ? 0.0 : ((v & 1) ? -Ti[u - v] : Ti[u - v]);
+        const double sr = pr + mr, dr = pr - mr;
+        const double si = u == v ? pi : pi + mi, di = u == v ? pi : pi - mi;
+#pragma unroll
+        for (int w = 0; w < 2; w++) {
+          if (w == 1 && u == v) continue;
+          const int m = w == 0 ? u : v, l = w == 0 ? v : u;
+          const double ssi = w == 0 ? si : di, ddi = w == 0 ? di : si;
+#pragma unroll
+          for (int n = 0; n <= P; n++) {
+            const int k = s - n;
+            if (n < m || k < l) continue;
+            if (H != 2 && (n & 1) != H) continue;
+            const double a = M[rre(k, l)], b = M[rim(k, l)];
+            F[rre(n, m)] = fma(a, sr, F[rre(n, m)]);
+            F[rim(n, m)] = fma(a, ssi, F[rim(n, m)]);
+            F[rre(n, m)] = fma(b, ddi, F[rre(n, m)]);
+            F[rim(n, m)] = fma(-b, dr, F[rim(n, m)]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q <= P; q++) {
+      if (q > s) continue;
+      Br[q] = Ar[q];
+      Bi[q] = Ai[q];
+      Ar[q] = Tr[q];
+      Ai[q] = Ti[q];
+    }
+    if (s == (P < 2 ? P : 2)) mid();
   }
-  cplx* out = part + (size_t)ci * NF;
-#pragma unroll
-  for (int n = 0; n <= P; n++) {
-    if (H != 2 && (n & 1) != H) continue;
-#pragma unroll
-    for (int m = 0; m <= n; m++) out[hpos(n, m)] = F[hpos(n, m)];
+}
+
+// Source rows: the cells' multipoles in the real layout with the cell centre,
+// one contiguous row per cell (k_m2l_rows). The tail of the multipole is
+// staged through LDS in 64-byte segments (SEG of them); the first NDIR
+// doubles and the centre are read by each lane itself. Lanes reading whole
+// rows by themselves touch 64 cache lines per load and made the kernel wait
+// on the address unit (P = 7: 36 loads x 64 lines per source against 9600
+// cycles of arithmetic, with one wave a SIMD and so no overlap). Four lanes
+// now read a segment of one row, and the copy to LDS runs without registers
+// while the wave computes. Measured (kernel alone): P = 7, 8.4M bodies, 152M
+// directed pairs 20.7 -> 10.4 ms; P = 8, 1M bodies, 38.8M pairs 10.0 -> 4.6 ms;
+// P = 6, 250k bodies 0.66 -> 0.35 ms. The rows' traffic (88 GB at P = 7, 8.4
+// TB/s, mostly from the memory-side cache) and FP64 issue now bound it
+// together. P = 8 keeps its first degrees out of LDS so that
+// four waves fit a CU; from P = 9 on the rows are read directly.
+template <int P>
+struct M2lRow {
+  static constexpr int NM = (P + 1) * (P + 1);
+  static constexpr bool STAGED = P <= 8;
+  static constexpr int NDIR = P <= 7 ? 1 : P == 8 ? 9 : NM;
+  static constexpr int SEG = (NM - NDIR + 7) / 8;
+  static constexpr int DIR = (3 + NDIR + 7) / 8 * 8;  // centre + direct part
+  static constexpr int WORDS = SEG * 8 + DIR;          // staged part first, 64-byte rows
+};
+
+template <int P>
+__global__ void __launch_bounds__(256) k_m2l_rows(uint32_t nc, const cplx* __restrict__ moments,
+                                                 const double* __restrict__ ccx,
+                                                 const double* __restrict__ ccy,
+                                                 const double* __restrict__ ccz,
+                                                 double* __restrict__ rows) {
+  using R = M2lRow<P>;
+  const size_t g = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const uint32_t c = (uint32_t)(g / R::WORDS);
+  if (c >= nc) return;
+  const int i = (int)(g - (size_t)c * R::WORDS);
+  // position i -> multipole entry e (-1: none) or centre coordinate
+  const int d = i - R::SEG * 8;
+  const int e = d < 0 ? (i + R::NDIR < R::NM ? i + R::NDIR : -1) : (d >= 3 && d - 3 < R::NDIR ? d - 3 : -1);
+  double v = 0.0;
+  if (e >= 0) {
+    int n = 0;
+    while ((n + 1) * (n + 1) <= e) n++;
+    const int r = e - n * n;  // 0: m = 0; 2m-1: re, 2m: im
+    const cplx q = moments[(size_t)c * hdim(P) + hidx(n, (r + 1) / 2)];
+    v = r > 0 && (r & 1) == 0 ? q.im : q.re;
+  } else if (d >= 0 && d < 3) {
+    v = d == 0 ? ccx[c] : d == 1 ? ccy[c] : ccz[c];
   }
+  rows[g] = v;
 }
 
 // SPLIT: two blocks per 64 chunks, the even-n and the odd-n half of F (the
 // pair of blocks is adjacent after the XCD remap, so on one XCD's L2).
-// Orders whose accumulators are split over two waves (register pressure),
-// and the waves per SIMD the split kernels are compiled for.
+// Orders whose accumulators are split over two waves (register pressure).
+// From 9: at P = 8 one wave measured 5.3 ms and two 5.6 (1M bodies).
 #ifndef FMMH_M2L_SPLIT_FROM
-#define FMMH_M2L_SPLIT_FROM 8
+#define FMMH_M2L_SPLIT_FROM 9
 #endif
-#ifndef FMMH_M2L_SPLIT_WAVES
-#define FMMH_M2L_SPLIT_WAVES 1
-#endif
+
+typedef __attribute__((address_space(3))) char lds_char;
+typedef __attribute__((address_space(1))) const char gbl_char;
+
+// Piece I of a row group's segments to LDS. The instruction adds its offset
+// (64 I) to both addresses, so the LDS side is passed less that much.
+template <int SEG, int I = 0>
+__device__ __forceinline__ void m2l_copy_segments(gbl_char* from, lds_char* to) {
+  if constexpr (I < SEG) {
+    __builtin_amdgcn_global_load_lds(from, to + I * (1024 - 64), 16, 64 * I, 0);
+    m2l_copy_segments<SEG, I + 1>(from, to);
+  }
+}
+
+template <int P, int H>
+__device__ __forceinline__ void m2l_chunks64(uint32_t ci, bool live, const M2lChunk ck,
+                                             const uint64_t* __restrict__ skeys, uint64_t smask,
+                                             const double* __restrict__ rows, double soft2,
+                                             double2* stage, double* __restrict__ part) {
+  using R = M2lRow<P>;
+  const int lane = threadIdx.x;
+  lds_char* stage3 = (lds_char*)stage;
+  const uint32_t cnt = live ? ck.end - ck.begin : 0u;
+  uint32_t trips = cnt;  // the wave runs its longest chunk's trip count
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) trips = max(trips, (uint32_t)__shfl_xor((int)trips, o, 64));
+  trips = (uint32_t)wave_uniform((int)trips);
+  if (trips == 0) return;
+  double F[R::NM];
+#pragma unroll
+  for (int i = 0; i < R::NM; i++) F[i] = 0.0;
+  // a lane past its chunk's end goes on reading the chunk's last source (a
+  // dead lane cell 0), so every row address stays valid
+  auto source = [&](uint32_t j) -> uint32_t {
+    return cnt ? (uint32_t)(skeys[ck.begin + min(j, cnt - 1)] & smask) : 0u;
+  };
+  // copy of the rows' staged part into LDS, [16-row group][segment][row][4]
+  // of 16 bytes, the four pieces of a row rotated by its number so that 16
+  // lanes reading one piece of 16 rows hit all banks
+  auto copy = [&](uint32_t src) {
+    if constexpr (R::STAGED) {
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        const uint32_t rs = (uint32_t)__shfl((int)src, g * 16 + (lane >> 2), 64);
+        m2l_copy_segments<R::SEG>(
+            (gbl_char*)(rows + (size_t)rs * R::WORDS) + ((lane & 3) ^ ((lane >> 4) & 3)) * 16,
+            stage3 + g * R::SEG * 1024);
+      }
+    }
+  };
+  const int swz = (lane >> 2) & 3;
+  const double2* mine = stage + (lane >> 4) * R::SEG * 64 + (lane & 15) * 4;
+  uint32_t src = source(0);
+  double dir[R::DIR];
+  auto direct = [&](uint32_t sc) {
+    const double2* d2 = (const double2*)(rows + (size_t)sc * R::WORDS + R::SEG * 8);
+#pragma unroll
+    for (int i = 0; i < (3 + R::NDIR + 1) / 2; i++) {
+      const double2 v = d2[i];
+      dir[2 * i] = v.x;
+      dir[2 * i + 1] = v.y;
+    }
+  };
+  direct(src);
+  copy(src);
+  double tx = 0.0, ty = 0.0, tz = 0.0;
+  {
+    const double* t = rows + (size_t)ck.target * R::WORDS + R::SEG * 8;
+    tx = t[0];
+    ty = t[1];
+    tz = t[2];
+  }
+  uint32_t src_n = source(1);
+  for (uint32_t j = 0; j < trips; j++) {
+    double M[R::NM];
+    const double x = tx - dir[0], y = ty - dir[1], z = tz - dir[2];
+#pragma unroll
+    for (int i = 0; i < R::NDIR; i++) M[i] = dir[3 + i];
+    if constexpr (R::STAGED) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copy has landed
+#pragma unroll
+      for (int e = 0; e < R::SEG * 4; e++) {
+        const double2 v = mine[(e >> 2) * 64 + ((e & 3) ^ swz)];
+        if (R::NDIR + 2 * e < R::NM) M[R::NDIR + 2 * e] = v.x;
+        if (R::NDIR + 2 * e + 1 < R::NM) M[R::NDIR + 2 * e + 1] = v.y;
+      }
+    }
+    // the next source's copy starts once this one's row has been read (while
+    // the first degrees are computed) and runs under the rest
+    m2l_accumulate64<P, H>(j < cnt, x, y, z, soft2, M, F, [&] {
+      if (j + 1 < trips) {
+        if constexpr (R::STAGED) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const uint32_t cur = src_n;
+        src_n = source(j + 2);
+        if constexpr (R::STAGED) direct(cur);
+        copy(cur);
+        src = cur;
+      }
+    });
+    if constexpr (!R::STAGED) {
+      if (j + 1 < trips) direct(src);
+    }
+  }
+  if (!live) return;
+  double* out = part + (size_t)ci * R::NM;
+#pragma unroll
+  for (int n = 0; n <= P; n++) {
+    if (H != 2 && (n & 1) != H) continue;
+    out[rre(n, 0)] = 2.0 * F[rre(n, 0)];
+#pragma unroll
+    for (int m = 1; m <= P; m++) {
+      if (m > n) continue;
+      out[rre(n, m)] = F[rre(n, m)];
+      out[rim(n, m)] = F[rim(n, m)];
+    }
+  }
+}
 
 template <int P, bool SPLIT>
 __global__ void __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(SPLIT ? FMMH_M2L_SPLIT_WAVES : 1))) k_m2l(const M2lChunk* __restrict__ chunks, uint32_t nchunks,
-                                           const uint64_t* __restrict__ skeys, uint64_t smask,
-                                           const double* __restrict__ ccx,
-                                           const double* __restrict__ ccy,
-                                           const double* __restrict__ ccz,
-                                           const cplx* __restrict__ moments, double soft2,
-                                           cplx* __restrict__ part) {
+__attribute__((amdgpu_waves_per_eu(1))) k_m2l(const M2lChunk* __restrict__ chunks,
+                                              uint32_t nchunks, const uint64_t* __restrict__ skeys,
+                                              uint64_t smask, const double* __restrict__ rows,
+                                              double soft2, double* __restrict__ part) {
+  __shared__ double2 stage[M2lRow<P>::STAGED ? M2lRow<P>::SEG * 256 : 1];
   const uint32_t lb = xcd_block(blockIdx.x, gridDim.x);
+  const uint32_t ci = (SPLIT ? lb >> 1 : lb) * 64 + threadIdx.x;
+  const bool live = ci < nchunks;
+  M2lChunk ck{0, 0, 0};
+  if (live) ck = chunks[ci];
   if constexpr (SPLIT) {
-    const uint32_t ci = (lb >> 1) * blockDim.x + threadIdx.x;
-    if (ci >= nchunks) return;
     if (lb & 1)
-      m2l_chunk<P, 1>(chunks[ci], ci, skeys, smask, ccx, ccy, ccz, moments, soft2, part);
+      m2l_chunks64<P, 1>(ci, live, ck, skeys, smask, rows, soft2, stage, part);
     else
-      m2l_chunk<P, 0>(chunks[ci], ci, skeys, smask, ccx, ccy, ccz, moments, soft2, part);
+      m2l_chunks64<P, 0>(ci, live, ck, skeys, smask, rows, soft2, stage, part);
   } else {
-    const uint32_t ci = lb * blockDim.x + threadIdx.x;
-    if (ci >= nchunks) return;
-    m2l_chunk<P, 2>(chunks[ci], ci, skeys, smask, ccx, ccy, ccz, moments, soft2, part);
+    m2l_chunks64<P, 2>(ci, live, ck, skeys, smask, rows, soft2, stage, part);
   }
 }
 
 template <int P>
 void m2l_t(const M2lChunk* chunks, uint32_t nchunks, const uint64_t* skeys, uint64_t smask,
-                  DevCells c, const cplx* moments, double soft2, cplx* part, hipStream_t s) {
+           uint32_t nc, DevCells c, const cplx* moments, double soft2, double* rows, double* part,
+           hipStream_t s) {
   if (!nchunks) return;
   constexpr bool split = P >= FMMH_M2L_SPLIT_FROM;
+  const size_t rt = (size_t)nc * M2lRow<P>::WORDS;
+  hipLaunchKernelGGL(k_m2l_rows<P>, dim3((rt + 255) / 256), dim3(256), 0, s, nc, moments, c.cx,
+                     c.cy, c.cz, rows);
   const uint32_t nb = (nchunks + 63) / 64 * (split ? 2 : 1);
   hipLaunchKernelGGL((k_m2l<P, split>), dim3(nb), dim3(64), 0, s, chunks, nchunks, skeys, smask,
-                     c.cx, c.cy, c.cz, moments, soft2, part);
+                     (const double*)rows, soft2, part);
 }
-
 
 // ------------------------------------------------------- FP32 (mixed form)
 // The same chunked M2L on radius-scaled FP32 operands. Per target t a scale
@@ -321,8 +563,8 @@ void m2l32_t(const M2lChunk* chunks, uint32_t nchunks, const uint64_t* skeys, ui
 
 // One translation unit per range of orders instantiates the launches.
 #define FMMH_M2L_INSTANTIATE(P)                                                             \
-  template void m2l_t<P>(const M2lChunk*, uint32_t, const uint64_t*, uint64_t, DevCells,    \
-                         const cplx*, double, cplx*, hipStream_t);                          \
+  template void m2l_t<P>(const M2lChunk*, uint32_t, const uint64_t*, uint64_t, uint32_t,    \
+                         DevCells, const cplx*, double, double*, double*, hipStream_t);     \
   template void m2l32_t<P>(const M2lChunk*, uint32_t, const uint64_t*, uint64_t, DevCells,  \
                            const double*, const cplxf*, double, cplxf*, hipStream_t);
 
