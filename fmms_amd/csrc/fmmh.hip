@@ -107,6 +107,7 @@ struct fmmh_ctx {
   Buf cpm;                              // {cx, cy, cz, mass} per cell
   std::vector<uint32_t> int_off;   // level L's internal cells: [int_off[L], int_off[L+1])
   Buf scan_tmp, sort_tmp;
+  Buf fprec;  // f pre-pass cell records
   Buf moments, locals, pows, fvals, fmin, fact, binom;
   Buf front_a, front_b, m2l, p2p, ctr;
   Buf mkeys, mkeys_alt, tptr, pkeys, pkeys_alt, pptr, list_tot;
@@ -133,7 +134,7 @@ struct fmmh_ctx {
                   &c_cx, &c_cy, &c_cz, &c_mass, &c_rho, &c_rope, &c_last, &lvl_cells,
                   &leaf_flags, &leaf_off, &leaf_ids, &leaf_of_slot, &int_pos, &int_cells, &lvl_dev, &split_bnd, &leaf_bc, &lbc_keys, &lbc_keys_alt, &cpm,
                   &scan_tmp, &sort_tmp,
-                  &moments, &locals, &pows, &fvals, &fmin, &fact, &binom, &front_a, &front_b,
+                  &fprec, &moments, &locals, &pows, &fvals, &fmin, &fact, &binom, &front_a, &front_b,
                   &m2l, &p2p, &ctr, &mkeys, &mkeys_alt, &tptr, &pkeys, &pkeys_alt, &pptr, &list_tot,
                   &nch, &choff, &chunks, &part, &far, &p2p_work, &walkrec, &walk_code, &walk_blk, &pl_n, &pl_items,
                   &pl_reds, &pl_partial, &m2l_lam, &m2l_m32, &m2l_rows, &loc32, &rt_tab, &direct_ids, &direct_out, &direct_part, &lf_part, &lf_state, &lf_flag, &ctrace, &clap,
@@ -482,7 +483,9 @@ struct fmmh_ctx {
     ensure(pows, (size_t)nc * (p + 1) * 8);
     ensure(fvals, n * 8);
     launch_pows(p, nc, (const cplx*)moments.p, (double*)fact.p, (double*)pows.p, s);
-    launch_fprepass((uint32_t)n, nc, c, b, keys_sorted, vlev, (double*)fvals.p, s);
+    ensure(fprec, (size_t)nc * fp_rec_bytes());
+    launch_pack_fp(nc, c, fprec.p, s);
+    launch_fprepass((uint32_t)n, nc, fprec.p, b.xyzm, keys_sorted, vlev, (double*)fvals.p, s);
     for (int L = (int)max_level; L >= 0; L--)
       launch_fmin((uint32_t*)lvl_cells.p + lvl_off[L], lvl_off[L + 1] - lvl_off[L], c,
                   (double*)fvals.p, (double*)fmin.p, s);

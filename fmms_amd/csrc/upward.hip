@@ -327,106 +327,170 @@ void launch_pows(int p, uint32_t nc, const cplx* moments, const double* fact, do
                      pows);
 }
 
-// f pre-pass (mac.rs:99-147) as a wave-coherent stackless walk. The 64
-// lanes (64 consecutive slots) share one traversal pointer over the
-// mirrored DFS (children 7..0, exactly the reference stack's pop order); a
-// lane that accepts a cell's monopole sleeps until the wave reaches that
-// cell's rope, so each lane accumulates precisely its own reference
-// sequence of terms, in order. Cell and body loads are wave-uniform.
-// Ensembles (vlev > 0): a lane walks only its own system's subtree. A
-// virtual cell (level < vlev) is opened by the lanes whose system it holds
+// f pre-pass (mac.rs:99-147) as a wave-coherent stackless walk. The lanes
+// of a wave (64 / SUB consecutive slots, SUB lanes each) share one traversal
+// pointer over the mirrored DFS (children 7..0, exactly the reference
+// stack's pop order); a body that accepts a cell's monopole sleeps until the
+// wave reaches that cell's rope, so each accumulates precisely its own
+// reference sequence of terms, in order.
+// Ensembles (vlev > 0): a body walks only its own system's subtree. A
+// virtual cell (level < vlev) is opened by the bodies whose system it holds
 // and skipped by the others; a real cell of another system is skipped; so
-// every lane meets its system's cells in the standalone order.
-struct FpCells {
-  const uint8_t* __restrict__ leaf;
-  const uint32_t* __restrict__ first;
-  const uint32_t* __restrict__ count;
-  const double* __restrict__ cx;
-  const double* __restrict__ cy;
-  const double* __restrict__ cz;
-  const double* __restrict__ rho;
-  const double* __restrict__ mass;
-  const int32_t* __restrict__ rope;
-  const int32_t* __restrict__ last_child;
-  const uint8_t* __restrict__ level;
+// every body meets its system's cells in the standalone order.
+//
+// A step is bound by the latency of the cell it moves to, so a cell is one
+// 64-byte record (one scalar load; nine arrays before) and both candidates
+// for the next step, the rope and the last child, are loaded before the
+// current cell is computed. SUB = 4: four lanes take four consecutive bodies
+// of a leaf and divide, then each adds the four terms in slot order (read
+// from its neighbours by lane permutation), so the sequence is unchanged
+// while the division, most of the arithmetic, is done once per four bodies,
+// and there are four times as many, smaller waves.
+// Measured: 1M bodies 3.93 -> 1.77 ms, 250k 1.12 -> 0.71, 16k 0.65 -> 0.24,
+// 1k 0.235 -> 0.10.
+struct __align__(64) FpRec {
+  double cx, cy, cz, rho2, mass;
+  int32_t rope, last;  // last: -1 in a leaf
+  uint32_t first, count, level, pad;
 };
 
-__global__ void __launch_bounds__(64) k_fprepass(uint32_t n, uint32_t max_steps, FpCells c,
-                                                const double* __restrict__ bx,
-                                                const double* __restrict__ by,
-                                                const double* __restrict__ bz,
-                                                const double* __restrict__ bm,
-                                                const uint64_t* __restrict__ keys_sorted,
-                                                int vlev, double* __restrict__ f) {
+__global__ void __launch_bounds__(256) k_pack_fp(uint32_t nc, DevCells c, FpRec* __restrict__ rec) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= nc) return;
+  FpRec r;
+  r.cx = c.cx[i];
+  r.cy = c.cy[i];
+  r.cz = c.cz[i];
+  r.rho2 = c.rho[i] * c.rho[i];
+  r.mass = c.mass[i];
+  r.rope = c.rope[i];
+  r.last = c.last_child[i];
+  r.first = c.first[i];
+  r.count = c.count[i];
+  r.level = c.level[i];
+  r.pad = 0;
+  rec[i] = r;
+}
+
+// Value of lane (4 q + J) in every lane of quad q.
+template <int J>
+__device__ __forceinline__ double quad_read(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  constexpr int ctl = J * 0x55;  // quad_perm [J, J, J, J]
+  const uint32_t lo =
+      (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, ctl, 0xf, 0xf, true);
+  const uint32_t hi =
+      (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), ctl, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+template <int SUB>
+__global__ void __launch_bounds__(64) k_fprepass(uint32_t n, uint32_t max_steps,
+                                                const FpRec* __restrict__ rec,
+                                                const double4* __restrict__ body,
+                                                const uint64_t* __restrict__ keys_sorted, int vlev,
+                                                double* __restrict__ f) {
   const int ACTIVE = -2, NEVER = -3;
-  const uint32_t i = blockIdx.x * 64 + threadIdx.x;
+  const uint32_t i = blockIdx.x * (64 / SUB) + threadIdx.x / SUB;
+  const uint32_t sub = threadIdx.x % SUB;
   const bool valid = i < n;
   const int sh = 63 - 3 * vlev;
   const uint32_t mysys = (valid && vlev) ? (uint32_t)(keys_sorted[i] >> sh) : 0u;
-  const double px = valid ? bx[i] : 0.0, py = valid ? by[i] : 0.0, pz = valid ? bz[i] : 0.0;
+  const double4 me = body[valid ? i : 0];
+  const double px = me.x, py = me.y, pz = me.z;
   double fi = 0.0;
   int resume = valid ? ACTIVE : NEVER;
   int cur = 0;
+  FpRec r = rec[0];
   // The mirrored DFS visits each cell at most once, so a wave needs at most
   // ncells steps; the cap only guards against a corrupt tree.
-  for (uint32_t step = 0; cur >= 0 && step < max_steps; step++) {
-    cur = wave_uniform(cur);
+  for (uint32_t step = 0; step < max_steps; step++) {
+    const int rope = wave_uniform(r.rope), last = wave_uniform(r.last);
+    // both candidates for the next step, in flight while this one is computed
+    const FpRec r_rope = rec[rope >= 0 ? rope : 0];
+    const FpRec r_last = rec[last >= 0 ? last : 0];
     if (resume == cur) resume = ACTIVE;
     bool act = resume == ACTIVE;
     bool virt = false;
     if (vlev) {
-      const uint32_t f0 = c.first[cur];
-      const uint32_t slo = (uint32_t)(keys_sorted[f0] >> sh);
-      virt = (int)c.level[cur] < vlev;
+      const uint32_t slo = (uint32_t)(keys_sorted[r.first] >> sh);
+      virt = (int)r.level < vlev;
       if (act) {
-        const uint32_t shi =
-            virt ? (uint32_t)(keys_sorted[f0 + c.count[cur] - 1] >> sh) : slo;
-        if (mysys < slo || mysys > shi) {  // not this lane's system
-          resume = c.rope[cur];
+        const uint32_t shi = virt ? (uint32_t)(keys_sorted[r.first + r.count - 1] >> sh) : slo;
+        if (mysys < slo || mysys > shi) {  // not this body's system
+          resume = rope;
           act = false;
         }
       }
     }
-    if (c.leaf[cur]) {
-      const uint32_t f0 = c.first[cur], e = f0 + c.count[cur];
-      for (uint32_t k = f0; k < e; k++) {
-        const double xk = bx[k], yk = by[k], zk = bz[k], mk = bm[k];
-        if (act && k != i) {
-          double dx = px - xk, dy = py - yk, dz = pz - zk;
-          double r2 = dx * dx + dy * dy + dz * dz;
-          if (r2 > 0.0) fi += mk / r2;
+    bool open = false;
+    if (last < 0) {
+      const uint32_t f0 = r.first, e = f0 + r.count;
+      if (SUB == 1) {
+#pragma unroll 4
+        for (uint32_t k = f0; k < e; k++) {
+          const double4 q = body[k];
+          const double dx = px - q.x, dy = py - q.y, dz = pz - q.z;
+          const double r2 = dx * dx + dy * dy + dz * dz;
+          if (act && k != i && r2 > 0.0) fi += q.w / r2;
+        }
+      } else {
+        for (uint32_t k0 = f0; k0 < e; k0 += SUB) {
+          const uint32_t k = k0 + sub;
+          const double4 q = body[min(k, e - 1)];
+          const double dx = px - q.x, dy = py - q.y, dz = pz - q.z;
+          const double r2 = dx * dx + dy * dy + dz * dz;
+          // an absent term is +0: fi + 0 is fi
+          const double t = (act && k < e && k != i && r2 > 0.0) ? q.w / r2 : 0.0;
+          fi += quad_read<0>(t);
+          fi += quad_read<1>(t);
+          fi += quad_read<2>(t);
+          fi += quad_read<3>(t);
         }
       }
-      cur = c.rope[cur];
-    } else {
-      const double cxv = c.cx[cur], cyv = c.cy[cur], czv = c.cz[cur];
-      const double rh = c.rho[cur], ms = c.mass[cur];
-      const int rope = c.rope[cur];
-      bool open = false;
-      if (act && virt) {
-        open = true;  // a virtual cell on the way to the lane's system root
-      } else if (act) {
-        double dx = px - cxv, dy = py - cyv, dz = pz - czv;
-        double d2 = dx * dx + dy * dy + dz * dz;
-        if (d2 > rh * rh) {
-          fi += ms / d2;
-          resume = rope;
-        } else {
-          open = true;
-        }
+    } else if (act && virt) {
+      open = true;  // a virtual cell on the way to the body's system root
+    } else if (act) {
+      const double dx = px - r.cx, dy = py - r.cy, dz = pz - r.cz;
+      const double d2 = dx * dx + dy * dy + dz * dz;
+      if (d2 > r.rho2) {
+        fi += r.mass / d2;
+        resume = rope;
+      } else {
+        open = true;
       }
-      cur = __ballot(open) ? c.last_child[cur] : rope;
     }
+    const bool down = __ballot(open) != 0;
+    cur = down ? last : rope;
+    if (cur < 0) break;
+    if (down)
+      r = r_last;
+    else
+      r = r_rope;
   }
-  if (valid) f[i] = fi;
+  if (valid && sub == 0) f[i] = fi;
 }
 
-void launch_fprepass(uint32_t n, uint32_t nc, DevCells c, DevBodies b,
+// Four lanes per body while all those waves are resident at once (8192: 256
+// CUs x 32); past that the extra waves only queue. SUB = 4 against 1: 1k 0.10
+// and 0.21 ms, 16k 0.24 and 0.50, 250k 0.76 and 0.71, 1M 3.40 and 1.77.
+constexpr uint32_t FP_SUB4_N = 8192 * 16;
+
+size_t fp_rec_bytes() { return sizeof(FpRec); }
+
+void launch_pack_fp(uint32_t nc, DevCells c, void* rec, hipStream_t s) {
+  if (nc == 0) return;
+  hipLaunchKernelGGL(k_pack_fp, dim3((nc + 255) / 256), dim3(256), 0, s, nc, c, (FpRec*)rec);
+}
+
+void launch_fprepass(uint32_t n, uint32_t nc, const void* rec, const double4* body,
                      const uint64_t* keys_sorted, int vlev, double* f, hipStream_t s) {
-  FpCells fc{c.leaf, c.first, c.count, c.cx, c.cy, c.cz, c.rho, c.mass, c.rope, c.last_child,
-             c.level};
-  hipLaunchKernelGGL(k_fprepass, dim3((n + 63) / 64), dim3(64), 0, s, n, nc + 1, fc, b.x, b.y, b.z,
-                     b.m, keys_sorted, vlev, f);
+  if (n <= FP_SUB4_N)
+    hipLaunchKernelGGL(k_fprepass<4>, dim3((n + 15) / 16), dim3(64), 0, s, n, nc + 1,
+                       (const FpRec*)rec, body, keys_sorted, vlev, f);
+  else
+    hipLaunchKernelGGL(k_fprepass<1>, dim3((n + 63) / 64), dim3(64), 0, s, n, nc + 1,
+                       (const FpRec*)rec, body, keys_sorted, vlev, f);
 }
 
 // fmin (mac.rs:151-173), one level at a time, deepest first.
