@@ -59,6 +59,9 @@ struct Budget {
   size_t limit;
 };
 
+// The build's flag words: [0] non-finite input, [4..] cells per level.
+constexpr size_t TREE_FLAGS = 4 + TREE_HIST;
+
 }  // namespace
 
 struct fmmh_ctx {
@@ -96,16 +99,14 @@ struct fmmh_ctx {
   Buf bx, by, bz, bm, bxyzm;
   Buf bpack;  // (x, y, z, m) in id order, written with the keys for the gather
   Buf bbox_partial, bbox, flags;
-  Buf chain, top, cstart;
-  Buf bfs_first, bfs_count, bfs_parent, bfs_oct, bfs_level, bfs_dfs, nchild, child_off;
+  Buf chain, cstart;  // per slot: cells starting there, and their scan
   Buf c_first, c_count, c_children, c_parent, c_leaf, c_level, c_cx, c_cy, c_cz, c_mass, c_rho,
       c_rope, c_last;
-  Buf lvl_cells, leaf_flags, leaf_off, leaf_ids, leaf_of_slot;
-  Buf int_pos, int_cells, lvl_dev;  // internal cells per level (BFS order)
-  Buf split_bnd;                    // octant boundaries of a level's cells (9 words each)
-  Buf leaf_bc, lbc_keys, lbc_keys_alt;  // leaves ordered by body count
+  Buf lvl_cells;  // cells by level, a level's internal cells first
+  Buf leaf_ids, leaf_of_slot;
+  Buf leaf_bc;    // leaves ordered by body count
   Buf cpm;                              // {cx, cy, cz, mass} per cell
-  std::vector<uint32_t> int_off;   // level L's internal cells: [int_off[L], int_off[L+1])
+  std::vector<uint32_t> n_int;     // internal cells per level
   Buf scan_tmp, sort_tmp;
   Buf fprec;  // f pre-pass cell records
   Buf moments, locals, pows, fvals, fmin, fact, binom;
@@ -128,11 +129,10 @@ struct fmmh_ctx {
 
   fmmh_ctx() {
     Buf* all[] = {&in_pos, &in_mass, &out_acc, &out_pot, &keys, &keys_alt, &vals, &vals_alt,
-                  &bx, &by, &bz, &bm, &bxyzm, &bpack, &bbox_partial, &bbox, &flags, &chain, &top, &cstart,
-                  &bfs_first, &bfs_count, &bfs_parent, &bfs_oct, &bfs_level, &bfs_dfs, &nchild,
-                  &child_off, &c_first, &c_count, &c_children, &c_parent, &c_leaf, &c_level,
+                  &bx, &by, &bz, &bm, &bxyzm, &bpack, &bbox_partial, &bbox, &flags, &chain, &cstart,
+                  &c_first, &c_count, &c_children, &c_parent, &c_leaf, &c_level,
                   &c_cx, &c_cy, &c_cz, &c_mass, &c_rho, &c_rope, &c_last, &lvl_cells,
-                  &leaf_flags, &leaf_off, &leaf_ids, &leaf_of_slot, &int_pos, &int_cells, &lvl_dev, &split_bnd, &leaf_bc, &lbc_keys, &lbc_keys_alt, &cpm,
+                  &leaf_ids, &leaf_of_slot, &leaf_bc, &cpm,
                   &scan_tmp, &sort_tmp,
                   &fprec, &moments, &locals, &pows, &fvals, &fmin, &fact, &binom, &front_a, &front_b,
                   &m2l, &p2p, &ctr, &mkeys, &mkeys_alt, &tptr, &pkeys, &pkeys_alt, &pptr, &list_tot,
@@ -224,22 +224,8 @@ struct fmmh_ctx {
   DevBodies bodies() {
     return DevBodies{(double*)bx.p, (double*)by.p, (double*)bz.p, (double*)bm.p, (double4*)bxyzm.p};
   }
-  DevBfs bfs() {
-    return DevBfs{(uint32_t*)bfs_first.p, (uint32_t*)bfs_count.p, (int32_t*)bfs_parent.p,
-                  (uint8_t*)bfs_oct.p,    (uint8_t*)bfs_level.p,  (uint32_t*)bfs_dfs.p};
-  }
-
-  void ensure_bfs(size_t cap, bool keep) {
-    ensure(bfs_first, cap * 4, keep);
-    ensure(bfs_count, cap * 4, keep);
-    ensure(bfs_parent, cap * 4, keep);
-    ensure(bfs_oct, cap, keep);
-    ensure(bfs_level, cap, keep);
-    ensure(bfs_dfs, cap * 4, false);
-  }
-
   void ensure_scan(size_t n_elems) {
-    ensure(scan_tmp, scan_tmp_words(n_elems) * 4 + 64);
+    ensure(scan_tmp, scan_tmp_words(n_elems) * 8 + 64);
   }
 
   // ------------------------------------------------------------------ build
@@ -262,14 +248,13 @@ struct fmmh_ctx {
     ensure(bpack, n * 32);
     ensure(bbox_partial, 6 * 1024 * 8);
     ensure(bbox, nsys * sizeof(BBox));
-    ensure(flags, 64);
-    ensure(chain, n * 4);
-    ensure(top, n);
-    ensure(cstart, n * 4);
+    ensure(flags, TREE_FLAGS * 4);
+    ensure(chain, n * 8);
+    ensure(cstart, n * 8);
     ensure(sort_tmp, radix_tmp_words(n) * 4 + 64);
     ensure_scan(n);
     mark(ST_TREE);
-    HCHECK(hipMemsetAsync(flags.p, 0, 64, s));
+    HCHECK(hipMemsetAsync(flags.p, 0, TREE_FLAGS * 4, s));
     uint64_t* off = nullptr;
     if (nsys == 1) {
       launch_bbox(pos, n, (double*)bbox_partial.p, (BBox*)bbox.p, s);
@@ -302,40 +287,26 @@ struct fmmh_ctx {
       }
     }
     launch_gather_packed((const double4*)bpack.p, order, n, bodies(), s);
-    // level-by-level octant splits
-    HCHECK(hipMemsetAsync(chain.p, 0, n * 4, s));
-    HCHECK(hipMemsetAsync(top.p, 0, n, s));
-    size_t cap = std::max<size_t>(1024, 4 * (n / std::max(1, prm.n_leaf)) + 64);
-    ensure_bfs(cap, false);
-    ensure(nchild, cap * 4);
-    ensure(child_off, cap * 4);
-    launch_tree_init(bfs(), n, (uint32_t*)chain.p, (uint8_t*)top.p, s);
-    if (read1((const uint32_t*)flags.p) != 0) throw int(FMMH_E_NONFINITE);
-    lvl_off.assign({0u, 1u});
-    for (int L = 0;; L++) {
-      uint32_t s0 = lvl_off[L], cnt = lvl_off[L + 1] - s0;
-      ensure(nchild, (size_t)cnt * 4);
-      ensure(child_off, (size_t)cnt * 4);
-      ensure(split_bnd, (size_t)cnt * 36);
-      ensure_scan(cnt);
-      launch_split_count(bfs(), s0, cnt, keys_sorted, (uint32_t)prm.n_leaf, vlev,
-                         (uint32_t*)nchild.p, (uint32_t*)split_bnd.p, s);
-      uint32_t* tot = nullptr;
-      scan_exclusive_u32((uint32_t*)nchild.p, (uint32_t*)child_off.p, cnt, (uint32_t*)scan_tmp.p, s,
-                         &tot);
-      uint32_t total = read1(tot);
-      if (total == 0) break;
-      size_t need = (size_t)lvl_off[L + 1] + total;
-      if (need > bfs_first.cap / 4) ensure_bfs(need + need / 2, true);
-      launch_split_emit(bfs(), s0, cnt, lvl_off[L + 1], (uint32_t)prm.n_leaf, vlev,
-                        (uint32_t*)split_bnd.p, (uint32_t*)child_off.p, (uint32_t*)chain.p,
-                        (uint8_t*)top.p, s);
-      lvl_off.push_back((uint32_t)need);
+    // cells per slot and per level, one host read for the lot
+    uint32_t* fl = (uint32_t*)flags.p;
+    launch_chain(keys_sorted, n, (uint32_t)prm.n_leaf, vlev, (uint64_t*)chain.p, fl + 4, s);
+    uint64_t* tot = nullptr;
+    scan_exclusive_u64((uint64_t*)chain.p, (uint64_t*)cstart.p, n, (uint64_t*)scan_tmp.p, s, &tot);
+    uint32_t* h = (uint32_t*)host_stage(TREE_FLAGS * 4);
+    HCHECK(hipMemcpyAsync(h, fl, TREE_FLAGS * 4, hipMemcpyDeviceToHost, s));
+    HCHECK(hipStreamSynchronize(s));
+    if (h[0] != 0) throw int(FMMH_E_NONFINITE);
+    const uint32_t* hist = h + 4;
+    lvl_off.assign(1, 0u);
+    n_int.clear();
+    nleaves = 0;
+    for (int L = 0; 2 * L < TREE_HIST && hist[2 * L] + hist[2 * L + 1] > 0; L++) {
+      n_int.push_back(hist[2 * L]);
+      nleaves += hist[2 * L + 1];
+      lvl_off.push_back(lvl_off.back() + hist[2 * L] + hist[2 * L + 1]);
     }
     nc = lvl_off.back();
     max_level = (uint32_t)lvl_off.size() - 2;
-    scan_exclusive_u32((uint32_t*)chain.p, (uint32_t*)cstart.p, n, (uint32_t*)scan_tmp.p, s, nullptr);
-    launch_dfs_ids(bfs(), nc, (uint32_t*)cstart.p, (uint8_t*)top.p, s);
     ensure(c_first, nc * 4);
     ensure(c_count, nc * 4);
     ensure(c_children, (size_t)nc * 32);
@@ -350,36 +321,22 @@ struct fmmh_ctx {
     ensure(c_rope, nc * 4);
     ensure(c_last, nc * 4);
     ensure(lvl_cells, nc * 4);
-    ensure(leaf_flags, nc * 4);
-    ensure(leaf_off, nc * 4);
-    ensure(leaf_ids, nc * 4);
+    ensure(leaf_ids, (size_t)nleaves * 4);
+    ensure(leaf_bc, (size_t)nleaves * 4);
     ensure(leaf_of_slot, n * 4);
-    ensure_scan(nc);
-    HCHECK(hipMemsetAsync(c_children.p, 0xFF, (size_t)nc * 32, s));
-    launch_scatter_cells(bfs(), nc, (uint32_t)prm.n_leaf, vlev, cells(), (uint32_t*)lvl_cells.p, s);
-    launch_leaf_flags(cells(), nc, (uint32_t*)leaf_flags.p, s);
-    uint32_t* tot = nullptr;
-    scan_exclusive_u32((uint32_t*)leaf_flags.p, (uint32_t*)leaf_off.p, nc, (uint32_t*)scan_tmp.p, s,
-                       &tot);
-    launch_leaf_compact(cells(), nc, (uint32_t*)leaf_off.p, (uint32_t*)leaf_ids.p,
-                        (uint32_t*)leaf_of_slot.p, s);
-    nleaves = read1(tot);
-    internal_lists();
-    ensure(leaf_bc, (size_t)nleaves * 4 + 4);
-    ensure(lbc_keys, (size_t)nleaves * 8 + 8);
-    ensure(lbc_keys_alt, (size_t)nleaves * 8 + 8);
-    ensure(sort_tmp, radix_tmp_words(nleaves) * 4 + 64);
-    launch_leaves_by_count((uint32_t*)leaf_ids.p, nleaves, cells(), (uint64_t*)lbc_keys.p,
-                           (uint64_t*)lbc_keys_alt.p, (uint32_t*)sort_tmp.p, (uint32_t*)leaf_bc.p,
-                           s);
+    ensure(sort_tmp, radix_tmp_words(nc) * 4 + 64);
+    launch_cells(keys_sorted, n, (const uint64_t*)chain.p, (const uint64_t*)cstart.p, nc, cells(),
+                 (uint32_t*)leaf_ids.p, (uint32_t*)leaf_of_slot.p, s);
+    cells_by_level((const uint8_t*)c_level.p, (const uint8_t*)c_leaf.p, nc, (uint32_t*)lvl_cells.p,
+                   (uint32_t*)sort_tmp.p, s);
+    leaves_by_count((const uint32_t*)leaf_ids.p, (const uint32_t*)c_count.p, nleaves,
+                    (uint32_t*)leaf_bc.p, (uint32_t*)sort_tmp.p, s);
     // geometry: every leaf at once (from its bodies), then internal cells
     // bottom-up level by level (from their children)
     launch_geometry_leaves((uint32_t*)leaf_ids.p, nleaves, cells(), bodies(), prm.center_mode, s);
     for (int L = (int)max_level - 1; L >= 0; L--)
-      launch_geometry((uint32_t*)lvl_cells.p + lvl_off[L], lvl_off[L + 1] - lvl_off[L], cells(),
-                      bodies(), prm.center_mode, s, 2);
-    for (int L = 0; L <= (int)max_level; L++)
-      launch_ropes((uint32_t*)lvl_cells.p + lvl_off[L], lvl_off[L + 1] - lvl_off[L], cells(), s);
+      launch_geometry(int_cells(L), n_int[L], cells(), prm.center_mode, s);
+    launch_ropes(nc, cells(), s);
     ensure(walkrec, (size_t)nc * walk_rec_bytes());
     ensure(cpm, (size_t)nc * sizeof(double4));
     launch_pack_walk(nc, cells(), walkrec.p, (double4*)cpm.p, s);
@@ -388,27 +345,9 @@ struct fmmh_ctx {
     built = true;
   }
 
-  // Internal cells of each level, for the per-level upward kernels.
-  void internal_lists() {
-    ensure(int_pos, (size_t)nc * 4);
-    ensure(int_cells, (size_t)nc * 4);
-    launch_internal_flags((uint32_t*)lvl_cells.p, nc, cells(), (uint32_t*)leaf_flags.p, s);
-    uint32_t* itot = nullptr;
-    scan_exclusive_u32((uint32_t*)leaf_flags.p, (uint32_t*)int_pos.p, nc, (uint32_t*)scan_tmp.p, s,
-                       &itot);
-    launch_internal_compact((uint32_t*)lvl_cells.p, nc, cells(), (uint32_t*)int_pos.p,
-                            (uint32_t*)int_cells.p, s);
-    const uint32_t nl = (uint32_t)lvl_off.size();
-    ensure(lvl_dev, (size_t)nl * 8);
-    uint32_t* h = (uint32_t*)host_stage((size_t)nl * 4);
-    std::memcpy(h, lvl_off.data(), (size_t)nl * 4);
-    HCHECK(hipMemcpyAsync(lvl_dev.p, h, (size_t)nl * 4, hipMemcpyHostToDevice, s));
-    launch_level_pick((uint32_t*)int_pos.p, itot, nc, (uint32_t*)lvl_dev.p, nl,
-                      (uint32_t*)lvl_dev.p + nl, s);
-    HCHECK(hipMemcpyAsync(h, (uint32_t*)lvl_dev.p + nl, (size_t)nl * 4, hipMemcpyDeviceToHost, s));
-    HCHECK(hipStreamSynchronize(s));
-    int_off.assign(h, h + nl);
-  }
+  // Internal cells of a level, for the per-level kernels (n_int[L] of them):
+  // the first of the level's cells in lvl_cells.
+  const uint32_t* int_cells(int L) const { return (const uint32_t*)lvl_cells.p + lvl_off[L]; }
 
   // --------------------------------------------------------------- evaluate
   // Lists of the last full evaluation, kept for frozen evaluations until the
@@ -437,26 +376,25 @@ struct fmmh_ctx {
       launch_m2l_scale(nc, c, (const BBox*)bbox.p, keys_sorted, vlev, lam, s);
       launch_p2m32(p, (uint32_t*)leaf_bc.p, nleaves, c, b, lam, m32, s);
       for (int L = (int)max_level - 1; L >= ltop; L--)
-        launch_m2m32(p, (uint32_t*)int_cells.p + int_off[L], int_off[L + 1] - int_off[L], c, lam,
+        launch_m2m32(p, int_cells(L), n_int[L], c, lam,
                      m32, s);
       launch_m32_to_f64(p, nc, c, ltop, lam, m32, mom, s);  // children of the top levels
       for (int L = std::min(ltop, (int)max_level) - 1; L >= 0; L--)
-        launch_m2m(p, (uint32_t*)int_cells.p + int_off[L], int_off[L + 1] - int_off[L], c, mom, s);
+        launch_m2m(p, int_cells(L), n_int[L], c, mom, s);
     } else if (p <= TEMPLATED_MAX_P) {
       launch_p2m(p, (uint32_t*)leaf_bc.p, nleaves, c, b, mom, s);
       for (int L = (int)max_level - 1; L >= 0; L--)
-        launch_m2m(p, (uint32_t*)int_cells.p + int_off[L], int_off[L + 1] - int_off[L], c, mom, s);
+        launch_m2m(p, int_cells(L), n_int[L], c, mom, s);
     } else {
       launch_p2m_gen(p, (uint32_t*)leaf_ids.p, nleaves, c, b, mom, s);
       for (int L = (int)max_level - 1; L >= 0; L--)
-        launch_m2m_gen(p, (uint32_t*)lvl_cells.p + lvl_off[L], lvl_off[L + 1] - lvl_off[L], c, mom,
-                       s);
+        launch_m2m_gen(p, int_cells(L), n_int[L], c, mom, s);
     }
     if (prm.softening > 0.0) {  // trace moments of the softened far field
       double* q = (double*)ctrace.p;
       launch_trace_leaf((uint32_t*)leaf_ids.p, nleaves, c, b, q, s);
       for (int L = (int)max_level - 1; L >= 0; L--)
-        launch_trace_up((uint32_t*)int_cells.p + int_off[L], int_off[L + 1] - int_off[L], c, p, mom,
+        launch_trace_up(int_cells(L), n_int[L], c, p, mom,
                         q, s, up32() ? m2l_m32.p : nullptr, (const double*)m2l_lam.p,
                         vlev + FP64_TOP);
     }

@@ -15,7 +15,17 @@ namespace fmmh {
 size_t scan_tmp_words(size_t n);
 void scan_exclusive_u32(const uint32_t* in, uint32_t* out, size_t n, uint32_t* tmp,
                         hipStream_t s, uint32_t** total_dev);
+// The same for two u32 counts packed in a u64 (tmp: scan_tmp_words(n) u64).
+void scan_exclusive_u64(const uint64_t* in, uint64_t* out, size_t n, uint64_t* tmp, hipStream_t s,
+                        uint64_t** total_dev);
 size_t radix_tmp_words(size_t n);
+// Cell ids ordered by level, each level's internal cells before its leaves
+// (both in id order); leaf ids ordered by body count (up to 255). tmp:
+// radix_tmp_words(n).
+void cells_by_level(const uint8_t* level, const uint8_t* leaf, uint32_t nc, uint32_t* out,
+                    uint32_t* tmp, hipStream_t s);
+void leaves_by_count(const uint32_t* leaf_ids, const uint32_t* count, uint32_t nleaves,
+                     uint32_t* out, uint32_t* tmp, hipStream_t s);
 int radix_sort_u64(uint64_t* keys, uint32_t* vals, uint64_t* k_alt, uint32_t* v_alt, size_t n,
                    int bit_lo, int bit_hi, uint32_t* tmp, hipStream_t s);
 // Directed entries of undirected pairs (x, y): 2i -> (y << sbits | x), 2i+1
@@ -49,16 +59,6 @@ struct DevBodies {  // slot (Morton) order, bodies.rs:13-22
   double4* xyzm;  // the same bodies interleaved (one 32-byte load per body)
 };
 
-// BFS (level-order) scratch of the tree build.
-struct DevBfs {
-  uint32_t* first;
-  uint32_t* count;
-  int32_t* parent;  // BFS index of the parent
-  uint8_t* oct;
-  uint8_t* level;
-  uint32_t* dfs;    // DFS id of each BFS cell
-};
-
 // -------------------------------------------------------------- tree.hip
 void launch_bbox(const double* pos, size_t n, double* partial, BBox* out, hipStream_t s);
 // Ensembles of nsys systems (body ranges off[s]..off[s+1], device array).
@@ -78,35 +78,22 @@ void launch_gather(const double* pos, const double* mass, const uint32_t* order,
                    DevBodies b, hipStream_t s);
 void launch_gather_packed(const double4* pk, const uint32_t* order, size_t n, DevBodies b,
                           hipStream_t s);
-void launch_tree_init(DevBfs bfs, size_t n, uint32_t* chain, uint8_t* top, hipStream_t s);
-void launch_split_count(DevBfs bfs, uint32_t s0, uint32_t cnt, const uint64_t* keys,
-                        uint32_t n_leaf, int vlev, uint32_t* nchild, uint32_t* bounds,
-                        hipStream_t s);
-void launch_split_emit(DevBfs bfs, uint32_t s0, uint32_t cnt, uint32_t e0, uint32_t n_leaf,
-                       int vlev, const uint32_t* bounds, const uint32_t* child_off,
-                       uint32_t* chain, uint8_t* top, hipStream_t s);
-void launch_dfs_ids(DevBfs bfs, uint32_t nc, const uint32_t* cstart, const uint8_t* top,
-                    hipStream_t s);
-void launch_scatter_cells(DevBfs bfs, uint32_t nc, uint32_t n_leaf, int vlev, DevCells c,
-                          uint32_t* lvl_cells, hipStream_t s);
-// which = 0: all cells of the list, 1: its leaves only, 2: its internal cells only.
+// Cells of the sorted keys: chain[i] = cells starting at slot i << 32 | (any
+// ? 1 : 0), hist[2 level + leaf] = cells per level (zeroed by the caller); then,
+// with start = the exclusive scan of chain, every cell's first, count, level,
+// leaf, parent and children, the leaf ids in slot order and each slot's leaf.
+constexpr int TREE_HIST = 2 * 22;
+void launch_chain(const uint64_t* keys, size_t n, uint32_t n_leaf, int vlev, uint64_t* chain,
+                  uint32_t* hist, hipStream_t s);
+void launch_cells(const uint64_t* keys, size_t n, const uint64_t* chain, const uint64_t* start,
+                  uint32_t nc, DevCells c, uint32_t* leaf_ids, uint32_t* leaf_of_slot,
+                  hipStream_t s);
 void launch_geometry_leaves(const uint32_t* leaf_ids, uint32_t nleaves, DevCells c, DevBodies b,
                             int center_mode, hipStream_t s);
-void launch_geometry(const uint32_t* lvl_cells, uint32_t cnt, DevCells c, DevBodies b,
-                     int center_mode, hipStream_t s, int which);
-void launch_ropes(const uint32_t* lvl_cells, uint32_t cnt, DevCells c, hipStream_t s);
-void launch_leaf_flags(DevCells c, uint32_t nc, uint32_t* flags, hipStream_t s);
-void launch_leaves_by_count(const uint32_t* leaf_ids, uint32_t nleaves, DevCells c,
-                            uint64_t* keys, uint64_t* keys_alt, uint32_t* tmp, uint32_t* out,
-                            hipStream_t s);
-void launch_internal_flags(const uint32_t* lvl_cells, uint32_t nc, DevCells c, uint32_t* flags,
-                           hipStream_t s);
-void launch_internal_compact(const uint32_t* lvl_cells, uint32_t nc, DevCells c,
-                             const uint32_t* pos, uint32_t* out, hipStream_t s);
-void launch_level_pick(const uint32_t* pos, const uint32_t* total, uint32_t nc, const uint32_t* at,
-                       uint32_t nl, uint32_t* out, hipStream_t s);
-void launch_leaf_compact(DevCells c, uint32_t nc, const uint32_t* off, uint32_t* leaf_ids,
-                         uint32_t* leaf_of_slot, hipStream_t s);
+// Internal cells of one level, their children done.
+void launch_geometry(const uint32_t* cells, uint32_t cnt, DevCells c, int center_mode,
+                     hipStream_t s);
+void launch_ropes(uint32_t nc, DevCells c, hipStream_t s);
 
 // ------------------------------------------------------------ upward.hip
 bool launch_p2m(int p, const uint32_t* leaf_ids, uint32_t nleaves, DevCells c, DevBodies b,

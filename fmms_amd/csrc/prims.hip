@@ -1,5 +1,5 @@
 // prims.hip — HBM-bound primitives for gfx950: device-wide exclusive scan
-// (u32) and a stable LSD radix sort of (u64 key, u32 value) pairs.
+// (u32, and two packed counts) and a stable LSD radix sort of (u64 key, u32 value) pairs.
 //
 // Radix sort: digits of up to 8 bits, as even as the passes allow (19 target
 // bits as 7 + 7 + 5), tiles of 2048 elements per 256-thread block (4 waves x
@@ -24,16 +24,22 @@ constexpr int SCAN_I = 16;
 constexpr int SCAN_TILE = SCAN_T * SCAN_I;
 
 // Block-wide exclusive scan of one value per thread (256 threads).
-__device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* total, uint32_t* sh) {
+template <class T>
+__device__ __forceinline__ T block_excl_scan(T v, T* total, T* sh) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  uint32_t wt;
-  uint32_t x = wave_excl_scan(v, &wt);
-  if (lane == 0) sh[w] = wt;
+  T x = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const T y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) sh[w] = x;
+  x -= v;
   __syncthreads();
-  uint32_t off = 0, tot = 0;
+  T off = 0, tot = 0;
 #pragma unroll
   for (int i = 0; i < SCAN_T / 64; i++) {
-    uint32_t s = sh[i];
+    T s = sh[i];
     if (i < w) off += s;
     tot += s;
   }
@@ -42,27 +48,28 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* total,
   return x + off;
 }
 
-__global__ void __launch_bounds__(SCAN_T) k_scan_tiles(const uint32_t* __restrict__ in,
-                                                      uint32_t* __restrict__ out, size_t n,
-                                                      uint32_t* __restrict__ tile_sums) {
-  __shared__ uint32_t tile[SCAN_TILE];
-  __shared__ uint32_t sh[SCAN_T / 64];
+template <class T>
+__global__ void __launch_bounds__(SCAN_T) k_scan_tiles(const T* __restrict__ in,
+                                                      T* __restrict__ out, size_t n,
+                                                      T* __restrict__ tile_sums) {
+  __shared__ T tile[SCAN_TILE];
+  __shared__ T sh[SCAN_T / 64];
   const size_t base = (size_t)blockIdx.x * SCAN_TILE;
 #pragma unroll
   for (int j = 0; j < SCAN_I; j++) {
     size_t e = base + (size_t)j * SCAN_T + threadIdx.x;
-    tile[j * SCAN_T + threadIdx.x] = e < n ? in[e] : 0u;
+    tile[j * SCAN_T + threadIdx.x] = e < n ? in[e] : T(0);
   }
   __syncthreads();
-  uint32_t v[SCAN_I];
-  uint32_t s = 0;
+  T v[SCAN_I];
+  T s = 0;
 #pragma unroll
   for (int j = 0; j < SCAN_I; j++) {
     v[j] = s;
     s += tile[threadIdx.x * SCAN_I + j];
   }
-  uint32_t total;
-  uint32_t off = block_excl_scan(s, &total, sh);
+  T total;
+  T off = block_excl_scan(s, &total, sh);
 #pragma unroll
   for (int j = 0; j < SCAN_I; j++) tile[threadIdx.x * SCAN_I + j] = v[j] + off;
   __syncthreads();
@@ -76,23 +83,25 @@ __global__ void __launch_bounds__(SCAN_T) k_scan_tiles(const uint32_t* __restric
 }
 
 // One block scans the tile sums in place; tile_sums[ntiles] = grand total.
-__global__ void __launch_bounds__(SCAN_T) k_scan_sums(uint32_t* __restrict__ sums, size_t ntiles) {
-  __shared__ uint32_t sh[SCAN_T / 64];
-  uint32_t carry = 0;
+template <class T>
+__global__ void __launch_bounds__(SCAN_T) k_scan_sums(T* __restrict__ sums, size_t ntiles) {
+  __shared__ T sh[SCAN_T / 64];
+  T carry = 0;
   for (size_t b = 0; b < ntiles; b += SCAN_T) {
     size_t e = b + threadIdx.x;
-    uint32_t v = e < ntiles ? sums[e] : 0u;
-    uint32_t total;
-    uint32_t x = block_excl_scan(v, &total, sh);
+    T v = e < ntiles ? sums[e] : T(0);
+    T total;
+    T x = block_excl_scan(v, &total, sh);
     if (e < ntiles) sums[e] = x + carry;
     carry += total;
   }
   if (threadIdx.x == 0) sums[ntiles] = carry;
 }
 
-__global__ void __launch_bounds__(SCAN_T) k_scan_add(uint32_t* __restrict__ out, size_t n,
-                                                    const uint32_t* __restrict__ sums) {
-  const uint32_t add = sums[blockIdx.x];
+template <class T>
+__global__ void __launch_bounds__(SCAN_T) k_scan_add(T* __restrict__ out, size_t n,
+                                                    const T* __restrict__ sums) {
+  const T add = sums[blockIdx.x];
   const size_t base = (size_t)blockIdx.x * SCAN_TILE;
   if (add == 0) return;
 #pragma unroll
@@ -105,12 +114,13 @@ __global__ void __launch_bounds__(SCAN_T) k_scan_add(uint32_t* __restrict__ out,
 // Up to SCAN_T tiles: each block adds the totals of the tiles before it
 // (one per thread, then a block sum), so no separate pass scans the tile
 // totals; the last block stores the grand total in sums[ntiles].
-__global__ void __launch_bounds__(SCAN_T) k_scan_add_small(uint32_t* __restrict__ out, size_t n,
-                                                          uint32_t* __restrict__ sums,
+template <class T>
+__global__ void __launch_bounds__(SCAN_T) k_scan_add_small(T* __restrict__ out, size_t n,
+                                                          T* __restrict__ sums,
                                                           uint32_t ntiles) {
-  __shared__ uint32_t sh[SCAN_T / 64];
-  const uint32_t v = threadIdx.x < blockIdx.x ? sums[threadIdx.x] : 0u;
-  uint32_t add;
+  __shared__ T sh[SCAN_T / 64];
+  const T v = threadIdx.x < blockIdx.x ? sums[threadIdx.x] : T(0);
+  T add;
   block_excl_scan(v, &add, sh);
   if (blockIdx.x == ntiles - 1 && threadIdx.x == 0) sums[ntiles] = add + sums[ntiles - 1];
   if (add == 0) return;
@@ -124,24 +134,36 @@ __global__ void __launch_bounds__(SCAN_T) k_scan_add_small(uint32_t* __restrict_
 
 size_t scan_tmp_words(size_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE + 1; }
 
-// Exclusive scan; in may equal out. tmp needs scan_tmp_words(n) words; the
+// Exclusive scan; in may equal out. tmp needs scan_tmp_words(n) elements; the
 // grand total lands in tmp[ntiles] (device) and *total_dev points at it.
-void scan_exclusive_u32(const uint32_t* in, uint32_t* out, size_t n, uint32_t* tmp,
-                        hipStream_t s, uint32_t** total_dev) {
+template <class T>
+static void scan_exclusive(const T* in, T* out, size_t n, T* tmp, hipStream_t s, T** total_dev) {
   size_t ntiles = (n + SCAN_TILE - 1) / SCAN_TILE;
   if (ntiles == 0) {
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_T), 0, s, tmp, (size_t)0);
+    hipLaunchKernelGGL(k_scan_sums<T>, dim3(1), dim3(SCAN_T), 0, s, tmp, (size_t)0);
   } else {
-    hipLaunchKernelGGL(k_scan_tiles, dim3(ntiles), dim3(SCAN_T), 0, s, in, out, n, tmp);
+    hipLaunchKernelGGL(k_scan_tiles<T>, dim3(ntiles), dim3(SCAN_T), 0, s, in, out, n, tmp);
     if (ntiles > (size_t)SCAN_T) {
-      hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_T), 0, s, tmp, ntiles);
-      hipLaunchKernelGGL(k_scan_add, dim3(ntiles), dim3(SCAN_T), 0, s, out, n, tmp);
+      hipLaunchKernelGGL(k_scan_sums<T>, dim3(1), dim3(SCAN_T), 0, s, tmp, ntiles);
+      hipLaunchKernelGGL(k_scan_add<T>, dim3(ntiles), dim3(SCAN_T), 0, s, out, n, tmp);
     } else if (ntiles > 1) {
-      hipLaunchKernelGGL(k_scan_add_small, dim3(ntiles), dim3(SCAN_T), 0, s, out, n, tmp,
+      hipLaunchKernelGGL(k_scan_add_small<T>, dim3(ntiles), dim3(SCAN_T), 0, s, out, n, tmp,
                          (uint32_t)ntiles);
     }
   }
   if (total_dev) *total_dev = tmp + ntiles;
+}
+
+void scan_exclusive_u32(const uint32_t* in, uint32_t* out, size_t n, uint32_t* tmp,
+                        hipStream_t s, uint32_t** total_dev) {
+  scan_exclusive<uint32_t>(in, out, n, tmp, s, total_dev);
+}
+
+// Two u32 counts per element, packed in the halves of a u64 (neither total
+// reaches 2^32).
+void scan_exclusive_u64(const uint64_t* in, uint64_t* out, size_t n, uint64_t* tmp, hipStream_t s,
+                        uint64_t** total_dev) {
+  scan_exclusive<uint64_t>(in, out, n, tmp, s, total_dev);
 }
 
 // ------------------------------------------------------------ radix sort
@@ -170,6 +192,24 @@ struct DirectedIn {
     if ((e & 1) == 0) return ((uint64_t)pr.y << sbits) | pr.x;
     if (sentinel && pr.x == pr.y) return (1ull << (2 * sbits)) - 1ull;
     return ((uint64_t)pr.x << sbits) | pr.y;
+  }
+};
+
+// Cells by level, internal ones before leaves: (2 level + leaf) << 32 | id.
+struct LevelIn {
+  const uint8_t* level;
+  const uint8_t* leaf;
+  __device__ __forceinline__ uint64_t operator()(size_t e) const {
+    return ((uint64_t)(2u * level[e] + leaf[e]) << 32) | (uint32_t)e;
+  }
+};
+// Leaves by body count (up to 255): count << 32 | cell id.
+struct LeafCountIn {
+  const uint32_t* leaf_ids;
+  const uint32_t* count;
+  __device__ __forceinline__ uint64_t operator()(size_t e) const {
+    const uint32_t id = leaf_ids[e];
+    return ((uint64_t)min(count[id], 255u) << 32) | id;
   }
 };
 
@@ -217,7 +257,13 @@ __global__ void __launch_bounds__(RS_T) k_rs_hist(KS ks, size_t n, int shift, in
 // (stable: wave order, then element order within a wave) and written from
 // LDS in that order, so the global writes of one digit are contiguous runs
 // instead of one line per lane.
-template <class KS, bool VALS>
+// OFFS: where the tile's global digit offsets come from. OFFS_SCAN: offs is the
+// scanned histogram. OFFS_HIST: offs is the histogram itself (few tiles), and
+// each block sums the rows and the counts of the tiles before it. OFFS_ONE: one
+// tile, whose own digit starts they are (no histogram at all).
+// LOW32: only the low 32 bits of the keys are written, to vout.
+enum { OFFS_SCAN = 0, OFFS_HIST = 1, OFFS_ONE = 2 };
+template <class KS, bool VALS, int OFFS, bool LOW32>
 __global__ void __launch_bounds__(RS_T) k_rs_scatter(KS ks, const uint32_t* __restrict__ vin,
                                                     uint64_t* __restrict__ kout,
                                                     uint32_t* __restrict__ vout, size_t n,
@@ -291,15 +337,37 @@ __global__ void __launch_bounds__(RS_T) k_rs_scatter(KS ks, const uint32_t* __re
   }
   __syncthreads();
   // global position of block slot i with digit d: offs[d][tile] + i - dstart[d]
-  for (uint32_t d = threadIdx.x; d < nb; d += RS_T)
-    dstart[d] = offs[(size_t)d * nblk + tile] - dstart[d];
+  if constexpr (OFFS == OFFS_SCAN) {
+    for (uint32_t d = threadIdx.x; d < nb; d += RS_T)
+      dstart[d] = offs[(size_t)d * nblk + tile] - dstart[d];
+  } else if constexpr (OFFS == OFFS_HIST) {
+    const uint32_t d = threadIdx.x;  // RS_NB == RS_T: one digit per thread
+    uint32_t tot = 0, before = 0;
+    if (d < nb) {
+      const uint32_t* row = offs + (size_t)d * nblk;
+#pragma unroll 8
+      for (uint32_t t = 0; t < nblk; t++) {
+        const uint32_t v = row[t];
+        tot += v;
+        before += t < tile ? v : 0u;
+      }
+    }
+    uint32_t all;
+    const uint32_t x = block_excl_scan(tot, &all, shs);
+    if (d < nb) dstart[d] = x + before - dstart[d];
+  } else {
+    for (uint32_t d = threadIdx.x; d < nb; d += RS_T) dstart[d] = 0;  // block order is global order
+  }
   __syncthreads();
   const uint32_t cnt_blk = (uint32_t)min((size_t)RS_TILE, n - bbase);
   for (uint32_t i = threadIdx.x; i < cnt_blk; i += RS_T) {
     const uint64_t key = sk[i];
     const uint32_t d = (uint32_t)(key >> shift) & (nb - 1u);
     const size_t pos = (size_t)(uint32_t)(dstart[d] + i);
-    kout[pos] = key;
+    if (LOW32)
+      vout[pos] = (uint32_t)key;
+    else
+      kout[pos] = key;
     if (VALS) vout[pos] = sv[i];
   }
 }
@@ -310,22 +378,50 @@ size_t radix_tmp_words(size_t n) {
   return h + scan_tmp_words(h);
 }
 
+// Tiles up to which a scatter block sums the histogram itself: 64 words per
+// digit and block (64 KB from L2 at most) cost less than the scan's one or two
+// launches a pass.
+constexpr uint32_t RS_FUSE = 64;
+static_assert(RS_NB == RS_T, "one digit per thread");
+
 // One LSD pass of w bits at `shift`: histogram, scan, scatter.
-template <class KS>
+template <class KS, bool VALS, bool LOW32>
 static void radix_pass(KS ks, const uint32_t* vin, uint64_t* kout, uint32_t* vout, size_t n,
                        int shift, int w, uint32_t* tmp, hipStream_t s) {
   const uint32_t nblk = (uint32_t)((n + RS_TILE - 1) / RS_TILE);
   uint32_t* hist = tmp;
-  const size_t nh = ((size_t)1 << w) * nblk;
-  uint32_t* stmp = tmp + (size_t)RS_NB * nblk;
+  if (nblk == 1) {
+    hipLaunchKernelGGL((k_rs_scatter<KS, VALS, OFFS_ONE, LOW32>), dim3(1), dim3(RS_T), 0, s, ks,
+                       vin, kout, vout, n, shift, w, hist, nblk);
+    return;
+  }
   hipLaunchKernelGGL(k_rs_hist<KS>, dim3(nblk), dim3(RS_T), 0, s, ks, n, shift, w, hist, nblk);
-  scan_exclusive_u32(hist, hist, nh, stmp, s, nullptr);
-  if (vin)
-    hipLaunchKernelGGL((k_rs_scatter<KS, true>), dim3(nblk), dim3(RS_T), 0, s, ks, vin, kout, vout,
-                       n, shift, w, hist, nblk);
-  else
-    hipLaunchKernelGGL((k_rs_scatter<KS, false>), dim3(nblk), dim3(RS_T), 0, s, ks, nullptr, kout,
-                       nullptr, n, shift, w, hist, nblk);
+  if (nblk <= RS_FUSE) {
+    hipLaunchKernelGGL((k_rs_scatter<KS, VALS, OFFS_HIST, LOW32>), dim3(nblk), dim3(RS_T), 0, s,
+                       ks, vin, kout, vout, n, shift, w, hist, nblk);
+    return;
+  }
+  scan_exclusive_u32(hist, hist, ((size_t)1 << w) * nblk, tmp + (size_t)RS_NB * nblk, s, nullptr);
+  hipLaunchKernelGGL((k_rs_scatter<KS, VALS, OFFS_SCAN, LOW32>), dim3(nblk), dim3(RS_T), 0, s, ks,
+                     vin, kout, vout, n, shift, w, hist, nblk);
+}
+
+// One pass over the low `bits` bits of the upper halves of the source's
+// keys; their lower halves come out in that order.
+template <class KS>
+static void radix_order32(KS ks, size_t n, int bits, uint32_t* out, uint32_t* tmp, hipStream_t s) {
+  if (n == 0) return;
+  radix_pass<KS, false, true>(ks, nullptr, nullptr, out, n, 32, bits, tmp, s);
+}
+
+void cells_by_level(const uint8_t* level, const uint8_t* leaf, uint32_t nc, uint32_t* out,
+                    uint32_t* tmp, hipStream_t s) {
+  radix_order32(LevelIn{level, leaf}, nc, 6, out, tmp, s);
+}
+
+void leaves_by_count(const uint32_t* leaf_ids, const uint32_t* count, uint32_t nleaves,
+                     uint32_t* out, uint32_t* tmp, hipStream_t s) {
+  radix_order32(LeafCountIn{leaf_ids, count}, nleaves, 8, out, tmp, s);
 }
 
 // Digit width of the passes over `bits` bits: as few passes as RS_MAXW
@@ -348,7 +444,10 @@ int radix_sort_u64(uint64_t* keys, uint32_t* vals, uint64_t* k_alt, uint32_t* v_
     const uint32_t* vin = vals ? (flip ? v_alt : vals) : nullptr;
     uint64_t* kout = flip ? keys : k_alt;
     uint32_t* vout = flip ? vals : v_alt;
-    radix_pass(KeysIn{kin}, vin, kout, vout, n, shift, wp, tmp, s);
+    if (vals)
+      radix_pass<KeysIn, true, false>(KeysIn{kin}, vin, kout, vout, n, shift, wp, tmp, s);
+    else
+      radix_pass<KeysIn, false, false>(KeysIn{kin}, nullptr, kout, nullptr, n, shift, wp, tmp, s);
     flip ^= 1;
   }
   return flip;
@@ -367,9 +466,11 @@ int radix_sort_directed(const uint2* pairs, uint32_t np, int sbits, bool sentine
     const int wp = std::min(w, 2 * sbits - shift);
     uint64_t* kout = flip ? keys : k_alt;
     if (shift == sbits)
-      radix_pass(DirectedIn{pairs, sbits, sentinel}, nullptr, kout, nullptr, n, shift, wp, tmp, s);
+      radix_pass<DirectedIn, false, false>(DirectedIn{pairs, sbits, sentinel}, nullptr, kout,
+                                           nullptr, n, shift, wp, tmp, s);
     else
-      radix_pass(KeysIn{flip ? k_alt : keys}, nullptr, kout, nullptr, n, shift, wp, tmp, s);
+      radix_pass<KeysIn, false, false>(KeysIn{flip ? k_alt : keys}, nullptr, kout, nullptr, n,
+                                       shift, wp, tmp, s);
     flip ^= 1;
   }
   return flip;

@@ -3,14 +3,21 @@
 // Follows crates/fmm tree.rs:94-227 and reproduces its output bit for bit:
 //   bbox (min/max, order-free) -> 63-bit Morton keys with the reference's
 //   quantiser (every axis measured from the x minimum, tree.rs:37-46) ->
-//   stable LSD radix sort (prims.hip) -> level-by-level octant splits ->
-//   DFS-preorder ids -> geometry in the reference's arithmetic order.
+//   stable LSD radix sort (prims.hip) -> cells straight from the sorted keys
+//   -> geometry in the reference's arithmetic order.
 //
-// DFS preorder without recursion: preorder sorts cells by (first slot,
-// level), because the only cells sharing a first slot form a parent->first-
-// child chain at consecutive levels. So id = (cells whose range starts
-// before `first`) + (level - top level of the chain at `first`); the first
-// term is an exclusive scan over slots of the per-slot chain lengths.
+// The cells need no recursion and no level-by-level pass. A cell is a run of
+// slots sharing a key prefix, and the cells starting at one slot are a
+// parent -> first-child chain over consecutive levels, from the level at
+// which the slot parts from its predecessor to the first level that is not
+// split; a cell splits when it holds more than n_leaf bodies, which for the
+// chain is a comparison with the key n_leaf slots on. DFS preorder sorts
+// cells by (first slot, level), so a cell's id is the number of cells whose
+// range starts before its slot (an exclusive scan of the chain lengths) plus
+// its position in the chain. One host read (the counts per level) replaces
+// one per level: 100k bodies 36 launches and 10 reads -> 7 and 1.
+#include <algorithm>
+
 #include "common.h"
 #include "internal.h"
 
@@ -298,190 +305,173 @@ void launch_gather_packed(const double4* pk, const uint32_t* order, size_t n, De
   hipLaunchKernelGGL(k_gather_packed, dim3((n + TB - 1) / TB), dim3(TB), 0, s, pk, order, n, b);
 }
 
-__global__ void k_tree_init(DevBfs bfs, uint32_t n, uint32_t* chain, uint8_t* top) {
-  if (threadIdx.x != 0) return;
-  bfs.first[0] = 0;
-  bfs.count[0] = n;
-  bfs.parent[0] = -1;
-  bfs.oct[0] = 0;
-  bfs.level[0] = 0;
-  chain[0] = 1;
-  top[0] = 0;
+// Leading octal digits (levels) in which two 63-bit keys agree, 0..21.
+__device__ __forceinline__ int common_levels(uint64_t a, uint64_t b) {
+  const uint64_t x = a ^ b;
+  return x == 0 ? BITS : ((int)__clzll((long long)x) - 1) / 3;
+}
+__device__ __forceinline__ bool same_cell(uint64_t a, uint64_t b, int level) {
+  return ((a ^ b) >> (3 * (BITS - level))) == 0;
 }
 
-void launch_tree_init(DevBfs bfs, size_t n, uint32_t* chain, uint8_t* top, hipStream_t s) {
-  hipLaunchKernelGGL(k_tree_init, dim3(1), dim3(64), 0, s, bfs, (uint32_t)n, chain, top);
-}
-
-// tree.rs:414 leaf rule; the virtual levels of an ensemble (level < vlev,
-// cells holding several systems) always split.
-__device__ __forceinline__ bool is_internal(uint32_t count, int level, uint32_t n_leaf, int vlev) {
-  return level < vlev || !(count <= n_leaf || level >= BITS);
-}
-
-// Octant boundaries of an internal cell (tree.rs:420-443): bnd[o] is the
-// first slot whose octant digit at this level is >= o, so the children are
-// bnd[o]..bnd[o+1]. One wave finds them by a 65-ary search per boundary
-// (64 probes a round, all seven boundaries at once): a cell of N bodies
-// takes about log65(N) rounds of loads instead of 7 log2(N) dependent ones.
-__device__ __forceinline__ void octant_bounds_wave(const uint64_t* __restrict__ keys, uint32_t f,
-                                                   uint32_t c, int level, int lane,
-                                                   uint32_t bnd[9]) {
-  const int shift = 3 * (BITS - (level + 1));
-  uint32_t lo[8], hi[8];
-#pragma unroll
-  for (int o = 1; o < 8; o++) {
-    lo[o] = f;
-    hi[o] = f + c;
-  }
-  // digits are non-decreasing over the cell's slots, so every ballot below
-  // is a prefix of the wave; a round shrinks a bracket of length L > 64 to
-  // at most L/65 + 1 and settles one of length <= 64 (7 rounds cover 2^32)
-  for (int it = 0; it < 8; it++) {
-    bool more = false;
-#pragma unroll
-    for (int o = 1; o < 8; o++) {
-      const uint32_t len = hi[o] - lo[o];
-      if (len == 0) continue;
-      more = true;
-      if (len <= 64) {
-        const bool v = (uint32_t)lane < len;
-        const uint32_t d = v ? (uint32_t)((keys[lo[o] + (uint32_t)lane] >> shift) & 7u) : 8u;
-        lo[o] += (uint32_t)__popcll(__ballot(d < (uint32_t)o));
-        hi[o] = lo[o];
-      } else {
-        const uint32_t q = lo[o] + (uint32_t)(((uint64_t)(lane + 1) * len) / 65u);
-        const uint32_t d = (uint32_t)((keys[q] >> shift) & 7u);
-        const uint32_t t = (uint32_t)__popcll(__ballot(d < (uint32_t)o));
-        const uint32_t nlo = t == 0 ? lo[o] : lo[o] + (uint32_t)(((uint64_t)t * len) / 65u) + 1u;
-        const uint32_t nhi = t == 64 ? hi[o] : lo[o] + (uint32_t)(((uint64_t)(t + 1) * len) / 65u);
-        lo[o] = nlo;
-        hi[o] = nhi;
+// Levels [top, bottom] of the cells starting at slot i (tree.rs:414: a cell
+// splits when it has more than n_leaf bodies and its level is below 21; the
+// virtual levels of an ensemble, level < vlev, always split). top > bottom:
+// none.
+__device__ __forceinline__ void slot_chain(const uint64_t* __restrict__ keys, uint32_t n,
+                                           uint32_t i, uint32_t n_leaf, int vlev, int* top,
+                                           int* bottom) {
+  const uint64_t k = keys[i];
+  int t = 0;
+  if (i > 0) {
+    // the slot starts cells below level q, if the cell of level q that holds
+    // it and its predecessor splits
+    const int q = common_levels(keys[i - 1], k);
+    *top = 1;
+    *bottom = 0;
+    if (q == BITS) return;
+    if (q >= vlev) {
+      // more than n_leaf bodies around slots i - 1 and i: half as many on one
+      // side at least (rejects nearly every slot inside a leaf) ...
+      const uint32_t h = n_leaf - n_leaf / 2;
+      const bool hi = (uint64_t)i + h < n && same_cell(keys[i + h], k, q);
+      const bool lo = i >= h && same_cell(keys[i - h], k, q);
+      if (!hi && !lo) return;
+      // ... and n_leaf slots past the cell's start still in it
+      uint32_t a = i > n_leaf ? i - n_leaf : 0u, b = i;  // start in [a, b] unless before a
+      while (a < b) {
+        const uint32_t mid = a + (b - a) / 2;
+        if (same_cell(keys[mid], k, q))
+          b = mid;
+        else
+          a = mid + 1;
       }
+      if (!((uint64_t)a + n_leaf < n && same_cell(keys[a + n_leaf], k, q))) return;
     }
-    if (!more) break;
+    t = q + 1;
   }
-  bnd[0] = f;
+  const int g = (uint64_t)i + n_leaf < n ? common_levels(k, keys[i + n_leaf]) : -1;
+  *top = t;
+  *bottom = max(max(t, vlev), min(g, BITS - 1) + 1);
+}
+
+// Per slot the cells that start there (count << 32 | 1 if any: each chain
+// ends in exactly one leaf) and per level the internal cells and leaves
+// (hist[2 level + leaf]).
+__global__ void __launch_bounds__(TB) k_chain(const uint64_t* __restrict__ keys, uint32_t n,
+                                             uint32_t n_leaf, int vlev,
+                                             uint64_t* __restrict__ chain,
+                                             uint32_t* __restrict__ hist) {
+  __shared__ uint32_t h[TREE_HIST];
+  for (int q = threadIdx.x; q < TREE_HIST; q += TB) h[q] = 0;
+  __syncthreads();
+  for (uint64_t i = (uint64_t)blockIdx.x * TB + threadIdx.x; i < n; i += (uint64_t)gridDim.x * TB) {
+    int top, bot;
+    slot_chain(keys, n, (uint32_t)i, n_leaf, vlev, &top, &bot);
+    chain[i] = top <= bot ? ((uint64_t)(bot - top + 1) << 32) | 1ull : 0ull;
+    for (int l = top; l <= bot; l++) atomicAdd(&h[2 * l + (l == bot ? 1 : 0)], 1u);
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < TREE_HIST; q += TB)
+    if (h[q]) atomicAdd(&hist[q], h[q]);
+}
+
+void launch_chain(const uint64_t* keys, size_t n, uint32_t n_leaf, int vlev, uint64_t* chain,
+                  uint32_t* hist, hipStream_t s) {
+  const size_t nb = std::min<size_t>((n + TB - 1) / TB, 2048);
+  hipLaunchKernelGGL(k_chain, dim3(nb), dim3(TB), 0, s, keys, (uint32_t)n, n_leaf, vlev, chain,
+                     hist);
+}
+
+// Writes each slot's chain of cells (start = exclusive scan of chain: cells
+// << 32 | leaves before the slot): first slot, level, leaf flag, the links
+// inside the chain, and the leaf list. The chain's top cell gets its parent
+// from k_cell_links.
+__global__ void __launch_bounds__(TB) k_cell_emit(const uint64_t* __restrict__ keys, uint32_t n,
+                                                 const uint64_t* __restrict__ chain,
+                                                 const uint64_t* __restrict__ start, DevCells c,
+                                                 uint32_t* __restrict__ leaf_ids) {
+  const uint32_t i = blockIdx.x * TB + threadIdx.x;
+  if (i >= n) return;
+  const int m = (int)(chain[i] >> 32);
+  if (m == 0) return;
+  const uint64_t k = keys[i];
+  const int top = i == 0 ? 0 : common_levels(keys[i - 1], k) + 1;
+  const uint32_t id0 = (uint32_t)(start[i] >> 32);
+  for (int q = 0; q < m; q++) {
+    const uint32_t id = id0 + (uint32_t)q;
+    c.first[id] = i;
+    c.level[id] = (uint8_t)(top + q);
+    c.leaf[id] = q == m - 1 ? 1 : 0;
+    if (q > 0) c.parent[id] = (int32_t)(id - 1);
+    const int32_t next = q == m - 1 ? -1 : (int32_t)(id + 1);
+    const int oct = (int)((k >> (3 * (BITS - (top + q + 1)))) & 7u);  // unused in a leaf
+    int32_t* ch = c.children + (size_t)id * 8;
 #pragma unroll
-  for (int o = 1; o < 8; o++) bnd[o] = lo[o];
-  bnd[8] = f + c;
-}
-
-constexpr int SPLIT_WAVES = 4;
-
-// One wave per cell of a level: child count and octant boundaries, which
-// are kept (9 words a cell) for k_split_emit.
-__global__ void __launch_bounds__(64 * SPLIT_WAVES) k_split_count(DevBfs bfs, uint32_t s0,
-                                                                uint32_t cnt,
-                                                                const uint64_t* __restrict__ keys,
-                                                                uint32_t n_leaf, int vlev,
-                                                                uint32_t* __restrict__ nchild,
-                                                                uint32_t* __restrict__ bounds) {
-  const uint32_t i = blockIdx.x * SPLIT_WAVES + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (i >= cnt) return;
-  const uint32_t b = s0 + i;
-  const uint32_t f = bfs.first[b], c = bfs.count[b];
-  const int lvl = bfs.level[b];
-  uint32_t k = 0;
-  if (is_internal(c, lvl, n_leaf, vlev)) {
-    uint32_t bnd[9];
-    octant_bounds_wave(keys, f, c, lvl, lane, bnd);
-#pragma unroll
-    for (int o = 0; o < 8; o++) k += bnd[o + 1] > bnd[o] ? 1u : 0u;
-#pragma unroll
-    for (int o = 0; o < 9; o++)
-      if (lane == o) bounds[(size_t)i * 9 + o] = bnd[o];
+    for (int o = 0; o < 8; o++) ch[o] = o == oct ? next : -1;
   }
-  if (lane == 0) nchild[i] = k;
+  leaf_ids[(uint32_t)start[i]] = id0 + (uint32_t)(m - 1);
 }
 
-void launch_split_count(DevBfs bfs, uint32_t s0, uint32_t cnt, const uint64_t* keys,
-                        uint32_t n_leaf, int vlev, uint32_t* nchild, uint32_t* bounds,
-                        hipStream_t s) {
-  hipLaunchKernelGGL(k_split_count, dim3((cnt + SPLIT_WAVES - 1) / SPLIT_WAVES),
-                     dim3(64 * SPLIT_WAVES), 0, s, bfs, s0, cnt, keys, n_leaf, vlev, nchild,
-                     bounds);
-}
-
-__global__ void __launch_bounds__(TB) k_split_emit(DevBfs bfs, uint32_t s0, uint32_t cnt,
-                                                  uint32_t e0, uint32_t n_leaf, int vlev,
-                                                  const uint32_t* __restrict__ bounds,
-                                                  const uint32_t* __restrict__ child_off,
-                                                  uint32_t* __restrict__ chain,
-                                                  uint8_t* __restrict__ top) {
-  uint32_t i = blockIdx.x * TB + threadIdx.x;
-  if (i >= cnt) return;
-  uint32_t b = s0 + i;
-  uint32_t c = bfs.count[b];
-  int lvl = bfs.level[b];
-  if (!is_internal(c, lvl, n_leaf, vlev)) return;
-  const uint32_t* bnd = bounds + (size_t)i * 9;
-  uint32_t w = e0 + child_off[i];
-  for (int o = 0; o < 8; o++) {
-    uint32_t lo = bnd[o], hi = bnd[o + 1];
-    if (hi <= lo) continue;
-    bfs.first[w] = lo;
-    bfs.count[w] = hi - lo;
-    bfs.parent[w] = (int32_t)b;
-    bfs.oct[w] = (uint8_t)o;
-    bfs.level[w] = (uint8_t)(lvl + 1);
-    // Ranges of one level are disjoint, so each slot is touched at most once
-    // per launch; a slot seen for the first time starts a chain here.
-    if (chain[lo] == 0) top[lo] = (uint8_t)(lvl + 1);
-    chain[lo] += 1;
-    w++;
+// Per cell: body count (the end of its prefix run, found by galloping) and,
+// for the top cell of a chain, the link to its parent, the cell one level up
+// whose run holds the slot before. Leaves also mark their slots.
+__global__ void __launch_bounds__(TB) k_cell_links(const uint64_t* __restrict__ keys, uint32_t n,
+                                                  const uint64_t* __restrict__ start, uint32_t nc,
+                                                  DevCells c, uint32_t* __restrict__ leaf_of_slot) {
+  const uint32_t id = blockIdx.x * TB + threadIdx.x;
+  if (id >= nc) return;
+  const uint32_t f = c.first[id];
+  const int lev = c.level[id];
+  const uint64_t k = keys[f];
+  // end: the last slot known inside is f + in, the first known outside f + out
+  uint64_t in = 0, out = 1;
+  while (f + out < n && same_cell(keys[f + out], k, lev)) {
+    in = out;
+    out *= 2;
   }
-}
-
-void launch_split_emit(DevBfs bfs, uint32_t s0, uint32_t cnt, uint32_t e0, uint32_t n_leaf,
-                       int vlev, const uint32_t* bounds, const uint32_t* child_off,
-                       uint32_t* chain, uint8_t* top, hipStream_t s) {
-  hipLaunchKernelGGL(k_split_emit, dim3((cnt + TB - 1) / TB), dim3(TB), 0, s, bfs, s0, cnt, e0,
-                     n_leaf, vlev, bounds, child_off, chain, top);
-}
-
-__global__ void __launch_bounds__(TB) k_dfs_ids(DevBfs bfs, uint32_t nc,
-                                               const uint32_t* __restrict__ cstart,
-                                               const uint8_t* __restrict__ top) {
-  uint32_t b = blockIdx.x * TB + threadIdx.x;
-  if (b >= nc) return;
-  uint32_t f = bfs.first[b];
-  bfs.dfs[b] = cstart[f] + (uint32_t)bfs.level[b] - (uint32_t)top[f];
-}
-
-void launch_dfs_ids(DevBfs bfs, uint32_t nc, const uint32_t* cstart, const uint8_t* top,
-                    hipStream_t s) {
-  hipLaunchKernelGGL(k_dfs_ids, dim3((nc + TB - 1) / TB), dim3(TB), 0, s, bfs, nc, cstart, top);
-}
-
-__global__ void __launch_bounds__(TB) k_scatter_cells(DevBfs bfs, uint32_t nc, uint32_t n_leaf,
-                                                     int vlev, DevCells c,
-                                                     uint32_t* __restrict__ lvl_cells) {
-  uint32_t b = blockIdx.x * TB + threadIdx.x;
-  if (b >= nc) return;
-  uint32_t d = bfs.dfs[b];
-  uint32_t cnt = bfs.count[b];
-  int lvl = bfs.level[b];
-  c.first[d] = bfs.first[b];
-  c.count[d] = cnt;
-  c.level[d] = (uint8_t)lvl;
-  c.leaf[d] = is_internal(cnt, lvl, n_leaf, vlev) ? 0 : 1;
-  int32_t pb = bfs.parent[b];
-  if (pb >= 0) {
-    uint32_t pd = bfs.dfs[pb];
-    c.parent[d] = (int32_t)pd;
-    c.children[(size_t)pd * 8 + bfs.oct[b]] = (int32_t)d;
-  } else {
-    c.parent[d] = -1;
+  out = min(out, (uint64_t)(n - f));
+  while (out - in > 1) {
+    const uint64_t mid = in + (out - in) / 2;
+    if (same_cell(keys[f + mid], k, lev))
+      in = mid;
+    else
+      out = mid;
   }
-  lvl_cells[b] = d;
+  c.count[id] = (uint32_t)out;
+  if (c.leaf[id])
+    for (uint32_t j = 0; j < (uint32_t)out; j++) leaf_of_slot[f + j] = id;
+  if (id == 0) {
+    c.parent[0] = -1;
+    return;
+  }
+  if ((uint32_t)(start[f] >> 32) != id) return;  // not the chain's top
+  uint64_t back = 0, past = 1;  // f - back is in the parent's run, f - past is not
+  while (past <= f && same_cell(keys[f - past], k, lev - 1)) {
+    back = past;
+    past *= 2;
+  }
+  past = min(past, (uint64_t)f + 1);
+  while (past - back > 1) {
+    const uint64_t mid = back + (past - back) / 2;
+    if (same_cell(keys[f - mid], k, lev - 1))
+      back = mid;
+    else
+      past = mid;
+  }
+  const uint32_t head = (uint32_t)(start[f - back] >> 32);
+  const uint32_t pa = head + (uint32_t)(lev - 1) - (uint32_t)c.level[head];
+  c.parent[id] = (int32_t)pa;
+  c.children[(size_t)pa * 8 + ((k >> (3 * (BITS - lev))) & 7u)] = (int32_t)id;
 }
 
-void launch_scatter_cells(DevBfs bfs, uint32_t nc, uint32_t n_leaf, int vlev, DevCells c,
-                          uint32_t* lvl_cells, hipStream_t s) {
-  hipLaunchKernelGGL(k_scatter_cells, dim3((nc + TB - 1) / TB), dim3(TB), 0, s, bfs, nc, n_leaf,
-                     vlev, c, lvl_cells);
+void launch_cells(const uint64_t* keys, size_t n, const uint64_t* chain, const uint64_t* start,
+                  uint32_t nc, DevCells c, uint32_t* leaf_ids, uint32_t* leaf_of_slot,
+                  hipStream_t s) {
+  hipLaunchKernelGGL(k_cell_emit, dim3((n + TB - 1) / TB), dim3(TB), 0, s, keys, (uint32_t)n, chain,
+                     start, c, leaf_ids);
+  hipLaunchKernelGGL(k_cell_links, dim3((nc + TB - 1) / TB), dim3(TB), 0, s, keys, (uint32_t)n,
+                     start, nc, c, leaf_of_slot);
 }
 
 // ---------------------------------------------------------------- geometry
@@ -584,81 +574,66 @@ __device__ void ritter(int nitems, Get get, double out[3]) {
   }
 }
 
-// tree.rs:152-227, one thread per cell of a level (children done first).
-// which = 0: every cell of the list; 1: only its leaves; 2: only its internal cells.
+// tree.rs:152-227, one thread per internal cell of a level (children done
+// first). The children's data is gathered before any of it is used, so the
+// cell costs two dependent loads instead of two per child.
 __global__ void __launch_bounds__(TB) k_geometry(const uint32_t* __restrict__ cells, uint32_t cnt,
-                                                DevCells c, DevBodies b, int mode, int which) {
-  uint32_t i = blockIdx.x * TB + threadIdx.x;
+                                                DevCells c, int mode) {
+  const uint32_t i = blockIdx.x * TB + threadIdx.x;
   if (i >= cnt) return;
-  uint32_t id = cells[i];
-  if ((which == 1 && !c.leaf[id]) || (which == 2 && c.leaf[id])) return;
+  const uint32_t id = cells[i];
+  int q[8];
+  double qm[8], qx[8], qy[8], qz[8], qr[8];
+  const int32_t* ch = c.children + (size_t)id * 8;
+#pragma unroll
+  for (int o = 0; o < 8; o++) q[o] = ch[o];
+#pragma unroll
+  for (int o = 0; o < 8; o++) {
+    const int a = q[o] >= 0 ? q[o] : (int)id;  // absent: read, not used
+    qm[o] = c.mass[a];
+    qx[o] = c.cx[a];
+    qy[o] = c.cy[a];
+    qz[o] = c.cz[a];
+    qr[o] = c.rho[a];
+  }
   double ms = 0.0;
   double cen[3];
-  double rho = 0.0;
-  if (c.leaf[id]) {
-    uint32_t f = c.first[id], e = f + c.count[id];
-    for (uint32_t k = f; k < e; k++) ms += b.m[k];
-    if (mode == 0) {  // com_of_slots, tree.rs:257-275
-      double com[3] = {0.0, 0.0, 0.0};
-      for (uint32_t k = f; k < e; k++) {
-        double m = b.m[k];
-        com[0] += m * b.x[k];
-        com[1] += m * b.y[k];
-        com[2] += m * b.z[k];
-      }
-      cen[0] = com[0] / ms;
-      cen[1] = com[1] / ms;
-      cen[2] = com[2] / ms;
-    } else {
-      ritter(
-          (int)(e - f),
-          [&](int q, double* qc, double* qr) {
-            qc[0] = b.x[f + q];
-            qc[1] = b.y[f + q];
-            qc[2] = b.z[f + q];
-            *qr = 0.0;
-          },
-          cen);
-    }
-    for (uint32_t k = f; k < e; k++) rho = fmax(rho, dist3(b.x[k], b.y[k], b.z[k], cen[0], cen[1], cen[2]));
-  } else {
-    const int32_t* ch = c.children + (size_t)id * 8;
-    for (int o = 0; o < 8; o++)
-      if (ch[o] >= 0) ms += c.mass[ch[o]];
-    if (mode == 0) {
-      double com[3] = {0.0, 0.0, 0.0};
-      for (int o = 0; o < 8; o++) {
-        int q = ch[o];
-        if (q < 0) continue;
-        double m = c.mass[q];
-        com[0] += m * c.cx[q];
-        com[1] += m * c.cy[q];
-        com[2] += m * c.cz[q];
-      }
-      cen[0] = com[0] / ms;
-      cen[1] = com[1] / ms;
-      cen[2] = com[2] / ms;
-    } else {
-      int list[8];
-      int nl = 0;
-      for (int o = 0; o < 8; o++)
-        if (ch[o] >= 0) list[nl++] = ch[o];
-      ritter(
-          nl,
-          [&](int q, double* qc, double* qr) {
-            int cc = list[q];
-            qc[0] = c.cx[cc];
-            qc[1] = c.cy[cc];
-            qc[2] = c.cz[cc];
-            *qr = c.rho[cc];
-          },
-          cen);
-    }
+#pragma unroll
+  for (int o = 0; o < 8; o++)
+    if (q[o] >= 0) ms += qm[o];
+  if (mode == 0) {
+    double com[3] = {0.0, 0.0, 0.0};
+#pragma unroll
     for (int o = 0; o < 8; o++) {
-      int q = ch[o];
-      if (q < 0) continue;
-      rho = fmax(rho, c.rho[q] + dist3(c.cx[q], c.cy[q], c.cz[q], cen[0], cen[1], cen[2]));
+      if (q[o] < 0) continue;
+      com[0] += qm[o] * qx[o];
+      com[1] += qm[o] * qy[o];
+      com[2] += qm[o] * qz[o];
     }
+    cen[0] = com[0] / ms;
+    cen[1] = com[1] / ms;
+    cen[2] = com[2] / ms;
+  } else {
+    int list[8];
+    int nl = 0;
+    for (int o = 0; o < 8; o++)
+      if (ch[o] >= 0) list[nl++] = ch[o];
+    ritter(
+        nl,
+        [&](int e, double* ec, double* er) {
+          const int cc = list[e];
+          ec[0] = c.cx[cc];
+          ec[1] = c.cy[cc];
+          ec[2] = c.cz[cc];
+          *er = c.rho[cc];
+        },
+        cen);
+  }
+  double rho = 0.0;
+#pragma unroll
+  for (int o = 0; o < 8; o++) {
+    if (q[o] < 0) continue;
+    rho = fmax(rho, qr[o] + dist3(qx[o], qy[o], qz[o], cen[0], cen[1], cen[2]));
   }
   c.mass[id] = ms;
   c.cx[id] = cen[0];
@@ -667,8 +642,7 @@ __global__ void __launch_bounds__(TB) k_geometry(const uint32_t* __restrict__ ce
   c.rho[id] = rho;
 }
 
-// Leaf geometry with one wave per leaf: the same values as k_geometry's
-// leaf branch (tree.rs:152-227, 257-275, 290-389). Order-dependent sums
+// Leaf geometry with one wave per leaf (tree.rs:152-227, 257-275, 290-389). Order-dependent sums
 // (mass, centre of mass) run in slot order over bodies read from the lanes
 // that hold them; the farthest-point searches, the box and the radius and
 // rho maxima spread over the lanes (a maximum, ties to the lowest slot, does
@@ -842,138 +816,42 @@ void launch_geometry_leaves(const uint32_t* leaf_ids, uint32_t nleaves, DevCells
                      dim3(64 * GEO_WAVES), 0, s, leaf_ids, nleaves, c, b, center_mode);
 }
 
-void launch_geometry(const uint32_t* lvl_cells, uint32_t cnt, DevCells c, DevBodies b,
-                     int center_mode, hipStream_t s, int which) {
+void launch_geometry(const uint32_t* cells, uint32_t cnt, DevCells c, int center_mode,
+                     hipStream_t s) {
   if (cnt == 0) return;
-  hipLaunchKernelGGL(k_geometry, dim3((cnt + TB - 1) / TB), dim3(TB), 0, s, lvl_cells, cnt, c, b,
-                     center_mode, which);
+  hipLaunchKernelGGL(k_geometry, dim3((cnt + TB - 1) / TB), dim3(TB), 0, s, cells, cnt, c,
+                     center_mode);
 }
 
 // Ropes of the mirrored DFS (children visited 7..0): the cell visited after
-// a child's subtree is its next lower existing sibling, else the parent's rope.
-__global__ void __launch_bounds__(TB) k_ropes(const uint32_t* __restrict__ cells, uint32_t cnt,
-                                             DevCells c) {
-  uint32_t i = blockIdx.x * TB + threadIdx.x;
-  if (i >= cnt) return;
-  uint32_t id = cells[i];
-  if (id == 0) c.rope[0] = -1;
-  if (c.leaf[id]) {
-    c.last_child[id] = -1;
-    return;
-  }
-  int32_t prev = (id == 0) ? -1 : c.rope[id];
-  const int32_t* ch = c.children + (size_t)id * 8;
-  for (int o = 0; o < 8; o++) {
-    int q = ch[o];
-    if (q < 0) continue;
-    c.rope[q] = prev;
-    prev = q;
-  }
-  c.last_child[id] = prev;
-}
-
-void launch_ropes(const uint32_t* lvl_cells, uint32_t cnt, DevCells c, hipStream_t s) {
-  if (cnt == 0) return;
-  hipLaunchKernelGGL(k_ropes, dim3((cnt + TB - 1) / TB), dim3(TB), 0, s, lvl_cells, cnt, c);
-}
-
-__global__ void __launch_bounds__(TB) k_leaf_flags(DevCells c, uint32_t nc, uint32_t* flags) {
-  uint32_t i = blockIdx.x * TB + threadIdx.x;
-  if (i < nc) flags[i] = c.leaf[i];
-}
-
-void launch_leaf_flags(DevCells c, uint32_t nc, uint32_t* flags, hipStream_t s) {
-  hipLaunchKernelGGL(k_leaf_flags, dim3((nc + TB - 1) / TB), dim3(TB), 0, s, c, nc, flags);
-}
-
-__global__ void __launch_bounds__(TB) k_leaf_compact(DevCells c, uint32_t nc,
-                                                    const uint32_t* __restrict__ off,
-                                                    uint32_t* __restrict__ leaf_ids,
-                                                    uint32_t* __restrict__ leaf_of_slot) {
-  uint32_t i = blockIdx.x * TB + threadIdx.x;
-  if (i >= nc || !c.leaf[i]) return;
-  leaf_ids[off[i]] = i;
-  uint32_t f = c.first[i], e = f + c.count[i];
-  for (uint32_t k = f; k < e; k++) leaf_of_slot[k] = i;
-}
-
-void launch_leaf_compact(DevCells c, uint32_t nc, const uint32_t* off, uint32_t* leaf_ids,
-                         uint32_t* leaf_of_slot, hipStream_t s) {
-  hipLaunchKernelGGL(k_leaf_compact, dim3((nc + TB - 1) / TB), dim3(TB), 0, s, c, nc, off, leaf_ids,
-                     leaf_of_slot);
-}
-
-// Internal cells of every level in BFS order (levels stay contiguous):
-// flag, exclusive scan, compact; then each level's start in the compacted
-// list is picked at the level's BFS offset.
-__global__ void __launch_bounds__(TB) k_internal_flags(const uint32_t* __restrict__ lvl_cells,
-                                                      uint32_t nc, DevCells c,
-                                                      uint32_t* __restrict__ flags) {
-  uint32_t i = blockIdx.x * TB + threadIdx.x;
-  if (i < nc) flags[i] = c.leaf[lvl_cells[i]] ? 0u : 1u;
-}
-
-__global__ void __launch_bounds__(TB) k_internal_compact(const uint32_t* __restrict__ lvl_cells,
-                                                        uint32_t nc, DevCells c,
-                                                        const uint32_t* __restrict__ pos,
-                                                        uint32_t* __restrict__ out) {
-  uint32_t i = blockIdx.x * TB + threadIdx.x;
+// a cell's subtree is its next lower existing sibling, else its parent's
+// rope. Each cell climbs to the first ancestor with a lower sibling (one
+// launch for all levels; a pass per level before).
+__global__ void __launch_bounds__(TB) k_ropes(uint32_t nc, DevCells c) {
+  const uint32_t i = blockIdx.x * TB + threadIdx.x;
   if (i >= nc) return;
-  const uint32_t id = lvl_cells[i];
-  if (!c.leaf[id]) out[pos[i]] = id;
+  int32_t last = -1;
+  const int32_t* ch = c.children + (size_t)i * 8;
+#pragma unroll
+  for (int o = 0; o < 8; o++)
+    if (ch[o] >= 0) last = ch[o];
+  c.last_child[i] = last;
+  int32_t rope = -1;
+  int32_t cur = (int32_t)i;
+  for (int l = 0; l <= BITS && rope < 0; l++) {
+    const int32_t pa = c.parent[cur];
+    if (pa < 0) break;
+    const int32_t* sib = c.children + (size_t)pa * 8;
+#pragma unroll
+    for (int o = 0; o < 8; o++)  // ids rise with the octant: the highest one below cur
+      if (sib[o] >= 0 && sib[o] < cur) rope = sib[o];
+    cur = pa;
+  }
+  c.rope[i] = rope;
 }
 
-__global__ void k_level_pick(const uint32_t* __restrict__ pos, const uint32_t* __restrict__ total,
-                             uint32_t nc, const uint32_t* __restrict__ at, uint32_t nl,
-                             uint32_t* __restrict__ out) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nl) out[i] = at[i] < nc ? pos[at[i]] : *total;
-}
-
-// Leaves ordered by body count (for per-leaf kernels whose waves should see
-// leaves of similar size): key = min(count, 65535) << 32 | leaf id, sorted
-// on bits 32..47, then the ids read back.
-__global__ void __launch_bounds__(TB) k_leaf_count_keys(const uint32_t* __restrict__ leaf_ids,
-                                                       uint32_t nleaves, DevCells c,
-                                                       uint64_t* __restrict__ keys) {
-  uint32_t i = blockIdx.x * TB + threadIdx.x;
-  if (i >= nleaves) return;
-  const uint32_t id = leaf_ids[i];
-  keys[i] = ((uint64_t)min(c.count[id], 65535u) << 32) | id;
-}
-
-__global__ void __launch_bounds__(TB) k_low32(const uint64_t* __restrict__ keys, uint32_t n,
-                                             uint32_t* __restrict__ out) {
-  uint32_t i = blockIdx.x * TB + threadIdx.x;
-  if (i < n) out[i] = (uint32_t)keys[i];
-}
-
-void launch_leaves_by_count(const uint32_t* leaf_ids, uint32_t nleaves, DevCells c,
-                            uint64_t* keys, uint64_t* keys_alt, uint32_t* tmp, uint32_t* out,
-                            hipStream_t s) {
-  if (nleaves == 0) return;
-  const dim3 g((nleaves + TB - 1) / TB);
-  hipLaunchKernelGGL(k_leaf_count_keys, g, dim3(TB), 0, s, leaf_ids, nleaves, c, keys);
-  const int fl = radix_sort_u64(keys, nullptr, keys_alt, nullptr, nleaves, 32, 48, tmp, s);
-  hipLaunchKernelGGL(k_low32, g, dim3(TB), 0, s, fl ? keys_alt : keys, nleaves, out);
-}
-
-void launch_internal_flags(const uint32_t* lvl_cells, uint32_t nc, DevCells c, uint32_t* flags,
-                           hipStream_t s) {
-  hipLaunchKernelGGL(k_internal_flags, dim3((nc + TB - 1) / TB), dim3(TB), 0, s, lvl_cells, nc, c,
-                     flags);
-}
-
-void launch_internal_compact(const uint32_t* lvl_cells, uint32_t nc, DevCells c,
-                             const uint32_t* pos, uint32_t* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_internal_compact, dim3((nc + TB - 1) / TB), dim3(TB), 0, s, lvl_cells, nc,
-                     c, pos, out);
-}
-
-void launch_level_pick(const uint32_t* pos, const uint32_t* total, uint32_t nc, const uint32_t* at,
-                       uint32_t nl, uint32_t* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_level_pick, dim3((nl + 63) / 64), dim3(64), 0, s, pos, total, nc, at, nl,
-                     out);
+void launch_ropes(uint32_t nc, DevCells c, hipStream_t s) {
+  hipLaunchKernelGGL(k_ropes, dim3((nc + TB - 1) / TB), dim3(TB), 0, s, nc, c);
 }
 
 }  // namespace fmmh
