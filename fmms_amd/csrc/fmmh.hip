@@ -111,15 +111,15 @@ struct fmmh_ctx {
   Buf fprec;  // f pre-pass cell records
   Buf moments, locals, pows, fvals, fmin, fact, binom;
   Buf front_a, front_b, m2l, p2p, ctr;
-  Buf mkeys, mkeys_alt, tptr, pkeys, pkeys_alt, pptr, list_tot;
-  Buf nch, choff, chunks, part;
+  Buf mkeys, mkeys_alt, tptr, pkeys, pkeys_alt, pptr;
+  Buf plan, chunks, part;
   Buf far, p2p_work, walkrec;
   Buf walk_code, walk_blk;  // the walk's per-pair decisions, per-block counts
-  Buf pl_n, pl_items, pl_reds, pl_partial;  // P2P work plan
+  Buf pl_longs, pl_items, pl_reds, pl_partial;  // P2P work plan
   Buf m2l_lam, m2l_m32;                     // mixed form: FP32 M2L scales, scaled moments
   Buf m2l_rows;                             // FP64 form: source rows
   Buf loc32;                                // mixed form: FP32 locals scaled by lam^n
-  uint32_t p_nitems = 0, p_nsplit = 0;
+  uint32_t p_nitems = 0, p_nsplit = 0, p_nlong = 0;
   Buf rt_tab;  // p > TEMPLATED_MAX_P: the rotation M2L's tables
   Buf ctrace, clap;  // softened far field: q = sum m |x - z|^2; L, G, H per cell
   int rot_p = -1;
@@ -135,8 +135,8 @@ struct fmmh_ctx {
                   &leaf_ids, &leaf_of_slot, &leaf_bc, &cpm,
                   &scan_tmp, &sort_tmp,
                   &fprec, &moments, &locals, &pows, &fvals, &fmin, &fact, &binom, &front_a, &front_b,
-                  &m2l, &p2p, &ctr, &mkeys, &mkeys_alt, &tptr, &pkeys, &pkeys_alt, &pptr, &list_tot,
-                  &nch, &choff, &chunks, &part, &far, &p2p_work, &walkrec, &walk_code, &walk_blk, &pl_n, &pl_items,
+                  &m2l, &p2p, &ctr, &mkeys, &mkeys_alt, &tptr, &pkeys, &pkeys_alt, &pptr,
+                  &plan, &chunks, &part, &far, &p2p_work, &walkrec, &walk_code, &walk_blk, &pl_longs, &pl_items,
                   &pl_reds, &pl_partial, &m2l_lam, &m2l_m32, &m2l_rows, &loc32, &rt_tab, &direct_ids, &direct_out, &direct_part, &lf_part, &lf_state, &lf_flag, &ctrace, &clap,
                   &d_sysoff};
     bufs.assign(std::begin(all), std::end(all));
@@ -454,29 +454,33 @@ struct fmmh_ctx {
     psorted = (const uint64_t*)(fl ? pkeys_alt.p : pkeys.p);
     launch_csr_ptr(psorted, 2 * n_p2p, sbits, nc, (uint32_t*)pptr.p, s);
     p2p_counted = false;
-    // the P2P plan's three totals and the M2L chunk count, copied into one
-    // small buffer on the device and read back together
-    ensure(list_tot, 16);
-    uint32_t* dtot = (uint32_t*)list_tot.p;
-    HCHECK(hipMemsetAsync(dtot, 0, 16, s));
-    plan_p2p_count(dtot);
+    // M2L chunks and P2P items per cell, scanned; the totals in one read
     const uint32_t ch = p <= TEMPLATED_MAX_P ? (uint32_t)tun.m2l_chunk : M2L_ROT_CHUNK;
-    size_t maxck = m2l_max_chunks(2 * n_m2l, nc, ch);
-    ensure(nch, ((size_t)nc + 1) * 4);
-    ensure(choff, ((size_t)nc + 1) * 4);
-    ensure(chunks, maxck * m2l_chunk_bytes());
-    ensure_scan(nc + 1);
-    uint32_t* tot = nullptr;
-    m2l_build_chunks((uint32_t*)tptr.p, nc, ch, (uint32_t*)nch.p, (uint32_t*)choff.p,
-                     (uint32_t*)scan_tmp.p, chunks.p, s, &tot);
-    // choff[nc] = total chunks (the reduce reads choff[t+1])
-    HCHECK(hipMemcpyAsync((uint32_t*)choff.p + nc, tot, 4, hipMemcpyDeviceToDevice, s));
-    HCHECK(hipMemcpyAsync(dtot + 3, tot, 4, hipMemcpyDeviceToDevice, s));
-    const uint4 t = read1((const uint4*)dtot);
-    p_nitems = t.x;
-    p_nsplit = t.z;
-    plan_p2p_emit(t.y);
-    nchunks = t.w;
+    const bool f32 = prm.precision == FMMH_PREC_FP32BULK;
+    uint4* pl = ensure<uint4>(plan, ((size_t)nc + 2) * sizeof(uint4));
+    ensure(scan_tmp, scan_tmp_words(4 * ((size_t)nc + 1)) * sizeof(uint4));
+    HCHECK(hipMemsetAsync(pl + nc + 1, 0, sizeof(uint4), s));
+    plan_count(nc, cells(), (const uint32_t*)tptr.p, ch, (const uint32_t*)pptr.p, psorted, sbits,
+               tun.p2p_item_work, f32, pl, s);
+    scan_exclusive_u32x4(pl, (size_t)nc + 1, (uint4*)scan_tmp.p, s);
+    struct Totals {
+      uint4 v[2];
+    };
+    const Totals t = read1((const Totals*)(pl + nc));
+    nchunks = t.v[0].x;
+    p_nitems = t.v[0].y;
+    p_nsplit = t.v[0].w;
+    // long items first where they are few: a system whose typical leaf has that
+    // many sources gains nothing from it and would lose the leaf order's reuse
+    p_nlong = (uint64_t)t.v[1].x * 16 <= p_nitems ? t.v[1].x : 0u;
+    ensure(chunks, std::max<size_t>(nchunks, 1) * m2l_chunk_bytes());
+    ensure(pl_items, (size_t)std::max<uint32_t>(p_nitems, 1) * sizeof(uint4));
+    ensure(pl_reds, (size_t)std::max<uint32_t>(p_nsplit, 1) * sizeof(uint4));
+    ensure(pl_longs, (size_t)p_nlong * 4);
+    ensure(pl_partial, (size_t)std::max<uint32_t>(t.v[0].z, 1) * sizeof(double4));
+    plan_emit(nc, cells(), (const uint32_t*)tptr.p, ch, (const uint32_t*)pptr.p, psorted, sbits,
+              tun.p2p_item_work, f32, pl, chunks.p, (uint4*)pl_items.p, (uint4*)pl_reds.p,
+              p_nlong ? (uint32_t*)(pl + nc + 1) + 1 : nullptr, (uint32_t*)pl_longs.p, s);
     ensure(part, m2l_part_bytes(p, std::max<size_t>(nchunks, 1), mixed32()));
     if (p > TEMPLATED_MAX_P) {
       rot_tables();
@@ -488,39 +492,6 @@ struct fmmh_ctx {
       ensure(loc32, (size_t)nc * m2l32_moment_bytes(p));
     }
     ensure(far, n * sizeof(double4));
-  }
-
-  // P2P work items (near.hip): per leaf the item count, partial-sum slots and
-  // split flag, scanned in place into offsets (the three totals to
-  // tot[0..2]), then, once the totals are on the host, the items themselves.
-  void plan_p2p_count(uint32_t* tot) {
-    p_nitems = p_nsplit = 0;
-    if (nleaves == 0) return;
-    const size_t w = (size_t)nleaves + 1;
-    ensure(pl_n, 3 * w * 4);
-    uint32_t* nitem = (uint32_t*)pl_n.p;
-    p2p_plan_count((const uint32_t*)leaf_ids.p, nleaves, (const uint32_t*)pptr.p, psorted, sbits,
-                   (const uint32_t*)c_count.p, tun.p2p_item_work, nitem, nitem + w, nitem + 2 * w,
-                   s);
-    ensure_scan(w);
-    for (int k = 0; k < 3; k++) {
-      uint32_t* col = nitem + k * w;
-      uint32_t* t = nullptr;
-      scan_exclusive_u32(col, col, w, (uint32_t*)scan_tmp.p, s, &t);
-      HCHECK(hipMemcpyAsync(tot + k, t, 4, hipMemcpyDeviceToDevice, s));
-    }
-  }
-
-  void plan_p2p_emit(uint32_t nslots) {
-    if (nleaves == 0) return;
-    const size_t w = (size_t)nleaves + 1;
-    uint32_t* nitem = (uint32_t*)pl_n.p;
-    ensure(pl_items, (size_t)std::max<uint32_t>(p_nitems, 1) * sizeof(uint4));
-    ensure(pl_reds, (size_t)std::max<uint32_t>(p_nsplit, 1) * sizeof(uint4));
-    ensure(pl_partial, (size_t)std::max<uint32_t>(nslots, 1) * sizeof(double4));
-    p2p_plan_emit((const uint32_t*)leaf_ids.p, nleaves, (const uint32_t*)pptr.p, psorted, sbits,
-                  (const uint32_t*)c_count.p, tun.p2p_item_work, nitem, nitem + w, nitem + 2 * w,
-                  (uint4*)pl_items.p, (uint4*)pl_reds.p, s);
   }
 
   // The mixed form's FP32 M2L, L2L and L2P (templated orders only).
@@ -545,14 +516,14 @@ struct fmmh_ctx {
                    vlev, mom, soft2, (double*)m2l_lam.p, m2l_m32.p, part.p, s,
                    up32() ? vlev + FP64_TOP : 255);
       mark(ST_M2L_REDUCE);
-      launch_m2l_reduce32(p, nc, (uint32_t*)choff.p, part.p, (const double*)m2l_lam.p, loc, s);
+      launch_m2l_reduce32(p, nc, (const uint4*)plan.p, part.p, (const double*)m2l_lam.p, loc, s);
     } else if (!gen) {
       launch_m2l_kernel(p, nc, chunks.p, nchunks, msorted, sbits, c, mom, soft2,
                         (double*)m2l_rows.p, (double*)part.p, s);
       mark(ST_M2L_REDUCE);
-      launch_m2l_reduce(p, nc, (uint32_t*)choff.p, (const double*)part.p, loc, s);
+      launch_m2l_reduce(p, nc, (const uint4*)plan.p, (const double*)part.p, loc, s);
     } else {
-      HCHECK(launch_m2l_rot(p, nc, chunks.p, nchunks, (uint32_t*)choff.p, msorted, sbits, c, mom,
+      HCHECK(launch_m2l_rot(p, nc, chunks.p, nchunks, (const uint4*)plan.p, msorted, sbits, c, mom,
                             soft2, (const double*)rt_tab.p, rot_off, (cplx*)part.p, loc, s));
       mark(ST_M2L_REDUCE);
     }
@@ -582,8 +553,8 @@ struct fmmh_ctx {
       launch_l2p(p, (uint32_t)n, (uint32_t*)leaf_of_slot.p, c, b, loc, lap, (double4*)far.p, s);
     else
       launch_l2p_gen(p, (uint32_t*)leaf_ids.p, nleaves, c, b, loc, lap, (double4*)far.p, s);
-    const P2PPlan pl{(const uint4*)pl_items.p, p_nitems, (const uint4*)pl_reds.p, p_nsplit,
-                     (double4*)pl_partial.p};
+    const P2PPlan pl{(const uint4*)pl_items.p, p_nitems, p_nlong, (const uint32_t*)pl_longs.p,
+                     (const uint4*)pl_reds.p, p_nsplit, (double4*)pl_partial.p};
     const bool f32 = prm.precision == FMMH_PREC_FP32BULK;
     mark(ST_P2P);
     if (f32)

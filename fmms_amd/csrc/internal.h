@@ -18,6 +18,8 @@ void scan_exclusive_u32(const uint32_t* in, uint32_t* out, size_t n, uint32_t* t
 // The same for two u32 counts packed in a u64 (tmp: scan_tmp_words(n) u64).
 void scan_exclusive_u64(const uint64_t* in, uint64_t* out, size_t n, uint64_t* tmp, hipStream_t s,
                         uint64_t** total_dev);
+// Four counts per element, in place (tmp: scan_tmp_words(4 n) uint4).
+void scan_exclusive_u32x4(uint4* a, size_t n, uint4* tmp, hipStream_t s);
 size_t radix_tmp_words(size_t n);
 // Cell ids ordered by level, each level's internal cells before its leaves
 // (both in id order); leaf ids ordered by body count (up to 255). tmp:
@@ -156,12 +158,8 @@ void launch_csr_ptr(const uint64_t* keys, uint32_t nnz, int sbits, uint32_t ntar
 
 // --------------------------------------------------------------- m2l.hip
 // Chunks of at most `ch` sources per target (the M2L work unit).
-size_t m2l_max_chunks(uint32_t nnz, uint32_t nc, uint32_t ch);
 size_t m2l_part_bytes(int p, size_t maxchunks, bool fp32);
 size_t m2l_chunk_bytes();
-void m2l_build_chunks(const uint32_t* tptr, uint32_t nc, uint32_t ch, uint32_t* nch,
-                      uint32_t* choff, uint32_t* scan_tmp, void* chunks, hipStream_t s,
-                      uint32_t** total_dev);
 // FP64 form, p <= 10: rows [nc] x m2l_row_bytes(p) is scratch (the sources'
 // multipoles and centres as contiguous rows), part gets the chunk partials.
 size_t m2l_row_bytes(int p);
@@ -181,9 +179,9 @@ bool launch_m2l32(int p, uint32_t nc, const void* chunks, uint32_t nchunks, cons
 void launch_m2l_scale(uint32_t nc, DevCells c, const BBox* bb, const uint64_t* keys_sorted,
                       int vlev, double* lam, hipStream_t s);
 size_t m2l32_moment_bytes(int p);
-bool launch_m2l_reduce32(int p, uint32_t nc, const uint32_t* choff, const void* part,
+bool launch_m2l_reduce32(int p, uint32_t nc, const uint4* plan, const void* part,
                          const double* lam, cplx* locals, hipStream_t s);
-bool launch_m2l_reduce(int p, uint32_t nc, const uint32_t* choff, const double* part, cplx* locals,
+bool launch_m2l_reduce(int p, uint32_t nc, const uint4* plan, const double* part, cplx* locals,
                        hipStream_t s);
 
 // ----------------------------------------------------------- upward32.hip
@@ -213,7 +211,7 @@ void launch_m2m_gen(int p, const uint32_t* cells, uint32_t cnt, DevCells c, cplx
 constexpr uint32_t M2L_ROT_CHUNK = 64;
 void rot_tables_host(int p, std::vector<double>& tab, std::vector<uint32_t>& off);
 hipError_t launch_m2l_rot(int p, uint32_t nc, const void* chunks, uint32_t nchunks,
-                          const uint32_t* choff, const uint64_t* skeys, int sbits, DevCells c,
+                          const uint4* plan, const uint64_t* skeys, int sbits, DevCells c,
                           const cplx* moments, double soft2, const double* tab,
                           const std::vector<uint32_t>& off, cplx* part, cplx* locals,
                           hipStream_t s);
@@ -293,19 +291,25 @@ __device__ __forceinline__ void l2p_trace_walk(const double* __restrict__ lap,
 struct P2PPlan {
   const uint4* items;
   uint32_t nitems;
+  uint32_t nlong;         // items launched first, by index
+  const uint32_t* longs;
   const uint4* reds;
   uint32_t nsplit;
   double4* partial;
 };
-// item_work: a leaf whose targets x sources exceed it is cut into items.
-void p2p_plan_count(const uint32_t* leaf_ids, uint32_t nleaves, const uint32_t* pptr,
-                    const uint64_t* skeys, int sbits, const uint32_t* ccount, uint64_t item_work,
-                    uint32_t* nitem, uint32_t* npart, uint32_t* nsplit, hipStream_t s);
-void p2p_plan_emit(const uint32_t* leaf_ids, uint32_t nleaves, const uint32_t* pptr,
-                   const uint64_t* skeys, int sbits, const uint32_t* ccount, uint64_t item_work,
-                   const uint32_t* ioff, const uint32_t* poff, const uint32_t* roff, uint4* items,
-                   uint4* reds, hipStream_t s);
-// skeys: the target-sorted directed P2P entries (source in the low sbits)
+// Work plan of the lists: plan[t] = {M2L chunks of <= ch sources, P2P items,
+// partial-sum slots, cut leaves} of cell t, scanned by the caller over nc + 1
+// entries (plan[nc] = the totals); plan[nc + 1].x, zeroed before, counts the
+// long items. item_work: a leaf whose targets x sources exceed it
+// is cut into items; fp32: the mixed form's cut. nlong: a zeroed counter, or
+// null (no item is launched first).
+void plan_count(uint32_t nc, DevCells c, const uint32_t* tptr, uint32_t ch, const uint32_t* pptr,
+                const uint64_t* skeys, int sbits, uint64_t item_work, bool fp32, uint4* plan,
+                hipStream_t s);
+void plan_emit(uint32_t nc, DevCells c, const uint32_t* tptr, uint32_t ch, const uint32_t* pptr,
+               const uint64_t* skeys, int sbits, uint64_t item_work, bool fp32, const uint4* plan,
+               void* chunks, uint4* items, uint4* reds, uint32_t* nlong, uint32_t* longs,
+               hipStream_t s);
 void launch_p2p(const P2PPlan& pl, DevCells c, const double4* body, const uint64_t* skeys,
                 int sbits, double soft2, const double4* far, const uint32_t* order,
                 double* accel, double* pot, hipStream_t s);

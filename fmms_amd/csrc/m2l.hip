@@ -61,24 +61,6 @@ __global__ void __launch_bounds__(256) k_m2l_prep32(uint32_t nc, const cplx* __r
   }
 }
 
-__global__ void __launch_bounds__(256) k_m2l_nchunks(const uint32_t* __restrict__ tptr, uint32_t nc,
-                                                    uint32_t ch, uint32_t* __restrict__ nch) {
-  uint32_t t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= nc) return;
-  uint32_t s = tptr[t + 1] - tptr[t];
-  nch[t] = (s + ch - 1) / ch;
-}
-
-__global__ void __launch_bounds__(256) k_m2l_emit(const uint32_t* __restrict__ tptr, uint32_t nc,
-                                                 uint32_t ch, const uint32_t* __restrict__ choff,
-                                                 M2lChunk* __restrict__ chunks) {
-  uint32_t t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= nc) return;
-  uint32_t b = tptr[t], e = tptr[t + 1];
-  uint32_t w = choff[t];
-  for (uint32_t j = b; j < e; j += ch) chunks[w++] = M2lChunk{t, j, min(e, j + ch)};
-}
-
 constexpr int RED_AHEAD = 8;  // chunk partials loaded ahead of the in-order sum
 
 // locals[t] = sum over the target's chunk partials in chunk order (partials
@@ -86,7 +68,7 @@ constexpr int RED_AHEAD = 8;  // chunk partials loaded ahead of the in-order sum
 // each m); both halves of m written (F_n^{-m} = (-1)^m conj(F_n^m)); empty
 // targets get 0.
 template <int P>
-__global__ void __launch_bounds__(256) k_m2l_reduce(uint32_t nc, const uint32_t* __restrict__ choff,
+__global__ void __launch_bounds__(256) k_m2l_reduce(uint32_t nc, const uint4* __restrict__ plan,
                                                    const double* __restrict__ part,
                                                    cplx* __restrict__ locals) {
   constexpr int D = hdim(P), NF = hnpos(P);
@@ -100,7 +82,7 @@ __global__ void __launch_bounds__(256) k_m2l_reduce(uint32_t nc, const uint32_t*
   cplx s = cplx{0.0, 0.0};
   constexpr int W = (P + 1) * (P + 1);
   const int ir = n * n + (m ? 2 * m - 1 : 0), ii = n * n + 2 * m;  // m = 0: ii unused
-  const uint32_t c0 = choff[t], c1 = choff[t + 1];
+  const uint32_t c0 = plan[t].x, c1 = plan[t + 1].x;
   uint32_t c = c0;
   for (; c + RED_AHEAD <= c1; c += RED_AHEAD) {  // loads issued together, added in order
     double vr[RED_AHEAD], vi[RED_AHEAD];
@@ -131,7 +113,7 @@ __global__ void __launch_bounds__(256) k_m2l_reduce(uint32_t nc, const uint32_t*
 // Mixed form: FP32 chunk partials of the scaled F, summed in FP64 in chunk
 // order, then F_n = lam_t^-(n+1) * sum.
 template <int P>
-__global__ void __launch_bounds__(256) k_m2l_reduce32(uint32_t nc, const uint32_t* __restrict__ choff,
+__global__ void __launch_bounds__(256) k_m2l_reduce32(uint32_t nc, const uint4* __restrict__ plan,
                                                      const cplxf* __restrict__ part,
                                                      const double* __restrict__ lam,
                                                      cplx* __restrict__ locals) {
@@ -144,7 +126,7 @@ __global__ void __launch_bounds__(256) k_m2l_reduce32(uint32_t nc, const uint32_
   while ((n + 1) * (n + 2) / 2 <= e) n++;
   int m = e - n * (n + 1) / 2;
   double sr = 0.0, si = 0.0;
-  const uint32_t c0 = choff[t], c1 = choff[t + 1];
+  const uint32_t c0 = plan[t].x, c1 = plan[t + 1].x;
   uint32_t c = c0;
   for (; c + RED_AHEAD <= c1; c += RED_AHEAD) {  // loads issued together, added in order
     cplxf v[RED_AHEAD];
@@ -173,9 +155,6 @@ __global__ void __launch_bounds__(256) k_m2l_reduce32(uint32_t nc, const uint32_
   }
 }
 
-// Scratch layout handed in by the context: nch/choff (nc+1 words each) and
-// chunk/partial arrays sized for the worst case sum_t ceil(S_t/CH).
-size_t m2l_max_chunks(uint32_t nnz, uint32_t nc, uint32_t ch) { return (size_t)nnz / ch + nc + 1; }
 // One chunk's partial: FP32 complex halves in the mixed form, (p+1)^2 doubles
 // in the FP64 form, complex halves in the runtime orders' kernel.
 size_t m2l_part_bytes(int p, size_t maxchunks, bool fp32) {
@@ -186,20 +165,11 @@ size_t m2l_part_bytes(int p, size_t maxchunks, bool fp32) {
 }
 
 template <int P>
-static void m2l_reduce_t(uint32_t nc, const uint32_t* choff, const double* part, cplx* locals,
+static void m2l_reduce_t(uint32_t nc, const uint4* plan, const double* part, cplx* locals,
                          hipStream_t s) {
   size_t th = (size_t)nc * hnpos(P);
-  hipLaunchKernelGGL(k_m2l_reduce<P>, dim3((th + 255) / 256), dim3(256), 0, s, nc, choff, part,
+  hipLaunchKernelGGL(k_m2l_reduce<P>, dim3((th + 255) / 256), dim3(256), 0, s, nc, plan, part,
                      locals);
-}
-
-void m2l_build_chunks(const uint32_t* tptr, uint32_t nc, uint32_t ch, uint32_t* nch,
-                      uint32_t* choff, uint32_t* scan_tmp, void* chunks, hipStream_t s,
-                      uint32_t** total_dev) {
-  hipLaunchKernelGGL(k_m2l_nchunks, dim3((nc + 255) / 256), dim3(256), 0, s, tptr, nc, ch, nch);
-  scan_exclusive_u32(nch, choff, (size_t)nc, scan_tmp, s, total_dev);
-  hipLaunchKernelGGL(k_m2l_emit, dim3((nc + 255) / 256), dim3(256), 0, s, tptr, nc, ch, choff,
-                     (M2lChunk*)chunks);
 }
 
 #define FMMH_P_SWITCH3(p, CALL) \
@@ -260,19 +230,19 @@ bool launch_m2l32(int p, uint32_t nc, const void* chunks, uint32_t nchunks, cons
 
 size_t m2l32_moment_bytes(int p) { return (size_t)hnpos(p) * sizeof(cplxf); }
 
-bool launch_m2l_reduce32(int p, uint32_t nc, const uint32_t* choff, const void* part,
+bool launch_m2l_reduce32(int p, uint32_t nc, const uint4* plan, const void* part,
                          const double* lam, cplx* locals, hipStream_t s) {
 #define CALL(P)                                                                                  \
   hipLaunchKernelGGL(k_m2l_reduce32<P>, dim3(((size_t)nc * hnpos(P) + 255) / 256), dim3(256), 0, \
-                     s, nc, choff, (const cplxf*)part, lam, locals)
+                     s, nc, plan, (const cplxf*)part, lam, locals)
   FMMH_P_SWITCH3(p, CALL)
 #undef CALL
   return true;
 }
 
-bool launch_m2l_reduce(int p, uint32_t nc, const uint32_t* choff, const double* part, cplx* locals,
+bool launch_m2l_reduce(int p, uint32_t nc, const uint4* plan, const double* part, cplx* locals,
                        hipStream_t s) {
-#define CALL(P) m2l_reduce_t<P>(nc, choff, part, locals, s)
+#define CALL(P) m2l_reduce_t<P>(nc, plan, part, locals, s)
   FMMH_P_SWITCH3(p, CALL)
 #undef CALL
   return true;

@@ -431,13 +431,13 @@ __global__ void __launch_bounds__(ROT_T) k_m2l_rot(int p, const M2lChunk* __rest
 // locals[t] = g * sum over the target's chunk partials in chunk order, both
 // signs of m; targets without sources get 0.
 __global__ void __launch_bounds__(256) k_m2l_reduce_rot(int p, uint32_t nc,
-                                                       const uint32_t* __restrict__ choff,
+                                                       const uint4* __restrict__ plan,
                                                        const cplx* __restrict__ part,
                                                        const double* __restrict__ g,
                                                        cplx* __restrict__ locals) {
   const int NH = hnpos(p);
   const uint32_t t = blockIdx.x;
-  const uint32_t c0 = choff[t], c1 = choff[t + 1];
+  const uint32_t c0 = plan[t].x, c1 = plan[t + 1].x;
   cplx* out = locals + (size_t)t * hdim(p);
   for (int e = threadIdx.x; e < NH; e += 256) {
     int n = (int)((sqrt(8.0 * e + 1.0) - 1.0) * 0.5);
@@ -552,7 +552,7 @@ static hipError_t rot_t(int p, const M2lChunk* ck, uint32_t nchunks, const uint6
 }
 
 hipError_t launch_m2l_rot(int p, uint32_t nc, const void* chunks, uint32_t nchunks,
-                          const uint32_t* choff, const uint64_t* skeys, int sbits, DevCells c,
+                          const uint4* plan, const uint64_t* skeys, int sbits, DevCells c,
                           const cplx* moments, double soft2, const double* tab,
                           const std::vector<uint32_t>& off, cplx* part, cplx* locals,
                           hipStream_t s) {
@@ -565,7 +565,7 @@ hipError_t launch_m2l_rot(int p, uint32_t nc, const void* chunks, uint32_t nchun
                 : rot_t<6>(p, ck, nchunks, skeys, smask, c, moments, soft2, rt, part, s);
   if (e != hipSuccess) return e;
   if (nc)
-    hipLaunchKernelGGL(k_m2l_reduce_rot, dim3(nc), dim3(256), 0, s, p, nc, choff, part, rt.g, locals);
+    hipLaunchKernelGGL(k_m2l_reduce_rot, dim3(nc), dim3(256), 0, s, p, nc, plan, part, rt.g, locals);
   return hipSuccess;
 }
 

@@ -10,8 +10,11 @@
 // per body, each lane on a strided share of every tile, combined by
 // xor-shuffles at the end.
 // Softening (an extension; 0 = the reference): r^2 += eps^2.
+#include <algorithm>
+
 #include "common.h"
 #include "internal.h"
+#include "m2l_chunk.h"
 
 namespace fmmh {
 
@@ -22,37 +25,38 @@ constexpr uint32_t P2P_RMAX = 256;  // source ranges staged in LDS per pass
 // list, w = P2P_DIRECT (the item is the whole leaf: results go straight to
 // accel / pot) or the offset of its partial sums (one double4 per target).
 constexpr uint32_t P2P_OWN = 0x80000000u;
-constexpr uint32_t P2P_LEAF_MASK = 0x7fffffffu;
+constexpr uint32_t P2P_FIRST = 0x40000000u;  // launched among the first blocks (longs)
+constexpr uint32_t P2P_LEAF_MASK = 0x3fffffffu;
 constexpr uint32_t P2P_DIRECT = 0xffffffffu;
 
-struct TileLoad {
-  double4 v;
-  uint32_t fill;
+// The source stream of one segment: the item's nonempty source ranges back to
+// back, each as {stream position after it, slot - stream position in it}.
+// A tile is 64 consecutive stream positions. Its lanes find their ranges
+// together: 64 lanes look at the next 64 range ends and mark the lanes they
+// fall on (a forward lane permutation), and a lane's range is the tile's first
+// plus the marks up to it. The cost does not depend on the number of ranges;
+// walking them one by one took 13 dependent steps a tile at 5 bodies a leaf
+// (P2P of 1k bodies 44 us walked, 31 marked; of 1M at leaf capacity 16, 810
+// and 660 us) and was no faster at 30 bodies a leaf.
+struct StreamCursor {
+  uint32_t at;   // range holding the next tile's first position
+  uint32_t end;  // the lane's range end, ranges[at + lane].x
 };
 
-// Next tile of the packed source stream: advances the (range, offset)
-// cursor over up to 64 bodies; the lane's body is loaded (not yet waited on).
-__device__ __forceinline__ TileLoad gather_tile(const uint2* rng, uint32_t nr, uint32_t& r,
-                                                uint32_t& off, uint32_t lane,
-                                                const double4* __restrict__ body, double4 pad) {
-  uint32_t fill = 0;
-  int slot = -1;
-  while (fill < 64 && r < nr) {
-    const uint2 g = rng[r];
-    const uint32_t take = min(g.y - off, 64u - fill);
-    if (lane >= fill && lane < fill + take) slot = (int)(g.x + off + (lane - fill));
-    fill += take;
-    off += take;
-    if (off == g.y) {
-      r++;
-      off = 0;
-    }
-  }
-  TileLoad t;
-  t.v = body[slot >= 0 ? slot : 0];  // in-bounds load, then padded by value
-  if (slot < 0) t.v = pad;
-  t.fill = fill;
-  return t;
+// The lane's body of the tile at `pos` (loaded, not waited on; past the
+// stream's end any body: the caller pads).
+__device__ __forceinline__ double4 gather_tile(const uint2* ranges, uint32_t nr, uint32_t total,
+                                               uint32_t pos, StreamCursor& c, uint32_t lane,
+                                               const double4* __restrict__ body) {
+  const uint32_t e = c.at + lane < nr ? c.end - pos : 0xFFFFFFFFu;  // > 0: `at` holds pos
+  // ends past the tile are sent to lane 0, where no range can end
+  const int got = __builtin_amdgcn_ds_permute((int)(e < 64u ? e : 0u) * 4, 1);
+  const uint64_t marks = __ballot(got == 1) & ~1ull;
+  const uint32_t r = c.at + (uint32_t)__popcll(marks & (lanemask_lt() | (1ull << lane)));
+  const uint32_t d = ranges[min(r, nr - 1)].y;
+  c.at += (uint32_t)__popcll(__ballot(e <= 64u));
+  c.end = ranges[min(c.at + lane, nr - 1)].x;  // for the next tile
+  return body[pos + lane < total ? pos + lane + d : 0u];
 }
 
 // The two forms of the pairwise terms. FP64: absolute positions, the
@@ -98,11 +102,7 @@ __device__ __forceinline__ void p2p_tile(const typename P2PForm<F32>::T4* __rest
                                          typename P2PForm<F32>::T& ph) {
   using F = P2PForm<F32>;
   using T = typename F::T;
-  // FP32: 8 reads in flight per lane; FP64 (twice the registers per entry,
-  // longer rsqrt): 4
-#pragma unroll(F32 ? 8 : 4)
-  for (uint32_t i = 0; i < 64 / K; i++) {
-    const auto sj = ts[i * K];
+  auto pair = [&](const auto sj, uint32_t i) {
     const T dx = sj.x - xi, dy = sj.y - yi, dz = sj.z - zi;
     T r2 = F::fmat(dx, dx, F::fmat(dy, dy, F::fmat(dz, dz, soft2)));
     T mj = sj.w;
@@ -119,6 +119,25 @@ __device__ __forceinline__ void p2p_tile(const typename P2PForm<F32>::T4* __rest
     ay = F::fmat(s3, dy, ay);
     az = F::fmat(s3, dz, az);
     ph += minv;
+  };
+  if constexpr (F32) {  // 8 reads in flight per lane
+#pragma unroll 8
+    for (uint32_t i = 0; i < 64 / K; i++) pair(ts[i * K], i);
+  } else {
+    // four entries (twice the registers each) are read, then computed: the
+    // scheduling barrier keeps the compiler from sinking each read to its use,
+    // where the wave waits out the LDS latency once per entry (8.4M bodies:
+    // 32.0 ms without, 30.6 with; eight entries 32.8)
+    constexpr uint32_t N = 64 / K, U = N < 4 ? N : 4;
+#pragma unroll 1
+    for (uint32_t i0 = 0; i0 < N; i0 += U) {
+      typename F::T4 e[U];
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) e[u] = ts[(i0 + u) * K];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) pair(e[u], i0 + u);
+    }
   }
 }
 
@@ -194,24 +213,43 @@ __device__ __forceinline__ void acc2(double& s, double& c, double v) {
   s = t;
 }
 
-// Slot ranges of one segment of an item's source stream into LDS: rng[0] =
-// the leaf's own bodies when the stream starts with them (else empty), then
-// each directed entry's source leaf (first slot, count), the own leaf's entry
-// emptied. The barriers keep the previous pass's readers and this pass's
-// readers apart.
-__device__ __forceinline__ void stage_ranges(uint2* rng, const uint64_t* __restrict__ skeys,
+// One segment of an item's source stream into LDS: the leaf's own bodies
+// first when the stream starts with them, then each directed entry's source
+// leaf (its slots), the own leaf's entry left out. Returns the stream length
+// and the number of ranges. The barriers keep the previous pass's readers and
+// this pass's readers apart.
+__device__ __forceinline__ void stage_ranges(uint2* ranges, const uint64_t* __restrict__ skeys,
                                              uint64_t smask, const uint32_t* __restrict__ cfirst,
                                              const uint32_t* __restrict__ ccount, uint32_t ft,
-                                             uint32_t nt_all, bool pre, uint32_t seg, uint32_t nr,
-                                             uint32_t lane) {
+                                             uint32_t nt_all, bool pre, uint32_t seg, uint32_t n,
+                                             uint32_t lane, uint32_t* nr, uint32_t* total) {
   __syncthreads();
-  if (lane == 0) rng[0] = make_uint2(ft, pre ? nt_all : 0u);
-  for (uint32_t q = lane; q < nr; q += 64) {
-    const uint32_t src = (uint32_t)(skeys[seg + q] & smask);
-    uint2 g = make_uint2(cfirst[src], ccount[src]);
-    if (g.x == ft) g.y = 0;
-    rng[1 + q] = g;
+  uint32_t at = 0, len = 0;
+  if (pre) {
+    if (lane == 0) ranges[0] = make_uint2(nt_all, ft);
+    at = 1;
+    len = nt_all;
   }
+  for (uint32_t q0 = 0; q0 < n; q0 += 64) {
+    const uint32_t q = q0 + lane;
+    uint32_t first = 0, c = 0;
+    if (q < n) {
+      const uint32_t src = (uint32_t)(skeys[seg + q] & smask);
+      first = cfirst[src];
+      c = first == ft ? 0u : ccount[src];
+    }
+    uint32_t sum;
+    const uint32_t start = len + wave_excl_scan(c, &sum);
+    const uint64_t full = __ballot(c > 0u);
+    if (c > 0u) {
+      const uint32_t k = at + (uint32_t)__popcll(full & lanemask_lt());
+      ranges[k] = make_uint2(start + c, first - start);
+    }
+    at += (uint32_t)__popcll(full);
+    len += sum;
+  }
+  *nr = (uint32_t)wave_uniform((int)at);
+  *total = (uint32_t)wave_uniform((int)len);
   __syncthreads();
 }
 
@@ -224,23 +262,32 @@ __device__ __forceinline__ void stage_ranges(uint2* rng, const uint64_t* __restr
 // before the current one is computed. The mixed form (F32) sums each tile in
 // FP32 and compensates the final sums (sub-lane partials, then the far field).
 #define FMMH_P2P_PARAMS                                                                     \
-  const uint4 *__restrict__ items, const uint64_t *__restrict__ skeys, uint64_t smask,       \
+  const uint4 *__restrict__ items, uint32_t nlong, const uint32_t *__restrict__ longs, const uint64_t *__restrict__ skeys, uint64_t smask,       \
       const uint32_t *__restrict__ cfirst, const uint32_t *__restrict__ ccount,               \
       const double *__restrict__ ccx, const double *__restrict__ ccy,                         \
       const double *__restrict__ ccz, const double4 *__restrict__ body, double soft2,         \
       const double4 *__restrict__ far, const uint32_t *__restrict__ order,                    \
       double *__restrict__ accel, double *__restrict__ pot, double4 *__restrict__ partial
 #define FMMH_P2P_ARGS \
-  items, skeys, smask, cfirst, ccount, ccx, ccy, ccz, body, soft2, far, order, accel, pot, partial
+  items, nlong, longs, skeys, smask, cfirst, ccount, ccx, ccy, ccz, body, soft2, far, order,   \
+      accel, pot, partial
 
 template <bool F32>
 __device__ __forceinline__ void p2p_item(FMMH_P2P_PARAMS) {
   using F = P2PForm<F32>;
   using T = typename F::T;
   __shared__ typename F::T4 tile[64];
-  __shared__ uint2 rng[P2P_RMAX + 1];
+  __shared__ uint2 ranges[P2P_RMAX + 1];
   const uint32_t lane = threadIdx.x;
-  const uint4 it = items[xcd_block(blockIdx.x, gridDim.x)];
+  // the first nlong blocks take the long items, the others every item in
+  // leaf order but those
+  uint4 it;
+  if (blockIdx.x < nlong) {
+    it = items[longs[blockIdx.x]];
+  } else {
+    it = items[xcd_block(blockIdx.x - nlong, gridDim.x - nlong)];
+    if (it.x & P2P_FIRST) return;
+  }
   const uint32_t leaf = it.x & P2P_LEAF_MASK;
   const bool own = (it.x & P2P_OWN) != 0u;
   const uint32_t ft = cfirst[leaf], nt_all = ccount[leaf];
@@ -248,9 +295,12 @@ __device__ __forceinline__ void p2p_item(FMMH_P2P_PARAMS) {
   // the mixed form works relative to the leaf's centre; FP64 in place
   const double cx = F32 ? ccx[leaf] : 0.0, cy = F32 ? ccy[leaf] : 0.0,
                cz = F32 ? ccz[leaf] : 0.0;
-  const double4 pad = make_double4(cx + 1e18, cy + 1e18, cz + 1e18, 0.0);
+  typename F::T4 pad;  // past the stream's end: far away and massless
+  pad.x = pad.y = pad.z = T(1e18);
+  pad.w = T(0);
   const T s2 = (T)soft2;
   const uint32_t nseg = (je - jb + P2P_RMAX - 1) / P2P_RMAX;
+  uint32_t nr = 0, total = 0;
   for (uint32_t t0 = 0; t0 < nt_all; t0 += 64) {
     const uint32_t r = min(64u, nt_all - t0);
     uint32_t n[P2P_NQ];
@@ -279,18 +329,21 @@ __device__ __forceinline__ void p2p_item(FMMH_P2P_PARAMS) {
     const uint32_t npass = max(nseg, own ? 1u : 0u);
     for (uint32_t sg = 0; sg < npass; sg++) {
       const uint32_t seg = jb + sg * P2P_RMAX;
-      const uint32_t nr = seg < je ? min(P2P_RMAX, je - seg) : 0u;
+      const uint32_t nseq = seg < je ? min(P2P_RMAX, je - seg) : 0u;
       const bool pre = own && sg == 0;  // stream starts with the own leaf
       // an item of one segment stages its ranges once, for every group
-      if (nseg > 1 || t0 == 0) stage_ranges(rng, skeys, smask, cfirst, ccount, ft, nt_all, pre,
-                                            seg, nr, lane);
-      uint32_t rr = 0, off = 0, pos = 0;
-      TileLoad cur = gather_tile(rng, nr + 1, rr, off, lane, body, pad);
-      while (cur.fill > 0) {
-        tile[lane] = F::stage(cur.v, cx, cy, cz);
-        const uint32_t fill = cur.fill;
+      if (nseg > 1 || t0 == 0)
+        stage_ranges(ranges, skeys, smask, cfirst, ccount, ft, nt_all, pre, seg, nseq, lane, &nr,
+                     &total);
+      if (total == 0) continue;
+      // the next tile's bodies are on their way while one is computed (padded
+      // only when staged: a select on the loaded value would wait for it here)
+      StreamCursor cur{0u, ranges[min(lane, nr - 1)].x};
+      double4 next = gather_tile(ranges, nr, total, 0u, cur, lane, body);
+      for (uint32_t pos = 0; pos < total; pos += 64) {
+        tile[lane] = pos + lane < total ? F::stage(next, cx, cy, cz) : pad;
         __syncthreads();
-        cur = gather_tile(rng, nr + 1, rr, off, lane, body, pad);
+        if (pos + 64 < total) next = gather_tile(ranges, nr, total, pos + 64, cur, lane, body);
         const bool self_tile = pre && pos < nt_all;
 #pragma unroll
         for (int q = 0; q < P2P_NQ; q++) {
@@ -317,7 +370,6 @@ __device__ __forceinline__ void p2p_item(FMMH_P2P_PARAMS) {
                                       ay[q], az[q], ph[q]);
           }
         }
-        pos += fill;
         __syncthreads();
       }
     }
@@ -384,22 +436,39 @@ __global__ void __launch_bounds__(64) k_p2p_fp64(FMMH_P2P_PARAMS) {
   p2p_item<false>(FMMH_P2P_ARGS);
 }
 
-// ------------------------------------------------------- P2P work plan
-// A leaf's P2P work is its target count times its source bodies (own leaf
-// plus neighbour leaves). One block per leaf leaves the whole device waiting
-// on the few leaves whose neighbourhoods are huge (a large sparse leaf beside
-// a dense region), so a leaf whose work exceeds the context's item bound W
-// (fmmh_tuning.p2p_item_work, default 2^18) is cut into m = ceil(work / W)
-// work items (at most one per source unit).
+// ------------------------------------------------------- the lists' work plan
+// M2L: a target's sources in chunks of at most `ch`. P2P: a leaf's work is its
+// target count times its source bodies (own leaf plus neighbour leaves). One
+// block per leaf leaves the whole device waiting on the few leaves whose
+// neighbourhoods are huge (a large sparse leaf beside a dense region), so a
+// leaf is cut into m work items (at most one per source unit): m = work / W
+// where the work exceeds the context's item bound W (fmmh_tuning.p2p_item_work,
+// default 2^18), and in the FP64 form at least one item per P2P_CAP sources.
 // Source units are the own leaf (unit 0) and the neighbour ranges in list
 // order; unit u with P_u sources before it goes to item
 // min(m - 1, P_u / ceil(S / m)) (items may come out empty). Split items write
 // partial sums that k_p2p_reduce adds in item order. The cut depends on the
 // leaf's own counts only, so a system evaluates the same alone and in an
-// ensemble. One wave per leaf in both plan kernels.
+// ensemble.
+//
+// P2P_CAP: an item is one wave streaming its sources tile by tile, about 1.4
+// us per 64 sources however few the targets are, so a leaf of 10 bodies with
+// 26000 sources (2^18 pairs, one item) ran for 600 us: all of the near field's
+// time at 16k and at 100k bodies. P2P with no cap, 8192, 6144 and 4096 sources:
+// 100k bodies 414, 303, 247 and 243 us, 16k 620 (no cap), 182, 124 and 95; at
+// 8.4M bodies (4485 sources a leaf) 4096 costs 0.3 of 30.4 ms against no cap.
+// The mixed form keeps its items (their tiles are what its FP32 sums are
+// grouped by). In both forms the long items (over P2P_LONG64 / P2P_LONG32
+// sources), which would otherwise start wherever their leaf comes and end last,
+// are launched first, where they are few (by index, in no particular order: an
+// item's results do not depend on when it runs): 100k bodies 382 -> 267 us,
+// mixed ensemble of 1.5M bodies 4.39 -> 4.13 ms.
 constexpr int PLAN_T = 256;
+constexpr uint32_t P2P_CAP = 4096;
+constexpr uint32_t P2P_LONG64 = 2048, P2P_LONG32 = 8192;
+constexpr uint32_t PLAN_SHORT = 32;  // a list of so few neighbours is never a long one
 
-__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
+__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
@@ -407,114 +476,150 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
 
 struct LeafCut {
   uint32_t leaf, nt, jb, je;
-  uint64_t S, m;
+  uint32_t S, m;  // sources (distinct bodies, so below 2^32), items
 };
 
-// Source total and item count of leaf i (all lanes get the result).
-__device__ __forceinline__ LeafCut leaf_cut(uint32_t i, const uint32_t* __restrict__ leaf_ids,
-                                            const uint32_t* __restrict__ pptr,
+// How a form's leaves are cut: work per item, sources per item, and the
+// sources from which an item counts as long.
+struct CutRule {
+  uint64_t W;
+  uint32_t cap, lng;
+};
+
+// Source total and item count of a leaf (all lanes get the result).
+__device__ __forceinline__ LeafCut leaf_cut(uint32_t leaf, const uint32_t* __restrict__ pptr,
                                             const uint64_t* __restrict__ skeys, uint64_t smask,
-                                            const uint32_t* __restrict__ ccount, uint64_t W,
+                                            const uint32_t* __restrict__ ccount, CutRule cut,
                                             uint32_t lane) {
   LeafCut L;
-  L.leaf = leaf_ids[i];
-  L.nt = ccount[L.leaf];
-  L.jb = pptr[L.leaf];
-  L.je = pptr[L.leaf + 1];
-  uint64_t s = 0;
+  L.leaf = leaf;
+  L.nt = ccount[leaf];
+  L.jb = pptr[leaf];
+  L.je = pptr[leaf + 1];
+  uint32_t s = 0;
+#pragma unroll 4
   for (uint32_t j = L.jb + lane; j < L.je; j += 64) {
     const uint32_t src = (uint32_t)(skeys[j] & smask);
-    s += src == L.leaf ? 0u : ccount[src];
+    s += src == leaf ? 0u : ccount[src];
   }
-  L.S = (uint64_t)L.nt + wave_sum_u64(s);
+  L.S = L.nt + wave_sum_u32(s);
   const uint64_t work = (uint64_t)L.nt * L.S;
-  uint64_t m = work > W ? (work + W - 1) / W : 1;
+  uint64_t m = work > cut.W ? (work + cut.W - 1) / cut.W : 1;
+  if (L.S > cut.cap) m = max(m, (uint64_t)((L.S - 1) / cut.cap + 1));
   const uint64_t units = (uint64_t)(L.je - L.jb) + 1;
-  L.m = m > units ? units : m;
+  L.m = (uint32_t)min(m, units);
   return L;
 }
 
-__global__ void __launch_bounds__(PLAN_T) k_p2p_plan_count(const uint32_t* __restrict__ leaf_ids,
-                                                          uint32_t nleaves,
-                                                          const uint32_t* __restrict__ pptr,
-                                                          const uint64_t* __restrict__ skeys,
-                                                          uint64_t smask,
-                                                          const uint32_t* __restrict__ ccount,
-                                                          uint64_t W, uint32_t* __restrict__ nitem,
-                                                          uint32_t* __restrict__ npart,
-                                                          uint32_t* __restrict__ nsplit) {
-  const uint32_t i = blockIdx.x * (PLAN_T / 64) + (threadIdx.x >> 6);
-  const uint32_t lane = threadIdx.x & 63;
-  if (i > nleaves) return;
-  if (i == nleaves) {  // the scans' closing element
-    if (lane == 0) nitem[i] = npart[i] = nsplit[i] = 0u;
-    return;
+// Whether a leaf's items are launched first.
+__device__ __forceinline__ bool long_items(const LeafCut& L, CutRule cut) {
+  return L.je - L.jb > PLAN_SHORT && L.S / L.m > cut.lng;
+}
+
+// {M2L chunks, P2P items, partial-sum slots, cut leaves} of cell t in plan[t];
+// plan[nc] = 0 closes the scan and plan[nc + 1].x counts the long items. One
+// wave per cell at a time, at most PLAN_BLOCKS blocks, each adding its long
+// items at once: one addition per long leaf serialised on that word (2.6 ms
+// at 280k leaves).
+constexpr uint32_t PLAN_BLOCKS = 2048;
+
+__global__ void __launch_bounds__(PLAN_T) k_plan_count(
+    uint32_t nc, const uint8_t* __restrict__ leaf, const uint32_t* __restrict__ tptr, uint32_t ch,
+    const uint32_t* __restrict__ pptr, const uint64_t* __restrict__ skeys, uint64_t smask,
+    const uint32_t* __restrict__ ccount, CutRule cut, uint4* __restrict__ plan) {
+  __shared__ uint32_t lng[PLAN_T / 64];
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  uint32_t nl = 0;
+  for (uint32_t t = blockIdx.x * (PLAN_T / 64) + wave; t <= nc; t += gridDim.x * (PLAN_T / 64)) {
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if (t < nc) {
+      v.x = (tptr[t + 1] - tptr[t] + ch - 1) / ch;
+      if (leaf[t]) {
+        const LeafCut L = leaf_cut(t, pptr, skeys, smask, ccount, cut, lane);
+        v.y = L.m;
+        v.z = L.m > 1 ? L.m * L.nt : 0u;
+        v.w = L.m > 1 ? 1u : 0u;
+        if (long_items(L, cut)) nl += L.m;
+      }
+    }
+    if (lane == 0) plan[t] = v;
   }
-  const LeafCut L = leaf_cut(i, leaf_ids, pptr, skeys, smask, ccount, W, lane);
-  if (lane == 0) {
-    const uint32_t m = (uint32_t)L.m;
-    nitem[i] = m;
-    npart[i] = m > 1 ? m * L.nt : 0u;
-    nsplit[i] = m > 1 ? 1u : 0u;
+  if (lane == 0) lng[wave] = nl;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    nl = 0;
+    for (int w = 0; w < PLAN_T / 64; w++) nl += lng[w];
+    if (nl) atomicAdd(&plan[nc + 1].x, nl);
   }
 }
 
-__global__ void __launch_bounds__(PLAN_T) k_p2p_plan_emit(const uint32_t* __restrict__ leaf_ids,
-                                                         uint32_t nleaves,
-                                                         const uint32_t* __restrict__ pptr,
-                                                         const uint64_t* __restrict__ skeys,
-                                                         uint64_t smask,
-                                                         const uint32_t* __restrict__ ccount,
-                                                         uint64_t W,
-                                                         const uint32_t* __restrict__ ioff,
-                                                         const uint32_t* __restrict__ poff,
-                                                         const uint32_t* __restrict__ roff,
-                                                         uint4* __restrict__ items,
-                                                         uint4* __restrict__ reds) {
-  const uint32_t i = blockIdx.x * (PLAN_T / 64) + (threadIdx.x >> 6);
+// plan: the scanned counts. Writes the chunks, the items, the records of cut
+// leaves and, unless nlong is null, the indices of the long items (their slots
+// counted in *nlong).
+__global__ void __launch_bounds__(PLAN_T) k_plan_emit(
+    uint32_t nc, const uint8_t* __restrict__ leaf, const uint32_t* __restrict__ tptr, uint32_t ch,
+    const uint32_t* __restrict__ pptr, const uint64_t* __restrict__ skeys, uint64_t smask,
+    const uint32_t* __restrict__ ccount, CutRule cut, const uint4* __restrict__ plan,
+    M2lChunk* __restrict__ chunks, uint4* __restrict__ items, uint4* __restrict__ reds,
+    uint32_t* __restrict__ nlong, uint32_t* __restrict__ longs) {
+  const uint32_t t = blockIdx.x * (PLAN_T / 64) + (threadIdx.x >> 6);
   const uint32_t lane = threadIdx.x & 63;
-  if (i >= nleaves) return;
-  const uint32_t base = ioff[i];
-  if (ioff[i + 1] - base == 1) {  // one item (the count pass found m = 1): the whole list
-    if (lane == 0) {
-      const uint32_t leaf = leaf_ids[i];
-      items[base] = make_uint4(leaf | P2P_OWN, pptr[leaf], pptr[leaf + 1], P2P_DIRECT);
-    }
+  if (t >= nc) return;
+  const uint4 at = plan[t];
+  {
+    const uint32_t b = tptr[t], e = tptr[t + 1];
+    for (uint32_t k = lane; b + k * ch < e; k += 64)
+      chunks[at.x + k] = M2lChunk{t, b + k * ch, min(e, b + (k + 1) * ch)};
+  }
+  if (!leaf[t]) return;
+  const uint32_t base = at.y;
+  const uint32_t m = plan[t + 1].y - base;
+  // one item: the whole list, not read again
+  if (m == 1 && (!nlong || pptr[t + 1] - pptr[t] <= PLAN_SHORT)) {
+    if (lane == 0) items[base] = make_uint4(t | P2P_OWN, pptr[t], pptr[t + 1], P2P_DIRECT);
     return;
   }
-  const LeafCut L = leaf_cut(i, leaf_ids, pptr, skeys, smask, ccount, W, lane);
-  const uint32_t m = (uint32_t)L.m;
-  const uint32_t pb = poff[i];
+  const LeafCut L = leaf_cut(t, pptr, skeys, smask, ccount, cut, lane);
+  const bool lng = nlong && long_items(L, cut);
+  const uint32_t mark = lng ? P2P_FIRST : 0u;
+  if (lng) {
+    uint32_t w = 0;
+    if (lane == 0) w = atomicAdd(nlong, m);
+    w = (uint32_t)__shfl((int)w, 0, 64);
+    for (uint32_t k = lane; k < m; k += 64) longs[w + k] = base + k;
+  }
   uint32_t* it = (uint32_t*)(items + base);  // [m][4]: leaf|own, begin, end, slot
   for (uint32_t k = lane; k < m; k += 64) {
-    it[4 * k] = L.leaf | (k == 0 ? P2P_OWN : 0u);
-    it[4 * k + 3] = m > 1 ? pb + k * L.nt : P2P_DIRECT;
+    it[4 * k] = L.leaf | mark | (k == 0 ? P2P_OWN : 0u);
+    it[4 * k + 3] = m > 1 ? at.z + k * L.nt : P2P_DIRECT;
   }
   if (lane == 0) {
     it[1] = L.jb;
-    if (m > 1) reds[roff[i]] = make_uint4(L.leaf, pb, m, 0u);
+    if (m > 1) reds[at.w] = make_uint4(L.leaf, at.z, m, 0u);
   }
   // item boundaries: where the unit's item index steps up
-  const uint64_t T = (L.S + L.m - 1) / L.m;
-  uint64_t running = L.nt;  // sources before the first neighbour unit
+  const uint32_t T = (L.S - 1) / m + 1;
+  uint32_t running = L.nt;  // sources before the first neighbour unit
   uint32_t gprev = 0;       // item of unit 0 (the own leaf)
-  for (uint32_t c0 = L.jb; c0 < L.je; c0 += 64) {
+  auto unit = [&](uint32_t j) -> uint32_t {
+    if (j >= L.je) return 0u;
+    const uint32_t src = (uint32_t)(skeys[j] & smask);
+    return src == L.leaf ? 0u : ccount[src];
+  };
+  uint32_t next = unit(L.jb + lane);  // the following 64 units' counts, loaded ahead
+  for (uint32_t c0 = L.jb; m > 1 && c0 < L.je; c0 += 64) {
     const uint32_t j = c0 + lane;
     const bool valid = j < L.je;
-    uint64_t cnt = 0;
-    if (valid) {
-      const uint32_t src = (uint32_t)(skeys[j] & smask);
-      cnt = src == L.leaf ? 0u : ccount[src];
-    }
-    uint64_t incl = cnt;  // inclusive wave scan
+    const uint32_t cnt = next;
+    next = unit(j + 64);
+    uint32_t incl = cnt;  // inclusive wave scan
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      const uint64_t v = __shfl_up(incl, o, 64);
+      const uint32_t v = __shfl_up(incl, o, 64);
       if ((int)lane >= o) incl += v;
     }
-    const uint64_t P = running + incl - cnt;
-    const uint64_t gq = P / T;
-    const uint32_t g = valid ? (uint32_t)(gq < L.m - 1 ? gq : L.m - 1) : 0u;
+    const uint32_t P = running + incl - cnt;
+    const uint32_t g = valid ? min(P / T, m - 1) : 0u;
     const uint32_t gl = (uint32_t)__shfl_up(g, 1, 64);
     const uint32_t before = lane == 0 ? gprev : gl;
     if (valid && g > before)
@@ -573,27 +678,27 @@ __global__ void __launch_bounds__(64) k_p2p_reduce(const uint4* __restrict__ red
   }
 }
 
-// Work plan of the current P2P lists. nitem / npart / nsplit are nleaves + 1
-// words each (scanned in place); the totals come back through the host.
-void p2p_plan_count(const uint32_t* leaf_ids, uint32_t nleaves, const uint32_t* pptr,
-                    const uint64_t* skeys, int sbits, const uint32_t* ccount, uint64_t item_work,
-                    uint32_t* nitem, uint32_t* npart, uint32_t* nsplit, hipStream_t s) {
-  if (nleaves == 0) return;
-  const uint64_t smask = (1ull << sbits) - 1ull;
-  hipLaunchKernelGGL(k_p2p_plan_count, dim3((nleaves + 1 + PLAN_T / 64 - 1) / (PLAN_T / 64)),
-                     dim3(PLAN_T), 0, s, leaf_ids,
-                     nleaves, pptr, skeys, smask, ccount, item_work, nitem, npart, nsplit);
+static CutRule cut_rule(uint64_t item_work, bool fp32) {
+  return fp32 ? CutRule{item_work, 0xFFFFFFFFu, P2P_LONG32} : CutRule{item_work, P2P_CAP, P2P_LONG64};
 }
 
-void p2p_plan_emit(const uint32_t* leaf_ids, uint32_t nleaves, const uint32_t* pptr,
-                   const uint64_t* skeys, int sbits, const uint32_t* ccount, uint64_t item_work,
-                   const uint32_t* ioff, const uint32_t* poff, const uint32_t* roff, uint4* items,
-                   uint4* reds, hipStream_t s) {
-  if (nleaves == 0) return;
-  const uint64_t smask = (1ull << sbits) - 1ull;
-  hipLaunchKernelGGL(k_p2p_plan_emit, dim3((nleaves + PLAN_T / 64 - 1) / (PLAN_T / 64)),
-                     dim3(PLAN_T), 0, s, leaf_ids,
-                     nleaves, pptr, skeys, smask, ccount, item_work, ioff, poff, roff, items, reds);
+// plan: nc + 2 entries, zeroed at [nc + 1] by the caller; scanned by the
+// caller between the two.
+void plan_count(uint32_t nc, DevCells c, const uint32_t* tptr, uint32_t ch, const uint32_t* pptr,
+                const uint64_t* skeys, int sbits, uint64_t item_work, bool fp32, uint4* plan,
+                hipStream_t s) {
+  const uint32_t nb = std::min(PLAN_BLOCKS, (nc + 1 + PLAN_T / 64 - 1) / (PLAN_T / 64));
+  hipLaunchKernelGGL(k_plan_count, dim3(nb), dim3(PLAN_T), 0, s, nc, c.leaf, tptr, ch, pptr, skeys, (1ull << sbits) - 1ull, c.count,
+                     cut_rule(item_work, fp32), plan);
+}
+
+void plan_emit(uint32_t nc, DevCells c, const uint32_t* tptr, uint32_t ch, const uint32_t* pptr,
+               const uint64_t* skeys, int sbits, uint64_t item_work, bool fp32, const uint4* plan,
+               void* chunks, uint4* items, uint4* reds, uint32_t* nlong, uint32_t* longs,
+               hipStream_t s) {
+  hipLaunchKernelGGL(k_plan_emit, dim3((nc + PLAN_T / 64 - 1) / (PLAN_T / 64)), dim3(PLAN_T), 0, s,
+                     nc, c.leaf, tptr, ch, pptr, skeys, (1ull << sbits) - 1ull, c.count,
+                     cut_rule(item_work, fp32), plan, (M2lChunk*)chunks, items, reds, nlong, longs);
 }
 
 void launch_p2p_f32(const P2PPlan& pl, DevCells c, const double4* body, const uint64_t* skeys,
@@ -601,7 +706,8 @@ void launch_p2p_f32(const P2PPlan& pl, DevCells c, const double4* body, const ui
                     double* accel, double* pot, hipStream_t s) {
   if (pl.nitems == 0) return;
   const uint64_t smask = (1ull << sbits) - 1ull;
-  hipLaunchKernelGGL(k_p2p_mixed, dim3(pl.nitems), dim3(64), 0, s, pl.items, skeys, smask, c.first,
+  hipLaunchKernelGGL(k_p2p_mixed, dim3(pl.nitems + pl.nlong),
+                     dim3(64), 0, s, pl.items, pl.nlong, pl.longs, skeys, smask, c.first,
                      c.count, c.cx, c.cy, c.cz, body, soft2, far, order, accel, pot, pl.partial);
 }
 
@@ -621,7 +727,8 @@ void launch_p2p(const P2PPlan& pl, DevCells c, const double4* body, const uint64
                 double* pot, hipStream_t s) {
   if (pl.nitems == 0) return;
   const uint64_t smask = (1ull << sbits) - 1ull;
-  hipLaunchKernelGGL(k_p2p_fp64, dim3(pl.nitems), dim3(64), 0, s, pl.items, skeys, smask, c.first,
+  hipLaunchKernelGGL(k_p2p_fp64, dim3(pl.nitems + pl.nlong),
+                     dim3(64), 0, s, pl.items, pl.nlong, pl.longs, skeys, smask, c.first,
                      c.count, c.cx, c.cy, c.cz, body, soft2, far, order, accel, pot, pl.partial);
 }
 

@@ -20,8 +20,60 @@
 namespace fmmh {
 
 constexpr int SCAN_T = 256;
-constexpr int SCAN_I = 16;
-constexpr int SCAN_TILE = SCAN_T * SCAN_I;
+
+// Four counts scanned together.
+struct alignas(16) U4 {
+  uint32_t x, y, z, w;
+  U4() = default;
+  __device__ __forceinline__ U4(int v) : x(v), y(v), z(v), w(v) {}
+  __device__ __forceinline__ U4& operator+=(const U4& o) {
+    x += o.x;
+    y += o.y;
+    z += o.z;
+    w += o.w;
+    return *this;
+  }
+  __device__ __forceinline__ U4& operator-=(const U4& o) {
+    x -= o.x;
+    y -= o.y;
+    z -= o.z;
+    w -= o.w;
+    return *this;
+  }
+  __device__ __forceinline__ U4 operator+(const U4& o) const {
+    U4 r = *this;
+    r += o;
+    return r;
+  }
+};
+__device__ __forceinline__ bool is_zero(const U4& v) { return (v.x | v.y | v.z | v.w) == 0u; }
+template <class T>
+__device__ __forceinline__ bool is_zero(T v) {
+  return v == 0;
+}
+template <class T>
+__device__ __forceinline__ T lane_up(T v, int o) {
+  return __shfl_up(v, o, 64);
+}
+template <>
+__device__ __forceinline__ U4 lane_up<U4>(U4 v, int o) {
+  U4 r(0);
+  r.x = __shfl_up(v.x, o, 64);
+  r.y = __shfl_up(v.y, o, 64);
+  r.z = __shfl_up(v.z, o, 64);
+  r.w = __shfl_up(v.w, o, 64);
+  return r;
+}
+
+// Elements per thread and per tile (16 KB of LDS for u32 and the quadruples).
+template <class T>
+constexpr int scan_i() {
+  return sizeof(T) > 8 ? 4 : 16;
+}
+template <class T>
+constexpr int scan_tile() {
+  return SCAN_T * scan_i<T>();
+}
 
 // Block-wide exclusive scan of one value per thread (256 threads).
 template <class T>
@@ -30,7 +82,7 @@ __device__ __forceinline__ T block_excl_scan(T v, T* total, T* sh) {
   T x = v;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    const T y = __shfl_up(x, o, 64);
+    const T y = lane_up(x, o);
     if (lane >= o) x += y;
   }
   if (lane == 63) sh[w] = x;
@@ -52,6 +104,7 @@ template <class T>
 __global__ void __launch_bounds__(SCAN_T) k_scan_tiles(const T* __restrict__ in,
                                                       T* __restrict__ out, size_t n,
                                                       T* __restrict__ tile_sums) {
+  constexpr int SCAN_I = scan_i<T>(), SCAN_TILE = scan_tile<T>();
   __shared__ T tile[SCAN_TILE];
   __shared__ T sh[SCAN_T / 64];
   const size_t base = (size_t)blockIdx.x * SCAN_TILE;
@@ -101,9 +154,10 @@ __global__ void __launch_bounds__(SCAN_T) k_scan_sums(T* __restrict__ sums, size
 template <class T>
 __global__ void __launch_bounds__(SCAN_T) k_scan_add(T* __restrict__ out, size_t n,
                                                     const T* __restrict__ sums) {
+  constexpr int SCAN_I = scan_i<T>(), SCAN_TILE = scan_tile<T>();
   const T add = sums[blockIdx.x];
   const size_t base = (size_t)blockIdx.x * SCAN_TILE;
-  if (add == 0) return;
+  if (is_zero(add)) return;
 #pragma unroll
   for (int j = 0; j < SCAN_I; j++) {
     size_t e = base + (size_t)j * SCAN_T + threadIdx.x;
@@ -118,12 +172,13 @@ template <class T>
 __global__ void __launch_bounds__(SCAN_T) k_scan_add_small(T* __restrict__ out, size_t n,
                                                           T* __restrict__ sums,
                                                           uint32_t ntiles) {
+  constexpr int SCAN_I = scan_i<T>(), SCAN_TILE = scan_tile<T>();
   __shared__ T sh[SCAN_T / 64];
   const T v = threadIdx.x < blockIdx.x ? sums[threadIdx.x] : T(0);
   T add;
   block_excl_scan(v, &add, sh);
   if (blockIdx.x == ntiles - 1 && threadIdx.x == 0) sums[ntiles] = add + sums[ntiles - 1];
-  if (add == 0) return;
+  if (is_zero(add)) return;
   const size_t base = (size_t)blockIdx.x * SCAN_TILE;
 #pragma unroll
   for (int j = 0; j < SCAN_I; j++) {
@@ -132,13 +187,15 @@ __global__ void __launch_bounds__(SCAN_T) k_scan_add_small(T* __restrict__ out, 
   }
 }
 
-size_t scan_tmp_words(size_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE + 1; }
+size_t scan_tmp_words(size_t n) {
+  return (n + scan_tile<uint32_t>() - 1) / scan_tile<uint32_t>() + 1;
+}
 
 // Exclusive scan; in may equal out. tmp needs scan_tmp_words(n) elements; the
 // grand total lands in tmp[ntiles] (device) and *total_dev points at it.
 template <class T>
 static void scan_exclusive(const T* in, T* out, size_t n, T* tmp, hipStream_t s, T** total_dev) {
-  size_t ntiles = (n + SCAN_TILE - 1) / SCAN_TILE;
+  const size_t ntiles = (n + scan_tile<T>() - 1) / scan_tile<T>();
   if (ntiles == 0) {
     hipLaunchKernelGGL(k_scan_sums<T>, dim3(1), dim3(SCAN_T), 0, s, tmp, (size_t)0);
   } else {
@@ -164,6 +221,10 @@ void scan_exclusive_u32(const uint32_t* in, uint32_t* out, size_t n, uint32_t* t
 void scan_exclusive_u64(const uint64_t* in, uint64_t* out, size_t n, uint64_t* tmp, hipStream_t s,
                         uint64_t** total_dev) {
   scan_exclusive<uint64_t>(in, out, n, tmp, s, total_dev);
+}
+
+void scan_exclusive_u32x4(uint4* a, size_t n, uint4* tmp, hipStream_t s) {
+  scan_exclusive<U4>((const U4*)a, (U4*)a, n, (U4*)tmp, s, nullptr);
 }
 
 // ------------------------------------------------------------ radix sort
