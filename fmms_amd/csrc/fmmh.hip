@@ -741,7 +741,7 @@ struct fmmh_ctx {
     }
     ensure(m2l, (size_t)(32 * (size_t)nc + 1024) * 8);
     ensure(p2p, (size_t)(16 * (size_t)nc + 1024) * 8);
-    ensure(ctr, 64);
+    ensure(ctr, 2 * sizeof(WalkState));
     MacParams mp;
     mp.p = prm.p;
     mp.use_err = use_err ? 1 : 0;
@@ -754,8 +754,7 @@ struct fmmh_ctx {
     mp.soft_mac = prm.soft_mac;
     // the walk starts from the self pair of every (system) root: level vlev
     const uint32_t nf0 = lvl_off[vlev + 1] - lvl_off[vlev];
-    WalkState* st = (WalkState*)ctr.p;
-    HCHECK(hipMemsetAsync(st, 0, sizeof(WalkState), s));
+    WalkState* st = (WalkState*)ctr.p;  // [2]: round r reads st[r % 2], writes the other
     launch_front_init((const uint32_t*)lvl_cells.p + lvl_off[vlev], nf0, front_a.p, st, s);
     ensure(walk_blk, (size_t)3 * WALK_G * 4);
     Buf* fr[2] = {&front_a, &front_b};
@@ -769,11 +768,11 @@ struct fmmh_ctx {
       ensure(walk_code, (size_t)std::max(cap(front_a), cap(front_b)) * 2);
       const uint32_t batch = std::max<uint32_t>(4u, walk_batch);
       for (uint32_t k = 0; k < batch; k++, r++)
-        launch_walk_round(fr[r & 1u]->p, fr[(r + 1u) & 1u]->p, r, st, cap(*fr[(r + 1u) & 1u]),
-                          (uint2*)m2l.p, cap(m2l), (uint2*)p2p.p, cap(p2p),
+        launch_walk_round(fr[r & 1u]->p, fr[(r + 1u) & 1u]->p, r, st + (r & 1u),
+                          st + ((r + 1u) & 1u), cap(*fr[(r + 1u) & 1u]), (uint2*)m2l.p, cap(m2l), (uint2*)p2p.p, cap(p2p),
                           (uint16_t*)walk_code.p, (uint32_t*)walk_blk.p, walkrec.p,
-                          (const double*)c_mass.p, mp, s);
-      const WalkState h = read1((const WalkState*)st);
+                          (const double*)c_mass.p, mp, nc, s);
+      const WalkState h = read1((const WalkState*)(st + (r & 1u)));
       r = h.round;
       if (h.status != 0u) {
         // round r needs more room: its input frontier is kept, the rest grows
@@ -783,10 +782,14 @@ struct fmmh_ctx {
         }
         if (h.status & 2u) ensure(m2l, (size_t)h.need_m2l * 8 * 2, true);
         if (h.status & 4u) ensure(p2p, (size_t)h.need_p2p * 8 * 2, true);
-        HCHECK(hipMemsetAsync(&st->status, 0, sizeof(uint32_t), s));
+        WalkState* again = (WalkState*)host_stage(sizeof(WalkState));
+        *again = h;
+        again->status = 0u;
+        HCHECK(hipMemcpyAsync(st + (r & 1u), again, sizeof(WalkState), hipMemcpyHostToDevice, s));
+        HCHECK(hipStreamSynchronize(s));
         continue;
       }
-      if (h.fsize[r & 1u] == 0u) {
+      if (h.fsize == 0u) {
         n_m2l = h.n_m2l;
         n_p2p = h.n_p2p;
         walk_rounds = h.rounds;

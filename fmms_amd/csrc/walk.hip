@@ -47,13 +47,17 @@ __global__ void __launch_bounds__(256) k_pack_walk(uint32_t nc, DevCells c,
 size_t walk_rec_bytes() { return sizeof(WalkRec); }
 
 // Initial walk frontier: the self pairs (c, c) of the given cells (the root,
-// or every system root of an ensemble); its size goes to the walk state.
+// or every system root of an ensemble) and the first round's state.
 __global__ void __launch_bounds__(256) k_front_init(const uint32_t* __restrict__ cells,
                                                    uint32_t cnt, uint2* __restrict__ front,
                                                    WalkState* __restrict__ st) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   if (i < cnt) front[i] = make_uint2(cells[i], cells[i]);
-  if (i == 0) st->fsize[0] = cnt;
+  if (i == 0) {
+    WalkState w{};
+    w.fsize = cnt;
+    *st = w;
+  }
 }
 
 void launch_front_init(const uint32_t* cells, uint32_t cnt, void* front, WalkState* st,
@@ -153,17 +157,21 @@ __device__ __forceinline__ int decide(uint32_t a, uint32_t b, const WalkRec& ra,
 
 constexpr int CW_T = 256;
 
-// Sum of three counters over the block (CW_T threads); every thread gets it.
-__device__ __forceinline__ void block_sum3(uint32_t v[3], uint32_t (*sh)[3]) {
+// Sums of N counters over the block (CW_T threads); every thread gets them.
+template <int N>
+__device__ __forceinline__ void block_sum(uint32_t (&v)[N], uint32_t (*sh)[N]) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  for (int k = 0; k < 3; k++) {
+#pragma unroll
+  for (int k = 0; k < N; k++) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
   }
   if (lane == 0)
-    for (int k = 0; k < 3; k++) sh[w][k] = v[k];
+#pragma unroll
+    for (int k = 0; k < N; k++) sh[w][k] = v[k];
   __syncthreads();
-  for (int k = 0; k < 3; k++) {
+#pragma unroll
+  for (int k = 0; k < N; k++) {
     uint32_t t = 0;
     for (int q = 0; q < CW_T / 64; q++) t += sh[q][k];
     v[k] = t;
@@ -192,31 +200,40 @@ __device__ __forceinline__ void block_scan3(const uint32_t v[3], uint32_t x[3], 
   __syncthreads();
 }
 
-// The round's frontier slice of logical block lb: WALK_G blocks, each a
-// contiguous run of ceil(nf / WALK_G) pairs, in frontier order. Logical
-// blocks are spread so that each XCD takes a contiguous range of slices
-// (neighbouring pairs share cells, whose records then share one L2).
+// The round's frontier slice of logical block lb: contiguous runs of `chunk`
+// pairs in frontier order, over as many of the grid's blocks as there are
+// full batches for (a small frontier leaves the others idle, and the counts
+// to add up few). Logical blocks are spread so that each XCD takes a
+// contiguous range of slices (neighbouring pairs share cells, whose records
+// then share one L2).
 __device__ __forceinline__ uint32_t walk_block() { return xcd_block(blockIdx.x, gridDim.x); }
-__device__ __forceinline__ void walk_slice(uint32_t nf, uint32_t lb, uint32_t* b0, uint32_t* b1) {
-  const uint32_t chunk = (nf + WALK_G - 1) / WALK_G;
-  *b0 = min(lb * chunk, nf);
-  *b1 = min(*b0 + chunk, nf);
+struct WalkSlices {
+  uint32_t chunk, blocks;
+};
+__device__ __forceinline__ WalkSlices walk_slices(uint32_t nf) {
+  WalkSlices w;
+  w.chunk = max((nf + gridDim.x - 1) / gridDim.x, (uint32_t)CW_T);
+  w.blocks = (nf + w.chunk - 1) / w.chunk;
+  return w;
 }
 
-// One round of the breadth-first walk in three launches of fixed grids, with
+// One round of the breadth-first walk in two launches of fixed grids, with
 // outputs in frontier order and no host round trip: (1) every pair of the
-// round's frontier (its size read from the walk state) is decided, its
-// decision stored and its block's output counts written; (2) one block scans
-// the per-block counts and, when the round's outputs fit, advances the walk
-// state (next frontier size, list lengths); otherwise it records the sizes
-// needed and halts the walk at this round (every later kernel returns at
-// once); (3) every pair writes its outputs (child pairs to the next
+// round's frontier (its size read from the round's walk state) is decided, its
+// decision stored and its block's output counts written; (2) every block adds
+// up the counts of the blocks before its own and of them all, and when the
+// round's outputs fit, each pair writes its outputs (child pairs to the next
 // frontier, M2L and P2P pairs appended to the lists) at its block's offset
-// plus its rank in the block. The lists thus come out in one fixed order,
-// and a system's pairs keep their relative order whether it is walked alone
-// or in an ensemble.
+// plus its rank in the block; block 0 writes the next round's state. Rounds
+// alternate between two states, so no block reads what another writes. When
+// the outputs do not fit, every block finds the same, nothing is written but
+// the state with the sizes needed, and the walk is halted at this round (every
+// later launch passes the state on). The lists thus come out in one fixed
+// order, and a system's pairs keep their relative order whether it is walked
+// alone or in an ensemble. A third launch per round scanned the counts before:
+// 22 rounds at 1M bodies, 16 at 100k, one launch and about 4 us each.
 template <bool ERR>
-__global__ void __launch_bounds__(CW_T) k_walk_decide(const uint2* __restrict__ fin, uint32_t r,
+__global__ void __launch_bounds__(CW_T) k_walk_decide(const uint2* __restrict__ fin,
                                                     const WalkState* __restrict__ st,
                                                     uint16_t* __restrict__ code,
                                                     uint32_t* __restrict__ blk,
@@ -224,9 +241,11 @@ __global__ void __launch_bounds__(CW_T) k_walk_decide(const uint2* __restrict__ 
                                                     const double* __restrict__ mass, MacParams mp) {
   __shared__ uint32_t sh[CW_T / 64][3];
   if (st->status != 0u) return;
+  const uint32_t nf = st->fsize;
   const uint32_t lb = walk_block();
-  uint32_t b0, b1;
-  walk_slice(st->fsize[r & 1u], lb, &b0, &b1);
+  const WalkSlices w = walk_slices(nf);
+  if (lb >= w.blocks) return;
+  const uint32_t b0 = lb * w.chunk, b1 = min(b0 + w.chunk, nf);
   uint32_t v[3] = {0u, 0u, 0u};  // child pairs, M2L, P2P
   for (uint32_t t = b0 + threadIdx.x; t < b1; t += CW_T) {
     const uint2 pr = fin[t];
@@ -238,71 +257,16 @@ __global__ void __launch_bounds__(CW_T) k_walk_decide(const uint2* __restrict__ 
     v[1] += act == A_M2L ? 1u : 0u;
     v[2] += act == A_P2P ? 1u : 0u;
   }
-  block_sum3(v, sh);
+  block_sum(v, sh);
   if (threadIdx.x < 3) blk[WALK_G * threadIdx.x + lb] = v[threadIdx.x];
-}
-
-// One block of 1024 threads: exclusive scans of the three count columns
-// (WALK_G entries each, in place), then the walk state update.
-__global__ void __launch_bounds__(1024) k_walk_scan(uint32_t* __restrict__ blk, uint32_t r,
-                                                  WalkState* __restrict__ st, uint32_t cap_f,
-                                                  uint32_t cap_m2l, uint32_t cap_p2p) {
-  constexpr int PER = WALK_G / 1024;
-  __shared__ uint32_t sh[16][3];
-  if (st->status != 0u) return;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  uint32_t v[3][PER], sum[3], x[3], wt[3], tot[3];
-  for (int k = 0; k < 3; k++) {
-    sum[k] = 0;
-    for (int q = 0; q < PER; q++) {
-      v[k][q] = blk[WALK_G * k + PER * threadIdx.x + q];
-      sum[k] += v[k][q];
-    }
-    x[k] = wave_excl_scan(sum[k], &wt[k]);
-  }
-  if (lane == 0)
-    for (int k = 0; k < 3; k++) sh[w][k] = wt[k];
-  __syncthreads();
-  for (int k = 0; k < 3; k++) {
-    uint32_t off = 0, t = 0;
-    for (int q = 0; q < 16; q++) {
-      if (q < w) off += sh[q][k];
-      t += sh[q][k];
-    }
-    tot[k] = t;
-    uint32_t run = off + x[k];
-    for (int q = 0; q < PER; q++) {
-      blk[WALK_G * k + PER * threadIdx.x + q] = run;
-      run += v[k][q];
-    }
-  }
-  if (threadIdx.x != 0) return;
-  const uint64_t need_m2l = (uint64_t)st->n_m2l + tot[1];
-  const uint64_t need_p2p = (uint64_t)st->n_p2p + tot[2];
-  uint32_t bad = 0u;
-  if (tot[0] > cap_f) bad |= 1u;
-  if (need_m2l > cap_m2l) bad |= 2u;
-  if (need_p2p > cap_p2p) bad |= 4u;
-  if (bad) {
-    st->need_f = tot[0];
-    st->need_m2l = (uint32_t)min(need_m2l, (uint64_t)0xFFFFFFFFu);
-    st->need_p2p = (uint32_t)min(need_p2p, (uint64_t)0xFFFFFFFFu);
-    st->status = bad;
-    return;
-  }
-  if (st->fsize[r & 1u] > 0u) st->rounds++;
-  st->fsize[(r + 1u) & 1u] = tot[0];
-  st->m2l_base = st->n_m2l;
-  st->p2p_base = st->n_p2p;
-  st->n_m2l = (uint32_t)need_m2l;
-  st->n_p2p = (uint32_t)need_p2p;
-  st->round = r + 1u;
 }
 
 constexpr uint32_t WALK_STAGE = CW_T * 8;  // child pairs staged per batch
 
 __global__ void __launch_bounds__(CW_T) k_walk_emit(const uint2* __restrict__ fin, uint32_t r,
                                                   const WalkState* __restrict__ st,
+                                                  WalkState* __restrict__ st_next, uint32_t cap_f,
+                                                  uint32_t cap_m2l, uint32_t cap_p2p,
                                                   uint2* __restrict__ fout, uint2* __restrict__ m2l,
                                                   uint2* __restrict__ p2p,
                                                   const uint16_t* __restrict__ code,
@@ -310,14 +274,59 @@ __global__ void __launch_bounds__(CW_T) k_walk_emit(const uint2* __restrict__ fi
                                                   const WalkRec* __restrict__ rec) {
   __shared__ uint32_t sh[CW_T / 64][3];
   __shared__ uint2 stage[WALK_STAGE];
-  if (st->status != 0u) return;
+  const WalkState s0 = *st;
   const uint32_t lb = walk_block();
-  uint32_t b0, b1;
-  walk_slice(st->fsize[r & 1u], lb, &b0, &b1);
-  // the scan checked that the whole round fits its buffers
-  uint32_t fo = blk[lb];
-  uint32_t mo = st->m2l_base + blk[WALK_G + lb];
-  uint32_t po = st->p2p_base + blk[2 * WALK_G + lb];
+  if (s0.status != 0u) {  // halted at an earlier round
+    if (lb == 0 && threadIdx.x == 0) *st_next = s0;
+    return;
+  }
+  const uint32_t nf = s0.fsize;
+  const WalkSlices w = walk_slices(nf);
+  if (lb >= max(w.blocks, 1u)) return;
+  // counts of the blocks before this one, and of all
+  __shared__ uint32_t sh6[CW_T / 64][6];
+  uint32_t v6[6] = {0u, 0u, 0u, 0u, 0u, 0u};
+#pragma unroll
+  for (uint32_t q0 = 0; q0 < WALK_G; q0 += CW_T) {
+    const uint32_t q = q0 + threadIdx.x;
+    if (q >= w.blocks) continue;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const uint32_t v = blk[WALK_G * k + q];
+      v6[k] += q < lb ? v : 0u;
+      v6[3 + k] += v;
+    }
+  }
+  block_sum(v6, sh6);
+  const uint32_t* pre = v6;
+  const uint32_t* all = v6 + 3;
+  const uint64_t need_m2l = (uint64_t)s0.n_m2l + all[1];
+  const uint64_t need_p2p = (uint64_t)s0.n_p2p + all[2];
+  uint32_t bad = 0u;
+  if (all[0] > cap_f) bad |= 1u;
+  if (need_m2l > cap_m2l) bad |= 2u;
+  if (need_p2p > cap_p2p) bad |= 4u;
+  if (lb == 0 && threadIdx.x == 0) {
+    WalkState n = s0;
+    if (bad) {
+      n.status = bad;
+      n.need_f = all[0];
+      n.need_m2l = (uint32_t)min(need_m2l, (uint64_t)0xFFFFFFFFu);
+      n.need_p2p = (uint32_t)min(need_p2p, (uint64_t)0xFFFFFFFFu);
+    } else {
+      n.fsize = all[0];
+      n.n_m2l = (uint32_t)need_m2l;
+      n.n_p2p = (uint32_t)need_p2p;
+      n.round = r + 1u;
+      n.rounds = s0.rounds + (nf > 0u ? 1u : 0u);
+    }
+    *st_next = n;
+  }
+  if (bad || lb >= w.blocks) return;
+  const uint32_t b0 = lb * w.chunk, b1 = min(b0 + w.chunk, nf);
+  uint32_t fo = pre[0];
+  uint32_t mo = s0.n_m2l + pre[1];
+  uint32_t po = s0.n_p2p + pre[2];
   for (uint32_t t0 = b0; t0 < b1; t0 += CW_T) {
     const uint32_t t = t0 + threadIdx.x;
     const bool valid = t < b1;
@@ -362,19 +371,25 @@ __global__ void __launch_bounds__(CW_T) k_walk_emit(const uint2* __restrict__ fi
   }
 }
 
-void launch_walk_round(const void* fin, void* fout, uint32_t r, WalkState* st, uint32_t cap_f,
-                       uint2* m2l, uint32_t cap_m2l, uint2* p2p, uint32_t cap_p2p, uint16_t* code,
-                       uint32_t* blk, const void* rec, const double* mass, MacParams mac,
-                       hipStream_t s) {
+void launch_walk_round(const void* fin, void* fout, uint32_t r, const WalkState* st,
+                       WalkState* st_next, uint32_t cap_f, uint2* m2l, uint32_t cap_m2l, uint2* p2p,
+                       uint32_t cap_p2p, uint16_t* code, uint32_t* blk, const void* rec,
+                       const double* mass, MacParams mac, uint32_t nc, hipStream_t s) {
+  // Blocks: enough for the largest frontiers, which grow with the tree, but
+  // each round pays for the idle ones and for adding up the counts. 2048, 1024
+  // and 512 blocks: 590k cells (16M bodies) 3.8, 4.7 and 7.1 ms of walk;
+  // evaluations at 229k cells 12.70, 12.54 and 12.97 ms, at 64k 7.33, 7.31 and
+  // 7.49, at 40k (24 rounds) 2.81, 2.60 and 2.60.
+  const uint32_t g = nc >= (1u << 18) ? WALK_G : nc >= (1u << 15) ? WALK_G / 2 : WALK_G / 4;
   if (mac.use_err)
-    hipLaunchKernelGGL(k_walk_decide<true>, dim3(WALK_G), dim3(CW_T), 0, s, (const uint2*)fin, r,
-                       st, code, blk, (const WalkRec*)rec, mass, mac);
+    hipLaunchKernelGGL(k_walk_decide<true>, dim3(g), dim3(CW_T), 0, s, (const uint2*)fin, st,
+                       code, blk, (const WalkRec*)rec, mass, mac);
   else
-    hipLaunchKernelGGL(k_walk_decide<false>, dim3(WALK_G), dim3(CW_T), 0, s, (const uint2*)fin, r,
-                       st, code, blk, (const WalkRec*)rec, mass, mac);
-  hipLaunchKernelGGL(k_walk_scan, dim3(1), dim3(1024), 0, s, blk, r, st, cap_f, cap_m2l, cap_p2p);
-  hipLaunchKernelGGL(k_walk_emit, dim3(WALK_G), dim3(CW_T), 0, s, (const uint2*)fin, r, st,
-                     (uint2*)fout, m2l, p2p, code, blk, (const WalkRec*)rec);
+    hipLaunchKernelGGL(k_walk_decide<false>, dim3(g), dim3(CW_T), 0, s, (const uint2*)fin, st,
+                       code, blk, (const WalkRec*)rec, mass, mac);
+  hipLaunchKernelGGL(k_walk_emit, dim3(g), dim3(CW_T), 0, s, (const uint2*)fin, r, st, st_next,
+                     cap_f, cap_m2l, cap_p2p, (uint2*)fout, m2l, p2p, code, blk,
+                     (const WalkRec*)rec);
 }
 
 // Row pointers of the target-sorted directed entries over all cells:
