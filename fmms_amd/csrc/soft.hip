@@ -72,28 +72,41 @@ __global__ void __launch_bounds__(ST) k_trace_up(const uint32_t* __restrict__ ce
   const uint32_t id = cells[i];
   if (c.leaf[id]) return;
   const double zx = c.cx[id], zy = c.cy[id], zz = c.cz[id];
-  double acc = 0.0;
+  // gathered first, so a cell costs a few dependent loads and not a few per child
+  int ch[8];
+  double cx[8], cy[8], cz[8], cm[8], cq[8], px[8], py[8], pz[8];
+#pragma unroll
+  for (int o = 0; o < 8; o++) ch[o] = c.children[(size_t)id * 8 + o];
+#pragma unroll
   for (int o = 0; o < 8; o++) {
-    const int ch = c.children[(size_t)id * 8 + o];
-    if (ch < 0) continue;
-    const double dx = c.cx[ch] - zx, dy = c.cy[ch] - zy, dz = c.cz[ch] - zz;
-    double px, py, pz;
+    if (ch[o] < 0) continue;
+    cx[o] = c.cx[ch[o]];
+    cy[o] = c.cy[ch[o]];
+    cz[o] = c.cz[ch[o]];
+    cm[o] = c.mass[ch[o]];
+    cq[o] = q[ch[o]];
     // cells below level m32_below hold only scaled FP32 moments (the mixed
     // form's FP32 upward pass): M_1 = Mt_1 lam (m >= 0 layout: (1,0) at 1,
     // (1,1) at 2); the others hold FP64 moments
-    if (m32 && (int)c.level[ch] > m32_below) {
-      const cplxf* mc = m32 + (size_t)ch * NF;
-      const double l = lam[ch];
-      px = 2.0 * (double)mc[2].re * l;
-      py = 2.0 * (double)mc[2].im * l;
-      pz = (double)mc[1].re * l;
+    if (m32 && (int)c.level[ch[o]] > m32_below) {
+      const cplxf* mc = m32 + (size_t)ch[o] * NF;
+      const double l = lam[ch[o]];
+      px[o] = 2.0 * (double)mc[2].re * l;
+      py[o] = 2.0 * (double)mc[2].im * l;
+      pz[o] = (double)mc[1].re * l;
     } else {
-      const cplx* mc = mom + (size_t)ch * D;
-      px = 2.0 * mc[3].re;
-      py = 2.0 * mc[3].im;
-      pz = mc[2].re;
+      const cplx* mc = mom + (size_t)ch[o] * D;
+      px[o] = 2.0 * mc[3].re;
+      py[o] = 2.0 * mc[3].im;
+      pz[o] = mc[2].re;
     }
-    acc += q[ch] + 2.0 * (px * dx + py * dy + pz * dz) + c.mass[ch] * (dx * dx + dy * dy + dz * dz);
+  }
+  double acc = 0.0;
+#pragma unroll
+  for (int o = 0; o < 8; o++) {
+    if (ch[o] < 0) continue;
+    const double dx = cx[o] - zx, dy = cy[o] - zy, dz = cz[o] - zz;
+    acc += cq[o] + 2.0 * (px[o] * dx + py[o] * dy + pz[o] * dz) + cm[o] * (dx * dx + dy * dy + dz * dz);
   }
   q[id] = acc;
 }

@@ -239,6 +239,8 @@ __global__ void __launch_bounds__(M2M_T) k_m2m(const uint32_t* __restrict__ cell
     const int e = kM2mSched<P>.e_of[slot], b = kM2mSched<P>.base[slot];
     const int nt = has ? (int)kM2mSched<P>.nt[slot] : 0;
     cplx acc = cz();
+    // the terms' LDS reads overlap; the additions stay in order
+#pragma unroll 4
     for (int t = 0; t < nt; t++) {
       const uint32_t cd = code[b + t];
       const cplx uv = *(const cplx*)(ub + (cd & 0xFFFFu));
