@@ -6,6 +6,8 @@
 //     pot += Re Psi_0^0, a -= (Re Psi_1^1, Im Psi_1^1, Re Psi_1^0).
 // Upsilon is streamed degree by degree (harmonic.rs:141-173 recursion) and
 // only the m >= 0 halves of the expansions are held (registers, P static).
+#include <type_traits>
+
 #include "common.h"
 #include "harm32.h"
 #include "internal.h"
@@ -74,60 +76,110 @@ __device__ __forceinline__ void f_at(const cplx* F, int s, int q, double* br, do
   }
 }
 
-// L2L, one thread per child cell of a level: locals[child] += shift(parent).
+// L2L of a level: four waves per 64 child cells, each taking some of the
+// degrees of every child (lane = child), so a level's latency, which bounds
+// the small levels near the root and the deepest ones, is a quarter of one
+// thread doing a whole cell. The degrees are dealt out by work, (n + 1)
+// (P - n + 1)^2 products for degree n, longest first to the least loaded wave.
+// Per level at p = 8: 13.0 -> 8.0 us (1k bodies), 15.6 -> 9.4 (100k).
+constexpr int L2L_G = 4;
 template <int P>
-__global__ void __launch_bounds__(64) k_l2l(const uint32_t* __restrict__ cells, uint32_t cnt,
-                                           const int32_t* __restrict__ parent,
-                                           const double* __restrict__ cx,
-                                           const double* __restrict__ cy,
-                                           const double* __restrict__ cz,
-                                           cplx* __restrict__ locals) {
+struct L2lGroups {
+  int of[P + 1];
+};
+template <int P>
+constexpr L2lGroups<P> l2l_groups() {
+  L2lGroups<P> g{};
+  bool done[P + 1] = {};
+  int load[L2L_G] = {};
+  for (int i = 0; i <= P; i++) {
+    int best = -1, bw = -1;
+    for (int n = 0; n <= P; n++) {
+      const int w = (n + 1) * (P - n + 1) * (P - n + 1);
+      if (!done[n] && w > bw) {
+        bw = w;
+        best = n;
+      }
+    }
+    int q = 0;
+    for (int k = 1; k < L2L_G; k++)
+      if (load[k] < load[q]) q = k;
+    done[best] = true;
+    load[q] += bw;
+    g.of[best] = q;
+  }
+  return g;
+}
+// Calls f(integral_constant<N>) for every degree N of group GR, as separate
+// instantiations (unrolled loops over all degrees that skip the others' cost
+// the compiler minutes).
+template <int P, int GR, int N = 0, class F>
+__device__ __forceinline__ void l2l_degrees(F f) {
+  if constexpr (N <= P) {
+    if constexpr (l2l_groups<P>().of[N] == GR) f(std::integral_constant<int, N>{});
+    l2l_degrees<P, GR, N + 1>(f);
+  }
+}
+
+// Calls f with the wave's group as a template argument.
+template <class F>
+__device__ __forceinline__ void l2l_group(int g, F f) {
+  if (g == 0)
+    f(std::integral_constant<int, 0>{});
+  else if (g == 1)
+    f(std::integral_constant<int, 1>{});
+  else if (g == 2)
+    f(std::integral_constant<int, 2>{});
+  else
+    f(std::integral_constant<int, 3>{});
+}
+
+// locals[child] += shift(parent), degrees of group GR.
+template <int P, int GR>
+__device__ __forceinline__ void l2l_part(uint32_t c, uint32_t pa, const double* __restrict__ cx,
+                                         const double* __restrict__ cy,
+                                         const double* __restrict__ cz, cplx* __restrict__ locals) {
   constexpr int D = hdim(P), NF = hnpos(P);
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= cnt) return;
-  const uint32_t c = cells[i];
-  const int32_t pa = parent[c];
-  if (pa < 0) return;
   const double x = cx[pa] - cx[c], y = cy[pa] - cy[c], z = cz[pa] - cz[c];
   const double r2 = x * x + y * y + z * z;
-  cplx Fp[NF], G[NF];
+  cplx Fp[NF], G[NF];  // only the group's degrees of G, and what they read of Fp
   const cplx* lp = locals + (size_t)pa * D;
   cplx* lc = locals + (size_t)c * D;
 #pragma unroll
   for (int n = 0; n <= P; n++)
 #pragma unroll
-    for (int m = 0; m <= n; m++) {
-      Fp[hpos(n, m)] = lp[hidx(n, m)];
-      G[hpos(n, m)] = lc[hidx(n, m)];
-    }
+    for (int m = 0; m <= n; m++) Fp[hpos(n, m)] = lp[hidx(n, m)];
+  l2l_degrees<P, GR>([&](auto d) {
+    constexpr int n = decltype(d)::value;
+#pragma unroll
+    for (int m = 0; m <= n; m++) G[hpos(n, m)] = lc[hidx(n, m)];
+  });
   cplx U[P + 1], U1[P + 1], U2[P + 1];
 #pragma unroll
   for (int k = 0; k <= P; k++) {
     upsilon_degree<P>(k, x, y, z, r2, U, U1, U2);
+    l2l_degrees<P, GR>([&](auto d) {
+      constexpr int n = decltype(d)::value;
+      if (n + k > P) return;
 #pragma unroll
-    for (int n = 0; n <= P; n++) {
-      if (n + k > P) continue;
+      for (int m = 0; m <= n; m++) {
 #pragma unroll
-      for (int m = 0; m <= P; m++) {
-        if (m > n) continue;
-#pragma unroll
-        for (int l = -P; l <= P; l++) {
-          if (l < -k || l > k) continue;
+        for (int l = -k; l <= k; l++) {
           double ar, ai, br, bi;
           conj_y(U, l, &ar, &ai);
           f_at<P>(Fp, n + k, m + l, &br, &bi);
           cmac2(G[hpos(n, m)], ar, ai, br, bi);
         }
       }
-    }
+    });
 #pragma unroll
     for (int q = 0; q <= P; q++) {
       U2[q] = U1[q];
       U1[q] = U[q];
     }
   }
-#pragma unroll
-  for (int n = 0; n <= P; n++)
+  l2l_degrees<P, GR>([&](auto d) {
+    constexpr int n = decltype(d)::value;
 #pragma unroll
     for (int m = 0; m <= n; m++) {
       cplx g = G[hpos(n, m)];
@@ -137,6 +189,25 @@ __global__ void __launch_bounds__(64) k_l2l(const uint32_t* __restrict__ cells, 
         lc[hidx(n, -m)] = cplx{sg * g.re, -sg * g.im};
       }
     }
+  });
+}
+
+template <int P>
+__global__ void __launch_bounds__(64 * L2L_G) k_l2l(const uint32_t* __restrict__ cells,
+                                                   uint32_t cnt,
+                                                   const int32_t* __restrict__ parent,
+                                                   const double* __restrict__ cx,
+                                                   const double* __restrict__ cy,
+                                                   const double* __restrict__ cz,
+                                                   cplx* __restrict__ locals) {
+  const uint32_t i = blockIdx.x * 64 + (threadIdx.x & 63);
+  if (i >= cnt) return;
+  const uint32_t c = cells[i];
+  const int32_t pa = parent[c];
+  if (pa < 0) return;
+  l2l_group(wave_uniform((int)(threadIdx.x >> 6)), [&](auto g) {
+    l2l_part<P, decltype(g)::value>(c, (uint32_t)pa, cx, cy, cz, locals);
+  });
 }
 
 // L2P, one thread per body (slot): far-field acceleration and potential of
@@ -204,29 +275,103 @@ __global__ void __launch_bounds__(64) k_l2p(uint32_t n, const uint32_t* __restri
 //   L2L  Gt_n(child) = kappa^n sum_k sum_l conj(Y_k^l(u)) Ft_{n+k}^{m+l}(parent),
 //        u = (s_parent - s_child) / lam_parent, kappa = lam_child / lam_parent <= 1;
 //   L2P  Psi_n = lam^-n sum_k sum_l conj(Y_k^l(u)) Ft_{n+k}^{m+l}, u = (s - x) / lam.
-// One thread per cell of a level (parents' levels done before): the cell's
+// Four waves per 64 cells of a level (parents' levels done before): the cell's
 // own FP64 locals (M2L and the softened source-side terms) scaled to Ft, plus
 // its parent's Ft shifted to the cell. The own part enters divided by
 // kappa^n, so the shifted sum needs no per-term factor; the result is
 // multiplied by kappa^n once.
-template <int P>
-__global__ void __launch_bounds__(64) k_l2l32(const uint32_t* __restrict__ cells, uint32_t cnt,
-                                             const int32_t* __restrict__ parent,
-                                             const double* __restrict__ cx,
-                                             const double* __restrict__ cy,
-                                             const double* __restrict__ cz,
-                                             const double* __restrict__ lam,
-                                             const cplx* __restrict__ own,
-                                             cplxf* __restrict__ loc32) {
+template <int P, int GR>
+__device__ __forceinline__ void l2l32_part(uint32_t c, uint32_t pa, const double* __restrict__ cx,
+                                           const double* __restrict__ cy,
+                                           const double* __restrict__ cz,
+                                           const double* __restrict__ lam,
+                                           const cplx* __restrict__ own,
+                                           cplxf* __restrict__ loc32) {
   constexpr int D = hdim(P), NF = hnpos(P);
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= cnt) return;
-  const uint32_t c = cells[i];
-  const int32_t pa = parent[c];
   const double lc = lam[c];
   const cplx* lo = own + (size_t)c * D;
   cplxf* out = loc32 + (size_t)c * NF;
+  const double lp = lam[pa], il = 1.0 / lp;
+  const double kap = lc * il;
+  cplxf G[NF], Fp[NF];
+  {
+    const double ik = 1.0 / kap;
+    double sc[P + 1];  // lam_c^n kappa^-n = lam_p^n
+    sc[0] = 1.0;
+#pragma unroll
+    for (int n = 1; n <= P; n++) sc[n] = sc[n - 1] * (lc * ik);
+    l2l_degrees<P, GR>([&](auto d) {
+      constexpr int n = decltype(d)::value;
+#pragma unroll
+      for (int m = 0; m <= n; m++) {
+        const cplx v = lo[hidx(n, m)];
+        G[hpos(n, m)] = cplxf{(float)(v.re * sc[n]), (float)(v.im * sc[n])};
+      }
+    });
+  }
+  const cplxf* lpp = loc32 + (size_t)pa * NF;
+#pragma unroll
+  for (int e = 0; e < NF; e++) Fp[e] = lpp[e];
+  const float x = (float)((cx[pa] - cx[c]) * il), y = (float)((cy[pa] - cy[c]) * il),
+              z = (float)((cz[pa] - cz[c]) * il);
+  const float r2 = x * x + y * y + z * z;
+  cplxf U[P + 1], U1[P + 1], U2[P + 1];
+#pragma unroll
+  for (int k = 0; k <= P; k++) {
+    upsilon_degree32<P>(k, x, y, z, r2, U, U1, U2);
+    l2l_degrees<P, GR>([&](auto d) {
+      constexpr int n = decltype(d)::value;
+      if (n + k > P) return;
+#pragma unroll
+      for (int m = 0; m <= n; m++) {
+#pragma unroll
+        for (int l = -k; l <= k; l++) {
+          float ar, ai, br, bi;
+          conj_y32(U, l, &ar, &ai);
+          f_at32<P>(Fp, n + k, m + l, &br, &bi);
+          cmac2f(G[hpos(n, m)], ar, ai, br, bi);
+        }
+      }
+    });
+#pragma unroll
+    for (int q = 0; q <= P; q++) {
+      U2[q] = U1[q];
+      U1[q] = U[q];
+    }
+  }
+  float kn[P + 1];
+  const float kf = (float)kap;
+  kn[0] = 1.0f;
+#pragma unroll
+  for (int n = 1; n <= P; n++) kn[n] = kn[n - 1] * kf;
+  l2l_degrees<P, GR>([&](auto d) {
+    constexpr int n = decltype(d)::value;
+#pragma unroll
+    for (int m = 0; m <= n; m++)
+      out[hpos(n, m)] = cplxf{G[hpos(n, m)].re * kn[n], G[hpos(n, m)].im * kn[n]};
+  });
+}
+
+template <int P>
+__global__ void __launch_bounds__(64 * L2L_G) k_l2l32(const uint32_t* __restrict__ cells,
+                                                     uint32_t cnt,
+                                                     const int32_t* __restrict__ parent,
+                                                     const double* __restrict__ cx,
+                                                     const double* __restrict__ cy,
+                                                     const double* __restrict__ cz,
+                                                     const double* __restrict__ lam,
+                                                     const cplx* __restrict__ own,
+                                                     cplxf* __restrict__ loc32) {
+  constexpr int D = hdim(P), NF = hnpos(P);
+  const uint32_t i = blockIdx.x * 64 + (threadIdx.x & 63);
+  if (i >= cnt) return;
+  const uint32_t c = cells[i];
+  const int32_t pa = parent[c];
   if (pa < 0) {
+    if (threadIdx.x >= 64) return;
+    const double lc = lam[c];
+    const cplx* lo = own + (size_t)c * D;
+    cplxf* out = loc32 + (size_t)c * NF;
     double sc = 1.0;
 #pragma unroll
     for (int n = 0; n <= P; n++) {
@@ -239,62 +384,9 @@ __global__ void __launch_bounds__(64) k_l2l32(const uint32_t* __restrict__ cells
     }
     return;
   }
-  const double lp = lam[pa], il = 1.0 / lp;
-  const double kap = lc * il;
-  cplxf G[NF], Fp[NF];
-  {
-    const double ik = 1.0 / kap;
-    double sc = 1.0;  // lam_c^n kappa^-n = lam_p^n
-#pragma unroll
-    for (int n = 0; n <= P; n++) {
-#pragma unroll
-      for (int m = 0; m <= n; m++) {
-        const cplx v = lo[hidx(n, m)];
-        G[hpos(n, m)] = cplxf{(float)(v.re * sc), (float)(v.im * sc)};
-      }
-      sc *= lc * ik;
-    }
-  }
-  const cplxf* lpp = loc32 + (size_t)pa * NF;
-#pragma unroll
-  for (int e = 0; e < NF; e++) Fp[e] = lpp[e];
-  const float x = (float)((cx[pa] - cx[c]) * il), y = (float)((cy[pa] - cy[c]) * il),
-              z = (float)((cz[pa] - cz[c]) * il);
-  const float r2 = x * x + y * y + z * z;
-  cplxf U[P + 1], U1[P + 1], U2[P + 1];
-#pragma unroll
-  for (int k = 0; k <= P; k++) {
-    upsilon_degree32<P>(k, x, y, z, r2, U, U1, U2);
-#pragma unroll
-    for (int n = 0; n <= P; n++) {
-      if (n + k > P) continue;
-#pragma unroll
-      for (int m = 0; m <= P; m++) {
-        if (m > n) continue;
-#pragma unroll
-        for (int l = -P; l <= P; l++) {
-          if (l < -k || l > k) continue;
-          float ar, ai, br, bi;
-          conj_y32(U, l, &ar, &ai);
-          f_at32<P>(Fp, n + k, m + l, &br, &bi);
-          cmac2f(G[hpos(n, m)], ar, ai, br, bi);
-        }
-      }
-    }
-#pragma unroll
-    for (int q = 0; q <= P; q++) {
-      U2[q] = U1[q];
-      U1[q] = U[q];
-    }
-  }
-  float kn = 1.0f;
-  const float kf = (float)kap;
-#pragma unroll
-  for (int n = 0; n <= P; n++) {
-#pragma unroll
-    for (int m = 0; m <= n; m++) out[hpos(n, m)] = cplxf{G[hpos(n, m)].re * kn, G[hpos(n, m)].im * kn};
-    kn *= kf;
-  }
+  l2l_group(wave_uniform((int)(threadIdx.x >> 6)), [&](auto g) {
+    l2l32_part<P, decltype(g)::value>(c, (uint32_t)pa, cx, cy, cz, lam, own, loc32);
+  });
 }
 
 // L2P of the scaled locals, one thread per body; the offset from the leaf
@@ -382,7 +474,7 @@ __global__ void __launch_bounds__(256) k_loc32_export(uint32_t nc, const double*
 
 template <int P>
 static void l2l_t(const uint32_t* cells, uint32_t cnt, DevCells c, cplx* locals, hipStream_t s) {
-  hipLaunchKernelGGL(k_l2l<P>, dim3((cnt + 63) / 64), dim3(64), 0, s, cells, cnt, c.parent, c.cx,
+  hipLaunchKernelGGL(k_l2l<P>, dim3((cnt + 63) / 64), dim3(64 * L2L_G), 0, s, cells, cnt, c.parent, c.cx,
                      c.cy, c.cz, locals);
 }
 
@@ -412,7 +504,7 @@ bool launch_l2l32(int p, const uint32_t* cells, uint32_t cnt, DevCells c, const 
                   const cplx* own, void* loc32, hipStream_t s) {
   if (cnt == 0) return true;
 #define CALL(P)                                                                                  \
-  hipLaunchKernelGGL(k_l2l32<P>, dim3((cnt + 63) / 64), dim3(64), 0, s, cells, cnt, c.parent, \
+  hipLaunchKernelGGL(k_l2l32<P>, dim3((cnt + 63) / 64), dim3(64 * L2L_G), 0, s, cells, cnt, c.parent, \
                      c.cx, c.cy, c.cz, lam, own, (cplxf*)loc32)
   FMMH_P_SWITCH2(p, CALL)
 #undef CALL
