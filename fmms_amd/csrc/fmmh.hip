@@ -117,7 +117,7 @@ struct fmmh_ctx {
   Buf walk_code, walk_blk;  // the walk's per-pair decisions, per-block counts
   Buf pl_longs, pl_items, pl_reds, pl_partial;  // P2P work plan
   Buf m2l_lam, m2l_m32;                     // mixed form: FP32 M2L scales, scaled moments
-  Buf m2l_rows;                             // FP64 form: source rows
+  Buf m2l_rows;                             // M2L source rows
   Buf loc32;                                // mixed form: FP32 locals scaled by lam^n
   uint32_t p_nitems = 0, p_nsplit = 0, p_nlong = 0;
   Buf rt_tab;  // p > TEMPLATED_MAX_P: the rotation M2L's tables
@@ -490,6 +490,7 @@ struct fmmh_ctx {
       ensure(m2l_lam, (size_t)nc * sizeof(double));
       ensure(m2l_m32, (size_t)nc * m2l32_moment_bytes(p));
       ensure(loc32, (size_t)nc * m2l32_moment_bytes(p));
+      ensure(m2l_rows, (size_t)nc * m2l32_row_bytes(p));
     }
     ensure(far, n * sizeof(double4));
   }
@@ -513,7 +514,7 @@ struct fmmh_ctx {
     mark(ST_M2L);
     if (!gen && prm.precision == FMMH_PREC_FP32BULK) {
       launch_m2l32(p, nc, chunks.p, nchunks, msorted, sbits, c, (const BBox*)bbox.p, keys_sorted,
-                   vlev, mom, soft2, (double*)m2l_lam.p, m2l_m32.p, part.p, s,
+                   vlev, mom, soft2, (double*)m2l_lam.p, m2l_m32.p, (double*)m2l_rows.p, part.p, s,
                    up32() ? vlev + FP64_TOP : 255);
       mark(ST_M2L_REDUCE);
       launch_m2l_reduce32(p, nc, (const uint4*)plan.p, part.p, (const double*)m2l_lam.p, loc, s);

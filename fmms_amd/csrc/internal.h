@@ -155,7 +155,6 @@ void launch_csr_ptr(const uint64_t* keys, uint32_t nnz, int sbits, uint32_t ntar
                     uint32_t* ptr, hipStream_t s);
 
 // --------------------------------------------------------------- m2l.hip
-// Chunks of at most `ch` sources per target (the M2L work unit).
 size_t m2l_part_bytes(int p, size_t maxchunks, bool fp32);
 size_t m2l_chunk_bytes();
 // FP64 form, p <= 10: rows [nc] x m2l_row_bytes(p) is scratch (the sources'
@@ -165,14 +164,16 @@ bool launch_m2l_kernel(int p, uint32_t nc, const void* chunks, uint32_t nchunks,
                        const uint64_t* skeys, int sbits, DevCells c, const cplx* moments,
                        double soft2, double* rows, double* part, hipStream_t s);
 // Mixed form: the same M2L on radius-scaled FP32 operands (m2l_kernel.h);
-// lam [nc] doubles and m32 [nc] x m2l32_moment_bytes(p) are scratch.
+// lam [nc] doubles, m32 [nc] x m2l32_moment_bytes(p) and rows [nc] x
+// m2l32_row_bytes(p) are scratch.
 // prep_below: FP32 moments are made from the FP64 ones for the cells above
 // this level only (the cells below hold them from the FP32 upward pass);
 // 255 = every cell.
 bool launch_m2l32(int p, uint32_t nc, const void* chunks, uint32_t nchunks, const uint64_t* skeys,
                   int sbits, DevCells c, const BBox* bb, const uint64_t* keys_sorted, int vlev,
-                  const cplx* moments, double soft2, double* lam, void* m32, void* part,
-                  hipStream_t s, int prep_below = 255);
+                  const cplx* moments, double soft2, double* lam, void* m32, double* rows,
+                  void* part, hipStream_t s, int prep_below = 255);
+size_t m2l32_row_bytes(int p);
 // Per-cell scale of the mixed form: radius, floored at a quarter of the octant edge.
 void launch_m2l_scale(uint32_t nc, DevCells c, const BBox* bb, const uint64_t* keys_sorted,
                       int vlev, double* lam, hipStream_t s);

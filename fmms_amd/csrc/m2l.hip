@@ -14,8 +14,8 @@ void m2l_t(const M2lChunk* chunks, uint32_t nchunks, const uint64_t* skeys, uint
            hipStream_t s);
 template <int P>
 void m2l32_t(const M2lChunk* chunks, uint32_t nchunks, const uint64_t* skeys, uint64_t smask,
-             DevCells c, const double* lam, const cplxf* m32, double soft2, cplxf* part,
-             hipStream_t s);
+             uint32_t nc, DevCells c, const double* lam, const cplxf* m32, double soft2,
+             double* rows, cplxf* part, hipStream_t s);
 
 // Scale of each cell for the FP32 M2L: its radius, floored at a quarter of
 // its octant edge (the system's box side halved per level below the system
@@ -213,8 +213,8 @@ void launch_m2l_scale(uint32_t nc, DevCells c, const BBox* bb, const uint64_t* k
 
 bool launch_m2l32(int p, uint32_t nc, const void* chunks, uint32_t nchunks, const uint64_t* skeys,
                   int sbits, DevCells c, const BBox* bb, const uint64_t* keys_sorted, int vlev,
-                  const cplx* moments, double soft2, double* lam, void* m32, void* part,
-                  hipStream_t s, int prep_below) {
+                  const cplx* moments, double soft2, double* lam, void* m32, double* rows,
+                  void* part, hipStream_t s, int prep_below) {
   const uint64_t smask = (1ull << sbits) - 1ull;
   const M2lChunk* ck = (const M2lChunk*)chunks;
   if (nc == 0) return true;
@@ -222,10 +222,18 @@ bool launch_m2l32(int p, uint32_t nc, const void* chunks, uint32_t nchunks, cons
 #define CALL(P)                                                                            \
   hipLaunchKernelGGL(k_m2l_prep32<P>, dim3((nc + 255) / 256), dim3(256), 0, s, nc, moments, \
                      (const double*)lam, c.level, prep_below, (cplxf*)m32);                \
-  m2l32_t<P>(ck, nchunks, skeys, smask, c, lam, (const cplxf*)m32, soft2, (cplxf*)part, s)
+  m2l32_t<P>(ck, nchunks, skeys, smask, nc, c, lam, (const cplxf*)m32, soft2, rows,         \
+             (cplxf*)part, s)
   FMMH_P_SWITCH3(p, CALL)
 #undef CALL
   return true;
+}
+
+// Bytes of one cell's source row of the mixed form (M2lRow32<p>); 0: none.
+size_t m2l32_row_bytes(int p) {
+  if (p < 3 || p > 8) return 0;
+  const int nf = hnpos(p), seg = (nf - 2) / 8;
+  return (size_t)((seg * 8 + 4 + nf - 8 * seg + 7) / 8 * 8) * sizeof(double);
 }
 
 size_t m2l32_moment_bytes(int p) { return (size_t)hnpos(p) * sizeof(cplxf); }

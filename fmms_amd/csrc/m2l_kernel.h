@@ -44,9 +44,12 @@ __device__ __forceinline__ float m2l_rsqrt(float x) {
 }
 
 // FP32 (mixed form): F (m>=0 half, hpos layout) += M2L of source multipole M
-// (m>=0 half) at r, term by term (softening as in m2l_accumulate64).
-template <int P, int H, typename R, typename C>
-__device__ __forceinline__ void m2l_accumulate(R x, R y, R z, R soft2, const C* M, C* F) {
+// (m>=0 half) at r, term by term (softening as in m2l_accumulate64). on:
+// whether the lane has a pair (else Theta is 0 and nothing is added); mid()
+// runs before the products of degree MID.
+template <int P, int H, int MID, typename R, typename C, class Mid>
+__device__ __forceinline__ void m2l_accumulate(bool on, R x, R y, R z, R soft2, const C* M, C* F,
+                                               Mid mid) {
   const R rr2 = x * x + y * y + z * z;
   const R r2 = rr2 + soft2;
   const R ir = m2l_rsqrt(r2);
@@ -57,7 +60,7 @@ __device__ __forceinline__ void m2l_accumulate(R x, R y, R z, R soft2, const C* 
   for (int s = 0; s <= P; s++) {
     // Theta_s^q, q = 0..s (harmonic.rs:91-129 recursion, Dehnen eq. 52/54)
     if (s == 0) {
-      T[0] = C{ir, R(0)};
+      T[0] = C{on ? ir : R(0), R(0)};
     } else {
       const R a = (R)(2 * s - 1) * z;
 #pragma unroll
@@ -78,6 +81,7 @@ __device__ __forceinline__ void m2l_accumulate(R x, R y, R z, R soft2, const C* 
         }
       }
     }
+    if (s == MID) mid(T[s].re);
     // all terms with n + k == s
 #pragma unroll
     for (int n = 0; n <= P; n++) {
@@ -508,9 +512,9 @@ __device__ __forceinline__ void m2l_chunk32(const M2lChunk ck, uint32_t ci,
       }
       kk *= kap;
     }
-    m2l_accumulate<P, H, float, cplxf>((float)((tx - ccx[src]) * ilt),
-                                       (float)((ty - ccy[src]) * ilt),
-                                       (float)((tz - ccz[src]) * ilt), s2s, M, F);
+    m2l_accumulate<P, H, P, float, cplxf>(true, (float)((tx - ccx[src]) * ilt),
+                                          (float)((ty - ccy[src]) * ilt),
+                                          (float)((tz - ccz[src]) * ilt), s2s, M, F, [](float&) {});
   }
   cplxf* out = part + (size_t)ci * NF;
 #pragma unroll
@@ -519,6 +523,165 @@ __device__ __forceinline__ void m2l_chunk32(const M2lChunk ck, uint32_t ci,
 #pragma unroll
     for (int m = 0; m <= n; m++) out[hpos(n, m)] = F[hpos(n, m)];
   }
+}
+
+// Source rows of the staged orders 3..8: SEG 64-byte segments of the scaled
+// moments (from the NDIR-th on) that go through LDS, then centre, scale and the
+// first NDIR moments, which each lane reads itself. As in the FP64 form, rows
+// read lane by lane kept the address unit busy as long as the arithmetic (P =
+// 7: 18 loads of 64 lines a source), and the loads were waited for at the top
+// of each source, with two waves a SIMD; the copy now runs under the products of
+// the last degree, before which the row must be in registers anyway (earlier
+// it costs registers that P = 8 does not have: 2.44 ms there, 2.68 - 2.83 before
+// an earlier degree). Two waves a SIMD of 20 KB each fill the LDS. Kernel alone:
+// P = 8, 1M bodies 2.94 -> 2.44 ms; P = 7, 16.8M bodies 17.3 -> 15.2; P = 3 .. 6,
+// 250k bodies 198 / 244 / 380 / 446 -> 128 / 179 / 222 / 298 us, and 4 - 16 us (83
+// at 16.8M) for the rows. FP32 issue bounds it now (3.1 cycles an instruction).
+// P = 1, 2 have less than a segment, and P = 9, 10 no registers left: read
+// directly.
+template <int P>
+struct M2lRow32 {
+  static constexpr int NF = hnpos(P);
+  static constexpr bool STAGED = P >= 3 && P <= 8;
+  static constexpr int SEG = (NF - 2) / 8;
+  static constexpr int NDIR = NF - 8 * SEG;
+  static constexpr int WORDS = (SEG * 8 + 4 + NDIR + 7) / 8 * 8;  // of 8 bytes
+};
+
+template <int P>
+__global__ void __launch_bounds__(256) k_m2l_rows32(uint32_t nc, const cplxf* __restrict__ m32,
+                                                   const double* __restrict__ ccx,
+                                                   const double* __restrict__ ccy,
+                                                   const double* __restrict__ ccz,
+                                                   const double* __restrict__ lam,
+                                                   double* __restrict__ rows) {
+  using R = M2lRow32<P>;
+  const size_t g = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const uint32_t c = (uint32_t)(g / R::WORDS);
+  if (c >= nc) return;
+  const int i = (int)(g - (size_t)c * R::WORDS), d = i - R::SEG * 8;
+  const int e = d < 0 ? i + R::NDIR : d >= 4 && d - 4 < R::NDIR ? d - 4 : -1;
+  double v = 0.0;
+  if (e >= 0)
+    v = __builtin_bit_cast(double, m32[(size_t)c * R::NF + e]);
+  else if (d < 4)
+    v = d == 0 ? ccx[c] : d == 1 ? ccy[c] : d == 2 ? ccz[c] : lam[c];
+  rows[g] = v;
+}
+
+// The chunks of 64 lanes, rows staged as in m2l_chunks64 (same layout in LDS).
+template <int P>
+__device__ __forceinline__ void m2l_chunks32(uint32_t ci, bool live, const M2lChunk ck,
+                                             const uint64_t* __restrict__ skeys, uint64_t smask,
+                                             const double* __restrict__ rows, double soft2,
+                                             float4* stage, cplxf* __restrict__ part) {
+  using R = M2lRow32<P>;
+  const int lane = threadIdx.x;
+  lds_char* stage3 = (lds_char*)stage;
+  const uint32_t cnt = live ? ck.end - ck.begin : 0u;
+  uint32_t trips = cnt;  // the wave runs its longest chunk's trip count
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) trips = max(trips, (uint32_t)__shfl_xor((int)trips, o, 64));
+  trips = (uint32_t)wave_uniform((int)trips);
+  if (trips == 0) return;
+  cplxf F[R::NF];
+#pragma unroll
+  for (int i = 0; i < R::NF; i++) F[i] = cplxf{0.f, 0.f};
+  // past the end: the last one; a dead lane: the first key's
+  auto source = [&](uint32_t j) -> uint32_t {
+    return (uint32_t)(skeys[ck.begin + min(j, max(cnt, 1u) - 1)] & smask);
+  };
+  auto copy = [&](uint32_t src) {
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const uint32_t rs = (uint32_t)__shfl((int)src, g * 16 + (lane >> 2), 64);
+      m2l_copy_segments<R::SEG>(
+          (gbl_char*)(rows + (size_t)rs * R::WORDS) + ((lane & 3) ^ ((lane >> 4) & 3)) * 16,
+          stage3 + g * R::SEG * 1024);
+    }
+  };
+  const int swz = (lane >> 2) & 3;
+  const float4* mine = stage + (lane >> 4) * R::SEG * 64 + (lane & 15) * 4;
+  double cl[4];  // the source's centre and scale
+  cplxf dir[R::NDIR];
+  auto direct = [&](uint32_t sc) {
+    const double* d = rows + (size_t)sc * R::WORDS + R::SEG * 8;
+    const double2 a = *(const double2*)d, b = *(const double2*)(d + 2);
+    cl[0] = a.x;
+    cl[1] = a.y;
+    cl[2] = b.x;
+    cl[3] = b.y;
+    const float4* q = (const float4*)(d + 4);
+#pragma unroll
+    for (int i = 0; i < (R::NDIR + 1) / 2; i++) {
+      const float4 v = q[i];
+      dir[2 * i] = cplxf{v.x, v.y};
+      if (2 * i + 1 < R::NDIR) dir[2 * i + 1] = cplxf{v.z, v.w};
+    }
+  };
+  uint32_t src = source(0);
+  direct(src);
+  copy(src);
+  const double* t = rows + (size_t)ck.target * R::WORDS + R::SEG * 8;
+  const double tx = t[0], ty = t[1], tz = t[2], ilt = 1.0 / t[3];
+  const float s2s = (float)(soft2 * ilt * ilt);
+  src = source(1);
+  for (uint32_t j = 0; j < trips; j++) {
+    const float x = (float)((tx - cl[0]) * ilt), y = (float)((ty - cl[1]) * ilt),
+                z = (float)((tz - cl[2]) * ilt);
+    const float kap = (float)(cl[3] * ilt);
+    float kk[P + 1];
+    kk[0] = 1.f;
+#pragma unroll
+    for (int k = 1; k <= P; k++) kk[k] = kk[k - 1] * kap;
+    cplxf M[R::NF];
+#pragma unroll
+    for (int i = 0; i < R::NDIR; i++) M[i] = dir[i];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copy has landed
+#pragma unroll
+    for (int e = 0; e < R::SEG * 4; e++) {
+      const float4 v = mine[(e >> 2) * 64 + ((e & 3) ^ swz)];
+      M[R::NDIR + 2 * e] = cplxf{v.x, v.y};
+      M[R::NDIR + 2 * e + 1] = cplxf{v.z, v.w};
+    }
+#pragma unroll
+    for (int k = 0; k <= P; k++)
+#pragma unroll
+      for (int l = 0; l <= k; l++) {
+        M[hpos(k, l)].re *= kk[k];
+        M[hpos(k, l)].im *= kk[k];
+      }
+    m2l_accumulate<P, 2, P, float, cplxf>(j < cnt, x, y, z, s2s, M, F, [&](float& tq) {
+      // the row has been read; tq ties the point to the degrees (a branch or a
+      // free wait would move to the top of the loop, and the row's registers
+      // with it)
+      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(tq)::"memory");
+      direct(src);
+      copy(src);
+      src = source(j + 2);
+    });
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last copy, into a wave's LDS
+  if (!live) return;
+  cplxf* out = part + (size_t)ci * R::NF;
+#pragma unroll
+  for (int i = 0; i < R::NF; i++) out[i] = F[i];
+}
+
+template <int P>
+__global__ void __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(2))) k_m2l32_staged(const M2lChunk* __restrict__ chunks,
+                                                       uint32_t nchunks,
+                                                       const uint64_t* __restrict__ skeys,
+                                                       uint64_t smask,
+                                                       const double* __restrict__ rows,
+                                                       double soft2, cplxf* __restrict__ part) {
+  __shared__ float4 stage[M2lRow32<P>::SEG * 256];
+  const uint32_t ci = xcd_block(blockIdx.x, gridDim.x) * 64 + threadIdx.x;
+  const bool live = ci < nchunks;
+  M2lChunk ck{0, 0, 0};
+  if (live) ck = chunks[ci];
+  m2l_chunks32<P>(ci, live, ck, skeys, smask, rows, soft2, stage, part);
 }
 
 template <int P, bool SPLIT>
@@ -552,20 +715,29 @@ __global__ void __launch_bounds__(64) k_m2l32(const M2lChunk* __restrict__ chunk
 
 template <int P>
 void m2l32_t(const M2lChunk* chunks, uint32_t nchunks, const uint64_t* skeys, uint64_t smask,
-             DevCells c, const double* lam, const cplxf* m32, double soft2, cplxf* part,
-             hipStream_t s) {
+             uint32_t nc, DevCells c, const double* lam, const cplxf* m32, double soft2,
+             double* rows, cplxf* part, hipStream_t s) {
   if (!nchunks) return;
-  constexpr bool split = P >= FMMH_M2L32_SPLIT_FROM;
-  const uint32_t nb = (nchunks + 63) / 64 * (split ? 2 : 1);
-  hipLaunchKernelGGL((k_m2l32<P, split>), dim3(nb), dim3(64), 0, s, chunks, nchunks, skeys, smask,
-                     c.cx, c.cy, c.cz, lam, m32, soft2, part);
+  if constexpr (M2lRow32<P>::STAGED) {
+    const size_t rt = (size_t)nc * M2lRow32<P>::WORDS;
+    hipLaunchKernelGGL(k_m2l_rows32<P>, dim3((rt + 255) / 256), dim3(256), 0, s, nc, m32, c.cx,
+                       c.cy, c.cz, lam, rows);
+    hipLaunchKernelGGL(k_m2l32_staged<P>, dim3((nchunks + 63) / 64), dim3(64), 0, s, chunks,
+                       nchunks, skeys, smask, (const double*)rows, soft2, part);
+  } else {
+    constexpr bool split = P >= FMMH_M2L32_SPLIT_FROM;
+    const uint32_t nb = (nchunks + 63) / 64 * (split ? 2 : 1);
+    hipLaunchKernelGGL((k_m2l32<P, split>), dim3(nb), dim3(64), 0, s, chunks, nchunks, skeys,
+                       smask, c.cx, c.cy, c.cz, lam, m32, soft2, part);
+  }
 }
 
 // One translation unit per range of orders instantiates the launches.
 #define FMMH_M2L_INSTANTIATE(P)                                                             \
   template void m2l_t<P>(const M2lChunk*, uint32_t, const uint64_t*, uint64_t, uint32_t,    \
                          DevCells, const cplx*, double, double*, double*, hipStream_t);     \
-  template void m2l32_t<P>(const M2lChunk*, uint32_t, const uint64_t*, uint64_t, DevCells,  \
-                           const double*, const cplxf*, double, cplxf*, hipStream_t);
+  template void m2l32_t<P>(const M2lChunk*, uint32_t, const uint64_t*, uint64_t, uint32_t,  \
+                           DevCells, const double*, const cplxf*, double, double*, cplxf*,  \
+                           hipStream_t);
 
 }  // namespace fmmh
