@@ -71,19 +71,32 @@ void launch_pack_walk(uint32_t nc, DevCells c, void* rec, double4* cpm, hipStrea
                      cpm);
 }
 
-// mac.rs:23-61 error estimate of cell a acting on cell b (r > 0 here).
+// Which MAC a walk is compiled for: without the error estimate, with it at one
+// order p <= MAC_P_MAX, or at any.
+enum : int { MAC_THETA = -1, MAC_ANY_P = 0 };
+constexpr int MAC_P_MAX = 10;
+
+// mac.rs:23-61 error estimate of cell a acting on cell b (r > 0 here). With the
+// order known (PE > 0) the powers stay in registers and the cell's row of
+// pows is read at once; with a loop over p the table is scratch memory and every
+// term waits for its load: the walk's decisions at 1M bodies, p = 8, 1542 -> 531 us.
+template <int PE>
 __device__ __forceinline__ double error_estimate(uint32_t a, double rho_b, double mass_a,
                                                  double rho_a, double r, const MacParams& mp) {
-  const int p = mp.p;
+  constexpr int UN = PE > 0 ? PE + 1 : 1;
+  const int p = PE > 0 ? PE : mp.p;
   double r2 = r * r;
   double rp = 1.0;
+#pragma unroll UN
   for (int i = 0; i < p / 2; i++) rp *= r2;
   if (p % 2 == 1) rp *= r;
-  double rpows[FMMH_MAX_P + 1];
+  double rpows[(PE > 0 ? PE : FMMH_MAX_P) + 1];
   rpows[0] = 1.0;
+#pragma unroll UN
   for (int j = 1; j <= p; j++) rpows[j] = rpows[j - 1] * rho_b;
   const double* pw = mp.pows + (size_t)a * (p + 1);
   double s = 0.0;
+#pragma unroll UN
   for (int k = 0; k <= p; k++) s += mp.binom[k] * pw[k] * rpows[p - k];
   double e = s / (mass_a * rp);
   double denom = rho_a + rho_b;
@@ -95,7 +108,7 @@ __device__ __forceinline__ double error_estimate(uint32_t a, double rho_b, doubl
 // r2*theta_max^2 <= (rhoA+rhoB)^2 rejects; theta_max = 1 multiplies by 1.
 // Softening guard extension: eps^2 (rhoA+rhoB)^3 > tau r^5 rejects (the
 // softened far field's leading residual relative to the pair's field).
-template <bool ERR>
+template <int PE>
 __device__ __forceinline__ bool accept(uint32_t a, const WalkRec& ra, uint32_t b,
                                        const WalkRec& rb, double r2, const double* __restrict__ mass,
                                        const MacParams& mp) {
@@ -104,11 +117,11 @@ __device__ __forceinline__ bool accept(uint32_t a, const WalkRec& ra, uint32_t b
   if (mp.soft_mac > 0.0 && mp.soft2 > 0.0 &&
       mp.soft2 * (sum_rho * sum_rho * sum_rho) > mp.soft_mac * (r2 * r2 * sqrt(r2)))
     return false;
-  if (!ERR) return true;
+  if (PE == MAC_THETA) return true;
   double r = sqrt(r2);
   if (r == 0.0) return false;
   const double ma = mass[a];
-  double est = error_estimate(a, rb.rho, ma, ra.rho, r, mp);
+  double est = error_estimate<PE>(a, rb.rho, ma, ra.rho, r, mp);
   if (est == 0.0) return true;
   return est * ma / r2 < mp.eps * mp.fmin[b];
 }
@@ -122,10 +135,8 @@ __device__ __forceinline__ uint32_t nchild(const WalkRec& r) {
   return k;
 }
 
-// walk.rs:94-190 decision of one frontier pair; nch = its child pairs. ERR:
-// the error-controlled MAC (mp.use_err); the theta-only walk is compiled
-// without it (no scratch for the error estimate's power table).
-template <bool ERR>
+// walk.rs:94-190 decision of one frontier pair; nch = its child pairs.
+template <int PE>
 __device__ __forceinline__ int decide(uint32_t a, uint32_t b, const WalkRec& ra,
                                       const WalkRec& rb, const double* __restrict__ mass,
                                       const MacParams& mp, uint32_t* nch) {
@@ -141,7 +152,7 @@ __device__ __forceinline__ int decide(uint32_t a, uint32_t b, const WalkRec& ra,
   double r2ab = dx * dx + dy * dy + dz * dz;
   double ex = ra.cx - rb.cx, ey = ra.cy - rb.cy, ez = ra.cz - rb.cz;
   double r2ba = ex * ex + ey * ey + ez * ez;
-  if (accept<ERR>(a, ra, b, rb, r2ab, mass, mp) && accept<ERR>(b, rb, a, ra, r2ba, mass, mp))
+  if (accept<PE>(a, ra, b, rb, r2ab, mass, mp) && accept<PE>(b, rb, a, ra, r2ba, mass, mp))
     return A_M2L;
   if (la && lb) return A_P2P;
   bool split_b;
@@ -232,7 +243,7 @@ __device__ __forceinline__ WalkSlices walk_slices(uint32_t nf) {
 // order, and a system's pairs keep their relative order whether it is walked
 // alone or in an ensemble. A third launch per round scanned the counts before:
 // 22 rounds at 1M bodies, 16 at 100k, one launch and about 4 us each.
-template <bool ERR>
+template <int PE>
 __global__ void __launch_bounds__(CW_T) k_walk_decide(const uint2* __restrict__ fin,
                                                     const WalkState* __restrict__ st,
                                                     uint16_t* __restrict__ code,
@@ -251,7 +262,7 @@ __global__ void __launch_bounds__(CW_T) k_walk_decide(const uint2* __restrict__ 
     const uint2 pr = fin[t];
     const WalkRec ra = rec[pr.x], rb = rec[pr.y];
     uint32_t nch;
-    const int act = decide<ERR>(pr.x, pr.y, ra, rb, mass, mp, &nch);
+    const int act = decide<PE>(pr.x, pr.y, ra, rb, mass, mp, &nch);
     code[t] = (uint16_t)(act | (nch << 3));
     v[0] += nch;
     v[1] += act == A_M2L ? 1u : 0u;
@@ -371,6 +382,26 @@ __global__ void __launch_bounds__(CW_T) k_walk_emit(const uint2* __restrict__ fi
   }
 }
 
+template <int PE, class... A>
+static void decide_t(dim3 g, hipStream_t s, A... args) {
+  hipLaunchKernelGGL(k_walk_decide<PE>, g, dim3(CW_T), 0, s, args...);
+}
+
+// The kernel for the walk's MAC, orders PE and above.
+template <int PE>
+static void launch_decide(dim3 g, const uint2* fin, const WalkState* st, uint16_t* code,
+                          uint32_t* blk, const WalkRec* rec, const double* mass, MacParams mac,
+                          hipStream_t s) {
+  if (!mac.use_err)
+    decide_t<MAC_THETA>(g, s, fin, st, code, blk, rec, mass, mac);
+  else if (mac.p == PE)
+    decide_t<PE>(g, s, fin, st, code, blk, rec, mass, mac);
+  else if constexpr (PE < MAC_P_MAX)
+    launch_decide<PE + 1>(g, fin, st, code, blk, rec, mass, mac, s);
+  else
+    decide_t<MAC_ANY_P>(g, s, fin, st, code, blk, rec, mass, mac);
+}
+
 void launch_walk_round(const void* fin, void* fout, uint32_t r, const WalkState* st,
                        WalkState* st_next, uint32_t cap_f, uint2* m2l, uint32_t cap_m2l, uint2* p2p,
                        uint32_t cap_p2p, uint16_t* code, uint32_t* blk, const void* rec,
@@ -381,12 +412,7 @@ void launch_walk_round(const void* fin, void* fout, uint32_t r, const WalkState*
   // evaluations at 229k cells 12.70, 12.54 and 12.97 ms, at 64k 7.33, 7.31 and
   // 7.49, at 40k (24 rounds) 2.81, 2.60 and 2.60.
   const uint32_t g = nc >= (1u << 18) ? WALK_G : nc >= (1u << 15) ? WALK_G / 2 : WALK_G / 4;
-  if (mac.use_err)
-    hipLaunchKernelGGL(k_walk_decide<true>, dim3(g), dim3(CW_T), 0, s, (const uint2*)fin, st,
-                       code, blk, (const WalkRec*)rec, mass, mac);
-  else
-    hipLaunchKernelGGL(k_walk_decide<false>, dim3(g), dim3(CW_T), 0, s, (const uint2*)fin, st,
-                       code, blk, (const WalkRec*)rec, mass, mac);
+  launch_decide<1>(dim3(g), (const uint2*)fin, st, code, blk, (const WalkRec*)rec, mass, mac, s);
   hipLaunchKernelGGL(k_walk_emit, dim3(g), dim3(CW_T), 0, s, (const uint2*)fin, r, st, st_next,
                      cap_f, cap_m2l, cap_p2p, (uint2*)fout, m2l, p2p, code, blk,
                      (const WalkRec*)rec);
