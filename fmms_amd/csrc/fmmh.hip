@@ -246,7 +246,7 @@ struct fmmh_ctx {
     ensure(bm, n * 8);
     ensure(bxyzm, n * 32);
     ensure(bpack, n * 32);
-    ensure(bbox_partial, 6 * 1024 * 8);
+    ensure(bbox_partial, bbox_partial_bytes());
     ensure(bbox, nsys * sizeof(BBox));
     ensure(flags, TREE_FLAGS * 4);
     ensure(chain, n * 8);
@@ -257,7 +257,7 @@ struct fmmh_ctx {
     HCHECK(hipMemsetAsync(flags.p, 0, TREE_FLAGS * 4, s));
     uint64_t* off = nullptr;
     if (nsys == 1) {
-      launch_bbox(pos, n, (double*)bbox_partial.p, (BBox*)bbox.p, s);
+      launch_bbox(pos, n, nullptr, 1, (double*)bbox_partial.p, (BBox*)bbox.p, s);
       launch_keys(pos, mass, n, (const BBox*)bbox.p, (uint64_t*)keys.p, (uint32_t*)vals.p,
                   (uint32_t*)flags.p, (double4*)bpack.p, s);
     } else {
@@ -265,7 +265,7 @@ struct fmmh_ctx {
       uint64_t* h = (uint64_t*)host_stage((nsys + 1) * 8);
       std::memcpy(h, sys_off.data(), (nsys + 1) * 8);
       HCHECK(hipMemcpyAsync(off, h, (nsys + 1) * 8, hipMemcpyHostToDevice, s));
-      launch_bbox_sys(pos, off, nsys, (BBox*)bbox.p, s);
+      launch_bbox(pos, n, off, nsys, (double*)bbox_partial.p, (BBox*)bbox.p, s);
       launch_keys_sys(pos, mass, n, off, nsys, vlev, (const BBox*)bbox.p, (uint64_t*)keys.p,
                       (uint32_t*)vals.p, (uint32_t*)flags.p, (double4*)bpack.p, s);
     }

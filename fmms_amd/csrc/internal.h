@@ -62,10 +62,11 @@ struct DevBodies {  // slot (Morton) order, bodies.rs:13-22
 };
 
 // -------------------------------------------------------------- tree.hip
-void launch_bbox(const double* pos, size_t n, double* partial, BBox* out, hipStream_t s);
-// Ensembles of nsys systems (body ranges off[s]..off[s+1], device array).
-void launch_bbox_sys(const double* pos, const uint64_t* off, uint32_t nsys, BBox* out,
-                     hipStream_t s);
+// Boxes of nsys systems (body ranges off[s]..off[s+1], device array; one system:
+// off null); partial is scratch of bbox_partial_bytes().
+size_t bbox_partial_bytes();
+void launch_bbox(const double* pos, size_t n, const uint64_t* off, uint32_t nsys, double* partial,
+                 BBox* out, hipStream_t s);
 void launch_keys_sys(const double* pos, const double* mass, size_t n, const uint64_t* off,
                      uint32_t nsys, int vlev, const BBox* bbs, uint64_t* keys, uint32_t* vals,
                      uint32_t* flags, double4* pk, hipStream_t s);
