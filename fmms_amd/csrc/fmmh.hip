@@ -99,7 +99,7 @@ struct fmmh_ctx {
   Buf bx, by, bz, bm, bxyzm;
   Buf bpack;  // (x, y, z, m) in id order, written with the keys for the gather
   Buf bbox_partial, bbox, flags;
-  Buf chain, cstart;  // per slot: cells starting there, and their scan
+  Buf cstart;  // per slot: scan of the cells starting there
   Buf c_first, c_count, c_children, c_parent, c_leaf, c_level, c_cx, c_cy, c_cz, c_mass, c_rho,
       c_rope, c_last;
   Buf lvl_cells;  // cells by level, a level's internal cells first
@@ -117,19 +117,21 @@ struct fmmh_ctx {
   Buf walk_code, walk_blk;  // the walk's per-pair decisions, per-block counts
   Buf pl_longs, pl_items, pl_reds, pl_partial;  // P2P work plan
   Buf m2l_lam, m2l_m32;                     // mixed form: FP32 M2L scales, scaled moments
-  Buf m2l_rows;                             // M2L source rows
+  Buf m2l_rows;                             // M2L source rows, where ...
+  double* rows = nullptr;                   // ... the M2L sort's idle buffer is too small
   Buf loc32;                                // mixed form: FP32 locals scaled by lam^n
   uint32_t p_nitems = 0, p_nsplit = 0, p_nlong = 0;
   Buf rt_tab;  // p > TEMPLATED_MAX_P: the rotation M2L's tables
   Buf ctrace, clap;  // softened far field: q = sum m |x - z|^2; L, G, H per cell
   int rot_p = -1;
+  int mac_p = -1;  // order of fact, binom
   std::vector<uint32_t> rot_off;
   Buf direct_ids, direct_out, direct_part;
   Buf pinned;
 
   fmmh_ctx() {
     Buf* all[] = {&in_pos, &in_mass, &out_acc, &out_pot, &keys, &keys_alt, &vals, &vals_alt,
-                  &bx, &by, &bz, &bm, &bxyzm, &bpack, &bbox_partial, &bbox, &flags, &chain, &cstart,
+                  &bx, &by, &bz, &bm, &bxyzm, &bpack, &bbox_partial, &bbox, &flags, &cstart,
                   &c_first, &c_count, &c_children, &c_parent, &c_leaf, &c_level,
                   &c_cx, &c_cy, &c_cz, &c_mass, &c_rho, &c_rope, &c_last, &lvl_cells,
                   &leaf_ids, &leaf_of_slot, &leaf_bc, &cpm,
@@ -249,8 +251,7 @@ struct fmmh_ctx {
     ensure(bbox_partial, bbox_partial_bytes());
     ensure(bbox, nsys * sizeof(BBox));
     ensure(flags, TREE_FLAGS * 4);
-    ensure(chain, n * 8);
-    ensure(cstart, n * 8);
+    ensure(cstart, std::max<size_t>(n, 4) * 8);
     ensure(sort_tmp, radix_tmp_words(n) * 4 + 64);
     ensure_scan(n);
     mark(ST_TREE);
@@ -289,9 +290,10 @@ struct fmmh_ctx {
     launch_gather_packed((const double4*)bpack.p, order, n, bodies(), s);
     // cells per slot and per level, one host read for the lot
     uint32_t* fl = (uint32_t*)flags.p;
-    launch_chain(keys_sorted, n, (uint32_t)prm.n_leaf, vlev, (uint64_t*)chain.p, fl + 4, s);
+    uint64_t* chain = (uint64_t*)(keys_sorted == keys.p ? keys_alt.p : keys.p);  // the sort's other
+    launch_chain(keys_sorted, n, (uint32_t)prm.n_leaf, vlev, chain, fl + 4, s);
     uint64_t* tot = nullptr;
-    scan_exclusive_u64((uint64_t*)chain.p, (uint64_t*)cstart.p, n, (uint64_t*)scan_tmp.p, s, &tot);
+    scan_exclusive_u64(chain, (uint64_t*)cstart.p, n, (uint64_t*)scan_tmp.p, s, &tot);
     uint32_t* h = (uint32_t*)host_stage(TREE_FLAGS * 4);
     HCHECK(hipMemcpyAsync(h, fl, TREE_FLAGS * 4, hipMemcpyDeviceToHost, s));
     HCHECK(hipStreamSynchronize(s));
@@ -325,7 +327,7 @@ struct fmmh_ctx {
     ensure(leaf_bc, (size_t)nleaves * 4);
     ensure(leaf_of_slot, n * 4);
     ensure(sort_tmp, radix_tmp_words(nc) * 4 + 64);
-    launch_cells(keys_sorted, n, (const uint64_t*)chain.p, (const uint64_t*)cstart.p, nc, cells(),
+    launch_cells(keys_sorted, n, chain, (const uint64_t*)cstart.p, nc, cells(),
                  (uint32_t*)leaf_ids.p, (uint32_t*)leaf_of_slot.p, s);
     cells_by_level((const uint8_t*)c_level.p, (const uint8_t*)c_leaf.p, nc, (uint32_t*)lvl_cells.p,
                    (uint32_t*)sort_tmp.p, s);
@@ -400,11 +402,10 @@ struct fmmh_ctx {
     }
   }
 
-  // Multipole powers, f pre-pass and fmin (error-controlled MAC only).
-  void mac_inputs() {
+  // Factorials and binomials of the order, laid out once per context.
+  void mac_tables() {
     const int p = prm.p;
-    DevCells c = cells();
-    DevBodies b = bodies();
+    if (mac_p == p) return;
     std::vector<double> f(2 * p + 1, 1.0);
     for (size_t i = 1; i < f.size(); i++) f[i] = f[i - 1] * (double)i;  // moments.rs:11-17
     std::vector<double> bn(p + 1, 1.0);
@@ -417,6 +418,15 @@ struct fmmh_ctx {
     HCHECK(hipMemcpyAsync(fact.p, hf, f.size() * 8, hipMemcpyHostToDevice, s));
     HCHECK(hipMemcpyAsync(binom.p, hf + f.size(), bn.size() * 8, hipMemcpyHostToDevice, s));
     HCHECK(hipStreamSynchronize(s));
+    mac_p = p;
+  }
+
+  // Multipole powers, f pre-pass and fmin (error-controlled MAC only).
+  void mac_inputs() {
+    const int p = prm.p;
+    DevCells c = cells();
+    DevBodies b = bodies();
+    mac_tables();
     ensure(fmin, nc * 8);
     ensure(pows, (size_t)nc * (p + 1) * 8);
     ensure(fvals, n * 8);
@@ -424,9 +434,15 @@ struct fmmh_ctx {
     ensure(fprec, (size_t)nc * fp_rec_bytes());
     launch_pack_fp(nc, c, fprec.p, s);
     launch_fprepass((uint32_t)n, nc, fprec.p, b.xyzm, keys_sorted, vlev, (double*)fvals.p, s);
-    for (int L = (int)max_level; L >= 0; L--)
-      launch_fmin((uint32_t*)lvl_cells.p + lvl_off[L], lvl_off[L + 1] - lvl_off[L], c,
-                  (double*)fvals.p, (double*)fmin.p, s);
+    // the tree's scan (n words at least, and 4) is done with
+    launch_fmin((uint32_t)n, nc, c, (const double*)fvals.p, (double*)cstart.p, (double*)fmin.p, s);
+  }
+
+  // Room for the M2L source rows: the buffer that the directed sort did not end
+  // in, which nothing reads until the next lists, if it is large enough.
+  double* source_rows(size_t bytes) {
+    const Buf& idle = msorted == mkeys.p ? mkeys_alt : mkeys;
+    return idle.cap >= bytes ? (double*)idle.p : ensure<double>(m2l_rows, bytes);
   }
 
   // Directed lists grouped by target, P2P work count, M2L chunks.
@@ -485,12 +501,12 @@ struct fmmh_ctx {
     if (p > TEMPLATED_MAX_P) {
       rot_tables();
     } else if (!mixed32()) {
-      ensure(m2l_rows, (size_t)nc * m2l_row_bytes(p));
+      rows = source_rows((size_t)nc * m2l_row_bytes(p));
     } else {
       ensure(m2l_lam, (size_t)nc * sizeof(double));
       ensure(m2l_m32, (size_t)nc * m2l32_moment_bytes(p));
       ensure(loc32, (size_t)nc * m2l32_moment_bytes(p));
-      ensure(m2l_rows, (size_t)nc * m2l32_row_bytes(p));
+      rows = source_rows((size_t)nc * m2l32_row_bytes(p));
     }
     ensure(far, n * sizeof(double4));
   }
@@ -514,13 +530,13 @@ struct fmmh_ctx {
     mark(ST_M2L);
     if (!gen && prm.precision == FMMH_PREC_FP32BULK) {
       launch_m2l32(p, nc, chunks.p, nchunks, msorted, sbits, c, (const BBox*)bbox.p, keys_sorted,
-                   vlev, mom, soft2, (double*)m2l_lam.p, m2l_m32.p, (double*)m2l_rows.p, part.p, s,
+                   vlev, mom, soft2, (double*)m2l_lam.p, m2l_m32.p, rows, part.p, s,
                    up32() ? vlev + FP64_TOP : 255);
       mark(ST_M2L_REDUCE);
       launch_m2l_reduce32(p, nc, (const uint4*)plan.p, part.p, (const double*)m2l_lam.p, loc, s);
     } else if (!gen) {
       launch_m2l_kernel(p, nc, chunks.p, nchunks, msorted, sbits, c, mom, soft2,
-                        (double*)m2l_rows.p, (double*)part.p, s);
+                        rows, (double*)part.p, s);
       mark(ST_M2L_REDUCE);
       launch_m2l_reduce(p, nc, (const uint4*)plan.p, (const double*)part.p, loc, s);
     } else {

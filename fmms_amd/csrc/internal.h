@@ -111,7 +111,8 @@ size_t fp_rec_bytes();
 void launch_pack_fp(uint32_t nc, DevCells c, void* rec, hipStream_t s);
 void launch_fprepass(uint32_t n, uint32_t nc, const void* rec, const double4* body,
                      const uint64_t* keys_sorted, int vlev, double* f, hipStream_t s);
-void launch_fmin(const uint32_t* cells, uint32_t cnt, DevCells c, const double* f, double* fmin,
+size_t fmin_blocks_words(size_t n);
+void launch_fmin(uint32_t n, uint32_t nc, DevCells c, const double* f, double* blocks, double* fmin,
                  hipStream_t s);
 
 // -------------------------------------------------------------- walk.hip
