@@ -601,35 +601,57 @@ __global__ void __launch_bounds__(PLAN_T) k_plan_emit(
   const uint32_t T = (L.S - 1) / m + 1;
   uint32_t running = L.nt;  // sources before the first neighbour unit
   uint32_t gprev = 0;       // item of unit 0 (the own leaf)
-  auto unit = [&](uint32_t j) -> uint32_t {
-    if (j >= L.je) return 0u;
-    const uint32_t src = (uint32_t)(skeys[j] & smask);
-    return src == L.leaf ? 0u : ccount[src];
+  // PU consecutive units a lane, the following ones' counts loaded ahead: the
+  // longest leaf's chain of such steps bounds the launch (100k bodies, one unit a
+  // lane 102 us, four 66)
+  constexpr uint32_t PU = 4;
+  auto units = [&](uint32_t j0, uint32_t* cnt) {
+    uint32_t src[PU];
+#pragma unroll
+    for (uint32_t u = 0; u < PU; u++)
+      src[u] = j0 + u < L.je ? (uint32_t)(skeys[j0 + u] & smask) : L.leaf;
+#pragma unroll
+    for (uint32_t u = 0; u < PU; u++) cnt[u] = src[u] == L.leaf ? 0u : ccount[src[u]];
   };
-  uint32_t next = unit(L.jb + lane);  // the following 64 units' counts, loaded ahead
-  for (uint32_t c0 = L.jb; m > 1 && c0 < L.je; c0 += 64) {
-    const uint32_t j = c0 + lane;
-    const bool valid = j < L.je;
-    const uint32_t cnt = next;
-    next = unit(j + 64);
-    uint32_t incl = cnt;  // inclusive wave scan
+  uint32_t next[PU];
+  units(L.jb + PU * lane, next);
+  for (uint32_t c0 = L.jb; m > 1 && c0 < L.je; c0 += 64 * PU) {
+    const uint32_t j = c0 + PU * lane;
+    uint32_t cnt[PU], own = 0u;
+#pragma unroll
+    for (uint32_t u = 0; u < PU; u++) {
+      cnt[u] = next[u];
+      own += cnt[u];
+    }
+    units(j + 64 * PU, next);
+    uint32_t incl = own;  // inclusive wave scan
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const uint32_t v = __shfl_up(incl, o, 64);
       if ((int)lane >= o) incl += v;
     }
-    const uint32_t P = running + incl - cnt;
-    const uint32_t g = valid ? min(P / T, m - 1) : 0u;
-    const uint32_t gl = (uint32_t)__shfl_up(g, 1, 64);
-    const uint32_t before = lane == 0 ? gprev : gl;
-    if (valid && g > before)
-      for (uint32_t k = before + 1; k <= g; k++) {
-        it[4 * k + 1] = j;
-        it[4 * (k - 1) + 2] = j;
+    uint32_t P = running + incl - own;
+    uint32_t g[PU], glast = 0u;  // of the lane's last valid unit
+#pragma unroll
+    for (uint32_t u = 0; u < PU; u++) {
+      g[u] = min(P / T, m - 1);
+      if (j + u < L.je) glast = g[u];
+      P += cnt[u];
+    }
+    const uint32_t gl = (uint32_t)__shfl_up(glast, 1, 64);
+    uint32_t before = lane == 0 ? gprev : gl;
+#pragma unroll
+    for (uint32_t u = 0; u < PU; u++) {
+      if (j + u >= L.je) break;
+      for (uint32_t k = before + 1; k <= g[u]; k++) {
+        it[4 * k + 1] = j + u;
+        it[4 * (k - 1) + 2] = j + u;
       }
-    const uint32_t last = min(63u, L.je - 1 - c0);  // last valid lane of this chunk
-    gprev = (uint32_t)__shfl(g, (int)last, 64);
-    running += __shfl(incl, (int)last, 64);
+      before = g[u];
+    }
+    const uint32_t last = min(63u, (L.je - 1 - c0) / PU);  // last lane with a unit
+    gprev = (uint32_t)__shfl(glast, (int)last, 64);
+    running += __shfl(incl, 63, 64);
   }
   // items after the last unit's item are empty; the last item ends the list
   for (uint32_t k = gprev + lane; k < m; k += 64) {
