@@ -83,6 +83,7 @@ __device__ __forceinline__ void f_at(const cplx* F, int s, int q, double* br, do
 // (P - n + 1)^2 products for degree n, longest first to the least loaded wave.
 // Per level at p = 8: 13.0 -> 8.0 us (1k bodies), 15.6 -> 9.4 (100k).
 constexpr int L2L_G = 4;
+constexpr int L2L32_SPLIT_TO = 8;  // see k_l2l32_whole
 template <int P>
 struct L2lGroups {
   int of[P + 1];
@@ -352,6 +353,97 @@ __device__ __forceinline__ void l2l32_part(uint32_t c, uint32_t pa, const double
   });
 }
 
+// P = 9 and 10: one thread per cell. Dealt out to waves, the compiler contracts the
+// FP32 sums of these orders with other roundings (forces differ by 1e-9; to P = 8
+// the two are bit for bit the same), for 5 us a level.
+template <int P>
+__global__ void __launch_bounds__(64) k_l2l32_whole(const uint32_t* __restrict__ cells, uint32_t cnt,
+                                                   const int32_t* __restrict__ parent,
+                                                   const double* __restrict__ cx,
+                                                   const double* __restrict__ cy,
+                                                   const double* __restrict__ cz,
+                                                   const double* __restrict__ lam,
+                                                   const cplx* __restrict__ own,
+                                                   cplxf* __restrict__ loc32) {
+  constexpr int D = hdim(P), NF = hnpos(P);
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= cnt) return;
+  const uint32_t c = cells[i];
+  const int32_t pa = parent[c];
+  const double lc = lam[c];
+  const cplx* lo = own + (size_t)c * D;
+  cplxf* out = loc32 + (size_t)c * NF;
+  if (pa < 0) {
+    double sc = 1.0;
+#pragma unroll
+    for (int n = 0; n <= P; n++) {
+#pragma unroll
+      for (int m = 0; m <= n; m++) {
+        const cplx v = lo[hidx(n, m)];
+        out[hpos(n, m)] = cplxf{(float)(v.re * sc), (float)(v.im * sc)};
+      }
+      sc *= lc;
+    }
+    return;
+  }
+  const double lp = lam[pa], il = 1.0 / lp;
+  const double kap = lc * il;
+  cplxf G[NF], Fp[NF];
+  {
+    const double ik = 1.0 / kap;
+    double sc = 1.0;  // lam_c^n kappa^-n = lam_p^n
+#pragma unroll
+    for (int n = 0; n <= P; n++) {
+#pragma unroll
+      for (int m = 0; m <= n; m++) {
+        const cplx v = lo[hidx(n, m)];
+        G[hpos(n, m)] = cplxf{(float)(v.re * sc), (float)(v.im * sc)};
+      }
+      sc *= lc * ik;
+    }
+  }
+  const cplxf* lpp = loc32 + (size_t)pa * NF;
+#pragma unroll
+  for (int e = 0; e < NF; e++) Fp[e] = lpp[e];
+  const float x = (float)((cx[pa] - cx[c]) * il), y = (float)((cy[pa] - cy[c]) * il),
+              z = (float)((cz[pa] - cz[c]) * il);
+  const float r2 = x * x + y * y + z * z;
+  cplxf U[P + 1], U1[P + 1], U2[P + 1];
+#pragma unroll
+  for (int k = 0; k <= P; k++) {
+    upsilon_degree32<P>(k, x, y, z, r2, U, U1, U2);
+#pragma unroll
+    for (int n = 0; n <= P; n++) {
+      if (n + k > P) continue;
+#pragma unroll
+      for (int m = 0; m <= P; m++) {
+        if (m > n) continue;
+#pragma unroll
+        for (int l = -P; l <= P; l++) {
+          if (l < -k || l > k) continue;
+          float ar, ai, br, bi;
+          conj_y32(U, l, &ar, &ai);
+          f_at32<P>(Fp, n + k, m + l, &br, &bi);
+          cmac2f(G[hpos(n, m)], ar, ai, br, bi);
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q <= P; q++) {
+      U2[q] = U1[q];
+      U1[q] = U[q];
+    }
+  }
+  float kn = 1.0f;
+  const float kf = (float)kap;
+#pragma unroll
+  for (int n = 0; n <= P; n++) {
+#pragma unroll
+    for (int m = 0; m <= n; m++) out[hpos(n, m)] = cplxf{G[hpos(n, m)].re * kn, G[hpos(n, m)].im * kn};
+    kn *= kf;
+  }
+}
+
 template <int P>
 __global__ void __launch_bounds__(64 * L2L_G) k_l2l32(const uint32_t* __restrict__ cells,
                                                      uint32_t cnt,
@@ -504,8 +596,12 @@ bool launch_l2l32(int p, const uint32_t* cells, uint32_t cnt, DevCells c, const 
                   const cplx* own, void* loc32, hipStream_t s) {
   if (cnt == 0) return true;
 #define CALL(P)                                                                                  \
-  hipLaunchKernelGGL(k_l2l32<P>, dim3((cnt + 63) / 64), dim3(64 * L2L_G), 0, s, cells, cnt, c.parent, \
-                     c.cx, c.cy, c.cz, lam, own, (cplxf*)loc32)
+  if constexpr (P <= L2L32_SPLIT_TO)                                                             \
+    hipLaunchKernelGGL(k_l2l32<P>, dim3((cnt + 63) / 64), dim3(64 * L2L_G), 0, s, cells, cnt,     \
+                       c.parent, c.cx, c.cy, c.cz, lam, own, (cplxf*)loc32);                      \
+  else                                                                                           \
+    hipLaunchKernelGGL(k_l2l32_whole<P>, dim3((cnt + 63) / 64), dim3(64), 0, s, cells, cnt,       \
+                       c.parent, c.cx, c.cy, c.cz, lam, own, (cplxf*)loc32)
   FMMH_P_SWITCH2(p, CALL)
 #undef CALL
   return true;
