@@ -47,7 +47,7 @@ sys.path.insert(0, ROOT)
 METRIC = "body-forces/sec @ rel err ≤1e-5, mixed vs FP64 GPU; p50/p99 step latency"
 FP64_PEAK_TFLOPS = 78.6  # MI355X FP64 vector / matrix peak
 # MI355X FP32 vector peak (published; reached only with packed FP32 math,
-# which this build leaves off: unpacked FP32 issues at the FP64 rate).
+# which this build leaves off; unpacked FP32 is priced at the FP64 peak).
 FP32_PEAK_TFLOPS = 157.3
 # Softening guard of the MAC on the halos and ensemble workloads (softening
 # reaching into the far field of small cells): M2L only where

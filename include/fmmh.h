@@ -64,7 +64,7 @@ extern "C" {
 #define FMMH_FLAG_TIMING 1u   /* record per-stage device times (hipEvents) */
 
 typedef struct fmmh_params {
-  int p;            /* expansion order (Fmm.p); 1..FMMH_MAX_P (rotation M2L from p = 20) */
+  int p;            /* expansion order (Fmm.p); 1..FMMH_MAX_P (rotation M2L above p = 10) */
   double eps_mac;   /* error-controlled MAC tolerance (Fmm.eps, mac.rs:8-11,92);
                        +INFINITY = theta-only MAC, no f pre-pass */
   double theta_max; /* opening angle bound; 1.0 = the reference's hard-coded theta<1 */
@@ -115,9 +115,10 @@ int fmmh_accel_device(fmmh_ctx* ctx, size_t n, const double* d_pos, const double
  * fmms_amd.autotune picks them (with p and n_leaf) by measurement. */
 typedef struct fmmh_tuning {
   int m2l_chunk;          /* sources per M2L work chunk (one thread's serial work), 1..1024;
-                             default 32 */
+                             default 32; p <= 10 (above, chunks are 64 sources) */
   uint64_t p2p_item_work; /* a leaf whose targets x sources exceed this is cut into P2P work
-                             items of about equal source count, 64..2^40; default 2^18 */
+                             items of about equal source count, 64..2^40; default 2^18
+                             (the FP64 form also cuts at 4096 sources an item) */
 } fmmh_tuning;
 void fmmh_default_tuning(fmmh_tuning* out);
 int fmmh_set_tuning(fmmh_ctx* ctx, const fmmh_tuning* t);
@@ -224,7 +225,8 @@ const char* fmmh_stage_name(int stage);
 int fmmh_work_counts(const fmmh_ctx* ctx, uint64_t* out8);
 /* P2P work plan of the current lists (no counterpart in the reference, whose
  * threads take leaf pairs from a shared list): [work items, leaves cut into
- * several items]. A leaf whose targets x sources exceed 2^18 is cut into
+ * several items]. A leaf whose targets x sources exceed
+ * p2p_item_work (in FP64: or whose items would pass 4096 sources) is cut into
  * items of about equal source count, added back in a fixed order. */
 int fmmh_p2p_plan_counts(const fmmh_ctx* ctx, uint64_t* out2);
 
