@@ -97,7 +97,9 @@ struct fmmh_ctx {
   Buf in_pos, in_mass, out_acc, out_pot;
   Buf keys, keys_alt, vals, vals_alt;
   Buf bx, by, bz, bm, bxyzm;
-  Buf bpack;  // (x, y, z, m) in id order, written with the keys for the gather
+  // (x, y, z, m) in id order, written with the keys for the build's gather; then
+  // the bodies' far field (double4 by slot), from L2P to the final sums
+  Buf bpack;
   Buf bbox_partial, bbox, flags;
   Buf cstart;  // per slot: scan of the cells starting there
   Buf c_first, c_count, c_children, c_parent, c_leaf, c_level, c_cx, c_cy, c_cz, c_mass, c_rho,
@@ -113,12 +115,12 @@ struct fmmh_ctx {
   Buf front_a, front_b, m2l, p2p, ctr;
   Buf mkeys, mkeys_alt, tptr, pkeys, pkeys_alt, pptr;
   Buf plan, chunks, part;
-  Buf far, p2p_work, walkrec;
+  Buf p2p_work, walkrec;
   Buf walk_code, walk_blk;  // the walk's per-pair decisions, per-block counts
   Buf pl_longs, pl_items, pl_reds, pl_partial;  // P2P work plan
   Buf m2l_lam, m2l_m32;                     // mixed form: FP32 M2L scales, scaled moments
-  Buf m2l_rows;                             // M2L source rows, where ...
-  double* rows = nullptr;                   // ... the M2L sort's idle buffer is too small
+  Buf m2l_rows;  // M2L source rows, where no idle buffer holds them
+  double* rows = nullptr;
   Buf loc32;                                // mixed form: FP32 locals scaled by lam^n
   uint32_t p_nitems = 0, p_nsplit = 0, p_nlong = 0;
   Buf rt_tab;  // p > TEMPLATED_MAX_P: the rotation M2L's tables
@@ -138,7 +140,7 @@ struct fmmh_ctx {
                   &scan_tmp, &sort_tmp,
                   &fprec, &moments, &locals, &pows, &fvals, &fmin, &fact, &binom, &front_a, &front_b,
                   &m2l, &p2p, &ctr, &mkeys, &mkeys_alt, &tptr, &pkeys, &pkeys_alt, &pptr,
-                  &plan, &chunks, &part, &far, &p2p_work, &walkrec, &walk_code, &walk_blk, &pl_longs, &pl_items,
+                  &plan, &chunks, &part, &p2p_work, &walkrec, &walk_code, &walk_blk, &pl_longs, &pl_items,
                   &pl_reds, &pl_partial, &m2l_lam, &m2l_m32, &m2l_rows, &loc32, &rt_tab, &direct_ids, &direct_out, &direct_part, &lf_part, &lf_state, &lf_flag, &ctrace, &clap,
                   &d_sysoff};
     bufs.assign(std::begin(all), std::end(all));
@@ -248,7 +250,7 @@ struct fmmh_ctx {
     ensure(bm, n * 8);
     ensure(bxyzm, n * 32);
     ensure(bpack, n * 32);
-    ensure(bbox_partial, bbox_partial_bytes());
+    ensure(bbox_partial, bbox_partial_bytes(n, nsys));
     ensure(bbox, nsys * sizeof(BBox));
     ensure(flags, TREE_FLAGS * 4);
     ensure(cstart, std::max<size_t>(n, 4) * 8);
@@ -438,9 +440,12 @@ struct fmmh_ctx {
     launch_fmin((uint32_t)n, nc, c, (const double*)fvals.p, (double*)cstart.p, (double*)fmin.p, s);
   }
 
-  // Room for the M2L source rows: the buffer that the directed sort did not end
-  // in, which nothing reads until the next lists, if it is large enough.
+  // Room for the M2L source rows: the locals, which the reduction writes after
+  // the last row has been read (every order from 2 up fits), or the buffer that
+  // the directed sort did not end in, which nothing reads until the next lists.
+  // A buffer of their own was 8 - 11 % of a context with short lists.
   double* source_rows(size_t bytes) {
+    if (locals.cap >= bytes) return (double*)locals.p;
     const Buf& idle = msorted == mkeys.p ? mkeys_alt : mkeys;
     return idle.cap >= bytes ? (double*)idle.p : ensure<double>(m2l_rows, bytes);
   }
@@ -508,7 +513,6 @@ struct fmmh_ctx {
       ensure(loc32, (size_t)nc * m2l32_moment_bytes(p));
       rows = source_rows((size_t)nc * m2l32_row_bytes(p));
     }
-    ensure(far, n * sizeof(double4));
   }
 
   // The mixed form's FP32 M2L, L2L and L2P (templated orders only).
@@ -564,23 +568,23 @@ struct fmmh_ctx {
     }
     mark(ST_L2P);
     if (l32)
-      launch_l2p(p, (uint32_t)n, (uint32_t*)leaf_of_slot.p, c, b, loc, lap, (double4*)far.p, s,
+      launch_l2p(p, (uint32_t)n, (uint32_t*)leaf_of_slot.p, c, b, loc, lap, (double4*)bpack.p, s,
                  (const double*)m2l_lam.p, loc32.p);
     else if (!gen)
-      launch_l2p(p, (uint32_t)n, (uint32_t*)leaf_of_slot.p, c, b, loc, lap, (double4*)far.p, s);
+      launch_l2p(p, (uint32_t)n, (uint32_t*)leaf_of_slot.p, c, b, loc, lap, (double4*)bpack.p, s);
     else
-      launch_l2p_gen(p, (uint32_t*)leaf_ids.p, nleaves, c, b, loc, lap, (double4*)far.p, s);
+      launch_l2p_gen(p, (uint32_t*)leaf_ids.p, nleaves, c, b, loc, lap, (double4*)bpack.p, s);
     const P2PPlan pl{(const uint4*)pl_items.p, p_nitems, p_nlong, (const uint32_t*)pl_longs.p,
                      (const uint4*)pl_reds.p, p_nsplit, (double4*)pl_partial.p};
     const bool f32 = prm.precision == FMMH_PREC_FP32BULK;
     mark(ST_P2P);
     if (f32)
-      launch_p2p_f32(pl, c, b.xyzm, psorted, sbits, soft2, (const double4*)far.p, order, acc, pot,
+      launch_p2p_f32(pl, c, b.xyzm, psorted, sbits, soft2, (const double4*)bpack.p, order, acc, pot,
                      s);
     else
-      launch_p2p(pl, c, b.xyzm, psorted, sbits, soft2, (const double4*)far.p, order, acc, pot, s);
+      launch_p2p(pl, c, b.xyzm, psorted, sbits, soft2, (const double4*)bpack.p, order, acc, pot, s);
     mark(ST_P2P_REDUCE);
-    launch_p2p_reduce(pl, c, (const double4*)far.p, order, acc, pot, f32, s);
+    launch_p2p_reduce(pl, c, (const double4*)bpack.p, order, acc, pot, f32, s);
     mark(ST_COUNT);
   }
 

@@ -63,8 +63,8 @@ struct DevBodies {  // slot (Morton) order, bodies.rs:13-22
 
 // -------------------------------------------------------------- tree.hip
 // Boxes of nsys systems (body ranges off[s]..off[s+1], device array; one system:
-// off null); partial is scratch of bbox_partial_bytes().
-size_t bbox_partial_bytes();
+// off null); partial is scratch of bbox_partial_bytes(n, nsys).
+size_t bbox_partial_bytes(size_t n, uint32_t nsys);
 void launch_bbox(const double* pos, size_t n, const uint64_t* off, uint32_t nsys, double* partial,
                  BBox* out, hipStream_t s);
 void launch_keys_sys(const double* pos, const double* mass, size_t n, const uint64_t* off,

@@ -111,13 +111,19 @@ __global__ void __launch_bounds__(TB) k_bbox_final(const double* __restrict__ pa
 // Blocks per system: BBOX_BLOCKS in all, each with a body a thread at least on
 // average. One block per system left most of the chip idle: 48 systems of 31k
 // bodies 291 -> 21 + 5 us. Minima and maxima do not depend on the split.
-size_t bbox_partial_bytes() { return (size_t)6 * BBOX_BLOCKS * sizeof(double); }
+static uint32_t bbox_blocks(size_t n, uint32_t nsys) {
+  const size_t most = std::max<size_t>(1, BBOX_BLOCKS / nsys);
+  return (uint32_t)std::min(most, std::max<size_t>(1, (n / nsys + TB - 1) / TB));
+}
+
+size_t bbox_partial_bytes(size_t n, uint32_t nsys) {
+  const uint32_t nb = bbox_blocks(n, nsys);
+  return nb > 1 ? (size_t)6 * nsys * nb * sizeof(double) : 0;  // a system's only block keeps none
+}
 
 void launch_bbox(const double* pos, size_t n, const uint64_t* off, uint32_t nsys, double* partial,
                  BBox* out, hipStream_t s) {
-  const size_t most = std::max<size_t>(1, BBOX_BLOCKS / nsys);
-  const uint32_t nb =
-      (uint32_t)std::min(most, std::max<size_t>(1, (n / nsys + TB - 1) / TB));
+  const uint32_t nb = bbox_blocks(n, nsys);
   hipLaunchKernelGGL(k_bbox_partial, dim3(nsys * nb), dim3(TB), 0, s, pos, n, off, nb, partial, out);
   if (nb > 1) hipLaunchKernelGGL(k_bbox_final, dim3(nsys), dim3(TB), 0, s, partial, nb, out);
 }
