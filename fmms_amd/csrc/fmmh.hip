@@ -126,6 +126,8 @@ struct fmmh_ctx {
   Buf rt_tab;  // p > TEMPLATED_MAX_P: the rotation M2L's tables
   Buf ctrace, clap;  // softened far field: q = sum m |x - z|^2; L, G, H per cell
   int rot_p = -1;
+  cplx* rot_part = nullptr;  // rotation M2L: room for the partials of a slice of chunks
+  size_t rot_slice = 0;
   int mac_p = -1;  // order of fact, binom
   std::vector<uint32_t> rot_off;
   Buf direct_ids, direct_out, direct_part;
@@ -446,8 +448,40 @@ struct fmmh_ctx {
   // A buffer of their own was 8 - 11 % of a context with short lists.
   double* source_rows(size_t bytes) {
     if (locals.cap >= bytes) return (double*)locals.p;
-    const Buf& idle = msorted == mkeys.p ? mkeys_alt : mkeys;
+    const Buf& idle = idle_keys(msorted, mkeys, mkeys_alt);
     return idle.cap >= bytes ? (double*)idle.p : ensure<double>(m2l_rows, bytes);
+  }
+
+  // The key buffer that a directed sort did not end in: idle until the next lists.
+  const Buf& idle_keys(const uint64_t* sorted, const Buf& a, const Buf& b) const {
+    return sorted == a.p ? b : a;
+  }
+
+  // Room for the chunk partials of the orders above 10, all of them at once up to
+  // ROT_PART_MAX (5.2 KB a chunk at p = 24, 13.8 at p = 40: a buffer for any number
+  // of them doubled a context): an idle key buffer if they fit there, or a buffer
+  // of their own, or, where the context's budget has no room for that, what is
+  // idle, and the chunks run in more slices. Each slice has a tail of its own:
+  // order 24, 30k bodies, 10.8k chunks, in one 9.44 ms an evaluation, in two 9.61.
+  static constexpr size_t ROT_PART_MAX = (size_t)64 << 20;
+  void rot_room() {
+    const size_t one = m2l_part_bytes(prm.p, 1, false);
+    const size_t want = std::min<size_t>(nchunks, std::max<size_t>(1, ROT_PART_MAX / one));
+    const Buf& km = idle_keys(msorted, mkeys, mkeys_alt);
+    const Buf& kp = idle_keys(psorted, pkeys, pkeys_alt);
+    const Buf& idle = km.cap >= kp.cap ? km : kp;
+    const size_t limit = (size_t)prm.hbm_budget_bytes;
+    // the pair count on request (fmmh_work_counts) comes after an evaluation
+    const size_t later = (1 + p2p_count_scratch(n_p2p)) * 8;
+    const bool fits = part.cap >= want * one || !limit ||
+                      used - part.cap + want * one + later <= limit;
+    if (idle.cap >= want * one || (!fits && idle.cap >= one)) {
+      rot_part = (cplx*)idle.p;
+      rot_slice = std::min(want, idle.cap / one);
+    } else {
+      rot_slice = fits ? want : 1;
+      rot_part = ensure<cplx>(part, rot_slice * one);
+    }
   }
 
   // Directed lists grouped by target, P2P work count, M2L chunks.
@@ -502,10 +536,13 @@ struct fmmh_ctx {
     plan_emit(nc, cells(), (const uint32_t*)tptr.p, ch, (const uint32_t*)pptr.p, psorted, sbits,
               tun.p2p_item_work, f32, pl, chunks.p, (uint4*)pl_items.p, (uint4*)pl_reds.p,
               p_nlong ? (uint32_t*)(pl + nc + 1) + 1 : nullptr, (uint32_t*)pl_longs.p, s);
-    ensure(part, m2l_part_bytes(p, std::max<size_t>(nchunks, 1), mixed32()));
     if (p > TEMPLATED_MAX_P) {
       rot_tables();
-    } else if (!mixed32()) {
+      rot_room();
+      return;
+    }
+    ensure(part, m2l_part_bytes(p, std::max<size_t>(nchunks, 1), mixed32()));
+    if (!mixed32()) {
       rows = source_rows((size_t)nc * m2l_row_bytes(p));
     } else {
       ensure(m2l_lam, (size_t)nc * sizeof(double));
@@ -545,7 +582,8 @@ struct fmmh_ctx {
       launch_m2l_reduce(p, nc, (const uint4*)plan.p, (const double*)part.p, loc, s);
     } else {
       HCHECK(launch_m2l_rot(p, nc, chunks.p, nchunks, (const uint4*)plan.p, msorted, sbits, c, mom,
-                            soft2, (const double*)rt_tab.p, rot_off, (cplx*)part.p, loc, s));
+                            soft2, (const double*)rt_tab.p, rot_off, rot_part, rot_slice, loc,
+                            s));
       mark(ST_M2L_REDUCE);
     }
     double* lap = nullptr;

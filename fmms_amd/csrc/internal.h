@@ -210,11 +210,13 @@ void launch_m2m_gen(int p, const uint32_t* cells, uint32_t cnt, DevCells c, cplx
 // batches. A fixed length, since a target's sums are grouped by it and a system
 // in an ensemble has to get its standalone sums bit for bit.
 constexpr uint32_t M2L_ROT_CHUNK = 64;
+// part holds `slice` chunk partials (1 at least if there are chunks); the chunks
+// run in slices of that many.
 void rot_tables_host(int p, std::vector<double>& tab, std::vector<uint32_t>& off);
 hipError_t launch_m2l_rot(int p, uint32_t nc, const void* chunks, uint32_t nchunks,
                           const uint4* plan, const uint64_t* skeys, int sbits, DevCells c,
                           const cplx* moments, double soft2, const double* tab,
-                          const std::vector<uint32_t>& off, cplx* part, cplx* locals,
+                          const std::vector<uint32_t>& off, cplx* part, size_t slice, cplx* locals,
                           hipStream_t s);
 void launch_l2l_gen(int p, const uint32_t* cells, uint32_t cnt, DevCells c, cplx* locals,
                     hipStream_t s);

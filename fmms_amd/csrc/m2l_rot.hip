@@ -342,8 +342,10 @@ __host__ __device__ constexpr size_t rot_lds_bytes(int p) {
   return (size_t)NP * ((size_t)rot_wrow(p, p + 1) * 16 + (size_t)(p + 1) * 40);
 }
 
+// Chunks c0, c0 + 1, ... (one per block) into part[0], part[1], ...
 template <int STMAX>
-__global__ void __launch_bounds__(ROT_T) k_m2l_rot(int p, const M2lChunk* __restrict__ chunks,
+__global__ void __launch_bounds__(ROT_T) k_m2l_rot(int p, uint32_t c0,
+                                                  const M2lChunk* __restrict__ chunks,
                                                   const uint64_t* __restrict__ skeys,
                                                   uint64_t smask, DevCells c,
                                                   const cplx* __restrict__ moments, double soft2,
@@ -358,7 +360,7 @@ __global__ void __launch_bounds__(ROT_T) k_m2l_rot(int p, const M2lChunk* __rest
   Cx* eb = ea + (p + 1) * NP;
   double* fa = (double*)(eb + (p + 1) * NP);
   const uint32_t ci = xcd_block(blockIdx.x, gridDim.x);
-  const M2lChunk ck = chunks[ci];
+  const M2lChunk ck = chunks[c0 + ci];
   const double tx = c.cx[ck.target], ty = c.cy[ck.target], tz = c.cz[ck.target];
   const int lane = threadIdx.x & 63, wave = wave_uniform((int)(threadIdx.x >> 6));
   double acc[SL][NT];
@@ -429,26 +431,35 @@ __global__ void __launch_bounds__(ROT_T) k_m2l_rot(int p, const M2lChunk* __rest
 }
 
 // locals[t] = g * sum over the target's chunk partials in chunk order, both
-// signs of m; targets without sources get 0.
-__global__ void __launch_bounds__(256) k_m2l_reduce_rot(int p, uint32_t nc,
+// signs of m; targets without sources get 0. part holds the chunks c0..c1-1: a
+// target whose chunks go on past c1 keeps its sum so far, unscaled, in the
+// m >= 0 entries, and the next slice adds to it, so the slices change no sum.
+__global__ void __launch_bounds__(256) k_m2l_reduce_rot(int p, uint32_t nc, uint32_t c0, uint32_t c1,
                                                        const uint4* __restrict__ plan,
                                                        const cplx* __restrict__ part,
                                                        const double* __restrict__ g,
                                                        cplx* __restrict__ locals) {
   const int NH = hnpos(p);
   const uint32_t t = blockIdx.x;
-  const uint32_t c0 = plan[t].x, c1 = plan[t + 1].x;
+  const uint32_t b = plan[t].x, e1 = plan[t + 1].x;
+  const bool none = b == e1;  // no sources: written once, with the first slice
+  if (none ? c0 > 0u : e1 <= c0 || b >= c1) return;
+  const bool begun = !none && b < c0, done = none || e1 <= c1;
   cplx* out = locals + (size_t)t * hdim(p);
   for (int e = threadIdx.x; e < NH; e += 256) {
     int n = (int)((sqrt(8.0 * e + 1.0) - 1.0) * 0.5);
     while (n * (n + 1) / 2 > e) n--;
     while ((n + 1) * (n + 2) / 2 <= e) n++;
     const int m = e - n * (n + 1) / 2;
-    cplx s = cplx{0.0, 0.0};
-    for (uint32_t k = c0; k < c1; k++) {
-      const cplx v = part[(size_t)k * NH + e];
+    cplx s = begun ? out[hidx(n, m)] : cplx{0.0, 0.0};
+    for (uint32_t k = max(b, c0); k < min(e1, c1); k++) {
+      const cplx v = part[(size_t)(k - c0) * NH + e];
       s.re += v.re;
       s.im += v.im;
+    }
+    if (!done) {
+      out[hidx(n, m)] = s;
+      continue;
     }
     s.re *= g[e];
     s.im *= g[e];
@@ -539,33 +550,40 @@ static RotTables rot_view(int p, const double* tab, const std::vector<uint32_t>&
 }
 
 template <int STMAX>
-static hipError_t rot_t(int p, const M2lChunk* ck, uint32_t nchunks, const uint64_t* skeys,
-                        uint64_t smask, DevCells c, const cplx* moments, double soft2,
+static hipError_t rot_t(int p, const M2lChunk* ck, uint32_t c0, uint32_t nchunks,
+                        const uint64_t* skeys, uint64_t smask, DevCells c, const cplx* moments, double soft2,
                         const RotTables& rt, cplx* part, hipStream_t s) {
   const size_t lds = rot_lds_bytes(p);
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_m2l_rot<STMAX>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((k_m2l_rot<STMAX>), dim3(nchunks), dim3(ROT_T), lds, s, p, ck, skeys, smask,
-                     c, moments, soft2, rt, part);
+  hipLaunchKernelGGL((k_m2l_rot<STMAX>), dim3(nchunks), dim3(ROT_T), lds, s, p, c0, ck, skeys,
+                     smask, c, moments, soft2, rt, part);
   return hipSuccess;
 }
 
 hipError_t launch_m2l_rot(int p, uint32_t nc, const void* chunks, uint32_t nchunks,
                           const uint4* plan, const uint64_t* skeys, int sbits, DevCells c,
                           const cplx* moments, double soft2, const double* tab,
-                          const std::vector<uint32_t>& off, cplx* part, cplx* locals,
+                          const std::vector<uint32_t>& off, cplx* part, size_t slice, cplx* locals,
                           hipStream_t s) {
   const uint64_t smask = (1ull << sbits) - 1ull;
   const RotTables rt = rot_view(p, tab, off);
   const M2lChunk* ck = (const M2lChunk*)chunks;
-  hipError_t e = hipSuccess;
-  if (nchunks)
-    e = p <= 31 ? rot_t<4>(p, ck, nchunks, skeys, smask, c, moments, soft2, rt, part, s)
-                : rot_t<6>(p, ck, nchunks, skeys, smask, c, moments, soft2, rt, part, s);
-  if (e != hipSuccess) return e;
-  if (nc)
-    hipLaunchKernelGGL(k_m2l_reduce_rot, dim3(nc), dim3(256), 0, s, p, nc, plan, part, rt.g, locals);
+  if (nc == 0) return hipSuccess;
+  uint32_t c0 = 0;
+  do {  // once without chunks: every local is 0
+    const uint32_t m = (uint32_t)std::min<size_t>(slice, nchunks - c0);
+    if (m) {
+      const hipError_t e =
+          p <= 31 ? rot_t<4>(p, ck, c0, m, skeys, smask, c, moments, soft2, rt, part, s)
+                  : rot_t<6>(p, ck, c0, m, skeys, smask, c, moments, soft2, rt, part, s);
+      if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(k_m2l_reduce_rot, dim3(nc), dim3(256), 0, s, p, nc, c0, c0 + m, plan, part,
+                       rt.g, locals);
+    c0 += m;
+  } while (c0 < nchunks);
   return hipSuccess;
 }
 

@@ -36,3 +36,22 @@ def test_source_rows(n, p, eps, theta, n_leaf, budget):
     free, tight, frozen = _pair(n, budget, p=p, eps=eps, theta_max=theta, n_leaf=n_leaf)
     assert np.array_equal(free.accel, tight.accel) and np.array_equal(free.pot, tight.pot)
     assert np.array_equal(free.accel, frozen.accel) and np.array_equal(free.pot, frozen.pot)
+
+
+# orders above 10: the chunk partials do not fit at once and run in slices
+@pytest.mark.parametrize("n,p,eps,theta,n_leaf,precision,budget", [
+    (200, 16, math.inf, 0.7, 8, "fp64", 1507892),
+    (1000, 24, math.inf, 0.5, 64, "fp64", 2635976),
+    (5000, 16, math.inf, 0.5, 32, "fp64", 13126196),
+    (5000, 40, math.inf, 0.5, 64, "fp64", 21893620),
+    (30000, 12, 1e-6, 1.0, 16, "fp64", 102337458),
+    (30000, 12, math.inf, 0.5, 64, "fp32bulk", 41461066),
+    (30000, 16, math.inf, 0.5, 32, "fp64", 91418884),
+    (30000, 24, math.inf, 0.5, 64, "fp64", 70305818),
+])
+def test_rotation_partials(n, p, eps, theta, n_leaf, precision, budget):
+    free, tight, frozen = _pair(n, budget, p=p, eps=eps, theta_max=theta, n_leaf=n_leaf,
+                                precision=precision,
+                                softening=1e-3 if precision == "fp32bulk" else 0.0)
+    assert np.array_equal(free.accel, tight.accel) and np.array_equal(free.pot, tight.pot)
+    assert np.array_equal(free.accel, frozen.accel) and np.array_equal(free.pot, frozen.pot)
