@@ -66,7 +66,7 @@ constexpr size_t TREE_FLAGS = 4 + TREE_HIST;
 
 struct fmmh_ctx {
   fmmh_params prm;
-  fmmh_tuning tun = {32, (uint64_t)1 << 18};
+  fmmh_tuning tun = {32, P2P_ITEM_WORK};
   hipStream_t s = nullptr;
   std::string err;
   size_t used = 0;
@@ -512,11 +512,13 @@ struct fmmh_ctx {
     // M2L chunks and P2P items per cell, scanned; the totals in one read
     const uint32_t ch = p <= TEMPLATED_MAX_P ? (uint32_t)tun.m2l_chunk : M2L_ROT_CHUNK;
     const bool f32 = prm.precision == FMMH_PREC_FP32BULK;
+    // items longer than the default are the caller's choice: no cap on their sources
+    const uint32_t cap = f32 || tun.p2p_item_work > P2P_ITEM_WORK ? P2P_NO_CAP : P2P_CAP;
     uint4* pl = ensure<uint4>(plan, ((size_t)nc + 2) * sizeof(uint4));
     ensure(scan_tmp, scan_tmp_words(4 * ((size_t)nc + 1)) * sizeof(uint4));
     HCHECK(hipMemsetAsync(pl + nc + 1, 0, sizeof(uint4), s));
     plan_count(nc, cells(), (const uint32_t*)tptr.p, ch, (const uint32_t*)pptr.p, psorted, sbits,
-               tun.p2p_item_work, f32, pl, s);
+               tun.p2p_item_work, cap, f32, pl, s);
     scan_exclusive_u32x4(pl, (size_t)nc + 1, (uint4*)scan_tmp.p, s);
     struct Totals {
       uint4 v[2];
@@ -534,7 +536,7 @@ struct fmmh_ctx {
     ensure(pl_longs, (size_t)p_nlong * 4);
     ensure(pl_partial, (size_t)std::max<uint32_t>(t.v[0].z, 1) * sizeof(double4));
     plan_emit(nc, cells(), (const uint32_t*)tptr.p, ch, (const uint32_t*)pptr.p, psorted, sbits,
-              tun.p2p_item_work, f32, pl, chunks.p, (uint4*)pl_items.p, (uint4*)pl_reds.p,
+              tun.p2p_item_work, cap, f32, pl, chunks.p, (uint4*)pl_items.p, (uint4*)pl_reds.p,
               p_nlong ? (uint32_t*)(pl + nc + 1) + 1 : nullptr, (uint32_t*)pl_longs.p, s);
     if (p > TEMPLATED_MAX_P) {
       rot_tables();
@@ -1161,7 +1163,7 @@ int fmmh_evaluate_frozen(fmmh_ctx* ctx, size_t n, const double* pos, const doubl
 
 void fmmh_default_tuning(fmmh_tuning* out) {
   out->m2l_chunk = 32;
-  out->p2p_item_work = (uint64_t)1 << 18;
+  out->p2p_item_work = P2P_ITEM_WORK;
 }
 
 int fmmh_set_tuning(fmmh_ctx* ctx, const fmmh_tuning* t) {

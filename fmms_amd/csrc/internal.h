@@ -304,15 +304,19 @@ struct P2PPlan {
 // partial-sum slots, cut leaves} of cell t, scanned by the caller over nc + 1
 // entries (plan[nc] = the totals); plan[nc + 1].x, zeroed before, counts the
 // long items. item_work: a leaf whose targets x sources exceed it
-// is cut into items; fp32: the mixed form's cut. nlong: a zeroed counter, or
-// null (no item is launched first).
+// is cut into items; cap: and one with more sources than this (P2P_NO_CAP: none);
+// fp32: the mixed form's long items. nlong: a zeroed counter, or null (no item is
+// launched first).
+constexpr uint64_t P2P_ITEM_WORK = (uint64_t)1 << 18;  // the default item bound
+constexpr uint32_t P2P_CAP = 4096;                     // the FP64 form's cap (near.hip)
+constexpr uint32_t P2P_NO_CAP = 0xFFFFFFFFu;
 void plan_count(uint32_t nc, DevCells c, const uint32_t* tptr, uint32_t ch, const uint32_t* pptr,
-                const uint64_t* skeys, int sbits, uint64_t item_work, bool fp32, uint4* plan,
-                hipStream_t s);
+                const uint64_t* skeys, int sbits, uint64_t item_work, uint32_t cap, bool fp32,
+                uint4* plan, hipStream_t s);
 void plan_emit(uint32_t nc, DevCells c, const uint32_t* tptr, uint32_t ch, const uint32_t* pptr,
-               const uint64_t* skeys, int sbits, uint64_t item_work, bool fp32, const uint4* plan,
-               void* chunks, uint4* items, uint4* reds, uint32_t* nlong, uint32_t* longs,
-               hipStream_t s);
+               const uint64_t* skeys, int sbits, uint64_t item_work, uint32_t cap, bool fp32,
+               const uint4* plan, void* chunks, uint4* items, uint4* reds, uint32_t* nlong,
+               uint32_t* longs, hipStream_t s);
 void launch_p2p(const P2PPlan& pl, DevCells c, const double4* body, const uint64_t* skeys,
                 int sbits, double soft2, const double4* far, const uint32_t* order,
                 double* accel, double* pot, hipStream_t s);

@@ -443,7 +443,8 @@ __global__ void __launch_bounds__(64) k_p2p_fp64(FMMH_P2P_PARAMS) {
 // neighbourhoods are huge (a large sparse leaf beside a dense region), so a
 // leaf is cut into m work items (at most one per source unit): m = work / W
 // where the work exceeds the context's item bound W (fmmh_tuning.p2p_item_work,
-// default 2^18), and in the FP64 form at least one item per P2P_CAP sources.
+// default 2^18), and in the FP64 form, up to that default, at least one item per
+// P2P_CAP sources; a caller who asks for longer items gets them.
 // Source units are the own leaf (unit 0) and the neighbour ranges in list
 // order; unit u with P_u sources before it goes to item
 // min(m - 1, P_u / ceil(S / m)) (items may come out empty). Split items write
@@ -464,7 +465,6 @@ __global__ void __launch_bounds__(64) k_p2p_fp64(FMMH_P2P_PARAMS) {
 // item's results do not depend on when it runs): 100k bodies 382 -> 267 us,
 // mixed ensemble of 1.5M bodies 4.39 -> 4.13 ms.
 constexpr int PLAN_T = 256;
-constexpr uint32_t P2P_CAP = 4096;
 constexpr uint32_t P2P_LONG64 = 2048, P2P_LONG32 = 8192;
 constexpr uint32_t PLAN_SHORT = 32;  // a list of so few neighbours is never a long one
 
@@ -700,27 +700,27 @@ __global__ void __launch_bounds__(64) k_p2p_reduce(const uint4* __restrict__ red
   }
 }
 
-static CutRule cut_rule(uint64_t item_work, bool fp32) {
-  return fp32 ? CutRule{item_work, 0xFFFFFFFFu, P2P_LONG32} : CutRule{item_work, P2P_CAP, P2P_LONG64};
+static CutRule cut_rule(uint64_t item_work, uint32_t cap, bool fp32) {
+  return CutRule{item_work, cap, fp32 ? P2P_LONG32 : P2P_LONG64};
 }
 
 // plan: nc + 2 entries, zeroed at [nc + 1] by the caller; scanned by the
 // caller between the two.
 void plan_count(uint32_t nc, DevCells c, const uint32_t* tptr, uint32_t ch, const uint32_t* pptr,
-                const uint64_t* skeys, int sbits, uint64_t item_work, bool fp32, uint4* plan,
-                hipStream_t s) {
+                const uint64_t* skeys, int sbits, uint64_t item_work, uint32_t cap, bool fp32,
+                uint4* plan, hipStream_t s) {
   const uint32_t nb = std::min(PLAN_BLOCKS, (nc + 1 + PLAN_T / 64 - 1) / (PLAN_T / 64));
   hipLaunchKernelGGL(k_plan_count, dim3(nb), dim3(PLAN_T), 0, s, nc, c.leaf, tptr, ch, pptr, skeys, (1ull << sbits) - 1ull, c.count,
-                     cut_rule(item_work, fp32), plan);
+                     cut_rule(item_work, cap, fp32), plan);
 }
 
 void plan_emit(uint32_t nc, DevCells c, const uint32_t* tptr, uint32_t ch, const uint32_t* pptr,
-               const uint64_t* skeys, int sbits, uint64_t item_work, bool fp32, const uint4* plan,
-               void* chunks, uint4* items, uint4* reds, uint32_t* nlong, uint32_t* longs,
-               hipStream_t s) {
+               const uint64_t* skeys, int sbits, uint64_t item_work, uint32_t cap, bool fp32,
+               const uint4* plan, void* chunks, uint4* items, uint4* reds, uint32_t* nlong,
+               uint32_t* longs, hipStream_t s) {
   hipLaunchKernelGGL(k_plan_emit, dim3((nc + PLAN_T / 64 - 1) / (PLAN_T / 64)), dim3(PLAN_T), 0, s,
                      nc, c.leaf, tptr, ch, pptr, skeys, (1ull << sbits) - 1ull, c.count,
-                     cut_rule(item_work, fp32), plan, (M2lChunk*)chunks, items, reds, nlong, longs);
+                     cut_rule(item_work, cap, fp32), plan, (M2lChunk*)chunks, items, reds, nlong, longs);
 }
 
 void launch_p2p_f32(const P2PPlan& pl, DevCells c, const double4* body, const uint64_t* skeys,

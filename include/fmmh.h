@@ -118,7 +118,8 @@ typedef struct fmmh_tuning {
                              default 32; p <= 10 (above, chunks are 64 sources) */
   uint64_t p2p_item_work; /* a leaf whose targets x sources exceed this is cut into P2P work
                              items of about equal source count, 64..2^40; default 2^18
-                             (the FP64 form also cuts at 4096 sources an item) */
+                             (up to which the FP64 form also cuts at 4096 sources an
+                             item; a larger bound is taken as it is) */
 } fmmh_tuning;
 void fmmh_default_tuning(fmmh_tuning* out);
 int fmmh_set_tuning(fmmh_ctx* ctx, const fmmh_tuning* t);
@@ -226,8 +227,8 @@ int fmmh_work_counts(const fmmh_ctx* ctx, uint64_t* out8);
 /* P2P work plan of the current lists (no counterpart in the reference, whose
  * threads take leaf pairs from a shared list): [work items, leaves cut into
  * several items]. A leaf whose targets x sources exceed
- * p2p_item_work (in FP64: or whose items would pass 4096 sources) is cut into
- * items of about equal source count, added back in a fixed order. */
+ * p2p_item_work (in FP64 with a bound up to the default: or whose items would
+ * pass 4096 sources) is cut into items of about equal source count, added back in a fixed order. */
 int fmmh_p2p_plan_counts(const fmmh_ctx* ctx, uint64_t* out2);
 
 /* FP64 direct sum at sampled targets, on the device: acc [nt][3], pot [nt]
