@@ -118,6 +118,7 @@ struct fmmh_ctx {
   Buf p2p_work, walkrec;
   Buf walk_code, walk_blk;  // the walk's per-pair decisions, per-block counts
   Buf pl_longs, pl_items, pl_reds, pl_partial;  // P2P work plan
+  double4* p2p_partial = nullptr;               // its partial sums: pl_partial or an idle buffer
   Buf m2l_lam, m2l_m32;                     // mixed form: FP32 M2L scales, scaled moments
   Buf m2l_rows;  // M2L source rows, where no idle buffer holds them
   double* rows = nullptr;
@@ -484,6 +485,17 @@ struct fmmh_ctx {
     }
   }
 
+  // Room for the partial sums of cut leaves in what P2P leaves idle: the M2L's
+  // chunk partials and the key buffers the sorts did not end in (null: none is
+  // large enough). A buffer of their own, at the FP64 form's cap, took systems
+  // that are mostly near field 2 - 4 % over their footprint without the cap.
+  double4* partial_room(size_t slots) const {
+    for (const Buf* b : {&part, &idle_keys(psorted, pkeys, pkeys_alt),
+                         &idle_keys(msorted, mkeys, mkeys_alt)})
+      if (b->cap >= slots * sizeof(double4)) return (double4*)b->p;
+    return nullptr;
+  }
+
   // Directed lists grouped by target, P2P work count, M2L chunks.
   void build_lists() {
     const int p = prm.p;
@@ -513,45 +525,67 @@ struct fmmh_ctx {
     const uint32_t ch = p <= TEMPLATED_MAX_P ? (uint32_t)tun.m2l_chunk : M2L_ROT_CHUNK;
     const bool f32 = prm.precision == FMMH_PREC_FP32BULK;
     // items longer than the default are the caller's choice: no cap on their sources
-    const uint32_t cap = f32 || tun.p2p_item_work > P2P_ITEM_WORK ? P2P_NO_CAP : P2P_CAP;
+    uint32_t cap = f32 || tun.p2p_item_work > P2P_ITEM_WORK ? P2P_NO_CAP : P2P_CAP;
     uint4* pl = ensure<uint4>(plan, ((size_t)nc + 2) * sizeof(uint4));
     ensure(scan_tmp, scan_tmp_words(4 * ((size_t)nc + 1)) * sizeof(uint4));
-    HCHECK(hipMemsetAsync(pl + nc + 1, 0, sizeof(uint4), s));
-    plan_count(nc, cells(), (const uint32_t*)tptr.p, ch, (const uint32_t*)pptr.p, psorted, sbits,
-               tun.p2p_item_work, cap, f32, pl, s);
-    scan_exclusive_u32x4(pl, (size_t)nc + 1, (uint4*)scan_tmp.p, s);
-    struct Totals {
-      uint4 v[2];
+    size_t slots = 0;  // partial sums
+    auto count = [&] {
+      HCHECK(hipMemsetAsync(pl + nc + 1, 0, sizeof(uint4), s));
+      plan_count(nc, cells(), (const uint32_t*)tptr.p, ch, (const uint32_t*)pptr.p, psorted, sbits,
+                 tun.p2p_item_work, cap, f32, pl, s);
+      scan_exclusive_u32x4(pl, (size_t)nc + 1, (uint4*)scan_tmp.p, s);
+      struct Totals {
+        uint4 v[2];
+      };
+      const Totals t = read1((const Totals*)(pl + nc));
+      nchunks = t.v[0].x;
+      p_nitems = t.v[0].y;
+      p_nsplit = t.v[0].w;
+      slots = t.v[0].z;
+      // long items first where they are few: a system whose typical leaf has that
+      // many sources gains nothing from it and would lose the leaf order's reuse
+      p_nlong = (uint64_t)t.v[1].x * 16 <= p_nitems ? t.v[1].x : 0u;
     };
-    const Totals t = read1((const Totals*)(pl + nc));
-    nchunks = t.v[0].x;
-    p_nitems = t.v[0].y;
-    p_nsplit = t.v[0].w;
-    // long items first where they are few: a system whose typical leaf has that
-    // many sources gains nothing from it and would lose the leaf order's reuse
-    p_nlong = (uint64_t)t.v[1].x * 16 <= p_nitems ? t.v[1].x : 0u;
+    count();
     ensure(chunks, std::max<size_t>(nchunks, 1) * m2l_chunk_bytes());
-    ensure(pl_items, (size_t)std::max<uint32_t>(p_nitems, 1) * sizeof(uint4));
-    ensure(pl_reds, (size_t)std::max<uint32_t>(p_nsplit, 1) * sizeof(uint4));
+    if (p > TEMPLATED_MAX_P) {
+      rot_tables();
+    } else {
+      ensure(part, m2l_part_bytes(p, std::max<size_t>(nchunks, 1), mixed32()));
+      if (!mixed32()) {
+        rows = source_rows((size_t)nc * m2l_row_bytes(p));
+      } else {
+        ensure(m2l_lam, (size_t)nc * sizeof(double));
+        ensure(m2l_m32, (size_t)nc * m2l32_moment_bytes(p));
+        ensure(loc32, (size_t)nc * m2l32_moment_bytes(p));
+        rows = source_rows((size_t)nc * m2l32_row_bytes(p));
+      }
+    }
+    // the items last: a budget that has no room for the capped ones gets the plan
+    // without the cap (the same sums, cut elsewhere)
+    auto bytes_items = [&] { return (size_t)std::max<uint32_t>(p_nitems, 1) * sizeof(uint4); };
+    auto bytes_reds = [&] { return (size_t)std::max<uint32_t>(p_nsplit, 1) * sizeof(uint4); };
+    const size_t limit = (size_t)prm.hbm_budget_bytes;
+    if (limit && cap != P2P_NO_CAP) {
+      auto more = [](const Buf& b, size_t bytes) { return bytes > b.cap ? bytes - b.cap : 0; };
+      const size_t need = more(pl_items, bytes_items()) + more(pl_reds, bytes_reds()) +
+                          more(pl_longs, (size_t)p_nlong * 4) +
+                          (partial_room(slots) ? 0 : more(pl_partial, slots * sizeof(double4)));
+      if (used + need > limit) {
+        cap = P2P_NO_CAP;
+        count();
+      }
+    }
+    ensure(pl_items, bytes_items());
+    ensure(pl_reds, bytes_reds());
     ensure(pl_longs, (size_t)p_nlong * 4);
-    ensure(pl_partial, (size_t)std::max<uint32_t>(t.v[0].z, 1) * sizeof(double4));
+    if (!partial_room(slots)) ensure(pl_partial, slots * sizeof(double4));
     plan_emit(nc, cells(), (const uint32_t*)tptr.p, ch, (const uint32_t*)pptr.p, psorted, sbits,
               tun.p2p_item_work, cap, f32, pl, chunks.p, (uint4*)pl_items.p, (uint4*)pl_reds.p,
               p_nlong ? (uint32_t*)(pl + nc + 1) + 1 : nullptr, (uint32_t*)pl_longs.p, s);
-    if (p > TEMPLATED_MAX_P) {
-      rot_tables();
-      rot_room();
-      return;
-    }
-    ensure(part, m2l_part_bytes(p, std::max<size_t>(nchunks, 1), mixed32()));
-    if (!mixed32()) {
-      rows = source_rows((size_t)nc * m2l_row_bytes(p));
-    } else {
-      ensure(m2l_lam, (size_t)nc * sizeof(double));
-      ensure(m2l_m32, (size_t)nc * m2l32_moment_bytes(p));
-      ensure(loc32, (size_t)nc * m2l32_moment_bytes(p));
-      rows = source_rows((size_t)nc * m2l32_row_bytes(p));
-    }
+    if (p > TEMPLATED_MAX_P) rot_room();
+    p2p_partial = partial_room(slots);
+    if (!p2p_partial) p2p_partial = (double4*)pl_partial.p;
   }
 
   // The mixed form's FP32 M2L, L2L and L2P (templated orders only).
@@ -615,7 +649,7 @@ struct fmmh_ctx {
     else
       launch_l2p_gen(p, (uint32_t*)leaf_ids.p, nleaves, c, b, loc, lap, (double4*)bpack.p, s);
     const P2PPlan pl{(const uint4*)pl_items.p, p_nitems, p_nlong, (const uint32_t*)pl_longs.p,
-                     (const uint4*)pl_reds.p, p_nsplit, (double4*)pl_partial.p};
+                     (const uint4*)pl_reds.p, p_nsplit, p2p_partial};
     const bool f32 = prm.precision == FMMH_PREC_FP32BULK;
     mark(ST_P2P);
     if (f32)

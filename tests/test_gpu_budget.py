@@ -55,3 +55,25 @@ def test_rotation_partials(n, p, eps, theta, n_leaf, precision, budget):
                                 softening=1e-3 if precision == "fp32bulk" else 0.0)
     assert np.array_equal(free.accel, tight.accel) and np.array_equal(free.pot, tight.pot)
     assert np.array_equal(free.accel, frozen.accel) and np.array_equal(free.pot, frozen.pot)
+
+
+# mostly near field: leaves cut at the FP64 form's cap on an item's sources; with
+# a budget that only holds the plan without the cap the sums are cut elsewhere
+@pytest.mark.parametrize("n,p,theta,n_leaf,budget,same", [
+    (20000, 1, 0.05, 32, 131047136, True),
+    (40000, 2, 0.02, 64, 149665794, True),
+    (40000, 3, 0.1, 96, 76462492, True),
+    (50000, 12, 0.2, 64, 231556320, True),
+    (12000, 2, 0.02, 128, 7459156, True),
+    (40000, 2, 0.02, 192, 42340338, False),
+])
+def test_cut_leaves(n, p, theta, n_leaf, budget, same):
+    free, tight, frozen = _pair(n, budget, p=p, eps=math.inf, theta_max=theta, n_leaf=n_leaf,
+                                softening=1e-2 if n == 12000 else 0.0)
+    assert np.array_equal(tight.accel, frozen.accel) and np.array_equal(tight.pot, frozen.pot)
+    if same:
+        assert np.array_equal(free.accel, tight.accel) and np.array_equal(free.pot, tight.pot)
+    else:  # the same sums in another order
+        an = np.linalg.norm(free.accel, axis=1)
+        assert np.all(np.linalg.norm(tight.accel - free.accel, axis=1) <= 1e-13 * an + 1e-15 * an.max())
+        assert np.allclose(tight.pot, free.pot, rtol=1e-13, atol=0)
