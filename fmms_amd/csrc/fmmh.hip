@@ -101,7 +101,7 @@ struct fmmh_ctx {
   // the bodies' far field (double4 by slot), from L2P to the final sums
   Buf bpack;
   Buf bbox_partial, bbox, flags;
-  Buf cstart;  // per slot: scan of the cells starting there
+  Buf cstart;  // per slot: scan of the cells starting there; then fmin's block minima
   Buf c_first, c_count, c_children, c_parent, c_leaf, c_level, c_cx, c_cy, c_cz, c_mass, c_rho,
       c_rope, c_last;
   Buf lvl_cells;  // cells by level, a level's internal cells first
@@ -256,7 +256,7 @@ struct fmmh_ctx {
     ensure(bbox_partial, bbox_partial_bytes(n, nsys));
     ensure(bbox, nsys * sizeof(BBox));
     ensure(flags, TREE_FLAGS * 4);
-    ensure(cstart, std::max<size_t>(n, 4) * 8);
+    ensure(cstart, std::max(n, fmin_blocks_words(n)) * 8);
     ensure(sort_tmp, radix_tmp_words(n) * 4 + 64);
     ensure_scan(n);
     mark(ST_TREE);
@@ -439,7 +439,7 @@ struct fmmh_ctx {
     ensure(fprec, (size_t)nc * fp_rec_bytes());
     launch_pack_fp(nc, c, fprec.p, s);
     launch_fprepass((uint32_t)n, nc, fprec.p, b.xyzm, keys_sorted, vlev, (double*)fvals.p, s);
-    // the tree's scan (n words at least, and 4) is done with
+    // the tree's scan is done with
     launch_fmin((uint32_t)n, nc, c, (const double*)fvals.p, (double*)cstart.p, (double*)fmin.p, s);
   }
 
