@@ -395,7 +395,7 @@ struct fmmh_ctx {
     } else {
       launch_p2m_gen(p, (uint32_t*)leaf_ids.p, nleaves, c, b, mom, s);
       for (int L = (int)max_level - 1; L >= 0; L--)
-        launch_m2m_gen(p, int_cells(L), n_int[L], c, mom, s);
+        HCHECK(launch_m2m_gen(p, int_cells(L), n_int[L], c, mom, s));
     }
     if (prm.softening > 0.0) {  // trace moments of the softened far field
       double* q = (double*)ctrace.p;
@@ -741,13 +741,23 @@ struct fmmh_ctx {
                            const fmmh_leapfrog_opts& o, double* part, double* st) {
     drop_graph();
     const uint32_t age = tree_evals;  // capture records the step, it does not run it
-    capturing = true;
-    HCHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    frozen_step(pos, vel, mass, acc, pot, o, part, st);
     hipGraph_t g = nullptr;
-    const hipError_t e = hipStreamEndCapture(s, &g);
-    capturing = false;
-    tree_evals = age;
+    hipError_t e = hipSuccess;
+    HCHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+    capturing = true;
+    auto end = [&] {
+      e = hipStreamEndCapture(s, &g);
+      capturing = false;
+      tree_evals = age;
+    };
+    try {
+      frozen_step(pos, vel, mass, acc, pot, o, part, st);
+    } catch (...) {  // a step that fails leaves the stream out of capture
+      end();
+      if (g) (void)hipGraphDestroy(g);
+      throw;
+    }
+    end();
     if (e != hipSuccess) {
       if (g) (void)hipGraphDestroy(g);
       throw HipError{std::string("hipStreamEndCapture: ") + hipGetErrorString(e)};

@@ -170,19 +170,21 @@ void launch_p2m_gen(int p, const uint32_t* leaf_ids, uint32_t nleaves, DevCells 
                      leaf_ids, nleaves, c, b, moments);
 }
 
-void launch_m2m_gen(int p, const uint32_t* cells, uint32_t cnt, DevCells c, cplx* moments,
-                    hipStream_t s) {
-  if (cnt == 0) return;
+hipError_t launch_m2m_gen(int p, const uint32_t* cells, uint32_t cnt, DevCells c, cplx* moments,
+                          hipStream_t s) {
+  if (cnt == 0) return hipSuccess;
   // children per pass: as many as leave tables and moments within 150 KB (4 up to p = 31)
   const size_t D = (size_t)hdim(p);
   int nch = 8;
   while (nch > 1 && (2 * (size_t)nch * D + M2MG_T) * sizeof(cplx) > 150 * 1024) nch /= 2;
   const size_t lds = (2 * (size_t)nch * D + M2MG_T) * sizeof(cplx);
   const int per = M2MG_T / nch;
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_m2m_gen),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_m2m_gen),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (err != hipSuccess) return err;
   hipLaunchKernelGGL(k_m2m_gen, dim3(cnt, (D + per - 1) / per), dim3(M2MG_T), lds, s, p, nch, cells,
                      c, moments);
+  return hipSuccess;
 }
 
 }  // namespace fmmh

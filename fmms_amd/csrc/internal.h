@@ -203,8 +203,8 @@ constexpr int FP64_TOP = 3;
 constexpr int TEMPLATED_MAX_P = 10;  // above this the runtime-p kernels run
 void launch_p2m_gen(int p, const uint32_t* leaf_ids, uint32_t nleaves, DevCells c, DevBodies b,
                     cplx* moments, hipStream_t s);
-void launch_m2m_gen(int p, const uint32_t* cells, uint32_t cnt, DevCells c, cplx* moments,
-                    hipStream_t s);
+hipError_t launch_m2m_gen(int p, const uint32_t* cells, uint32_t cnt, DevCells c, cplx* moments,
+                          hipStream_t s);
 // m2l_rot.hip: the swap matrices and scale factors of order p (host), and the
 // M2L (chunk partials in part, then the locals). Sources per chunk: four
 // batches. A fixed length, since a target's sums are grouped by it and a system
