@@ -459,7 +459,7 @@ struct fmmh_ctx {
   }
 
   // Room for the chunk partials of the orders above 10, all of them at once up to
-  // ROT_PART_MAX (5.2 KB a chunk at p = 24, 13.8 at p = 40: a buffer for any number
+  // ROT_PART_MAX or an eighth of the context's other memory (5.2 KB a chunk at p = 24, 13.8 at p = 40: a buffer for any number
   // of them doubled a context): an idle key buffer if they fit there, or a buffer
   // of their own, or, where the context's budget has no room for that, what is
   // idle, and the chunks run in more slices. Each slice has a tail of its own:
@@ -467,7 +467,8 @@ struct fmmh_ctx {
   static constexpr size_t ROT_PART_MAX = (size_t)64 << 20;
   void rot_room() {
     const size_t one = m2l_part_bytes(prm.p, 1, false);
-    const size_t want = std::min<size_t>(nchunks, std::max<size_t>(1, ROT_PART_MAX / one));
+    const size_t most = std::max(ROT_PART_MAX, (used - part.cap) / 8);
+    const size_t want = std::min<size_t>(nchunks, std::max<size_t>(1, most / one));
     const Buf& km = idle_keys(msorted, mkeys, mkeys_alt);
     const Buf& kp = idle_keys(psorted, pkeys, pkeys_alt);
     const Buf& idle = km.cap >= kp.cap ? km : kp;
