@@ -198,11 +198,8 @@ bool launch_m2l_kernel(int p, uint32_t nc, const void* chunks, uint32_t nchunks,
   return true;
 }
 
-// Bytes of one cell's source row (M2lRow<p>), p <= 10.
-size_t m2l_row_bytes(int p) {
-  const int nm = hdim(p), ndir = p <= 7 ? 1 : p == 8 ? 9 : nm;
-  return (size_t)((nm - ndir + 7) / 8 * 8 + (3 + ndir + 7) / 8 * 8) * sizeof(double);
-}
+// Bytes of one cell's source row, p <= 10.
+size_t m2l_row_bytes(int p) { return (size_t)m2l_row_words(p) * sizeof(double); }
 
 void launch_m2l_scale(uint32_t nc, DevCells c, const BBox* bb, const uint64_t* keys_sorted,
                       int vlev, double* lam, hipStream_t s) {
@@ -229,12 +226,8 @@ bool launch_m2l32(int p, uint32_t nc, const void* chunks, uint32_t nchunks, cons
   return true;
 }
 
-// Bytes of one cell's source row of the mixed form (M2lRow32<p>); 0: none.
-size_t m2l32_row_bytes(int p) {
-  if (p < 3 || p > 8) return 0;
-  const int nf = hnpos(p), seg = (nf - 2) / 8;
-  return (size_t)((seg * 8 + 4 + nf - 8 * seg + 7) / 8 * 8) * sizeof(double);
-}
+// Bytes of one cell's source row of the mixed form; 0: none.
+size_t m2l32_row_bytes(int p) { return (size_t)m2l32_row_words(p) * sizeof(double); }
 
 size_t m2l32_moment_bytes(int p) { return (size_t)hnpos(p) * sizeof(cplxf); }
 

@@ -276,10 +276,11 @@ template <int P>
 struct M2lRow {
   static constexpr int NM = (P + 1) * (P + 1);
   static constexpr bool STAGED = P <= 8;
-  static constexpr int NDIR = P <= 7 ? 1 : P == 8 ? 9 : NM;
-  static constexpr int SEG = (NM - NDIR + 7) / 8;
-  static constexpr int DIR = (3 + NDIR + 7) / 8 * 8;  // centre + direct part
-  static constexpr int WORDS = SEG * 8 + DIR;          // staged part first, 64-byte rows
+  static constexpr int NDIR = m2l_row_direct(P);
+  static constexpr int SEG = m2l_row_segs(P);
+  static constexpr int DIR = m2l_row_tail(P);      // centre + direct part
+  static constexpr int WORDS = m2l_row_words(P);  // staged part first, 64-byte rows
+  static_assert(STAGED == (SEG > 0), "the direct part is the whole multipole or is followed by segments");
 };
 
 template <int P>
@@ -542,10 +543,10 @@ __device__ __forceinline__ void m2l_chunk32(const M2lChunk ck, uint32_t ci,
 template <int P>
 struct M2lRow32 {
   static constexpr int NF = hnpos(P);
-  static constexpr bool STAGED = P >= 3 && P <= 8;
-  static constexpr int SEG = (NF - 2) / 8;
-  static constexpr int NDIR = NF - 8 * SEG;
-  static constexpr int WORDS = (SEG * 8 + 4 + NDIR + 7) / 8 * 8;  // of 8 bytes
+  static constexpr bool STAGED = m2l32_staged(P);
+  static constexpr int SEG = m2l32_row_segs(P);
+  static constexpr int NDIR = m2l32_row_direct(P);
+  static constexpr int WORDS = m2l32_row_words(P);  // of 8 bytes
 };
 
 template <int P>
