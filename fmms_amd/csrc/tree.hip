@@ -383,7 +383,9 @@ __global__ void __launch_bounds__(TB) k_cell_emit(const uint64_t* __restrict__ k
     c.leaf[id] = q == m - 1 ? 1 : 0;
     if (q > 0) c.parent[id] = (int32_t)(id - 1);
     const int32_t next = q == m - 1 ? -1 : (int32_t)(id + 1);
-    const int oct = (int)((k >> (3 * (BITS - (top + q + 1)))) & 7u);  // unused in a leaf
+    // the octant of the next cell of the chain (a leaf has none, and at level 21
+    // the key has no digit left to shift to)
+    const int oct = next < 0 ? -1 : (int)((k >> (3 * (BITS - (top + q + 1)))) & 7u);
     int32_t* ch = c.children + (size_t)id * 8;
 #pragma unroll
     for (int o = 0; o < 8; o++) ch[o] = o == oct ? next : -1;
