@@ -73,8 +73,8 @@ __global__ void __launch_bounds__(64) k_p2m32_leaf(const uint32_t* __restrict__ 
 // equal trip counts). Column m: Y_m^m by the diagonal chain, then
 // Y_n^m = ((2n-1) z Y_{n-1}^m - r^2 Y_{n-2}^m) / (n^2 - m^2) (harmonic.rs:141-173).
 // The column is a template argument of the wave's code, so that the reciprocals
-// are constants and the chain is unrolled, and the following body is loaded
-// ahead (63k cells, p = 8: 197 -> 153 us; 42k cells 115 -> 87).
+// are constants and the chain is unrolled (63k cells, p = 8: 197 -> 153 us; 42k
+// cells 115 -> 87).
 template <int P, int M>
 __device__ __forceinline__ void p2m32_column(uint32_t id, uint32_t f, uint32_t e, double zx,
                                              double zy, double zz, double il,
@@ -84,7 +84,6 @@ __device__ __forceinline__ void p2m32_column(uint32_t id, uint32_t f, uint32_t e
   cplxf acc[P + 1];
 #pragma unroll
   for (int n = 0; n <= P; n++) acc[n] = cplxf{0.0f, 0.0f};
-  double4 next = xyzm[f];
   for (uint32_t k = f; k < e; k++) {
     const double4 q = xyzm[k];
     const float x = (float)((q.x - zx) * il), y = (float)((q.y - zy) * il),
