@@ -283,16 +283,22 @@ struct M2lRow {
   static_assert(STAGED == (SEG > 0), "the direct part is the whole multipole or is followed by segments");
 };
 
+// Blocks of the row kernels for `words` words in all, one a thread up to 2^30:
+// a launch holds fewer than 2^32 threads, and 34M cells at p = 10 have as many
+// words, so past that the threads take several.
+inline dim3 m2l_row_blocks(size_t words) {
+  const size_t most = (size_t)1 << 22, b = (words + 255) / 256;
+  return dim3((unsigned)(b < most ? b : most));
+}
+
 template <int P>
-__global__ void __launch_bounds__(256) k_m2l_rows(uint32_t nc, const cplx* __restrict__ moments,
-                                                 const double* __restrict__ ccx,
-                                                 const double* __restrict__ ccy,
-                                                 const double* __restrict__ ccz,
-                                                 double* __restrict__ rows) {
+__device__ __forceinline__ void m2l_row_word(size_t g, const cplx* __restrict__ moments,
+                                             const double* __restrict__ ccx,
+                                             const double* __restrict__ ccy,
+                                             const double* __restrict__ ccz,
+                                             double* __restrict__ rows) {
   using R = M2lRow<P>;
-  const size_t g = (size_t)blockIdx.x * 256 + threadIdx.x;
   const uint32_t c = (uint32_t)(g / R::WORDS);
-  if (c >= nc) return;
   const int i = (int)(g - (size_t)c * R::WORDS);
   // position i -> multipole entry e (-1: none) or centre coordinate
   const int d = i - R::SEG * 8;
@@ -308,6 +314,17 @@ __global__ void __launch_bounds__(256) k_m2l_rows(uint32_t nc, const cplx* __res
     v = d == 0 ? ccx[c] : d == 1 ? ccy[c] : ccz[c];
   }
   rows[g] = v;
+}
+
+template <int P>
+__global__ void __launch_bounds__(256) k_m2l_rows(uint32_t nc, const cplx* __restrict__ moments,
+                                                 const double* __restrict__ ccx,
+                                                 const double* __restrict__ ccy,
+                                                 const double* __restrict__ ccz,
+                                                 double* __restrict__ rows) {
+  const size_t words = (size_t)nc * M2lRow<P>::WORDS;
+  for (size_t g = (size_t)blockIdx.x * 256 + threadIdx.x; g < words; g += (size_t)gridDim.x * 256)
+    m2l_row_word<P>(g, moments, ccx, ccy, ccz, rows);
 }
 
 // SPLIT: two blocks per 64 chunks, the even-n and the odd-n half of F (the
@@ -463,9 +480,8 @@ void m2l_t(const M2lChunk* chunks, uint32_t nchunks, const uint64_t* skeys, uint
            hipStream_t s) {
   if (!nchunks) return;
   constexpr bool split = P >= FMMH_M2L_SPLIT_FROM;
-  const size_t rt = (size_t)nc * M2lRow<P>::WORDS;
-  hipLaunchKernelGGL(k_m2l_rows<P>, dim3((rt + 255) / 256), dim3(256), 0, s, nc, moments, c.cx,
-                     c.cy, c.cz, rows);
+  hipLaunchKernelGGL(k_m2l_rows<P>, m2l_row_blocks((size_t)nc * M2lRow<P>::WORDS), dim3(256), 0, s,
+                     nc, moments, c.cx, c.cy, c.cz, rows);
   const uint32_t nb = (nchunks + 63) / 64 * (split ? 2 : 1);
   hipLaunchKernelGGL((k_m2l<P, split>), dim3(nb), dim3(64), 0, s, chunks, nchunks, skeys, smask,
                      (const double*)rows, soft2, part);
@@ -550,16 +566,14 @@ struct M2lRow32 {
 };
 
 template <int P>
-__global__ void __launch_bounds__(256) k_m2l_rows32(uint32_t nc, const cplxf* __restrict__ m32,
-                                                   const double* __restrict__ ccx,
-                                                   const double* __restrict__ ccy,
-                                                   const double* __restrict__ ccz,
-                                                   const double* __restrict__ lam,
-                                                   double* __restrict__ rows) {
+__device__ __forceinline__ void m2l_row_word32(size_t g, const cplxf* __restrict__ m32,
+                                               const double* __restrict__ ccx,
+                                               const double* __restrict__ ccy,
+                                               const double* __restrict__ ccz,
+                                               const double* __restrict__ lam,
+                                               double* __restrict__ rows) {
   using R = M2lRow32<P>;
-  const size_t g = (size_t)blockIdx.x * 256 + threadIdx.x;
   const uint32_t c = (uint32_t)(g / R::WORDS);
-  if (c >= nc) return;
   const int i = (int)(g - (size_t)c * R::WORDS), d = i - R::SEG * 8;
   const int e = d < 0 ? i + R::NDIR : d >= 4 && d - 4 < R::NDIR ? d - 4 : -1;
   double v = 0.0;
@@ -568,6 +582,18 @@ __global__ void __launch_bounds__(256) k_m2l_rows32(uint32_t nc, const cplxf* __
   else if (d < 4)
     v = d == 0 ? ccx[c] : d == 1 ? ccy[c] : d == 2 ? ccz[c] : lam[c];
   rows[g] = v;
+}
+
+template <int P>
+__global__ void __launch_bounds__(256) k_m2l_rows32(uint32_t nc, const cplxf* __restrict__ m32,
+                                                   const double* __restrict__ ccx,
+                                                   const double* __restrict__ ccy,
+                                                   const double* __restrict__ ccz,
+                                                   const double* __restrict__ lam,
+                                                   double* __restrict__ rows) {
+  const size_t words = (size_t)nc * M2lRow32<P>::WORDS;
+  for (size_t g = (size_t)blockIdx.x * 256 + threadIdx.x; g < words; g += (size_t)gridDim.x * 256)
+    m2l_row_word32<P>(g, m32, ccx, ccy, ccz, lam, rows);
 }
 
 // The chunks of 64 lanes, rows staged as in m2l_chunks64 (same layout in LDS).
@@ -720,9 +746,8 @@ void m2l32_t(const M2lChunk* chunks, uint32_t nchunks, const uint64_t* skeys, ui
              double* rows, cplxf* part, hipStream_t s) {
   if (!nchunks) return;
   if constexpr (M2lRow32<P>::STAGED) {
-    const size_t rt = (size_t)nc * M2lRow32<P>::WORDS;
-    hipLaunchKernelGGL(k_m2l_rows32<P>, dim3((rt + 255) / 256), dim3(256), 0, s, nc, m32, c.cx,
-                       c.cy, c.cz, lam, rows);
+    hipLaunchKernelGGL(k_m2l_rows32<P>, m2l_row_blocks((size_t)nc * M2lRow32<P>::WORDS), dim3(256),
+                       0, s, nc, m32, c.cx, c.cy, c.cz, lam, rows);
     hipLaunchKernelGGL(k_m2l32_staged<P>, dim3((nchunks + 63) / 64), dim3(64), 0, s, chunks,
                        nchunks, skeys, smask, (const double*)rows, soft2, part);
   } else {

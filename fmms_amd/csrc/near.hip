@@ -553,18 +553,15 @@ __global__ void __launch_bounds__(PLAN_T) k_plan_count(
   }
 }
 
-// plan: the scanned counts. Writes the chunks, the items, the records of cut
-// leaves and, unless nlong is null, the indices of the long items (their slots
-// counted in *nlong).
-__global__ void __launch_bounds__(PLAN_T) k_plan_emit(
-    uint32_t nc, const uint8_t* __restrict__ leaf, const uint32_t* __restrict__ tptr, uint32_t ch,
-    const uint32_t* __restrict__ pptr, const uint64_t* __restrict__ skeys, uint64_t smask,
-    const uint32_t* __restrict__ ccount, CutRule cut, const uint4* __restrict__ plan,
-    M2lChunk* __restrict__ chunks, uint4* __restrict__ items, uint4* __restrict__ reds,
-    uint32_t* __restrict__ nlong, uint32_t* __restrict__ longs) {
-  const uint32_t t = blockIdx.x * (PLAN_T / 64) + (threadIdx.x >> 6);
-  const uint32_t lane = threadIdx.x & 63;
-  if (t >= nc) return;
+// Cell t by one wave; plan: the scanned counts. Writes the chunks, the items, the
+// records of cut leaves and, unless nlong is null, the indices of the long items
+// (their slots counted in *nlong).
+__device__ __forceinline__ void plan_emit_cell(
+    uint32_t t, uint32_t lane, const uint8_t* __restrict__ leaf, const uint32_t* __restrict__ tptr,
+    uint32_t ch, const uint32_t* __restrict__ pptr, const uint64_t* __restrict__ skeys,
+    uint64_t smask, const uint32_t* __restrict__ ccount, CutRule cut,
+    const uint4* __restrict__ plan, M2lChunk* __restrict__ chunks, uint4* __restrict__ items,
+    uint4* __restrict__ reds, uint32_t* __restrict__ nlong, uint32_t* __restrict__ longs) {
   const uint4 at = plan[t];
   {
     const uint32_t b = tptr[t], e = tptr[t + 1];
@@ -660,6 +657,19 @@ __global__ void __launch_bounds__(PLAN_T) k_plan_emit(
   }
 }
 
+__global__ void __launch_bounds__(PLAN_T) k_plan_emit(
+    uint32_t nc, const uint8_t* __restrict__ leaf, const uint32_t* __restrict__ tptr, uint32_t ch,
+    const uint32_t* __restrict__ pptr, const uint64_t* __restrict__ skeys, uint64_t smask,
+    const uint32_t* __restrict__ ccount, CutRule cut, const uint4* __restrict__ plan,
+    M2lChunk* __restrict__ chunks, uint4* __restrict__ items, uint4* __restrict__ reds,
+    uint32_t* __restrict__ nlong, uint32_t* __restrict__ longs) {
+  const uint32_t lane = threadIdx.x & 63;
+  for (uint32_t t = blockIdx.x * (PLAN_T / 64) + (threadIdx.x >> 6); t < nc;
+       t += gridDim.x * (PLAN_T / 64))
+    plan_emit_cell(t, lane, leaf, tptr, ch, pptr, skeys, smask, ccount, cut, plan, chunks, items, reds,
+                   nlong, longs);
+}
+
 // Split leaves: far field + the items' partial sums in item order, scattered
 // to particle-id order.
 // COMP (the mixed form): the item sums and the far field are added with
@@ -718,7 +728,10 @@ void plan_emit(uint32_t nc, DevCells c, const uint32_t* tptr, uint32_t ch, const
                const uint64_t* skeys, int sbits, uint64_t item_work, uint32_t cap, bool fp32,
                const uint4* plan, void* chunks, uint4* items, uint4* reds, uint32_t* nlong,
                uint32_t* longs, hipStream_t s) {
-  hipLaunchKernelGGL(k_plan_emit, dim3((nc + PLAN_T / 64 - 1) / (PLAN_T / 64)), dim3(PLAN_T), 0, s,
+  // a launch holds fewer than 2^32 threads: past 2^23 blocks (34M cells) a wave
+  // takes several cells
+  const uint32_t nb = std::min(1u << 23, (nc + PLAN_T / 64 - 1) / (PLAN_T / 64));
+  hipLaunchKernelGGL(k_plan_emit, dim3(nb), dim3(PLAN_T), 0, s,
                      nc, c.leaf, tptr, ch, pptr, skeys, (1ull << sbits) - 1ull, c.count,
                      cut_rule(item_work, cap, fp32), plan, (M2lChunk*)chunks, items, reds, nlong, longs);
 }
