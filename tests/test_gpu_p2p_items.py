@@ -1,11 +1,13 @@
 """The P2P work plan against its rule, recomputed from the lists: how many items
 the leaves are cut into, with the FP64 form's cap on an item's sources (default
 item bound) and without it (a larger bound is the caller's choice, the mixed form
-has none)."""
+has none); and systems in which a few items are long, which are launched first."""
 import math
 
 import numpy as np
 import pytest
+
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +59,34 @@ def test_item_counts(precision, work):
         an = np.linalg.norm(a.accel, axis=1)
         assert np.all(np.linalg.norm(r.accel - a.accel, axis=1) <= 1e-13 * an + 1e-15 * an.max())
         assert np.allclose(r.pot, a.pot, rtol=1e-13, atol=0)
+
+
+# sources above which an item is long, and neighbours up to which none is
+LONG = {"fp64": 2048, "fp32bulk": 8192}
+SHORT_LIST = 32
+
+
+@pytest.mark.parametrize("n,n_leaf,theta", [(20000, 16, 0.5), (20000, 8, 0.8), (30000, 16, 0.7)])
+def test_long_items_first(n, n_leaf, theta):
+    import fmms_amd as fa
+
+    pos, mass = O.plummer(n, seed=5)
+    mass = mass * np.linspace(0.5, 1.5, n)
+    kw = dict(p=2, eps=math.inf, n_leaf=n_leaf, theta_max=theta, softening=1e-2)
+    out = {}
+    for precision in ("fp64", "fp32bulk"):
+        g = fa.Fmm(None, None, precision=precision, **kw)
+        out[precision] = g.accel(pos, mass)
+        nt, s, units = leaf_sources(g)
+        m = leaf_items(nt, s, units, 1 << 18, CAP if precision == "fp64" else 0)
+        nlong = m[(units - 1 > SHORT_LIST) & (s // m > LONG[precision])].sum()
+        assert g.work_counts()["p2p_items"] == m.sum()
+        assert 0 < nlong and 16 * nlong <= m.sum()  # few: launched first
+    orc = O.OracleFmm(pos, mass, **kw)
+    a_ref, pot_ref = orc.run(pos, mass)
+    an = np.linalg.norm(a_ref, axis=1)
+    # the same sums in another order: the suite's FP64 bars, and the mixed form's
+    r, m = out["fp64"], out["fp32bulk"]
+    assert np.all(np.linalg.norm(r.accel - a_ref, axis=1) <= 1e-11 * an + 1e-13 * an.max())
+    assert np.allclose(r.pot, pot_ref, rtol=1e-11, atol=0)
+    assert np.all(np.linalg.norm(m.accel - r.accel, axis=1) <= 2e-5 * an + 2e-6 * an.max())
