@@ -25,8 +25,9 @@ static_assert(5 * (size_t)FMMH_DIRECT_NOALLOC_MAX_TARGETS <= DIRECT_SCRATCH_WORD
 // NT targets per block, in scalar registers: a thread reads a source once and
 // evaluates it against all of them. One target per block read 32 bytes from
 // the cache for every pair and divided by a square root: 4096 targets x 1M
-// sources 8.4 ms, now 3.4 (19 FP64 instructions and a rsqrt a pair are 3.3 ms at
-// the FP64 issue rate).
+// sources 8.4 ms, now 3.4 - 3.5 one launch after another (19 FP64 instructions and
+// a rsqrt a pair are 3.3 ms at the FP64 issue rate) and 4.1 for a launch by itself,
+// which the clock is still rising under.
 template <int NT>
 __global__ void __launch_bounds__(DT) k_direct_part(const double* __restrict__ pos,
                                                    const double* __restrict__ mass, size_t n,
@@ -144,8 +145,10 @@ __global__ void __launch_bounds__(DT) k_direct_reduce(const double* __restrict__
 // two blocks a CU; below, single targets have more blocks (groups against
 // singles in us: 10k bodies x 1000 targets, 250 blocks, 29 / 27; 100k x 100, 300
 // blocks, 35 / 33; 100k x 200, 600 blocks, 45 / 51; 1M x 32, 976 blocks,
-// 99 / 147; 100k x 400, 1200 blocks, 64 / 86). Eight a group: 1M x 100 202
-// instead of 177, 1M x 1000 987 instead of 912, 1M x 4096 3162 instead of 3404.
+// 99 / 147; 100k x 400, 1200 blocks, 64 / 86). Eight a group are slower up to
+// about a thousand targets (1M x 100 202 instead of 177, 1M x 1000 987 instead of
+// 912) and faster past that (1M x 4096 3162 instead of 3404): not taken, 0.2 ms of
+// a call of 5.4 there.
 static bool direct_groups(size_t n, size_t nt) {
   return (nt + DN - 1) / DN * std::min<size_t>(256, std::max<size_t>(1, n / 8192)) >= 512;
 }

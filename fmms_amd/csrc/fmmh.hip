@@ -4,8 +4,9 @@
 // build runs the Morton tree on the device (tree.hip); an evaluation runs
 // the upward pass, the optional f pre-pass, the dual walk, the target-grouped
 // M2L / L2L / L2P and the fused P2P + scatter. Sizes that decide launch
-// shapes (cells per level, walk frontier, list lengths) are read back once
-// per level / round; everything else stays on the device.
+// shapes are read back: the cells per level once a build, the walk's state once
+// a batch of rounds, the work plan's totals once; everything else stays on the
+// device.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -836,9 +837,9 @@ struct fmmh_ctx {
   }
 
   // The dual walk, breadth-first (walk.hip): per round the decisions and
-  // their per-block counts, then the outputs in frontier order; one readback
-  // per round gives the next frontier's size. An output buffer that ran out
-  // of room grows and the round's outputs are written again.
+  // their per-block counts, then the outputs in frontier order; the state that
+  // ends a batch of rounds is read back. An output buffer that ran out of room
+  // grows and the round's outputs are written again.
   void walk(bool use_err) {
     const size_t cap0 = (size_t)4 * nc + 1024;
     if (front_a.cap < cap0 * 8) {

@@ -26,10 +26,15 @@
 // What bounds it at p = 24: vector instructions (about 41k per wave and batch
 // of 16 pairs against 850 matrix instructions) and their latency at two waves
 // a SIMD. Measured, 670k directed pairs at p = 24 (30k bodies, evaluation
-// 145.4 -> 14.1 ms): the kernel before this one (one pair at a time per block,
-// full-length matrices read from L2 for every pair) took 136.7 ms, this one
-// 6.4 ms. W kept for every (k, m), half of it unread, held one block a CU: 7.6 ms.
-// It replaces the per-pair naive convolution of 11 <= p < 20 too.
+// 145.4 -> 14.1 ms with this kernel alone, 9.4 with M2M and the others of later):
+// the kernel before this one (one pair at a time per block, full-length matrices
+// read from L2 for every pair) took 136.7 ms, this one 6.4 ms. W kept for every
+// (k, m), half of it unread, held one block a CU: 7.6 ms.
+// It replaces the per-pair naive convolution of 11 <= p < 20 too, and rounds no
+// worse: against the 80-bit sum of the same moments and lists the far forces are
+// off by 1e-16 in the median at p = 11 .. 19 (3e-16 by convolution), by 2.5e-15 at
+// most in the 99th percentile on a clumped system (2.9e-15), and every degree's
+// locals, in the norm of their power, by 2.2e-15 (2.0e-15).
 #include <algorithm>
 #include <cmath>
 #include <type_traits>

@@ -1,5 +1,6 @@
 // prims.hip — HBM-bound primitives for gfx950: device-wide exclusive scan
-// (u32, and two packed counts) and a stable LSD radix sort of (u64 key, u32 value) pairs.
+// (u32, two counts packed in a u64, or four of them) and a stable LSD radix sort of
+// (u64 key, u32 value) pairs.
 //
 // Radix sort: digits of up to 8 bits, as even as the passes allow (19 target
 // bits as 7 + 7 + 5), tiles of 2048 elements per 256-thread block (4 waves x

@@ -74,7 +74,10 @@ typedef struct fmmh_params {
   int center_mode;  /* FMMH_CENTER_* */
   int precision;    /* FMMH_PREC_* */
   unsigned flags;   /* FMMH_FLAG_* */
-  double hbm_budget_bytes; /* device-memory budget of this context; 0 = no limit */
+  double hbm_budget_bytes; /* device-memory budget of this context; 0 = no limit. A
+                       call that cannot be done within it returns FMMH_E_OVER_BUDGET;
+                       scratch that only saves time (the M2L's partial sums at p > 10,
+                       the FP64 form's shorter P2P items) shrinks to it first. */
   double soft_mac;  /* softening guard of the MAC (extension, softening > 0 only): a pair
                        is rejected for M2L when softening^2 (rhoA + rhoB)^3 > soft_mac r^5,
                        the softened far field's leading residual relative to the pair's
