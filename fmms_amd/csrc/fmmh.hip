@@ -444,14 +444,15 @@ struct fmmh_ctx {
     launch_fmin((uint32_t)n, nc, c, (const double*)fvals.p, (double*)cstart.p, (double*)fmin.p, s);
   }
 
-  // Room for the M2L source rows: the locals, which the reduction writes after
-  // the last row has been read (every order from 2 up fits), or the buffer that
-  // the directed sort did not end in, which nothing reads until the next lists.
-  // A buffer of their own was 8 - 11 % of a context with short lists.
+  // Room for the M2L source rows: the buffer that the directed sort did not end
+  // in, which nothing reads until the next lists, or, with short lists, the
+  // locals, which the reduction writes after the last row has been read (every
+  // order from 2 up fits; 2 - 3 % slower to read: 250k bodies, p = 6, M2L 352 and
+  // 365 us). A buffer of their own was 8 - 11 % of a context with short lists.
   double* source_rows(size_t bytes) {
-    if (locals.cap >= bytes) return (double*)locals.p;
     const Buf& idle = idle_keys(msorted, mkeys, mkeys_alt);
-    return idle.cap >= bytes ? (double*)idle.p : ensure<double>(m2l_rows, bytes);
+    if (idle.cap >= bytes) return (double*)idle.p;
+    return locals.cap >= bytes ? (double*)locals.p : ensure<double>(m2l_rows, bytes);
   }
 
   // The key buffer that a directed sort did not end in: idle until the next lists.
