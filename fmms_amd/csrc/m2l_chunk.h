@@ -17,7 +17,7 @@ struct M2lChunk {
 // FP64 rows, orders up to 10: the first m2l_row_direct(p) doubles of the real
 // layout and the centre are read by each lane, the rest goes through LDS in
 // m2l_row_segs(p) segments of 64 bytes (m2l_kernel.h: why the line lies there).
-constexpr int m2l_row_direct(int p) { return p <= 7 ? 1 : p == 8 ? 9 : hdim(p); }
+constexpr int m2l_row_direct(int p) { return p == 8 ? 9 : 1; }
 constexpr int m2l_row_segs(int p) { return (hdim(p) - m2l_row_direct(p) + 7) / 8; }
 constexpr int m2l_row_tail(int p) { return (3 + m2l_row_direct(p) + 7) / 8 * 8; }
 constexpr int m2l_row_words(int p) { return 8 * m2l_row_segs(p) + m2l_row_tail(p); }

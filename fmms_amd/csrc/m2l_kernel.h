@@ -151,14 +151,15 @@ __host__ __device__ constexpr int rim(int n, int m) { return n * n + 2 * m; }
 // parts exchanged. F_n^0 is real: 2 Re(conj(M_k^l) Theta^l), accumulated
 // halved (the caller doubles it). At P = 7: 876 multiply-adds and 112 adds
 // for the sums, against 2100 term by term.
-// H = 2: every degree n of F; H = 0 / 1: only even / odd n (the two halves
-// of a chunk, run by two waves: about equal work, half the accumulators).
+// H, NC: only the degrees n of F with n % NC == H (one of the NC waves that share
+// a chunk's pairs; NC = 1: all).
 // on: whether the lane has a pair (else Theta is 0 and nothing is added).
-// mid() runs between the degrees s = 0..2 and the others.
-template <int P, int H, class Mid>
+// load(s) runs before the products of degree s, which read the degrees s - n of
+// M; mid() between the degrees s = 0..2 and the others.
+template <int P, int H, int NC, class Load, class Mid>
 __device__ __forceinline__ void m2l_accumulate64(bool on, double x, double y, double z,
                                                  double soft2, const double* M, double* F,
-                                                 Mid mid) {
+                                                 Load load, Mid mid) {
   // Softening: the harmonic derivatives of the Plummer kernel are those of
   // 1/r times (r/s)^{2n+1}, s^2 = r^2 + eps^2; in the recursion that is
   // 1/r^2 -> 1/s^2 and the (n-2) term scaled by r^2/s^2 (soft2 = 0: 1).
@@ -194,12 +195,13 @@ __device__ __forceinline__ void m2l_accumulate64(bool on, double x, double y, do
         }
       }
     }
+    load(s);
     // all terms with n + k == s: l = 0, and m = 0
     const double t0 = 0.5 * Tr[0];
 #pragma unroll
     for (int n = 0; n <= P; n++) {
       if (n > s) continue;
-      if (H != 2 && (n & 1) != H) continue;
+      if (n % NC != H) continue;
       const int k = s - n;
       F[rre(n, 0)] = fma(M[rre(k, 0)], t0, F[rre(n, 0)]);
 #pragma unroll
@@ -236,7 +238,7 @@ __device__ __forceinline__ void m2l_accumulate64(bool on, double x, double y, do
           for (int n = 0; n <= P; n++) {
             const int k = s - n;
             if (n < m || k < l) continue;
-            if (H != 2 && (n & 1) != H) continue;
+            if (n % NC != H) continue;
             const double a = M[rre(k, l)], b = M[rim(k, l)];
             F[rre(n, m)] = fma(a, sr, F[rre(n, m)]);
             F[rim(n, m)] = fma(a, ssi, F[rim(n, m)]);
@@ -271,16 +273,14 @@ __device__ __forceinline__ void m2l_accumulate64(bool on, double x, double y, do
 // P = 6, 250k bodies 0.66 -> 0.35 ms. The rows' traffic (88 GB at P = 7, 8.4
 // TB/s, mostly from the memory-side cache) and FP64 issue now bound it
 // together. P = 8 keeps its first degrees out of LDS so that
-// four waves fit a CU; from P = 9 on the rows are read directly.
+// four waves fit a CU; from P = 9 on four waves share the staged rows.
 template <int P>
 struct M2lRow {
   static constexpr int NM = (P + 1) * (P + 1);
-  static constexpr bool STAGED = P <= 8;
   static constexpr int NDIR = m2l_row_direct(P);
   static constexpr int SEG = m2l_row_segs(P);
   static constexpr int DIR = m2l_row_tail(P);      // centre + direct part
   static constexpr int WORDS = m2l_row_words(P);  // staged part first, 64-byte rows
-  static_assert(STAGED == (SEG > 0), "the direct part is the whole multipole or is followed by segments");
 };
 
 // Blocks of the row kernels for `words` words in all, one a thread up to 2^30:
@@ -327,14 +327,6 @@ __global__ void __launch_bounds__(256) k_m2l_rows(uint32_t nc, const cplx* __res
     m2l_row_word<P>(g, moments, ccx, ccy, ccz, rows);
 }
 
-// SPLIT: two blocks per 64 chunks, the even-n and the odd-n half of F (the
-// pair of blocks is adjacent after the XCD remap, so on one XCD's L2).
-// Orders whose accumulators are split over two waves (register pressure).
-// From 9: at P = 8 one wave measured 5.3 ms and two 5.6 (1M bodies).
-#ifndef FMMH_M2L_SPLIT_FROM
-#define FMMH_M2L_SPLIT_FROM 9
-#endif
-
 typedef __attribute__((address_space(3))) char lds_char;
 typedef __attribute__((address_space(1))) const char gbl_char;
 
@@ -348,47 +340,47 @@ __device__ __forceinline__ void m2l_copy_segments(gbl_char* from, lds_char* to) 
   }
 }
 
-template <int P, int H>
-__device__ __forceinline__ void m2l_chunks64(uint32_t ci, bool live, const M2lChunk ck,
-                                             const uint64_t* __restrict__ skeys, uint64_t smask,
-                                             const double* __restrict__ rows, double soft2,
-                                             double2* stage, double* __restrict__ part) {
+// What the kernels of 64 lanes, one chunk each, share: trips, sources, rows.
+template <int P>
+struct M2lLane {
   using R = M2lRow<P>;
-  const int lane = threadIdx.x;
-  lds_char* stage3 = (lds_char*)stage;
-  const uint32_t cnt = live ? ck.end - ck.begin : 0u;
-  uint32_t trips = cnt;  // the wave runs its longest chunk's trip count
+  const M2lChunk ck;
+  const uint64_t* skeys;
+  const uint64_t smask;
+  const double* rows;
+  const int lane;
+  uint32_t cnt, trips;
+  double dir[R::DIR];  // the source's centre and direct part
+
+  __device__ __forceinline__ M2lLane(bool live, const M2lChunk c, const uint64_t* k, uint64_t sm,
+                                     const double* r)
+      : ck(c), skeys(k), smask(sm), rows(r), lane((int)(threadIdx.x & 63)) {
+    cnt = live ? ck.end - ck.begin : 0u;
+    trips = cnt;  // the wave runs its longest chunk's trip count
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) trips = max(trips, (uint32_t)__shfl_xor((int)trips, o, 64));
-  trips = (uint32_t)wave_uniform((int)trips);
-  if (trips == 0) return;
-  double F[R::NM];
-#pragma unroll
-  for (int i = 0; i < R::NM; i++) F[i] = 0.0;
+    for (int o = 32; o > 0; o >>= 1) trips = max(trips, (uint32_t)__shfl_xor((int)trips, o, 64));
+    trips = (uint32_t)wave_uniform((int)trips);
+  }
   // a lane past its chunk's end goes on reading the chunk's last source (a
   // dead lane cell 0), so every row address stays valid
-  auto source = [&](uint32_t j) -> uint32_t {
+  __device__ __forceinline__ uint32_t source(uint32_t j) const {
     return cnt ? (uint32_t)(skeys[ck.begin + min(j, cnt - 1)] & smask) : 0u;
-  };
-  // copy of the rows' staged part into LDS, [16-row group][segment][row][4]
-  // of 16 bytes, the four pieces of a row rotated by its number so that 16
-  // lanes reading one piece of 16 rows hit all banks
-  auto copy = [&](uint32_t src) {
-    if constexpr (R::STAGED) {
-#pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const uint32_t rs = (uint32_t)__shfl((int)src, g * 16 + (lane >> 2), 64);
-        m2l_copy_segments<R::SEG>(
-            (gbl_char*)(rows + (size_t)rs * R::WORDS) + ((lane & 3) ^ ((lane >> 4) & 3)) * 16,
-            stage3 + g * R::SEG * 1024);
-      }
-    }
-  };
-  const int swz = (lane >> 2) & 3;
-  const double2* mine = stage + (lane >> 4) * R::SEG * 64 + (lane & 15) * 4;
-  uint32_t src = source(0);
-  double dir[R::DIR];
-  auto direct = [&](uint32_t sc) {
+  }
+  // copy of the staged part of the rows of 16 lanes' sources (16 g ..) into LDS,
+  // [16-row group][segment][row][4] of 16 bytes, the four pieces of a row rotated
+  // by its number so that 16 lanes reading one piece of 16 rows hit all banks
+  __device__ __forceinline__ void copy(uint32_t src, int g, lds_char* stage) const {
+    const uint32_t rs = (uint32_t)__shfl((int)src, g * 16 + (lane >> 2), 64);
+    m2l_copy_segments<R::SEG>(
+        (gbl_char*)(rows + (size_t)rs * R::WORDS) + ((lane & 3) ^ ((lane >> 4) & 3)) * 16,
+        stage + g * R::SEG * 1024);
+  }
+  // piece e (two doubles) of the lane's own row
+  __device__ __forceinline__ double2 piece(const double2* stage, int e) const {
+    const double2* mine = stage + (lane >> 4) * R::SEG * 64 + (lane & 15) * 4;
+    return mine[(e >> 2) * 64 + ((e & 3) ^ ((lane >> 2) & 3))];
+  }
+  __device__ __forceinline__ void direct(uint32_t sc) {
     const double2* d2 = (const double2*)(rows + (size_t)sc * R::WORDS + R::SEG * 8);
 #pragma unroll
     for (int i = 0; i < (3 + R::NDIR + 1) / 2; i++) {
@@ -396,52 +388,15 @@ __device__ __forceinline__ void m2l_chunks64(uint32_t ci, bool live, const M2lCh
       dir[2 * i] = v.x;
       dir[2 * i + 1] = v.y;
     }
-  };
-  direct(src);
-  copy(src);
-  double tx = 0.0, ty = 0.0, tz = 0.0;
-  {
-    const double* t = rows + (size_t)ck.target * R::WORDS + R::SEG * 8;
-    tx = t[0];
-    ty = t[1];
-    tz = t[2];
   }
-  uint32_t src_n = source(1);
-  for (uint32_t j = 0; j < trips; j++) {
-    double M[R::NM];
-    const double x = tx - dir[0], y = ty - dir[1], z = tz - dir[2];
-#pragma unroll
-    for (int i = 0; i < R::NDIR; i++) M[i] = dir[3 + i];
-    if constexpr (R::STAGED) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copy has landed
-#pragma unroll
-      for (int e = 0; e < R::SEG * 4; e++) {
-        const double2 v = mine[(e >> 2) * 64 + ((e & 3) ^ swz)];
-        if (R::NDIR + 2 * e < R::NM) M[R::NDIR + 2 * e] = v.x;
-        if (R::NDIR + 2 * e + 1 < R::NM) M[R::NDIR + 2 * e + 1] = v.y;
-      }
-    }
-    // the next source's copy starts once this one's row has been read (while
-    // the first degrees are computed) and runs under the rest
-    m2l_accumulate64<P, H>(j < cnt, x, y, z, soft2, M, F, [&] {
-      if (j + 1 < trips) {
-        if constexpr (R::STAGED) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        const uint32_t cur = src_n;
-        src_n = source(j + 2);
-        if constexpr (R::STAGED) direct(cur);
-        copy(cur);
-        src = cur;
-      }
-    });
-    if constexpr (!R::STAGED) {
-      if (j + 1 < trips) direct(src);
-    }
-  }
-  if (!live) return;
-  double* out = part + (size_t)ci * R::NM;
+};
+
+// The degrees n % NC == H of a chunk's partial.
+template <int P, int H, int NC>
+__device__ __forceinline__ void m2l_store64(const double* F, double* __restrict__ out) {
 #pragma unroll
   for (int n = 0; n <= P; n++) {
-    if (H != 2 && (n & 1) != H) continue;
+    if (n % NC != H) continue;
     out[rre(n, 0)] = 2.0 * F[rre(n, 0)];
 #pragma unroll
     for (int m = 1; m <= P; m++) {
@@ -452,26 +407,154 @@ __device__ __forceinline__ void m2l_chunks64(uint32_t ci, bool live, const M2lCh
   }
 }
 
-template <int P, bool SPLIT>
+template <int P>
 __global__ void __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(1))) k_m2l(const M2lChunk* __restrict__ chunks,
                                               uint32_t nchunks, const uint64_t* __restrict__ skeys,
                                               uint64_t smask, const double* __restrict__ rows,
                                               double soft2, double* __restrict__ part) {
-  __shared__ double2 stage[M2lRow<P>::STAGED ? M2lRow<P>::SEG * 256 : 1];
-  const uint32_t lb = xcd_block(blockIdx.x, gridDim.x);
-  const uint32_t ci = (SPLIT ? lb >> 1 : lb) * 64 + threadIdx.x;
+  using R = M2lRow<P>;
+  __shared__ double2 stage[R::SEG * 256];
+  const uint32_t ci = xcd_block(blockIdx.x, gridDim.x) * 64 + threadIdx.x;
   const bool live = ci < nchunks;
   M2lChunk ck{0, 0, 0};
   if (live) ck = chunks[ci];
-  if constexpr (SPLIT) {
-    if (lb & 1)
-      m2l_chunks64<P, 1>(ci, live, ck, skeys, smask, rows, soft2, stage, part);
-    else
-      m2l_chunks64<P, 0>(ci, live, ck, skeys, smask, rows, soft2, stage, part);
-  } else {
-    m2l_chunks64<P, 2>(ci, live, ck, skeys, smask, rows, soft2, stage, part);
+  M2lLane<P> ln(live, ck, skeys, smask, rows);
+  if (ln.trips == 0) return;
+  lds_char* stage3 = (lds_char*)stage;
+  double F[R::NM];
+#pragma unroll
+  for (int i = 0; i < R::NM; i++) F[i] = 0.0;
+  auto fetch = [&](uint32_t src) {
+    ln.direct(src);
+#pragma unroll
+    for (int g = 0; g < 4; g++) ln.copy(src, g, stage3);
+  };
+  fetch(ln.source(0));
+  const double* t = rows + (size_t)ck.target * R::WORDS + R::SEG * 8;
+  const double tx = t[0], ty = t[1], tz = t[2];
+  uint32_t src_n = ln.source(1);
+  for (uint32_t j = 0; j < ln.trips; j++) {
+    double M[R::NM];
+    const double x = tx - ln.dir[0], y = ty - ln.dir[1], z = tz - ln.dir[2];
+#pragma unroll
+    for (int i = 0; i < R::NDIR; i++) M[i] = ln.dir[3 + i];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copy has landed
+#pragma unroll
+    for (int e = 0; e < R::SEG * 4; e++) {
+      const double2 v = ln.piece(stage, e);
+      if (R::NDIR + 2 * e < R::NM) M[R::NDIR + 2 * e] = v.x;
+      if (R::NDIR + 2 * e + 1 < R::NM) M[R::NDIR + 2 * e + 1] = v.y;
+    }
+    // the next source's copy starts once this one's row has been read (while
+    // the first degrees are computed) and runs under the rest
+    m2l_accumulate64<P, 0, 1>(j < ln.cnt, x, y, z, soft2, M, F, [](int) {}, [&] {
+      if (j + 1 < ln.trips) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const uint32_t cur = src_n;
+        src_n = ln.source(j + 2);
+        fetch(cur);
+      }
+    });
   }
+  if (live) m2l_store64<P, 0, 1>(F, part + (size_t)ci * R::NM);
+}
+
+// P = 9 and 10: the accumulators and the row need more registers than a wave has
+// (a wave for each half of the degrees, rows read into registers: 227 and 617 of
+// them spilled). Four waves share the pairs of 64 chunks and one staged copy of
+// their rows; wave H takes the degrees n % 4 == H (of about equal work, 22 to 39
+// accumulators) and reads, for the products of degree s, the degrees s - n of the
+// row from LDS, a quarter of it on average, so that 256 registers do and two blocks
+// fit a CU. Each wave runs the recursion and makes the sums S and D for itself, on
+// top of its quarter of the products. M2L of 1M bodies at eps 1e-5, theta
+// 0.5 and leaf 96: P = 9, 34.0M directed pairs 18.0 -> 7.0 ms, 18.4M 9.3 -> 3.5;
+// P = 10, 29.8M 31.6 -> 8.0, 18.4M 18.2 -> 4.5 (term by term on two waves before
+// that: 13.5, 7.3, 14.7 and 9.1).
+constexpr int M2L_SHARED_FROM = 9, M2L_NC = 4;
+
+template <int P, int H>
+__device__ __forceinline__ void m2l_shared(uint32_t ci, bool live, const M2lChunk ck,
+                                           const uint64_t* __restrict__ skeys, uint64_t smask,
+                                           const double* __restrict__ rows, double soft2,
+                                           const double2* stage, double* __restrict__ part) {
+  using R = M2lRow<P>;
+  static_assert(R::NDIR == 1, "entry 2 e + 1 starts piece e");
+  M2lLane<P> ln(live, ck, skeys, smask, rows);
+  if (ln.trips == 0) return;  // of the block: its waves have the same chunks
+  lds_char* stage3 = (lds_char*)stage;
+  double F[R::NM];
+#pragma unroll
+  for (int i = 0; i < R::NM; i++) F[i] = 0.0;
+  uint32_t src = ln.source(0);
+  ln.direct(src);
+  ln.copy(src, H, stage3);
+  const double* t = rows + (size_t)ck.target * R::WORDS + R::SEG * 8;
+  const double tx = t[0], ty = t[1], tz = t[2];
+  src = ln.source(1);
+  for (uint32_t j = 0; j < ln.trips; j++) {
+    double M[R::NM];
+    const double x = tx - ln.dir[0], y = ty - ln.dir[1], z = tz - ln.dir[2];
+    M[0] = ln.dir[3];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's copy has landed ...
+    __syncthreads();                                  // ... and the block's
+    m2l_accumulate64<P, H, M2L_NC>(
+        j < ln.cnt, x, y, z, soft2, M, F,
+        [&](int s) {
+          // the products of the degrees before come first (nothing else keeps the
+          // compiler from reading all of the row here and multiplying later)
+#pragma unroll
+          for (int n = 0; n < P; n++) {
+            if (n >= s || n % M2L_NC != H) continue;
+#pragma unroll
+            for (int i = n * n; i <= n * n + 2 * n; i++) asm volatile("" : "+v"(F[i]));
+          }
+          asm volatile("" ::: "memory");
+#pragma unroll
+          for (int k = 1; k <= P; k++) {
+            if (k > s || (s - k) % M2L_NC != H) continue;
+#pragma unroll
+            for (int e = (k * k - 1) / 2; e <= (k * k + 2 * k - 1) / 2; e++) {
+              const double2 v = ln.piece(stage, e);
+              if (2 * e + 1 >= k * k) M[2 * e + 1] = v.x;
+              if (2 * e + 2 <= k * k + 2 * k) M[2 * e + 2] = v.y;
+            }
+          }
+          if (s != P) return;
+          // the last of the rows has been read by every wave: the next ones' copy
+          // runs under the products of degree P
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          __syncthreads();
+          if (j + 1 < ln.trips) {
+            ln.direct(src);
+            ln.copy(src, H, stage3);
+            src = ln.source(j + 2);
+          }
+        },
+        [] {});
+  }
+  if (live) m2l_store64<P, H, M2L_NC>(F, part + (size_t)ci * R::NM);
+}
+
+template <int P>
+__global__ void __launch_bounds__(64 * M2L_NC) __attribute__((amdgpu_waves_per_eu(2)))
+k_m2l_shared(const M2lChunk* __restrict__ chunks, uint32_t nchunks,
+             const uint64_t* __restrict__ skeys, uint64_t smask, const double* __restrict__ rows,
+             double soft2, double* __restrict__ part) {
+  __shared__ double2 stage[M2lRow<P>::SEG * 256];
+  const uint32_t ci = xcd_block(blockIdx.x, gridDim.x) * 64 + (threadIdx.x & 63);
+  const bool live = ci < nchunks;
+  M2lChunk ck{0, 0, 0};
+  if (live) ck = chunks[ci];
+  const int h = wave_uniform((int)(threadIdx.x >> 6));
+  if (h == 0)
+    m2l_shared<P, 0>(ci, live, ck, skeys, smask, rows, soft2, stage, part);
+  else if (h == 1)
+    m2l_shared<P, 1>(ci, live, ck, skeys, smask, rows, soft2, stage, part);
+  else if (h == 2)
+    m2l_shared<P, 2>(ci, live, ck, skeys, smask, rows, soft2, stage, part);
+  else
+    m2l_shared<P, 3>(ci, live, ck, skeys, smask, rows, soft2, stage, part);
 }
 
 template <int P>
@@ -479,12 +562,15 @@ void m2l_t(const M2lChunk* chunks, uint32_t nchunks, const uint64_t* skeys, uint
            uint32_t nc, DevCells c, const cplx* moments, double soft2, double* rows, double* part,
            hipStream_t s) {
   if (!nchunks) return;
-  constexpr bool split = P >= FMMH_M2L_SPLIT_FROM;
   hipLaunchKernelGGL(k_m2l_rows<P>, m2l_row_blocks((size_t)nc * M2lRow<P>::WORDS), dim3(256), 0, s,
                      nc, moments, c.cx, c.cy, c.cz, rows);
-  const uint32_t nb = (nchunks + 63) / 64 * (split ? 2 : 1);
-  hipLaunchKernelGGL((k_m2l<P, split>), dim3(nb), dim3(64), 0, s, chunks, nchunks, skeys, smask,
-                     (const double*)rows, soft2, part);
+  const dim3 nb((nchunks + 63) / 64);
+  if constexpr (P < M2L_SHARED_FROM)
+    hipLaunchKernelGGL(k_m2l<P>, nb, dim3(64), 0, s, chunks, nchunks, skeys, smask,
+                       (const double*)rows, soft2, part);
+  else
+    hipLaunchKernelGGL(k_m2l_shared<P>, nb, dim3(64 * M2L_NC), 0, s, chunks, nchunks, skeys, smask,
+                       (const double*)rows, soft2, part);
 }
 
 // ------------------------------------------------------- FP32 (mixed form)
