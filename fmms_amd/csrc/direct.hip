@@ -6,7 +6,8 @@
 // Each target's sources are cut into nsplit contiguous ranges, one 256-thread
 // block per (group of targets, range): a few sampled targets still fill the device.
 // Every block writes its five partial sums (ax, ay, az, pot, f) and a second
-// kernel adds them in range order, so the result does not depend on timing.
+// kernel adds them in range order, so the result does not depend on timing; the
+// only range of a small system is the result, in one launch.
 #include <cmath>
 #include <mutex>
 
@@ -22,6 +23,30 @@ constexpr size_t DIRECT_SCRATCH_WORDS = (size_t)1 << 20;
 static_assert(5 * (size_t)FMMH_DIRECT_NOALLOC_MAX_TARGETS <= DIRECT_SCRATCH_WORDS,
               "one range per target must fit the scratch");
 
+// Sums of 2 H values (a power of two) over the wave, by halving: as long as a lane
+// holds more than one of them, it hands half to the lane opposite and keeps the
+// other, so a block of four targets makes 32 exchanges instead of 120 (most of the
+// time of a small system's sums: 12 sources and 4414 targets 16.9 -> 7.5 us, 712 and
+// 17961 52.9 -> 27.4; with one target a block 10.6 and 37.7). v[0] of a lane is the sum of the value whose number is
+// returned, -1 in the lanes that hold a copy.
+template <int H, int O = 32>
+__device__ __forceinline__ int scatter_sums(double* v, int lane) {
+  if constexpr (H > 0) {
+    const bool up = (lane & O) != 0;
+#pragma unroll
+    for (int i = 0; i < H; i++) {
+      const double keep = up ? v[i + H] : v[i], send = up ? v[i] : v[i + H];
+      v[i] = keep + __shfl_xor(send, O, 64);
+    }
+    const int slot = scatter_sums<H / 2, O / 2>(v, lane);
+    return slot < 0 ? slot : slot + (up ? H : 0);
+  } else {  // lanes that differ in the bits left hold parts of one sum
+#pragma unroll
+    for (int o = O; o > 0; o >>= 1) v[0] += __shfl_xor(v[0], o, 64);
+    return (lane & (2 * O - 1)) == 0 ? 0 : -1;
+  }
+}
+
 // NT targets per block, in scalar registers: a thread reads a source once and
 // evaluates it against all of them. One target per block read 32 bytes from
 // the cache for every pair and divided by a square root: 4096 targets x 1M
@@ -33,7 +58,10 @@ __global__ void __launch_bounds__(DT) k_direct_part(const double* __restrict__ p
                                                    const double* __restrict__ mass, size_t n,
                                                    double soft2, const uint32_t* __restrict__ ids,
                                                    uint32_t nt, uint32_t nsplit, size_t chunk,
-                                                   double* __restrict__ part) {
+                                                   double* __restrict__ part,
+                                                   double* __restrict__ acc_out,
+                                                   double* __restrict__ pot_out,
+                                                   double* __restrict__ f_out) {
   __shared__ double sh[DT / 64][5 * NT];
   const uint32_t t0 = blockIdx.y * NT, k = blockIdx.x;
   uint32_t id[NT];
@@ -91,23 +119,27 @@ __global__ void __launch_bounds__(DT) k_direct_part(const double* __restrict__ p
   }
   // fixed-order reduction: lanes by halving, then the waves in order
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  constexpr int NV = NT == 1 ? 8 : 32;  // the sums, to a power of two
+  static_assert(5 * NT <= NV, "as many sums as are scattered");
+  double v[NV];
 #pragma unroll
-  for (int q = 0; q < NT; q++)
-#pragma unroll
-    for (int e = 0; e < 5; e++) {
-      double v = acc[q][e];
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-      if (lane == 0) sh[w][5 * q + e] = v;
-    }
+  for (int i = 0; i < NV; i++) v[i] = i < 5 * NT ? acc[i / 5][i % 5] : 0.0;
+  const int slot = scatter_sums<NV / 2>(v, lane);
+  if (slot >= 0 && slot < 5 * NT) sh[w][slot] = v[0];
   __syncthreads();
   for (int i = threadIdx.x; i < 5 * NT; i += DT) {
     const int q = i / 5;
     if (t0 + q >= nt) continue;
-    double v = 0.0;
-    for (int ww = 0; ww < DT / 64; ww++) v += sh[ww][i];
-    if (ids[t0 + q] >= n) v = __builtin_nan("");  // ids are device data
-    part[((size_t)(t0 + q) * nsplit + k) * 5 + (i - 5 * q)] = v;
+    double sum = 0.0;
+    for (int ww = 0; ww < DT / 64; ww++) sum += sh[ww][i];
+    if (ids[t0 + q] >= n) sum = __builtin_nan("");  // ids are device data
+    const int e = i - 5 * q;
+    if (nsplit > 1)
+      part[((size_t)(t0 + q) * nsplit + k) * 5 + e] = sum;
+    else if (e < 3)  // one range: its sums are the result
+      acc_out[3 * (size_t)(t0 + q) + e] = sum;
+    else if (e == 3 ? pot_out : f_out)
+      (e == 3 ? pot_out : f_out)[t0 + q] = sum;
   }
 }
 
@@ -170,10 +202,11 @@ void launch_direct(const double* pos, const double* mass, size_t n, double soft2
   const size_t chunk = (n + nsplit - 1) / nsplit;
   if (direct_groups(n, nt))
     hipLaunchKernelGGL(k_direct_part<DN>, dim3(nsplit, (nt + DN - 1) / DN), dim3(DT), 0, s, pos, mass,
-                       n, soft2, ids, nt, nsplit, chunk, part);
+                       n, soft2, ids, nt, nsplit, chunk, part, acc, pot, f);
   else
     hipLaunchKernelGGL(k_direct_part<1>, dim3(nsplit, nt), dim3(DT), 0, s, pos, mass, n, soft2, ids,
-                       nt, nsplit, chunk, part);
+                       nt, nsplit, chunk, part, acc, pot, f);
+  if (nsplit == 1) return;
   const size_t rb = ((size_t)nt * RL + DT - 1) / DT;
   hipLaunchKernelGGL(k_direct_reduce, dim3((unsigned)std::min<size_t>(rb, 1 << 16)), dim3(DT), 0, s,
                      part, nt, nsplit, acc, pot, f);
