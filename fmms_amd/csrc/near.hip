@@ -450,7 +450,7 @@ __global__ void __launch_bounds__(64) k_p2p_fp64(FMMH_P2P_PARAMS) {
 // min(m - 1, P_u / ceil(S / m)) (items may come out empty). Split items write
 // partial sums that k_p2p_reduce adds in item order. The cut depends on the
 // leaf's own counts only, so a system evaluates the same alone and in an
-// ensemble.
+// ensemble (unless a memory budget has left the cap out for one of the two).
 //
 // P2P_CAP: an item is one wave streaming its sources tile by tile, about 1.4
 // us per 64 sources however few the targets are, so a leaf of 10 bodies with
